@@ -226,8 +226,8 @@ def work(case):
 
 # largest (rel, max) of any output: four times what the path differs by from itself run in float32 on the same values
 # (float32: from the same rule in float64), capped where a sum over all tokens (the gradients of A_log and dt_bias) or an
-# output that is small beside a sum it passed through (a gated row, a decay's gradient) would go beyond 0.03 and 1
-_OFF = {"decode": (1e-2, 0.12), "prefill": (2e-2, 1.0), "rule": (2e-2, 0.25), "layer": (3e-2, 1.0), "kda": (3e-2, 1.0),
+# output that is small beside a sum it passed through (a gated row, a decay's gradient) would go beyond 0.03 and 0.9
+_OFF = {"decode": (1e-2, 0.12), "prefill": (2e-2, 0.9), "rule": (2e-2, 0.25), "layer": (3e-2, 0.9), "kda": (3e-2, 0.9),
         "kda_prefill": (2e-2, 0.25)}
 
 
