@@ -190,6 +190,10 @@ template <typename T> struct Vec16 {
 template <typename T> __device__ __forceinline__ Vec16<T> ld16(const T* p) {
   Vec16<T> v; v.raw = *reinterpret_cast<const u32x4*>(p); return v;
 }
+// data that no other workgroup reads: it passes through the caches without displacing anything
+template <typename T> __device__ __forceinline__ Vec16<T> ld16_stream(const T* p) {
+  Vec16<T> v; v.raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); return v;
+}
 template <typename T> __device__ __forceinline__ void st16(T* p, const Vec16<T>& v) {
   *reinterpret_cast<u32x4*>(p) = v.raw;
 }

@@ -13,10 +13,22 @@
 
 namespace gdn {
 
-__device__ __forceinline__ float sigmoid_(float p) { return 1.f / (1.f + __expf(-p)); }
+// 16-bit types: reciprocal instruction and one Newton step (within an ulp, a third of the instructions of the IEEE
+// division, which made these kernels bound by vector issue instead of memory); the exponent is capped where the
+// sigmoid leaves the normal range, so that the step never meets an infinity
+template <typename T> __device__ __forceinline__ float sigmoid_(float p) {
+  if constexpr (sizeof(T) == 4) {
+    return 1.f / (1.f + __expf(-p));
+  } else {
+    const float d = 1.f + __expf(fminf(-p, 88.f)), r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.f), r, r);
+  }
+}
 
-// round to T and back: the reference casts to the input dtype between the steps
-template <typename T> __device__ __forceinline__ float round_to(float x) { return Elem<T>::to_f(Elem<T>::from_f(x)); }
+// round to T and back: the reference casts to the input dtype between the steps (16-bit types: two elements at a time)
+template <typename T> __device__ __forceinline__ void round_piece(float* f) {
+  if constexpr (sizeof(T) == 2) unpack16<T>(pack16<T>(f), f);
+}
 
 template <typename T, typename TW> __device__ __forceinline__ void load_weight(float* w, const TW* p) {
   constexpr int V = Elem<T>::kVec;
@@ -32,24 +44,32 @@ template <typename T, typename TW> __device__ __forceinline__ void load_weight(f
 
 // sum of the squares of a piece's elements, added in element order
 template <typename T> __device__ __forceinline__ float piece_sumsq(const Vec16<T>& xv) {
-  float ss = 0.f;
+  float f[Elem<T>::kVec], ss = 0.f;
+  unpack16<T>(xv, f);
 #pragma unroll
-  for (int e = 0; e < Elem<T>::kVec; ++e) { const float f = xv.get(e); ss += f * f; }
+  for (int e = 0; e < Elem<T>::kVec; ++e) ss += f[e] * f[e];
   return ss;
 }
 
 // TW = T: weight in the input dtype, weight * xn is rounded to T as in the reference; TW = float: kept in fp32
 template <typename T, typename TW, int ACT = 0>
 __device__ __forceinline__ Vec16<T> rmsnorm_gated_piece(const Vec16<T>& xv, const Vec16<T>& gv, const float* w, float rstd) {
-  Vec16<T> out = zero16<T>();
+  constexpr int V = Elem<T>::kVec;
+  float t[V], gf[V], s[V];
+  unpack16<T>(xv, t);
+  unpack16<T>(gv, gf);
 #pragma unroll
-  for (int e = 0; e < Elem<T>::kVec; ++e) {
-    const float xn = round_to<T>(xv.get(e) * rstd);
-    const float t = sizeof(TW) == sizeof(T) ? round_to<T>(w[e] * xn) : w[e] * xn;
-    const float gf = gv.get(e);
-    out.set(e, ACT == 0 ? t * (gf * sigmoid_(gf)) : t * round_to<T>(sigmoid_(gf)));
-  }
-  return out;
+  for (int e = 0; e < V; ++e) t[e] *= rstd;
+  round_piece<T>(t);
+#pragma unroll
+  for (int e = 0; e < V; ++e) t[e] *= w[e];
+  if constexpr (sizeof(TW) == sizeof(T)) round_piece<T>(t);
+#pragma unroll
+  for (int e = 0; e < V; ++e) s[e] = ACT == 0 ? gf[e] * sigmoid_<T>(gf[e]) : sigmoid_<T>(gf[e]);
+  if constexpr (ACT != 0) round_piece<T>(s);
+#pragma unroll
+  for (int e = 0; e < V; ++e) t[e] *= s[e];
+  return pack16<T>(t);
 }
 
 }  // namespace gdn

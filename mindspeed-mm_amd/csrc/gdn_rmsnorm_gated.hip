@@ -4,6 +4,10 @@
 //     xn = x * rsqrt(mean(x^2) + eps)        (fp32, then cast to the input dtype)
 //     y  = (weight * xn) * silu(gate)        (gate in fp32; result cast to the input dtype)
 // Row-wise and bandwidth-bound: forward reads x, gate and writes y; backward reads x, gate, dy and writes dx, dgate.
+// The forward pass gives every workgroup 4 KB of each tensor and nothing more: handed out in order, such pieces keep what
+// is in flight close together, which the memory rewards (1M rows of 128 bf16: 164 us = 4.9 TB/s with 2048 workgroups
+// striding over the rows and element-wise conversions, 127 us = 6.3 TB/s now; the card's copy of 4 KB pieces reaches 6.2
+// to 6.5, of 32 KB pieces 5.4).  The backward pass needs few partial sums of dweight and strides (276 -> 234 us).
 // A row of N elements is held by N/VEC neighbouring lanes (16 bytes each); row sums use data-parallel-primitive moves.
 // With gate_activation = 1 the gate passes through a sigmoid instead (the KDA layer's norm, KimiK_3_MoeRMSNormGated,
 // mindspeed_mm/fsdp/models/kimi_k3/modeling_kimi_linear.py:75-96): s = cast(sigmoid(gate)).
@@ -37,18 +41,16 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_gated_fwd_kernel(const T* __
   const int c = threadIdx.x % LPR;
   float w[V];
   load_weight<T, TW>(w, weight + c * V);
-  for (int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR; row < (rows + RPB - 1) / RPB * RPB;
-       row += (int64_t)gridDim.x * RPB) {
-    const bool ok = row < rows;      // uniform trip count: every lane takes part in the row sums
-    const Vec16<T> xv = ok ? ld16(x + row * N + c * V) : zero16<T>();
-    const Vec16<T> gv = ok ? ld16(gate + row * N + c * V) : zero16<T>();
-    const float ss = row_lanes_sum<LPR>(piece_sumsq<T>(xv));
-    const float rstd = rsqrtf(ss * (1.f / N) + eps);
-    const Vec16<T> out = rmsnorm_gated_piece<T, TW, ACT>(xv, gv, w, rstd);
-    if (ok) {
-      __builtin_nontemporal_store(out.raw, reinterpret_cast<u32x4*>(y + row * N + c * V));
-      if (c == 0) rstd_out[row] = rstd;
-    }
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  const bool ok = row < rows;        // every lane takes part in the row sums: lanes past the end repeat the last row
+  const int64_t at = (ok ? row : rows - 1) * N + c * V;
+  const Vec16<T> xv = ld16_stream(x + at), gv = ld16_stream(gate + at);
+  const float ss = row_lanes_sum<LPR>(piece_sumsq<T>(xv));
+  const float rstd = rsqrtf(ss * (1.f / N) + eps);
+  const Vec16<T> out = rmsnorm_gated_piece<T, TW, ACT>(xv, gv, w, rstd);
+  if (ok) {
+    __builtin_nontemporal_store(out.raw, reinterpret_cast<u32x4*>(y + at));
+    if (c == 0) rstd_out[row] = rstd;
   }
 }
 
@@ -64,33 +66,55 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_gated_bwd_kernel(
   load_weight<T, TW>(w, weight + c * V);
 #pragma unroll
   for (int e = 0; e < V; ++e) dwa[e] = 0.f;
-  for (int64_t row = (int64_t)blockIdx.x * RPB + rg; row < (rows + RPB - 1) / RPB * RPB;
-       row += (int64_t)gridDim.x * RPB) {
+  const int64_t step = (int64_t)gridDim.x * RPB, stop = (rows + RPB - 1) / RPB * RPB;
+  int64_t row = (int64_t)blockIdx.x * RPB + rg;
+  // a trip's rows are requested one trip ahead; rows past the end repeat the last one with nothing added or stored
+  Vec16<T> xv, gv, dv;
+  float rstd;
+  auto request = [&](int64_t r) {
+    const int64_t rc = r < rows ? r : rows - 1, at = rc * N + c * V;
+    xv = ld16_stream(x + at);
+    gv = ld16_stream(gate + at);
+    dv = ld16_stream(dy + at);
+    rstd = rstd_in[rc];
+  };
+  request(row);
+  for (; row < stop; row += step) {   // uniform trip count: every lane takes part in the row sums
     const bool ok = row < rows;
-    const Vec16<T> xv = ok ? ld16(x + row * N + c * V) : zero16<T>();
-    const Vec16<T> gv = ok ? ld16(gate + row * N + c * V) : zero16<T>();
-    const Vec16<T> dv = ok ? ld16(dy + row * N + c * V) : zero16<T>();
-    const float rstd = ok ? rstd_in[row] : 0.f;
-    float dxn[V], xh[V], dot = 0.f;
-    Vec16<T> dgo = zero16<T>(), dxo = zero16<T>();
+    float xh[V], xn[V], t[V], gf[V], d[V], sg[V], dxn[V], dgo[V], dot = 0.f;
+    const float rs = ok ? rstd : 0.f;
+    unpack16<T>(xv, xh);
+    unpack16<T>(gv, gf);
+    unpack16<T>(dv, d);
+    request(row + step);
+#pragma unroll
+    for (int e = 0; e < V; ++e) { xh[e] *= rs; xn[e] = xh[e]; }
+    round_piece<T>(xn);
+#pragma unroll
+    for (int e = 0; e < V; ++e) t[e] = w[e] * xn[e];
+    if constexpr (sizeof(TW) == sizeof(T)) round_piece<T>(t);
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-      xh[e] = xv.get(e) * rstd;
-      const float xn = round_to<T>(xh[e]);
-      const float t = sizeof(TW) == sizeof(T) ? round_to<T>(w[e] * xn) : w[e] * xn;
-      const float gf = gv.get(e), sg = sigmoid_(gf), d = dv.get(e);
-      dgo.set(e, ACT == 0 ? d * t * sg * (1.f + gf * (1.f - sg)) : d * t * sg * (1.f - sg));
-      const float dt = ACT == 0 ? d * gf * sg : d * round_to<T>(sg);
-      dwa[e] += dt * xn;
+      sg[e] = sigmoid_<T>(gf[e]);
+      dgo[e] = ACT == 0 ? d[e] * t[e] * sg[e] * (1.f + gf[e] * (1.f - sg[e])) : d[e] * t[e] * sg[e] * (1.f - sg[e]);
+    }
+    if constexpr (ACT != 0) round_piece<T>(sg);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      const float dt = ACT == 0 ? d[e] * gf[e] * sg[e] : d[e] * sg[e];
+      xn[e] *= dt;
       dxn[e] = dt * w[e];
       dot += dxn[e] * xh[e];
     }
     dot = row_lanes_sum<LPR>(dot) * (1.f / N);
 #pragma unroll
-    for (int e = 0; e < V; ++e) dxo.set(e, rstd * (dxn[e] - xh[e] * dot));
+    for (int e = 0; e < V; ++e) dxn[e] = rs * (dxn[e] - xh[e] * dot);
     if (ok) {
-      __builtin_nontemporal_store(dxo.raw, reinterpret_cast<u32x4*>(dx + row * N + c * V));
-      __builtin_nontemporal_store(dgo.raw, reinterpret_cast<u32x4*>(dgate + row * N + c * V));
+      const int64_t at = row * N + c * V;
+#pragma unroll
+      for (int e = 0; e < V; ++e) dwa[e] += xn[e];
+      __builtin_nontemporal_store(pack16<T>(dxn).raw, reinterpret_cast<u32x4*>(dx + at));
+      __builtin_nontemporal_store(pack16<T>(dgo).raw, reinterpret_cast<u32x4*>(dgate + at));
     }
   }
   // workgroup partial of dweight: add the RPB row groups in a fixed order
@@ -121,15 +145,20 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_gated_dw_reduce_kernel(const
   if (threadIdx.x == 0) dw[i] = red[0];
 }
 
-static int rmsnorm_blocks(int64_t rows, int rpb) {
+// Two workgroups per CU, each a trip ahead with its requests.  Five streams share the memory: what counts is that the
+// rows in flight stay close together (2048 workgroups: 5.3 TB/s, 1024: 5.2, 768: 5.5, 512: 5.75, 384: 5.25, 256: 5.0 at
+// 1M rows of 128 bf16).
+static int rmsnorm_bwd_blocks(int64_t rows, int rpb) {
   const int64_t need = (rows + rpb - 1) / rpb;
-  return (int)(need < 2048 ? (need > 0 ? need : 1) : 2048);   // a few workgroups per CU, grid-stride over the rows
+  return (int)(need < 512 ? (need > 0 ? need : 1) : 512);
 }
 
 template <typename T, typename TW, int LPR>
 static int rmsnorm_fwd_launch(const void* x, const void* gate, const void* weight, void* y, float* rstd, int64_t rows,
                               float eps, int act, hipStream_t st) {
-  const dim3 grid(rmsnorm_blocks(rows, kThreads / LPR));
+  const int64_t nb = (rows + kThreads / LPR - 1) / (kThreads / LPR);
+  if (nb > 0x7fffffffLL) return -3;
+  const dim3 grid((unsigned)nb);
   if (act == 0)
     GDN_LAUNCH(kKernRmsNormFwd, st, (rmsnorm_gated_fwd_kernel<T, TW, LPR, 0>), grid, dim3(kThreads), 0, st, (const T*)x,
                (const T*)gate, (const TW*)weight, (T*)y, rstd, rows, eps);
@@ -143,7 +172,7 @@ template <typename T, typename TW, int LPR>
 static int rmsnorm_bwd_launch(const void* x, const void* gate, const void* weight, const float* rstd, const void* dy,
                               void* dx, void* dgate, float* dw, float* part, int64_t rows, int act, hipStream_t st) {
   constexpr int N = LPR * Elem<T>::kVec;
-  const int nb = rmsnorm_blocks(rows, kThreads / LPR);
+  const int nb = rmsnorm_bwd_blocks(rows, kThreads / LPR);
   if (act == 0)
     GDN_LAUNCH(kKernRmsNormBwd, st, (rmsnorm_gated_bwd_kernel<T, TW, LPR, 0>), dim3(nb), dim3(kThreads), 0, st, (const T*)x,
                (const T*)gate, (const TW*)weight, rstd, (const T*)dy, (T*)dx, (T*)dgate, part, rows);

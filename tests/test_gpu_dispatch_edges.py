@@ -1,0 +1,48 @@
+"""Each kernel at the sizes where its tiling or its dispatch turns over: one row or token past an edge, remainders, the
+smallest and the largest of a range, against the oracle with the bounds of the other parity tests."""
+import os
+import sys
+
+import pytest
+import torch
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import parity as P  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+F32, BF = torch.float32, torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from mindspeed_mm_amd.ops import _default_ops
+    return _default_ops()
+
+
+@pytest.mark.parametrize("dtype,rows,N", [
+    (BF, 1, 128), (BF, 17, 128),                   # one row; one row past a workgroup of the forward kernel
+    (BF, 16 * 512 + 1, 128), (BF, 3 * 16 * 512, 128),   # one row past the backward grid; whole trips of it
+    (BF, 4 * 512 + 3, 512), (F32, 64 * 512 + 5, 16),    # a row on a whole wave; a row on four lanes
+])
+@pytest.mark.parametrize("activation", ["silu", "sigmoid"])
+def test_rms_norm_gated_edges(ops, dtype, rows, N, activation):
+    P.check_rms_norm_gated(ops, "cuda", (rows,), N, dtype, activation=activation)
+
+
+@pytest.mark.parametrize("activation", ["silu", "sigmoid"])
+def test_rms_norm_gated_far_gates(ops, activation):
+    """Gates beyond the range of the exponential: the sigmoid is 0 or 1 there to the last bit of bf16 (e^-88 = 6e-39 is
+    below its smallest normal number), and nothing becomes inf or NaN."""
+    gate = torch.tensor([-1e4, -200.0, -89.0, -88.0, -87.0, 0.0, 87.0, 89.0, 200.0, 1e4], device="cuda", dtype=BF)
+    g = gate.repeat(13)[:128].repeat(40, 1)
+    x = torch.randn(40, 128, device="cuda", dtype=BF)
+    w = torch.ones(128, device="cuda", dtype=BF)
+    L = [t.clone().requires_grad_(True) for t in (x, g, w)]
+    y = ops.rms_norm_gated(*L, 1e-6, activation)
+    y.backward(torch.ones_like(y))
+    xn = (x.float() * torch.rsqrt(x.float().square().mean(-1, keepdim=True) + 1e-6)).to(BF).float()
+    s = torch.sigmoid(g.double())
+    ref = xn.double() * (g.double() * s if activation == "silu" else s)
+    # three roundings to bf16 (2^-9 each, the first shared) and the clamp's e^-88 times the gate
+    assert ((y.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e4 * 6.1e-39 * xn.abs().double() + 1e-37).all()
+    assert all(torch.isfinite(t.grad.float()).all() for t in L)
