@@ -7,8 +7,10 @@
 // decode update mindspeed_mm/fsdp/models/qwen3_5/modeling_qwen3_5.py:373-389.
 //
 // All kernels are HBM bound (2*W flop per element).  A thread owns 16 bytes of channels (8 bf16 /
-// 4 fp32) and walks a tile of consecutive tokens with the last W inputs in registers, so x is read
-// once; the backward pass recomputes the pre-activation in registers instead of re-reading y.
+// 4 fp32) and walks a tile of consecutive tokens with the last W inputs in registers; the backward pass recomputes the
+// pre-activation in registers instead of re-reading y.  Tiles are short: what is in flight then stays close together in
+// memory, which is worth more than the W-1 rows two neighbours both read (they meet in the caches), and a short input
+// still fills the device.
 #include "gdn_common.h"
 #include "gdn_profile.h"
 
@@ -35,22 +37,11 @@ struct SeqCursor {  // which sequence a flattened token index belongs to
   }
 };
 
-template <typename T, int V> struct ChanVec { float x[V]; };
-
-template <typename T> __device__ __forceinline__ void unpack_chan(float* dst, const Vec16<T>& v) {
-#pragma unroll
-  for (int e = 0; e < Elem<T>::kVec; ++e) dst[e] = v.get(e);
-}
+template <typename T> __device__ __forceinline__ void unpack_chan(float* dst, const Vec16<T>& v) { unpack16<T>(v, dst); }
 template <typename T> __device__ __forceinline__ void load_chan(float* dst, const T* p) { unpack_chan(dst, ld16(p)); }
-// tokens whose rows are requested together before any of them is used: a thread walks its channels token by token,
-// and without this only one 16-byte load per thread would be in flight
-constexpr int kConvAhead = 4;
 template <typename T> __device__ __forceinline__ void store_chan(T* p, const float* src) {
-  Vec16<T> v = zero16<T>();
-#pragma unroll
-  for (int e = 0; e < Elem<T>::kVec; ++e) v.set(e, src[e]);
   // streaming store: outputs are not read again by these kernels, the L2 stays with the sliding input window
-  __builtin_nontemporal_store(v.raw, reinterpret_cast<u32x4*>(p));
+  __builtin_nontemporal_store(pack16<T>(src).raw, reinterpret_cast<u32x4*>(p));
 }
 
 // input at flattened position tau for the sequence described by cur (tau may precede the sequence)
@@ -72,67 +63,85 @@ __device__ __forceinline__ void load_hist(float* dst, const T* x, const T* init,
 // v_rcp_f32 (1 ulp) instead of an IEEE division: ten instructions fewer per element
 __device__ __forceinline__ float sigmoidf_(float p) { return __builtin_amdgcn_rcpf(1.f + __expf(-p)); }
 
-template <typename T, int W>
+// TT tokens per workgroup.  A tile that lies inside one sequence, history included, takes straight-line code: its rows
+// and the W-1 before them are requested at once.  Tiles at a sequence's ends go token by token.
+// Bound by memory.  32768 x 8192 bf16, W = 4: 64 tokens per workgroup 206 us (5.2 TB/s), 16: 244, 8: 181 (5.9), 4: 189;
+// 4096 x 8192: 46 -> 23 us (64 tokens: too few waves in flight).
+template <typename T, int W, int TT, bool SILU, bool RES>
 __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) void conv1d_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ weight, const T* __restrict__ bias, const T* __restrict__ residual,
-    const T* __restrict__ init, const int64_t* __restrict__ cu, T* __restrict__ y, int64_t total, int T_len, int N,
-    int D, int tile, int silu) {
-  constexpr int V = Elem<T>::kVec;
+    const T* __restrict__ init, const int64_t* __restrict__ cu, T* __restrict__ y, T* __restrict__ fs, int64_t total,
+    int T_len, int N, int D) {
+  constexpr int V = Elem<T>::kVec, H = W - 1;
   // one linear grid, channel blocks fastest: the number of token tiles is not bounded by the y dimension's 65535
   const int nbd = (D / V + kConvThreads - 1) / kConvThreads, bx = blockIdx.x % nbd;
-  const int64_t by = blockIdx.x / nbd;
+  const int64_t t0 = (int64_t)(blockIdx.x / nbd) * TT;
   const int d0 = (bx * kConvThreads + threadIdx.x) * V;
   if (d0 >= D) return;
-  const int64_t t0 = by * tile;
-  const int64_t t1 = t0 + tile < total ? t0 + tile : total;
   float wgt[W][V], bs[V], win[W][V];
-#pragma unroll
-  for (int w = 0; w < W; ++w) load_chan(wgt[w], weight + (int64_t)w * D + d0);
-#pragma unroll
-  for (int e = 0; e < V; ++e) bs[e] = 0.f;
-  if (bias != nullptr) load_chan(bs, bias + d0);
   SeqCursor cur;
-  cur.init(cu, N, T_len, t0);
+  auto finish = [&](int64_t t, int u) {   // token t; the window's logical row j sits in slot (u + j) % W
+    float out[V];
 #pragma unroll
-  for (int w = 0; w < W - 1; ++w) load_hist(win[w], x, init, t0 - (W - 1) + w, cur, D, W, d0);
-  for (int64_t tb = t0; tb < t1; tb += kConvAhead) {
-    Vec16<T> xr[kConvAhead];
+    for (int e = 0; e < V; ++e) {
+      float a = bs[e];
 #pragma unroll
-    for (int u = 0; u < kConvAhead; ++u)
-      if (tb + u < t1) xr[u] = ld16(x + (tb + u) * D + d0);
+      for (int w = 0; w < W; ++w) a += win[(u + w) % W][e] * wgt[w][e];
+      out[e] = SILU ? a * sigmoidf_(a) : a;
+    }
+    if constexpr (RES) {
+      float r[V];
+      load_chan(r, residual + t * D + d0);
 #pragma unroll
-    for (int u = 0; u < kConvAhead; ++u) {
-      const int64_t t = tb + u;
-      if (t >= t1) break;
-      if (cur.advance_to(t)) {
+      for (int e = 0; e < V; ++e) out[e] += r[e];
+    }
+    store_chan(y + t * D + d0, out);
+  };
+  auto weights = [&] {
 #pragma unroll
-        for (int w = 0; w < W - 1; ++w) load_hist(win[w], x, init, t - (W - 1) + w, cur, D, W, d0);
+    for (int w = 0; w < W; ++w) load_chan(wgt[w], weight + (int64_t)w * D + d0);
+#pragma unroll
+    for (int e = 0; e < V; ++e) bs[e] = 0.f;
+    if (bias != nullptr) load_chan(bs, bias + d0);
+  };
+  if (t0 >= H && t0 + TT <= total) {
+    // the rows exist whatever sequence they belong to: they are on their way while the sequence is looked up
+    Vec16<T> xr[TT + H];
+    const T* xp = x + (t0 - H) * D;
+#pragma unroll
+    for (int i = 0; i < TT + H; ++i) xr[i] = ld16(xp + i * D + d0);
+    weights();
+    cur.init(cu, N, T_len, t0);
+    if (t0 - H >= cur.bos && t0 + TT <= cur.eos - (fs != nullptr ? 1 : 0)) {
+#pragma unroll
+      for (int w = 0; w < H; ++w) unpack_chan(win[w], xr[w]);
+#pragma unroll
+      for (int u = 0; u < TT; ++u) {   // sliding the window moves no register
+        unpack_chan(win[(u + H) % W], xr[u + H]);
+        finish(t0 + u, u);
       }
-      unpack_chan(win[W - 1], xr[u]);
-      float out[V];
+      return;
+    }
+  } else {
+    weights();
+    cur.init(cu, N, T_len, t0);
+  }
+  for (int64_t t = t0; t < t0 + TT && t < total; ++t) {
+    cur.advance_to(t);
 #pragma unroll
-      for (int e = 0; e < V; ++e) {
-        float a = bs[e];
+    for (int w = 0; w < W; ++w) load_hist(win[w], x, init, t - H + w, cur, D, W, d0);
+    finish(t, 0);
+    if (fs != nullptr && t + 1 == cur.eos) {   // the window is the sequence's final state [W] of each channel
 #pragma unroll
-        for (int w = 0; w < W; ++w) a += win[w][e] * wgt[w][e];
-        out[e] = silu ? a * sigmoidf_(a) : a;
-      }
-      if (residual != nullptr) {
-        float r[V];
-        load_chan(r, residual + t * D + d0);
+      for (int e = 0; e < V; ++e)
 #pragma unroll
-        for (int e = 0; e < V; ++e) out[e] += r[e];
-      }
-      store_chan(y + t * D + d0, out);
-#pragma unroll
-      for (int w = 0; w < W - 1; ++w)
-#pragma unroll
-        for (int e = 0; e < V; ++e) win[w][e] = win[w + 1][e];
+        for (int w = 0; w < W; ++w) fs[((int64_t)cur.n * D + d0 + e) * W + w] = Elem<T>::from_f(win[w][e]);
     }
   }
 }
 
-// final_state[n,d,w] = x[T_n - W + w] (falls back to the initial state / zero for T_n < W)
+// final_state[n,d,w] = x[T_n - W + w] (falls back to the initial state / zero for T_n < W).  Packed input only, where a
+// sequence may be empty; the forward kernel writes the state of a dense batch itself.
 template <typename T>
 __global__ void conv1d_final_state_kernel(const T* __restrict__ x, const T* __restrict__ init,
                                           const int64_t* __restrict__ cu, T* __restrict__ fs, int T_len, int N, int D,
@@ -154,36 +163,33 @@ __global__ void conv1d_final_state_kernel(const T* __restrict__ x, const T* __re
 // Backward.  With p the pre-activation and dyp = dy * act'(p):
 //   dx[s]   = sum_u dyp[s+u] * weight[W-1-u]   (s+u inside the sequence of s)  (+ dht at the last W tokens)
 //   dw[w]   = sum_t dyp[t] * xpad[t-(W-1)+w],   db = sum_t dyp[t]
-// Each thread writes its tile's partial dw/db to part[tile][W+1][D]; conv1d_reduce_kernel sums them.
-template <typename T, int W>
-__global__ __launch_bounds__(kConvThreads) void conv1d_bwd_kernel(
+// A workgroup walks the tiles by, by + G, by + 2 G, ... of its channels (G = gridDim.x / channel blocks), so that the
+// workgroups move through memory together, and writes one partial dw/db to part[by][W+1][D]; conv1d_reduce_kernel sums
+// them in a fixed order.
+template <typename T, int W, int TT, bool SILU>
+__global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 2 : 1) void conv1d_bwd_kernel(
     const T* __restrict__ x, const T* __restrict__ dy, const T* __restrict__ weight, const T* __restrict__ bias,
     const T* __restrict__ init, const T* __restrict__ dht, const int64_t* __restrict__ cu, T* __restrict__ dx,
-    float* __restrict__ part, int64_t total, int T_len, int N, int D, int tile, int silu) {
+    float* __restrict__ part, int64_t total, int T_len, int N, int D) {
   constexpr int V = Elem<T>::kVec;
   // one linear grid, channel blocks fastest: the number of token tiles is not bounded by the y dimension's 65535
   const int nbd = (D / V + kConvThreads - 1) / kConvThreads, bx = blockIdx.x % nbd;
   const int64_t by = blockIdx.x / nbd;
+  const int groups = gridDim.x / nbd;
   const int d0 = (bx * kConvThreads + threadIdx.x) * V;
   if (d0 >= D) return;
-  const int64_t t0 = by * tile;
-  const int64_t t1 = t0 + tile < total ? t0 + tile : total;
-  const int64_t tend = t1 + (W - 1) < total ? t1 + (W - 1) : total;  // halo: dyp of later tokens feeds dx
   float wgt[W][V], bs[V], win[W][V], dyw[W][V], dwa[W][V], dba[V];
 #pragma unroll
   for (int w = 0; w < W; ++w) {
     load_chan(wgt[w], weight + (int64_t)w * D + d0);
 #pragma unroll
-    for (int e = 0; e < V; ++e) { dwa[w][e] = 0.f; dyw[w][e] = 0.f; }
+    for (int e = 0; e < V; ++e) dwa[w][e] = 0.f;
   }
 #pragma unroll
   for (int e = 0; e < V; ++e) { bs[e] = 0.f; dba[e] = 0.f; }
   if (bias != nullptr) load_chan(bs, bias + d0);
   SeqCursor cur, lag;   // cur follows t (leading), lag follows s = t-(W-1) (the dx being emitted)
-  cur.init(cu, N, T_len, t0);
-  lag.init(cu, N, T_len, t0);
-#pragma unroll
-  for (int w = 0; w < W - 1; ++w) load_hist(win[w], x, init, t0 - (W - 1) + w, cur, D, W, d0);
+  int64_t t0, t1, tend;
   // t runs W-1 steps past the last dyp so that the final dx of the tile are flushed.  W tokens per trip: the windows
   // win (x[t-(W-1)+j]) and dyw (dyp[s+u], s = t-(W-1)) are rings whose logical index j sits in slot (uu + j) % W at
   // the uu-th token of a trip, so sliding a window moves no register.
@@ -215,7 +221,7 @@ __global__ __launch_bounds__(kConvThreads) void conv1d_bwd_kernel(
         unpack_chan(g, gr[uu]);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
-          if (silu) {
+          if constexpr (SILU) {
             float p = bs[e];
 #pragma unroll
             for (int w = 0; w < W; ++w) p += win[(uu + w) % W][e] * wgt[w][e];
@@ -260,14 +266,97 @@ __global__ __launch_bounds__(kConvThreads) void conv1d_bwd_kernel(
       }
     }
   };
+  // a tile whose tokens, history and halo lie inside one sequence: the same steps without a check, the window slots at
+  // the i-th token being (i + j) % W; P tokens are requested while P are worked on
+  auto inner_tile = [&] {
+    constexpr int H = W - 1, NTOK = TT + H, P = 2, NTRIP = (NTOK + P - 1) / P;
+    const T* xp = x + t0 * D;
+    const T* gp = dy + t0 * D;
+    T* op = dx + (t0 - H) * D;
+    Vec16<T> xr[2][P], gr[2][P], hr[W];
+    auto ask = [&](int k) {
+#pragma unroll
+      for (int u = 0; u < P; ++u)
+        if (k * P + u < NTOK) {
+          xr[k & 1][u] = ld16(xp + (k * P + u) * D + d0);
+          gr[k & 1][u] = ld16(gp + (k * P + u) * D + d0);
+        }
+    };
+#pragma unroll
+    for (int w = 0; w < H; ++w) hr[w] = ld16(xp + (w - H) * D + d0);
+    ask(0);
+#pragma unroll
+    for (int w = 0; w < H; ++w) unpack_chan(win[w], hr[w]);
+#pragma unroll
+    for (int k = 0; k < NTRIP; ++k) {
+      if (k + 1 < NTRIP) ask(k + 1);
+      GDN_SCHED_FENCE();
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        const int i = k * P + u;
+        if (i < NTOK) {
+          float* newest_g = dyw[(i + H) % W];
+          unpack_chan(win[(i + H) % W], xr[k & 1][u]);
+          unpack_chan(newest_g, gr[k & 1][u]);
+          if constexpr (SILU) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+              float p = bs[e];
+#pragma unroll
+              for (int w = 0; w < W; ++w) p += win[(i + w) % W][e] * wgt[w][e];
+              const float sg = sigmoidf_(p);
+              newest_g[e] *= sg * (1.f + p * (1.f - sg));
+            }
+          }
+          if (i < TT) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+              dba[e] += newest_g[e];
+#pragma unroll
+              for (int w = 0; w < W; ++w) dwa[w][e] += newest_g[e] * win[(i + w) % W][e];
+            }
+          }
+          if (i >= H) {
+            float out[V];
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+              out[e] = 0.f;
+#pragma unroll
+              for (int v = 0; v < W; ++v) out[e] += dyw[(i + v) % W][e] * wgt[W - 1 - v][e];
+            }
+            store_chan(op + i * D + d0, out);
+          }
+          GDN_SCHED_FENCE();
+        }
+      }
+    }
+  };
   Vec16<T> xa[W], ga[W], xb[W], gb[W];
-  request(xa, ga, t0);
-  for (int64_t tb = t0; tb < t1 + (W - 1); tb += 2 * W) {
-    request(xb, gb, tb + W);
-    trip(tb, xa, ga);
-    if (tb + W >= t1 + (W - 1)) break;
-    request(xa, ga, tb + 2 * W);
-    trip(tb + W, xb, gb);
+  for (t0 = by * TT; t0 < total; t0 += (int64_t)groups * TT) {
+    t1 = t0 + TT < total ? t0 + TT : total;
+    tend = t1 + (W - 1) < total ? t1 + (W - 1) : total;   // halo: dyp of later tokens feeds dx
+    cur.init(cu, N, T_len, t0);
+    if constexpr (W <= 4) {
+      if (t0 - (W - 1) >= cur.bos && t0 + TT + (dht != nullptr ? W : W - 1) <= cur.eos) {
+        inner_tile();
+        continue;
+      }
+    }
+    request(xa, ga, t0);
+    lag = cur;
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+#pragma unroll
+      for (int e = 0; e < V; ++e) dyw[w][e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < W - 1; ++w) load_hist(win[w], x, init, t0 - (W - 1) + w, cur, D, W, d0);
+    for (int64_t tb = t0; tb < t1 + (W - 1); tb += 2 * W) {
+      request(xb, gb, tb + W);
+      trip(tb, xa, ga);
+      if (tb + W >= t1 + (W - 1)) break;
+      request(xa, ga, tb + 2 * W);
+      trip(tb + W, xb, gb);
+    }
   }
   float* pp = part + by * (W + 1) * D;
 #pragma unroll
@@ -278,12 +367,22 @@ __global__ __launch_bounds__(kConvThreads) void conv1d_bwd_kernel(
   for (int e = 0; e < V; ++e) pp[(int64_t)W * D + d0 + e] = dba[e];
 }
 
-__global__ void conv1d_reduce_kernel(const float* __restrict__ part, float* __restrict__ dw, float* __restrict__ db,
-                                     int ntiles, int W, int D) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)(W + 1) * D) return;
+// 64 columns per workgroup, the partial sums dealt to its 16 waves; added in a fixed order
+__global__ __launch_bounds__(1024) void conv1d_reduce_kernel(const float* __restrict__ part, float* __restrict__ dw,
+                                                             float* __restrict__ db, int nparts, int W, int D) {
+  __shared__ float red[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t cols = (int64_t)(W + 1) * D, idx = (int64_t)blockIdx.x * 64 + lane;
   float s = 0.f;
-  for (int i = 0; i < ntiles; ++i) s += part[(int64_t)i * (W + 1) * D + idx];
+  if (idx < cols) {
+#pragma unroll 8
+    for (int i = wave; i < nparts; i += 16) s += part[(int64_t)i * cols + idx];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave != 0 || idx >= cols) return;
+#pragma unroll
+  for (int w = 1; w < 16; ++w) s += red[w][lane];
   if (idx < (int64_t)W * D) dw[idx] = s;
   else if (db != nullptr) db[idx - (int64_t)W * D] = s;
 }
@@ -378,30 +477,50 @@ __global__ __launch_bounds__(256) void conv1d_update_rows_kernel(const T* __rest
   *reinterpret_cast<RowVec*>(state + idx * W) = r.v;
 }
 
+constexpr int kConvFwdTile = 8;
+// Tokens per tile of the backward pass.  Bound by vector issue (about 40 instruction slots per element, halo tokens
+// included).  W = 4, D = 8192 bf16, 360 / 4096 / 32768 tokens: tiles of 256 on one workgroup each 200 / 208 / 362 us,
+// tiles of 32 29 / 54 / 337, tiles of 16 20 / 52 / 330.
+constexpr int conv_bwd_tile(int W) { return W <= 4 ? 16 : 64; }   // wide windows: fewer halo tokens computed twice
+constexpr int kConvMaxGroups = 256;
+// workgroups (and partial sums of dw, db) per channel block of the backward pass: as many as fit the device at once, no
+// more partial sums than it takes (512 workgroups in all instead of 1024: 427 us at 32768 x 8192, 2048: 328)
+static int conv_bwd_groups(int64_t total, int nbd, int W) {
+  const int64_t ntiles = (total + conv_bwd_tile(W) - 1) / conv_bwd_tile(W);
+  int most = 1024 / nbd;
+  most = most < 64 ? 64 : most > kConvMaxGroups ? kConvMaxGroups : most;
+  return (int)(ntiles < most ? ntiles : most);
+}
+
 template <typename T> struct ConvLaunch {
   static int fwd(const void* x, const void* weight, const void* bias, const void* residual, const void* init,
                  const int64_t* cu, void* y, void* fs, int B, int T_len, int N, int D, int W, int silu,
                  hipStream_t st) {
-    constexpr int V = Elem<T>::kVec;
+    constexpr int V = Elem<T>::kVec, TT = kConvFwdTile;
     const int64_t total = (int64_t)B * T_len;
-    const int tile = 64;
-    const int64_t nblocks = (int64_t)((D / V + kConvThreads - 1) / kConvThreads) * ((total + tile - 1) / tile);
+    const int64_t nblocks = (int64_t)((D / V + kConvThreads - 1) / kConvThreads) * ((total + TT - 1) / TT);
     if (nblocks > 0x7fffffffLL) return -3;
     dim3 grid((unsigned)nblocks);
+    const bool fs_inside = cu == nullptr && total > 0;   // every sequence has a last token
     if (total > 0) {
+      auto launch = [&](auto kern) {
+        GDN_LAUNCH(kKernConvFwd, st, kern, grid, dim3(kConvThreads), 0, st, (const T*)x, (const T*)weight, (const T*)bias,
+                   (const T*)residual, (const T*)init, cu, (T*)y, fs_inside ? (T*)fs : (T*)nullptr, total, T_len, N, D);
+      };
       switch (W) {
-#define GDN_CASE(W_)                                                                                              \
-  case W_:                                                                                                        \
-    GDN_LAUNCH(kKernConvFwd, st, (conv1d_fwd_kernel<T, W_>), grid, dim3(kConvThreads), 0, st, (const T*)x,   \
-                       (const T*)weight, (const T*)bias, (const T*)residual, (const T*)init, cu, (T*)y, total,    \
-                       T_len, N, D, tile, silu);                                                                  \
+#define GDN_CASE(W_)                                                                                \
+  case W_:                                                                                          \
+    if (residual != nullptr) silu ? launch(conv1d_fwd_kernel<T, W_, TT, true, true>)                \
+                                  : launch(conv1d_fwd_kernel<T, W_, TT, false, true>);              \
+    else silu ? launch(conv1d_fwd_kernel<T, W_, TT, true, false>)                                   \
+              : launch(conv1d_fwd_kernel<T, W_, TT, false, false>);                                 \
     break;
         GDN_CASE(1) GDN_CASE(2) GDN_CASE(3) GDN_CASE(4) GDN_CASE(5) GDN_CASE(6) GDN_CASE(7) GDN_CASE(8)
 #undef GDN_CASE
         default: return -3;
       }
     }
-    if (fs != nullptr) {
+    if (fs != nullptr && !fs_inside) {
       const int64_t n = (int64_t)N * D;
       GDN_LAUNCH(kKernConvState, st, (conv1d_final_state_kernel<T>), dim3((unsigned)((n + 255) / 256)), dim3(256),
                          0, st, (const T*)x, (const T*)init, cu, (T*)fs, T_len, N, D, W);
@@ -413,18 +532,19 @@ template <typename T> struct ConvLaunch {
                  int B, int T_len, int N, int D, int W, int silu, hipStream_t st) {
     constexpr int V = Elem<T>::kVec;
     const int64_t total = (int64_t)B * T_len;
-    const int tile = 256;
-    const int ntiles = (int)((total + tile - 1) / tile);
-    const int64_t nblocks = (int64_t)((D / V + kConvThreads - 1) / kConvThreads) * ntiles;
-    if (nblocks > 0x7fffffffLL) return -3;
-    dim3 grid((unsigned)nblocks);
+    const int nbd = (D / V + kConvThreads - 1) / kConvThreads;
+    const int groups = conv_bwd_groups(total, nbd, W);
+    dim3 grid((unsigned)(nbd * groups));
     if (total > 0) {
+      auto launch = [&](auto kern) {
+        GDN_LAUNCH(kKernConvBwd, st, kern, grid, dim3(kConvThreads), 0, st, (const T*)x, (const T*)dy, (const T*)weight,
+                   (const T*)bias, (const T*)init, (const T*)dht, cu, (T*)dx, workspace, total, T_len, N, D);
+      };
       switch (W) {
-#define GDN_CASE(W_)                                                                                              \
-  case W_:                                                                                                        \
-    GDN_LAUNCH(kKernConvBwd, st, (conv1d_bwd_kernel<T, W_>), grid, dim3(kConvThreads), 0, st, (const T*)x,   \
-                       (const T*)dy, (const T*)weight, (const T*)bias, (const T*)init, (const T*)dht, cu, (T*)dx, \
-                       workspace, total, T_len, N, D, tile, silu);                                                \
+#define GDN_CASE(W_)                                                                                \
+  case W_:                                                                                          \
+    silu ? launch(conv1d_bwd_kernel<T, W_, conv_bwd_tile(W_), true>)                                     \
+         : launch(conv1d_bwd_kernel<T, W_, conv_bwd_tile(W_), false>);                                   \
     break;
         GDN_CASE(1) GDN_CASE(2) GDN_CASE(3) GDN_CASE(4) GDN_CASE(5) GDN_CASE(6) GDN_CASE(7) GDN_CASE(8)
 #undef GDN_CASE
@@ -432,8 +552,8 @@ template <typename T> struct ConvLaunch {
       }
     }
     const int64_t nred = (int64_t)(W + 1) * D;
-    GDN_LAUNCH(kKernConvReduce, st, conv1d_reduce_kernel, dim3((unsigned)((nred + 255) / 256)), dim3(256), 0, st, workspace, dw, db,
-                       ntiles, W, D);
+    GDN_LAUNCH(kKernConvReduce, st, conv1d_reduce_kernel, dim3((unsigned)((nred + 63) / 64)), dim3(1024), 0, st, workspace, dw, db,
+                       groups, W, D);
     if (dh0 != nullptr) {
       const int64_t n = (int64_t)N * D;
       GDN_LAUNCH(kKernConvDh0, st, (conv1d_dh0_kernel<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
@@ -474,8 +594,9 @@ static int conv_check(int B, int T_len, int N, int D, int W, int dtype) {
 
 extern "C" int64_t gdn_conv1d_bwd_workspace_bytes(int B, int T, int D, int W) {
   const int64_t total = (int64_t)B * T;
-  const int64_t ntiles = (total + 255) / 256;
-  return (ntiles > 0 ? ntiles : 1) * (int64_t)(W + 1) * D * (int64_t)sizeof(float);
+  int64_t groups = (total + gdn::conv_bwd_tile(W) - 1) / gdn::conv_bwd_tile(W);
+  if (groups > gdn::kConvMaxGroups) groups = gdn::kConvMaxGroups;
+  return (groups > 0 ? groups : 1) * (int64_t)(W + 1) * D * (int64_t)sizeof(float);
 }
 
 extern "C" int gdn_conv1d_fwd(const void* x, const void* weight, const void* bias, const void* residual,
