@@ -684,6 +684,12 @@ template <int N> __device__ __forceinline__ float lane_group_sum(float v) {
   return v;
 }
 
+// sum over the wave, every lane gets the result
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+  v = lane_group_sum<32>(v);
+  return v + __shfl_xor(v, 32);
+}
+
 // Row sums of a 32x32 tile given as per-lane products x[r] (accumulator layout).  A halving butterfly over the 16
 // lanes of a DPP row: at each step a lane keeps the pair sums of the registers whose index bit matches its own lane bit, so 16 sums cost 15 exchanges instead of 64.  Lane l returns the sum over its DPP row of
 // register r = l & 15, i.e. a partial sum (16 of the 32 columns) of tile row acc_row(l & 15).

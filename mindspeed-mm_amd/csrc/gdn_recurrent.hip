@@ -3,8 +3,9 @@
 // (reference math: mindspeed_mm/fsdp/models/qwen3_5/modeling_qwen3_5.py:478-517).
 //
 // The kernel is bound by streaming the fp32 state [K,V] (64 KB at K=V=128) through HBM once in, once
-// out.  One workgroup of 256 threads owns a [K, BV] column slab of one state; the slab lives in
-// registers for all T tokens of the call.  With S_old the state before the token,
+// out (a batch of 256 with 32 heads: 1.08 GB in 190 us = 5.7 TB/s on states that no cache holds; 217 us with the loads and
+// the launch order left to themselves).  One workgroup of 256
+// threads owns a [K, BV] column slab of one state; the slab lives in registers for all T tokens of the call.  With S_old the state before the token,
 //     S^T k = e^g (S_old^T k),   S^T q = e^g (S_old^T q) + (k.q) delta
 // so both contractions are taken in ONE pass over the registers, then the rank-1 update is applied.
 // No MFMA: 6 flop per 8 bytes of state traffic, far below the matrix-core ridge.
@@ -13,6 +14,7 @@
 // the gates can be formed here from the layer's projections (g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b)
 // rounded to b's dtype as the layer's `b.sigmoid()` is; modeling_qwen3_5.py:833-841) instead of being passed in: a
 // decode step of the layer is then the convolution update followed by this kernel, with no copies in between.
+#include "gdn_chunk.h"
 #include "gdn_common.h"
 #include "gdn_profile.h"
 
@@ -27,34 +29,59 @@ struct RecurrentGates {   // either g, beta (fp32 [tokens,Hv]) or the projection
   const void* dt_bias;
 };
 
-template <typename T, typename TP, int DK, int BV>
-__global__ __launch_bounds__(256) void recurrent_kernel(
+// n consecutive values, n * sizeof(T) <= 16 bytes, in one load
+template <typename T, int n> __device__ __forceinline__ void load_run(float* dst, const T* p) {
+  constexpr int bytes = n * (int)sizeof(T);
+  float f[Elem<T>::kVec];
+  Vec16<T> x = zero16<T>();
+  if constexpr (bytes == 16) {
+    x = ld16(p);
+  } else if constexpr (bytes == 8) {
+    const u32x2 w = *reinterpret_cast<const u32x2*>(p);
+    x.raw[0] = w[0]; x.raw[1] = w[1];
+  } else if constexpr (bytes == 4) {
+    x.raw[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else {
+    static_assert(bytes == 2, "2 to 16 bytes");
+    x.raw[0] = *reinterpret_cast<const uint16_t*>(p);
+  }
+  unpack16<T>(x, f);
+#pragma unroll
+  for (int e = 0; e < n; ++e) dst[e] = f[e];
+}
+
+// A workgroup's slab is BV columns of one state, 4 of them per thread in RPT rows.  Everything a token needs is requested
+// at once: the slab, k and q (each wave normalises them by itself and keeps them in a part of the LDS of its own), v and
+// the gates; the only barrier of a token lies between the waves' partial sums over the rows.
+// waves per SIMD the registers have to allow: left to itself the compiler takes 280 for some of the smaller slabs
+constexpr int recurrent_waves(int dk, int bv) { return dk * bv < 128 * 128 ? 4 : 1; }
+
+template <typename T, typename TP, int DK, int BV, bool STREAM>
+__global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int64_t sq, int64_t sk, int64_t sv,
     RecurrentGates gates, const float* state_in, float* state_out, T* __restrict__ o, const int64_t* __restrict__ cu,
-    int B, int T_len, int Hqk, int Hv, int V, float scale, int use_l2norm) {
+    int T_len, int Hqk, int Hv, int V, float scale, int use_l2norm) {
   constexpr int CG = BV / 4;            // column groups (4 fp32 = 16 bytes each)
   constexpr int NRG = kThreads / CG;    // row groups
-  constexpr int RPT = DK / NRG;         // state rows held by a thread
-  constexpr int RGW = 64 / CG;          // row groups inside one wave
-  static_assert(DK % NRG == 0 && RPT >= 1, "tile shape");
-  __shared__ float ks[DK], qs[DK], red[4][CG][8], red3[4][3];
+  constexpr int RPT = DK / NRG;         // state rows held by a thread: rg, rg + NRG, ...
+  constexpr int EPL = DK / 64;          // elements of k and q per lane for the norms
+  static_assert(DK % NRG == 0 && RPT >= 1 && CG <= 64, "tile shape");
+  __shared__ float red[2][4][CG][8], kq_rows[4][DK][2];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cg = tid % CG, rg = tid / CG;
-  const int b = blockIdx.x / Hv, h = blockIdx.x % Hv, hq = h / (Hv / Hqk);
-  const int v0 = blockIdx.y * BV + cg * 4;
-  const int64_t sbase = ((int64_t)(b * Hv + h) * DK) * V + v0;
+  // the slabs of a state are neighbours in the launch order: what is in flight then stays close together in memory
+  const int nslab = V / BV, bh = blockIdx.x / nslab, b = bh / Hv, h = bh % Hv, hq = h / (Hv / Hqk);
+  const int v0 = (blockIdx.x % nslab) * BV + cg * 4;
+  const int64_t sbase = ((int64_t)bh * DK + rg) * V + v0;
 
-  float S[RPT][4];
+  f32x4 S[RPT];
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
-    const int row = rg + NRG * i;
-    if (state_in != nullptr) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(state_in + sbase + (int64_t)row * V);
-      S[i][0] = x[0]; S[i][1] = x[1]; S[i][2] = x[2]; S[i][3] = x[3];
-    } else {
-      S[i][0] = S[i][1] = S[i][2] = S[i][3] = 0.f;
-    }
+    const f32x4* p = reinterpret_cast<const f32x4*>(state_in + sbase + (int64_t)(NRG * i) * V);
+    if (state_in == nullptr) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    else if constexpr (STREAM) S[i] = __builtin_nontemporal_load(p);
+    else S[i] = *p;
   }
 
   // packed input (cu given): "sequence" b owns the tokens cu[b] .. cu[b+1] of the one batch row
@@ -62,43 +89,12 @@ __global__ __launch_bounds__(256) void recurrent_kernel(
   const int ntok = cu != nullptr ? (int)(cu[b + 1] - cu[b]) : T_len;
   for (int t = 0; t < ntok; ++t) {
     const int64_t tok = tok0 + t;
-    // ---- q, k of this token: optional l2 norm, q pre-scaled ----
-    float kv_ = 0.f, qv_ = 0.f;
-    if (tid < DK) {
-      kv_ = Elem<T>::to_f(k[tok * sk + hq * DK + tid]);
-      qv_ = Elem<T>::to_f(q[tok * sq + hq * DK + tid]);
-    }
-    const float sk = wave_sum(kv_ * kv_), sq = wave_sum(qv_ * qv_), skq = wave_sum(kv_ * qv_);
-    if (lane == 0) { red3[wave][0] = sk; red3[wave][1] = sq; red3[wave][2] = skq; }
-    __syncthreads();
-    const float tk = red3[0][0] + red3[1][0] + red3[2][0] + red3[3][0];
-    const float tq = red3[0][1] + red3[1][1] + red3[2][1] + red3[3][1];
-    float kq = red3[0][2] + red3[1][2] + red3[2][2] + red3[3][2];
-    float rk = 1.f, rq = scale;
-    if (use_l2norm) { rk = rsqrtf(tk + 1e-6f); rq = scale * rsqrtf(tq + 1e-6f); }
-    kq *= rk * rq;
-    if (tid < DK) { ks[tid] = kv_ * rk; qs[tid] = qv_ * rq; }
-    __syncthreads();
-
-    // ---- one pass over the slab: S_old^T k and S_old^T q ----
-    float pk[4] = {0.f, 0.f, 0.f, 0.f}, pq[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const float kk = ks[rg + NRG * i], qq = qs[rg + NRG * i];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) { pk[c] += S[i][c] * kk; pq[c] += S[i][c] * qq; }
-    }
-#pragma unroll
-    for (int m = CG; m < 64; m <<= 1) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) { pk[c] += __shfl_xor(pk[c], m); pq[c] += __shfl_xor(pq[c], m); }
-    }
-    if (lane < CG) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) { red[wave][cg][c] = pk[c]; red[wave][cg][4 + c] = pq[c]; }
-    }
-    __syncthreads();
-
+    const T* kp = k + tok * sk + hq * DK;
+    const T* qp = q + tok * sq + hq * DK;
+    float ke[EPL], qe[EPL], vv[4];
+    load_run<T, EPL>(ke, kp + lane * EPL);
+    load_run<T, EPL>(qe, qp + lane * EPL);
+    load_run<T, 4>(vv, v + tok * sv + h * V + v0);
     float eg, bt;
     if (gates.a == nullptr) {
       eg = __expf(gates.g[tok * Hv + h]);
@@ -111,25 +107,56 @@ __global__ __launch_bounds__(256) void recurrent_kernel(
       const float sg = 1.f / (1.f + expf(-Elem<T>::to_f(static_cast<const T*>(gates.b)[tok * Hv + h])));
       bt = Elem<T>::to_f(Elem<T>::from_f(sg));
     }
-    float delta[4], ov[4];
-    Vec16<T> vv;
-    if constexpr (sizeof(T) == 4) {
-      vv = ld16(v + tok * sv + h * V + v0);
-    } else {
-      const u32x2 w = *reinterpret_cast<const u32x2*>(v + tok * sv + h * V + v0);
-      vv.raw = u32x4{w[0], w[1], 0u, 0u};
+    // ---- optional l2 norm of k and q; q carries the scale ----
+    float tk = 0.f, tq = 0.f, kq = 0.f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) { tk += ke[e] * ke[e]; tq += qe[e] * qe[e]; kq += ke[e] * qe[e]; }
+    tk = wave_sum_dpp(tk);
+    tq = wave_sum_dpp(tq);
+    kq = wave_sum_dpp(kq);
+    float rk = 1.f, rq = scale;
+    if (use_l2norm) { rk = rsqrtf(tk + 1e-6f); rq = scale * rsqrtf(tq + 1e-6f); }
+    kq *= rk * rq;
+    float (*kw)[2] = kq_rows[wave];
+    GDN_WAVE_LDS_SYNC();   // the previous token's reads are done
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      kw[lane * EPL + e][0] = ke[e] * rk;
+      kw[lane * EPL + e][1] = qe[e] * rq;
+    }
+    GDN_WAVE_LDS_SYNC();
+
+    // ---- one pass over the slab: S_old^T k and S_old^T q ----
+    float pk[4] = {0.f, 0.f, 0.f, 0.f}, pq[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const float kk = kw[rg + NRG * i][0], qq = kw[rg + NRG * i][1];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) { pk[c] += S[i][c] * kk; pq[c] += S[i][c] * qq; }
     }
 #pragma unroll
+    for (int m = CG; m < 64; m <<= 1) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) { pk[c] += __shfl_xor(pk[c], m); pq[c] += __shfl_xor(pq[c], m); }
+    }
+    float (*rd)[CG][8] = red[t & 1];   // two sets: one is read while the next token's is written
+    if (lane < CG) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) { rd[wave][cg][c] = pk[c]; rd[wave][cg][4 + c] = pq[c]; }
+    }
+    GDN_LDS_BARRIER();
+    float delta[4], ov[4];
+#pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const float skv = red[0][cg][c] + red[1][cg][c] + red[2][cg][c] + red[3][cg][c];
-      const float sqv = red[0][cg][4 + c] + red[1][cg][4 + c] + red[2][cg][4 + c] + red[3][cg][4 + c];
-      delta[c] = bt * (vv.get(c) - eg * skv);
+      const float skv = rd[0][cg][c] + rd[1][cg][c] + rd[2][cg][c] + rd[3][cg][c];
+      const float sqv = rd[0][cg][4 + c] + rd[1][cg][4 + c] + rd[2][cg][4 + c] + rd[3][cg][4 + c];
+      delta[c] = bt * (vv[c] - eg * skv);
       ov[c] = eg * sqv + kq * delta[c];
     }
     // ---- rank-1 update in registers ----
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-      const float kk = ks[rg + NRG * i];
+      const float kk = kw[rg + NRG * i][0];
 #pragma unroll
       for (int c = 0; c < 4; ++c) S[i][c] = eg * S[i][c] + kk * delta[c];
     }
@@ -138,26 +165,16 @@ __global__ __launch_bounds__(256) void recurrent_kernel(
       if constexpr (sizeof(T) == 4) {
         *reinterpret_cast<f32x4*>(op) = f32x4{ov[0], ov[1], ov[2], ov[3]};
       } else {
-        Vec16<T> ow = zero16<T>();
-#pragma unroll
-        for (int c = 0; c < 4; ++c) ow.set(c, ov[c]);
-        *reinterpret_cast<u32x2*>(op) = u32x2{ow.raw[0], ow.raw[1]};
+        *reinterpret_cast<u32x2*>(op) = u32x2{f32x2_to_bf16x2(ov[0], ov[1]), f32x2_to_bf16x2(ov[2], ov[3])};
       }
     }
-    // red/ks/qs are rewritten only after the next token's first barrier
   }
 
   if (state_out != nullptr) {
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int row = rg + NRG * i;
-      // streaming store: the slab is not read again by this kernel, and keeping it out of the L2 on its way to
-      // memory leaves the cache to the loads (measured: 219 -> 163 us per batch-256 step)
-      __builtin_nontemporal_store(f32x4{S[i][0], S[i][1], S[i][2], S[i][3]},
-                                  reinterpret_cast<f32x4*>(state_out + sbase + (int64_t)row * V));
-    }
+    for (int i = 0; i < RPT; ++i)   // streaming store: the slab is not read again by this kernel
+      __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(state_out + sbase + (int64_t)(NRG * i) * V));
   }
-  (void)RGW; (void)B;
 }
 
 template <typename T, typename TP>
@@ -165,20 +182,36 @@ static int launch_recurrent(const void* q, const void* k, const void* v, int64_t
                             const RecurrentGates& gates, const float* state_in, float* state_out, void* o, int B,
                             int T_len, int Hqk, int Hv, int K, int V, float scale, int use_l2norm, hipStream_t stream,
                             const int64_t* cu = nullptr) {
-#define GDN_REC(DK_, BV_)                                                                                          \
-  GDN_LAUNCH(kKernRecurrent, stream, (recurrent_kernel<T, TP, DK_, BV_>), dim3(B * Hv, V / BV_), dim3(kThreads), 0, \
-             stream, (const T*)q, (const T*)k, (const T*)v, sq, sk, sv, gates, state_in, state_out, (T*)o, cu, B,     \
-             T_len, Hqk, Hv, V, scale, use_l2norm)
-  const bool wide = (V % 128 == 0);
-  if (K == 64 && wide) GDN_REC(64, 128);
-  else if (K == 64) GDN_REC(64, 64);
-  else if (K == 128 && wide) GDN_REC(128, 128);
-  else if (K == 128) GDN_REC(128, 64);
-  else if (K == 256 && wide) GDN_REC(256, 128);
-  else if (K == 256) GDN_REC(256, 64);
-  else return -3;
+  // Whole states (64 KB at K = V = 128) per workgroup where they give every CU one, else 32 columns: 8.1 -> 7.1 us for one
+  // sequence of 32 heads, 11.4 -> 10.4 for 8; 32 columns at 16 / 32 sequences 18 / 30 us against 14 / 24.
+  // State loads that pass by the caches, except where the states exceed the L2s and still fit the 256 MB memory-side cache,
+  // which then serves a part of them (64 sequences 46 us against 49; 128 sequences 107 against 97).
+  // Past that size two or three workgroups per CU instead of four (by the LDS they ask for): less memory in flight at
+  // once, 198 -> 190 us at 256 sequences; below it 47 -> 57 us at 64.
+  const int64_t states = (int64_t)B * Hv * (V / 128), bytes = (int64_t)B * Hv * K * V * 4;
+  const bool narrow = V % 128 != 0 || states <= device_compute_units(), beyond = bytes >= (256LL << 20);
+  const bool cached = bytes > (32LL << 20) && !beyond;
+#define GDN_REC(DK_, BV_, ST_, LDS_)                                                                                   \
+  GDN_LAUNCH(kKernRecurrent, stream, (recurrent_kernel<T, TP, DK_, BV_, ST_>), dim3((unsigned)(B * Hv * (V / BV_))),   \
+             dim3(kThreads), LDS_, stream, (const T*)q, (const T*)k, (const T*)v, sq, sk, sv, gates, state_in,         \
+             state_out, (T*)o, cu, T_len, Hqk, Hv, V, scale, use_l2norm)
+  // (K = 256: half as wide, which makes the slab the registers hold the same)
+#define GDN_REC_K(DK_)                                                           \
+  constexpr int kWide##DK_ = DK_ == 256 ? 64 : 128;                              \
+  if (K == DK_) {                                                                \
+    if (narrow && cached) GDN_REC(DK_, 32, false, 0);                            \
+    else if (narrow) GDN_REC(DK_, 32, true, 0);                                  \
+    else if (beyond) GDN_REC(DK_, kWide##DK_, true, 45000);                             \
+    else if (cached) GDN_REC(DK_, kWide##DK_, false, 0);                  \
+    else GDN_REC(DK_, kWide##DK_, true, 0);                                             \
+    return (int)hipGetLastError();                                               \
+  }
+  GDN_REC_K(64)
+  GDN_REC_K(128)
+  GDN_REC_K(256)
+  return -3;
+#undef GDN_REC_K
 #undef GDN_REC
-  return (int)hipGetLastError();
 }
 
 static int recurrent_check(int B, int T, int Hqk, int Hv, int V) {

@@ -58,3 +58,13 @@ def test_rms_norm_gated_far_gates(ops, activation):
 def test_conv1d_edges(ops, dtype, B, T, D, W, cu):
     P.check_conv(ops, "cuda", B, T, D, W, dtype, cu=cu, residual=True)
     P.check_conv(ops, "cuda", B, T, D, W, dtype, cu=cu, bias=False, state=False, activation=None)
+
+
+@pytest.mark.parametrize("dtype,B,T,Hqk,Hv,K,V", [
+    (BF, 8, 1, 16, 32, 128, 128), (BF, 9, 1, 16, 32, 128, 128),    # as many states as compute units; more: whole states
+    (BF, 17, 1, 16, 32, 128, 128),                                 # states larger than the L2s
+    (BF, 129, 1, 16, 32, 128, 128),                                # larger than the memory-side cache
+    (F32, 3, 2, 1, 2, 128, 192), (BF, 2, 3, 1, 1, 256, 64), (BF, 140, 2, 1, 2, 256, 128), (BF, 300, 1, 1, 1, 64, 256),
+])
+def test_recurrent_edges(ops, dtype, B, T, Hqk, Hv, K, V):
+    P.check_recurrent(ops, "cuda", B, T, Hqk, Hv, K, V, dtype)
