@@ -38,7 +38,8 @@ extern "C" {
  * workspace sized with with_backward = 0 writes neither per-chunk states nor v_new to memory.
  *
  * The workspace has two parts.  The prep part (with_backward = 2) holds what depends on q, k, g, beta only: the
- * cumulative decay, Tm, the intra-chunk Q K^T tiles and the K / Q^T tile images; the state part (with_backward = 3)
+ * cumulative decay, Tm, the intra-chunk Q K^T tiles and the K / Q^T tile images -- and, where few heads and long
+ * sequences make the recurrences run in segments, the states the segments start from; the state part (with_backward = 3)
  * holds the per-chunk states, v_new and room for their gradients.  with_backward = 1 is both, contiguous.  A forward
  * call in a 16-bit dtype that writes o (and no fused norm) needs the prep part only.  gdn_chunk_bwd_parts takes the
  * two parts as separate buffers, so that a caller can keep the prep part of its forward call (0.28 GB at B=2, T=8192,

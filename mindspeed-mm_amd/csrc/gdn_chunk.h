@@ -38,16 +38,40 @@ struct ChunkWorkspace {
   int64_t AQ;             // T [chunks,Hv,2,2]       scale tril(Q K^T . Gam), accumulator tiles: lane <-> column, registers <-> row
   int64_t KAF;            // T [chunks,Hqk,K/32,2]   K as A operand: tile = (32 tokens) x (32 columns of K)
   int64_t QTF;            // T [chunks,Hqk,K/32,2]   Q^T as A operand: tile = (32 columns of K) x (32 tokens)
-  int64_t prep_bytes;     // everything above: what chunk_prep_kernel leaves (no v, no state in it).  What follows, the "state
-                          // part", may live in a second buffer: the kernels take a base pointer for each part.
+  int64_t SEGH;           // f32 [N,P,Hv,K,V]        sequences in P > 1 segments: the state each segment starts from
+  int64_t SEGM;           // f32 [N,P-1,Hv,K,V+K]    and the maps of the segments but the last
+  int64_t prep_bytes;     // everything above: what chunk_prep_kernel leaves, and what a refill of the state part starts the
+                          // segments from.  What follows, the "state part", may live in a second buffer: the kernels take a
+                          // base pointer for each part.
   int64_t VF;             // T [chunks,Hv,V/32,2]    v_new = Tm (beta v - beta e^G K S), tile = (32-column block) x (32-token block)
   int64_t HF;             // T [chunks,Hv,V/32,K/32] state BEFORE each chunk, tile = (32 rows of K) x (32 columns of V)
   int64_t fwd_bytes;
   int64_t DVF;            // T [chunks,Hv,V/32,2]    d(v_new)
   int64_t DHF;            // T [chunks,Hv,V/32,K/32] gradient of the state AFTER each chunk; once the chunk-local kernel of a
                           //   head has read its part it may leave the group's dq, dk sums there for the next head's launch
+  int64_t SEGD, SEGDM;    // as SEGH, SEGM, for the state gradients; not shared with them: several backward passes may read
+                          // one forward pass's prep part at a time
   int64_t total_bytes;
 };
+
+int device_compute_units();   // defined with the forward launcher
+
+// Segments a sequence is cut into for the two recurrences (gdn_segments.h); 1 = not cut.  As many as give every slab of
+// 32 state columns a compute unit of its own, none shorter than kMinSegmentChunks on average; two segments would take as
+// many dependent steps as one.  Sequences of kMinCutChunks on average pay for the two launches in front of each
+// recurrence.  Forward pass, 128-wide heads, not cut -> cut: 4 heads 114 -> 80 us at 64 chunks, 207 -> 89 at 128; 8
+// heads 407 -> 145 at 256; 16 heads (4 segments) 114 -> 83 at 64, 829 -> 459 at 512.  At 48 chunks it is still 91 -> 77,
+// but a training step of that length waits for the host, and two more launches a pass cost it 235 -> 250.  Wider value
+// heads stay uncut: cut, they are as far from float32 in the mean (dg of slowly decaying heads 4.3e-3 to 5.2e-3, uncut
+// 4.3e-3 to 5.0e-3), but where the largest differences fall changes, and those lie at the stated bound (0.046 to 0.086
+// uncut, 0.050 to 0.082 cut, of a dg of 15).
+constexpr int kMinSegmentChunks = 16, kMinCutChunks = 64;
+inline int state_segments(const ChunkDims& d, int elem_bytes) {
+  if (elem_bytes != 2 || d.K != 128 || d.V != 128) return 1;
+  const int64_t slabs = (int64_t)d.N * d.Hv * (d.V / 32), chunks = d.tokens() / 64 / d.N;
+  const int64_t fit = device_compute_units() / slabs, p = fit < chunks / kMinSegmentChunks ? fit : chunks / kMinSegmentChunks;
+  return p >= 3 && chunks >= kMinCutChunks ? (int)p : 1;
+}
 
 inline int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
@@ -63,12 +87,17 @@ inline ChunkWorkspace chunk_workspace_layout(const ChunkDims& d, int elem_bytes)
   w.AQ = take(nc * 64 * d.Hv * 64 * elem_bytes);
   w.KAF = take(nc * 64 * d.Hqk * d.K * elem_bytes);
   w.QTF = take(nc * 64 * d.Hqk * d.K * elem_bytes);
+  const int64_t P = state_segments(d, elem_bytes), seg = P > 1 ? (int64_t)d.N * d.Hv * d.K * 4 : 0;
+  w.SEGH = take(seg * P * d.V);
+  w.SEGM = take(seg * (P - 1) * (d.V + d.K));
   w.prep_bytes = off;
   w.VF = take(nc * 64 * d.Hv * d.V * elem_bytes);
   w.HF = take(nc * d.Hv * d.V * d.K * elem_bytes);
   w.fwd_bytes = off;
   w.DVF = take(nc * 64 * d.Hv * d.V * elem_bytes);
   w.DHF = take(nc * d.Hv * d.V * d.K * elem_bytes);
+  w.SEGD = take(seg * P * d.V);
+  w.SEGDM = take(seg * (P - 1) * (d.V + d.K));
   w.total_bytes = off;
   return w;
 }
@@ -135,16 +164,14 @@ inline KdaWorkspace kda_workspace_layout(const ChunkDims& d, int elem_bytes) {
 // which one CU gets its requests served (about 35 GB/s measured, loads and stores together), whatever the number of
 // slabs the workgroup serves, so when the whole problem has no more slabs than the device has CUs every slab gets a
 // workgroup (and a CU) of its own; larger problems put two slabs in a workgroup, which share the tiles.
-int device_compute_units();   // defined with the forward launcher
-
-inline bool one_slab_per_workgroup(const ChunkDims& d, int compute_units) {
-  return (int64_t)d.N * d.Hv * (d.V / 32) <= compute_units;
+inline bool one_slab_per_workgroup(const ChunkDims& d, int compute_units, int segs = 1) {
+  return (int64_t)d.N * segs * d.Hv * (d.V / 32) <= compute_units;
 }
 // Two recurrences at once (a backward pass that refills the forward states on a second stream while the reverse
 // recurrence runs): with two slabs per workgroup each of them is as fast as with one and needs half of the compute
 // units, so both fit the device side by side.  Only needed where one slab per workgroup would take more than half.
-inline bool two_slabs_to_share_device(const ChunkDims& d, int compute_units) {
-  const int64_t slabs = (int64_t)d.N * d.Hv * (d.V / 32);
+inline bool two_slabs_to_share_device(const ChunkDims& d, int compute_units, int segs = 1) {
+  const int64_t slabs = (int64_t)d.N * segs * d.Hv * (d.V / 32);
   return slabs <= compute_units && 2 * slabs > compute_units;
 }
 

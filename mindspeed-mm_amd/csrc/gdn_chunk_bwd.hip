@@ -18,6 +18,7 @@
 #include "gdn_chunk.h"
 #include "gdn_common.h"
 #include "gdn_profile.h"
+#include "gdn_segments.h"
 
 namespace gdn {
 
@@ -52,13 +53,14 @@ template <int PIECES, int NT> struct DealB { static constexpr int kPer = (PIECES
 // KDA (one decay per key channel): kaf and kaf2 hold the two K images ready-made (rows x e^{G_last-G} and rows x
 // -beta e^{G}, channel by channel), qtf the transposed rows of q with scale and decay already applied (so dO is used
 // as it is), G holds e^{G_last} [chunks,Hv,DK]; the rows of dS decay each by their own factor.
-template <typename T, int DK, int NW, int NL, int STAGES, bool KDA = false>
+// segs, MAP: as in the forward recurrence; the map of a segment leaves in dh0.
+template <typename T, int DK, int NW, int NL, int STAGES, bool KDA = false, bool MAP = false>
 __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 && NL >= 4) ? 2 : 1) void chunk_state_bwd_kernel(
     const T* __restrict__ kaf, const T* __restrict__ kaf2, const T* __restrict__ qtf, const T* __restrict__ ai, const T* __restrict__ aqf,
     const T* __restrict__ dO, const float* __restrict__ G, const void* __restrict__ beta, int beta_same,
     const float* __restrict__ dht,
     float* __restrict__ dh0, T* __restrict__ dvf, T* __restrict__ dhf, const int64_t* __restrict__ cu,
-    const int* __restrict__ chunk_offsets, int T_len, int Hqk, int Hv, int V, float scale) {
+    const int* __restrict__ chunk_offsets, int T_len, int Hqk, int Hv, int V, float scale, int segs) {
   using SM = StateBwdSmem<T, DK, NW, STAGES, KDA>;
   static_assert(!KDA || 64 * NL >= DK, "a loader thread per key channel");
   constexpr int NT = 64 * NL, VEC = Elem<T>::kVec, NKT = DK / 32;   // NT loader threads
@@ -68,11 +70,13 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: the roles branch on a scalar
-  const int nh = xcd_grouped_head(blockIdx.x, gridDim.x, Hv / Hqk), n = nh / Hv, h = nh % Hv;
-  const int64_t bos = cu ? cu[n] : (int64_t)n * T_len;
-  const int len = cu ? (int)(cu[n + 1] - bos) : T_len;
-  const int nchunks = (len + kChunk - 1) / kChunk;
-  const int64_t chunk_base = cu ? chunk_offsets[n] : (int64_t)n * ((T_len + kChunk - 1) / kChunk);
+  const int nh = xcd_grouped_head(blockIdx.x, gridDim.x, Hv / Hqk), ns = nh / Hv, h = nh % Hv;
+  const SegmentRun run = segment_run(ns, MAP ? segs - 1 : segs, MAP ? 1 : 0, segs, cu, chunk_offsets, T_len);
+  const int64_t bos = run.bos, chunk_base = run.chunk_base;
+  const int len = run.len, nchunks = run.nchunks;
+  // MAP: the workgroup's columns belong to A, which starts from the identity and sees no dO
+  const bool of_a = MAP && (int)blockIdx.y * (32 * NW) >= V;
+  const int col0 = of_a ? 0 : (int)blockIdx.y * (32 * NW);   // of the rows of dO it reads
 
   // step s = 0 .. nchunks-1 handles chunk nchunks-1-s
   if (wave >= NW) {
@@ -110,7 +114,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 #pragma unroll
       for (int i = 0; i < CD; ++i) {   // dO rows of the slabs; rows past the end repeat the last one and are cleared below
         const int idc = imin(lt + i * NT, PD - 1), row = imin(idc / DPR, nvalid - 1), cc = idc % DPR;
-        pd[set][i] = ld16(dO + ((tok0 + row) * Hv + h) * V + blockIdx.y * (32 * NW) + cc * VEC);
+        pd[set][i] = ld16(dO + ((tok0 + row) * Hv + h) * V + col0 + cc * VEC);
         if constexpr (!KDA) pgd[set][i] = G[ch * 64 + row];
       }
       pnv[set] = nvalid;
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 #pragma unroll
       for (int i = 0; i < CD; ++i) {
         const int idc = imin(lt + i * NT, PD - 1);
-        const Vec16<T> x = idc / DPR < pnv[set] ? pd[set][i] : zero16<T>();
+        const Vec16<T> x = idc / DPR < pnv[set] && !of_a ? pd[set][i] : zero16<T>();
         st16(st + SM::off_do + idc * VEC, x);
         if constexpr (KDA) st16(st + SM::off_do + 64 * 32 * NW + idc * VEC, x);
         else st16(st + SM::off_do + 64 * 32 * NW + idc * VEC, scale16<T>(x, scale * __expf(pgd[set][i])));
@@ -218,10 +222,13 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 #pragma unroll
   for (int kt = 0; kt < NKT; ++kt) {
     dS[kt] = acc_zero();
-    if (dht != nullptr) {
+    if constexpr (MAP) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dS[kt][r] = v0 + acc_col() == V + 32 * kt + acc_row(r) ? 1.f : 0.f;
+    } else if (dht != nullptr) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        dS[kt][r] = dht[(((int64_t)n * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col()];
+        dS[kt][r] = dht[(((int64_t)ns * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col()];
     }
   }
   // As in the forward recurrence the vector work that does not depend on the running products (decay and packing of
@@ -264,7 +271,8 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
     const float eg = KDA ? 1.f : __expf(row[0]);
     const int64_t tile0 = ((chunk_base + c) * Hv + h) * (V / 32) + vblk;
 #pragma unroll
-    for (int kt = 0; kt < NKT; ++kt) dSb[kt].store_stream(dhf + (tile0 * NKT + kt) * 1024);
+    for (int kt = 0; kt < NKT; ++kt)
+      if constexpr (!MAP) dSb[kt].store_stream(dhf + (tile0 * NKT + kt) * 1024);
     // dV' = (scale tril(Q K^T . Gam))^T dO (from the forward pass's tiles) + (e^{G_last-G} . K) dS, one accumulation
     // chain per 32-token block.  The pair of A-operand tiles of K tile kt + 1 is requested from LDS before the matrix
     // instructions of K tile kt are issued (two register buffers); the decay of dS rides in between.
@@ -297,8 +305,10 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
     for (int t = 0; t < 3; ++t) tf[t].load_t(Tm + t * 1024);   // Tm^T tiles: (lane <-> column of Tm, registers <-> row)
     dvb[0].pack(a0);
     dvb[1].pack(a1);
-    dvb[0].store_stream(dvf + (tile0 * 2 + 0) * 1024);
-    dvb[1].store_stream(dvf + (tile0 * 2 + 1) * 1024);
+    if constexpr (!MAP) {
+      dvb[0].store_stream(dvf + (tile0 * 2 + 0) * 1024);
+      dvb[1].store_stream(dvf + (tile0 * 2 + 1) * 1024);
+    }
     // R = Tm^T dV' (upper triangular: R_0 = Tm00^T dV'_0 + Tm10^T dV'_1, R_1 = Tm11^T dV'_1)
     f32x16 y0 = acc_zero(), y1 = acc_zero();
     mma2(y0, tf[0], dvb[0], y1, tf[2], dvb[1]);
@@ -336,12 +346,14 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
     dSb[NKT - 1].pack(dS[NKT - 1]);
     if (STAGES == 1 && st + 1 < nchunks) GDN_LDS_BARRIER();   // (B)
   }
-  if (dh0 != nullptr) {
+  // the gradient before the run leaves as that of its sequence's initial state, or as the run's map
+  const int ldt = MAP ? V + DK : V;
+  if (dh0 != nullptr && (MAP || run.p == 0)) {
+    float* const to = dh0 + ((int64_t)(MAP ? ns : run.n) * Hv + h) * DK * ldt;
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        dh0[(((int64_t)n * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col()] = dS[kt][r];
+      for (int r = 0; r < 16; ++r) to[(int64_t)(32 * kt + acc_row(r)) * ldt + v0 + acc_col()] = dS[kt][r];
   }
 }
 
@@ -990,12 +1002,28 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
   const float* rstd_q = l2norm ? reinterpret_cast<const float*>(ws + L.rstd) : nullptr;
   const float* rstd_k = l2norm ? rstd_q + (int64_t)nc * 64 * d.Hqk : nullptr;
   if (phases & 2) {
+    const int segs = state_segments(d, (int)sizeof(T));
+    if constexpr (sizeof(T) == 2 && DK == 128 && NW == 4) {
+      if (segs > 1) {
+        float* maps = reinterpret_cast<float*>(ws_state + L.SEGDM);
+        float* starts = reinterpret_cast<float*>(ws_state + L.SEGD);
+        auto kern = chunk_state_bwd_kernel<T, DK, 2, NLS, STAGES, false, true>;
+        constexpr int smem = StateBwdSmem<T, DK, 2, STAGES>::bytes;
+        if (int e = set_lds_b(kern, smem)) return e;
+        GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
+                   (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, beta, beta_same,
+                   (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, segs);
+        GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
+                   (const float*)maps, dht, starts, segs, d.Hv, d.V);
+        dht = starts;
+      }
+    }
     auto kern = chunk_state_bwd_kernel<T, DK, NWS, NLS, STAGES>;
     constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
-    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * d.Hv, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)KAF,
+    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)KAF,
                (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, beta, beta_same, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V,
-               scale);
+               scale, segs);
   }
   if (phases & 4) {
     const TokenStrides gs = d.strides();
@@ -1065,8 +1093,9 @@ static int chunk_bwd_entry(const void* q, const void* k, const void* v, int64_t 
                                                           dk, dv, dg, dbeta, d_initial_state, ws, ws_state, phases, scale, \
                                                           use_qk_l2norm, st)
   const bool wide = (V % 128 == 0);
-  const bool solo = one_slab_per_workgroup(d, device_compute_units()) &&
-                    !(share_device && two_slabs_to_share_device(d, device_compute_units()));
+  const int segs = state_segments(d, dtype == 0 ? 4 : 2);
+  const bool solo = one_slab_per_workgroup(d, device_compute_units(), segs) &&
+                    !(share_device && two_slabs_to_share_device(d, device_compute_units(), segs));
   if (dtype == 1) {
     if (K == 128 && wide && solo) GDN_BWD(bf16_t, 128, 4, 1, 4, 2);
     if (K == 128 && wide) GDN_BWD(bf16_t, 128, 4, 2, 4, 2);

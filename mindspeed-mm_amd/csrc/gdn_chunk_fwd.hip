@@ -14,6 +14,7 @@
 #include "gdn_chunk.h"
 #include "gdn_common.h"
 #include "gdn_profile.h"
+#include "gdn_segments.h"
 #include "gdn_rmsnorm_gated.h"
 
 namespace gdn {
@@ -349,14 +350,15 @@ template <int PIECES, int NT> struct Deal { static constexpr int kPer = (PIECES 
 // e^{G_last-G} channel by channel, G holds e^{G_last} [chunks,Hv,DK] and beta the transformed beta in fp32; the state's
 // rows decay each by their own factor.  With OUT the output waves take (scale q . e^{G})^T from a third image, qim,
 // whose rows carry every factor of the output's first term (the other modes read their Q^T image through qtf).
-template <typename T, int DK, int NW, int NL, int STAGES, bool OUT, bool PRE_, bool KDA = false>
+// segs: segments of a sequence, each with its own initial state (gdn_segments.h); MAP: their maps [B | A] into ht.
+template <typename T, int DK, int NW, int NL, int STAGES, bool OUT, bool PRE_, bool KDA = false, bool MAP = false>
 __global__ __launch_bounds__(64 * (NW + (OUT ? NW * StateOutWaves<NW>::value : 0) + NL)) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 2 : 1)
 void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, const T* __restrict__ ai,
                         const T* __restrict__ aqf, const T* __restrict__ v, const float* __restrict__ G,
                         const void* __restrict__ beta, int beta_same, const float* __restrict__ h0, float* __restrict__ ht,
                         T* __restrict__ vf, T* __restrict__ hf, T* __restrict__ o, const int64_t* __restrict__ cu,
                         const int* __restrict__ chunk_offsets, int T_len, int Hqk, int Hv, int V, float scale,
-                        int64_t v_stride, const T* __restrict__ qim) {
+                        int64_t v_stride, const T* __restrict__ qim, int segs) {
   using SM = StateSmem<T, DK, NW, STAGES, OUT, PRE_, KDA>;
   static_assert(!KDA || 64 * NL >= DK, "a loader thread per key channel");
   constexpr int NT = 64 * NL, VEC = Elem<T>::kVec, NKT = DK / 32, OS = StateOutWaves<NW>::value, NWO = OUT ? NW * OS : 0;
@@ -367,20 +369,30 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: the roles branch on a scalar
-  const int nh = xcd_grouped_head(blockIdx.x, gridDim.x, Hv / Hqk), n = nh / Hv, h = nh % Hv;
-  const int64_t bos = cu ? cu[n] : (int64_t)n * T_len;
-  const int len = cu ? (int)(cu[n + 1] - bos) : T_len;
-  const int nchunks = (len + kChunk - 1) / kChunk;
-  const int64_t chunk_base = cu ? chunk_offsets[n] : (int64_t)n * ((T_len + kChunk - 1) / kChunk);
+  const int nh = xcd_grouped_head(blockIdx.x, gridDim.x, Hv / Hqk), ns = nh / Hv, h = nh % Hv;
+  const SegmentRun run = segment_run(ns, MAP ? segs - 1 : segs, 0, segs, cu, chunk_offsets, T_len);
+  const int64_t bos = run.bos, chunk_base = run.chunk_base;
+  const int len = run.len, nchunks = run.nchunks;
+  // MAP: the workgroup's columns belong to A, which starts from the identity and sees no v
+  const bool of_a = MAP && (int)blockIdx.y * (32 * NW) >= V;
+  const int col0 = of_a ? 0 : (int)blockIdx.y * (32 * NW);   // of the rows of v it reads
+  auto initial = [&](int row, int col) -> float {
+    if constexpr (MAP) return col == V + row ? 1.f : 0.f;
+    else return h0 != nullptr ? h0[(((int64_t)ns * Hv + h) * DK + row) * V + col] : 0.f;
+  };
+  // the state after the run leaves as the final state of its sequence, or as the run's map
+  const int ldt = MAP ? V + DK : V;
+  float* const hto = ht == nullptr || (!MAP && run.p != segs - 1)
+                         ? nullptr : ht + ((int64_t)(MAP ? ns : run.n) * Hv + h) * DK * ldt;
   // number of barriers every wave passes: one per chunk, plus one that hands the last V' to the output waves
   const int nsteps = nchunks + (OUT ? 1 : 0);
   if (nchunks == 0) {   // an empty sequence: its final state is its initial state
-    if (wave < NW && ht != nullptr) {
-      const int v0 = 32 * (blockIdx.y * NW + wave);
+    if (wave < NW && hto != nullptr) {
+      const int col = 32 * (blockIdx.y * NW + wave) + acc_col();
       for (int kt = 0; kt < NKT; ++kt)
         for (int r = 0; r < 16; ++r) {
-          const int64_t at = (((int64_t)n * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col();
-          ht[at] = h0 != nullptr ? h0[at] : 0.f;
+          const int row = 32 * kt + acc_row(r);
+          hto[(int64_t)row * ldt + col] = initial(row, col);
         }
     }
     return;
@@ -424,7 +436,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
 #pragma unroll
       for (int i = 0; i < CV; ++i) {   // rows past the end of the sequence repeat the last one (their beta is 0)
         const int idc = imin(lt + i * NT, PV - 1), row = imin(idc / VPR, nvalid - 1), cc = idc % VPR;
-        pv[set][i] = ld16(v + (tok0 + row) * v_stride + (int64_t)h * V + blockIdx.y * (32 * NW) + cc * VEC);
+        pv[set][i] = ld16(v + (tok0 + row) * v_stride + (int64_t)h * V + col0 + cc * VEC);
         if constexpr (PRE) pbv[set][i] = gate_raw<T>(beta, beta_same, (tok0 + row) * Hv + h);
       }
       pnv[set] = nvalid;
@@ -483,7 +495,8 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
 #pragma unroll
       for (int i = 0; i < CV; ++i) {
         const int idc = imin(lt + i * NT, PV - 1);
-        if constexpr (PRE) st16(st + SM::off_v + idc * VEC, scale16<T>(pv[set][i], idc / VPR < pnv[set] ? gate_val<T>(pbv[set][i], beta_same) : 0.f));
+        if (of_a) st16(st + SM::off_v + idc * VEC, zero16<T>());   // not v x 0: v may hold infinities
+        else if constexpr (PRE) st16(st + SM::off_v + idc * VEC, scale16<T>(pv[set][i], idc / VPR < pnv[set] ? gate_val<T>(pbv[set][i], beta_same) : 0.f));
         else st16(st + SM::off_v + idc * VEC, pv[set][i]);
       }
       float* row = reinterpret_cast<float*>(gdn_smem + buf * SM::stage + SM::off_row);
@@ -642,10 +655,9 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
 #pragma unroll
   for (int kt = 0; kt < NKT; ++kt) {
     S[kt] = acc_zero();
-    if (h0 != nullptr) {
+    if (MAP || h0 != nullptr) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        S[kt][r] = h0[(((int64_t)n * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col()];
+      for (int r = 0; r < 16; ++r) S[kt][r] = initial(32 * kt + acc_row(r), v0 + acc_col());
     }
   }
   // The wave issues its instructions in order and a matrix instruction occupies the matrix pipe for 32 cycles, in
@@ -787,12 +799,11 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     if (STAGES == 1 && c + 1 < nsteps) GDN_LDS_BARRIER();      // (B) done with the single stage
   }
   if constexpr (OUT) GDN_LDS_BARRIER();       // (A) of the extra step: the last V' is in LDS for the output wave
-  if (ht != nullptr) {
+  if (hto != nullptr) {
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        ht[(((int64_t)n * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col()] = S[kt][r];
+      for (int r = 0; r < 16; ++r) hto[(int64_t)(32 * kt + acc_row(r)) * ldt + v0 + acc_col()] = S[kt][r];
   }
 }
 
@@ -998,11 +1009,30 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
   // decided for the two-slab variant, the largest one: results must not depend on how many slabs a launch happens
   // to give a workgroup (a sequence computes the same bits alone and inside a packed batch)
   constexpr bool PRE = StatePre<T, DK, 2, STAGES, FUSE>::value && StatePre<T, DK, NWS, STAGES, FUSE>::value;
+  const int segs = state_segments(d, (int)sizeof(T));
+  if constexpr (FUSE && DK == 128 && NW == 4) {
+    if (segs > 1) {
+      float* starts = reinterpret_cast<float*>(ws + L.SEGH);
+      if (!skip_prep) {   // a refill finds the starts of the forward pass in the prep part
+        float* maps = reinterpret_cast<float*>(ws + L.SEGM);
+        auto kern = chunk_state_kernel<T, DK, 2, NLS, STAGES, false, PRE, false, true>;
+        constexpr int smem = StateSmem<T, DK, 2, STAGES, false, PRE>::bytes;
+        if (int e = set_lds(kern, smem)) return e;
+        GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
+                   (const T*)KAF, (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, beta, beta_same,
+                   (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T,
+                   d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr, segs);
+        GDN_LAUNCH(kKernStateFwd, st, (segment_chain_kernel<DK, false>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
+                   (const float*)maps, h0, starts, segs, d.Hv, d.V);
+      }
+      h0 = starts;
+    }
+  }
   auto launch_state = [&](auto kern, int smem, int waves, T* op) -> int {
     if (int e = set_lds(kern, smem)) return e;
-    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * d.Hv, d.V / (32 * NWS)), dim3(64 * waves), smem, st, (const T*)KAF,
+    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * waves), smem, st, (const T*)KAF,
                (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, beta, beta_same, h0, ht, VF, HF, op, cu,
-               (const int*)chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr);
+               (const int*)chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr, segs);
     return 0;
   };
   if constexpr (FUSE) {
@@ -1112,8 +1142,9 @@ int chunk_fwd_entry(const void* q, const void* k, const void* v, int64_t q_strid
   return chunk_fwd_launch<T_, DK_, NW_, NWS_, NLS_, ST_, FUSE_>(d, L, q, k, v, g, beta, beta_same, initial_state, cu_seqlens, o, final_state, \
                                                    ws, ws_state, skip_prep, scale, use_qk_l2norm, with_bwd, fn, st)
   const bool wide = (V % 128 == 0);
-  const bool solo = one_slab_per_workgroup(d, device_compute_units()) &&
-                    !(share_device && two_slabs_to_share_device(d, device_compute_units()));
+  const int segs = state_segments(d, dtype == 0 ? 4 : 2);
+  const bool solo = one_slab_per_workgroup(d, device_compute_units(), segs) &&
+                    !(share_device && two_slabs_to_share_device(d, device_compute_units(), segs));
   if (dtype == 1) {
     if (K == 128 && wide && solo) GDN_FWD(bf16_t, 128, 4, 1, 4, 2, true);
     if (K == 128 && wide) GDN_FWD(bf16_t, 128, 4, 2, 4, 2, true);

@@ -878,7 +878,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES, true>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
     GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, K2F, K1F, QBT,
-               Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale);
+               Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, 1);
   }
   {
     auto kern = chunk_bwd_local_kernel<T, DK, true>;

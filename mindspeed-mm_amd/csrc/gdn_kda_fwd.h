@@ -492,7 +492,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS * (1 + StateOutWaves<NWS>::value) + NLS)),
                smem, st, (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec,
                (const void*)bhat, 0, h0, ht, with_backward ? VF : (T*)nullptr, with_backward ? HF : (T*)nullptr, (T*)o, cu,
-               (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)QBT);
+               (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)QBT, 1);
     return (int)hipGetLastError();
   }
   {
@@ -501,7 +501,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     if (int e = set_lds(kern, smem)) return e;
     GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)K1F,
                (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const void*)bhat, 0, h0, ht, VF, HF,
-               (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)nullptr);
+               (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)nullptr, 1);
   }
   {
     auto kern = chunk_out_kernel<T, DK, NWO, false, T>;

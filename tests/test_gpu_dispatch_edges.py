@@ -68,3 +68,24 @@ def test_conv1d_edges(ops, dtype, B, T, D, W, cu):
 ])
 def test_recurrent_edges(ops, dtype, B, T, Hqk, Hv, K, V):
     P.check_recurrent(ops, "cuda", B, T, Hqk, Hv, K, V, dtype)
+
+
+@pytest.mark.parametrize("T,Hqk,Hv,V,cu", [
+    (4095, 1, 2, 128, None), (4096, 1, 2, 128, None), (4097, 2, 2, 128, None),   # a token short of being cut; uneven segments
+    (4159, 1, 3, 128, None),                                                     # a group of three heads, a short last chunk
+    (12400, 1, 2, 128, [0, 130, 130, 12400]),                                    # empty segments, an empty sequence
+])
+def test_recurrences_in_segments(ops, T, Hqk, Hv, V, cu):
+    """Few heads and long sequences: both recurrences run cut into segments.  Rebuilding the forward states in the backward
+    pass starts from the segments' saved states and has to give the same bits as keeping them."""
+    P.check_chunk(ops, "cuda", 1, T, Hqk, Hv, 128, V, BF, cu=cu, backward=True, h0_std=0.1)
+    x = P.gdn_inputs(1, T, Hqk, Hv, 128, V, BF, seed=3, N=len(cu) - 1 if cu else 1)
+    cu_t = torch.tensor(cu, dtype=torch.int64, device="cuda") if cu else None
+    got = []
+    for keep in (True, False):
+        leaf = [x[n].cuda().requires_grad_(True) for n in ("q", "k", "v", "g", "beta", "h0")]
+        o, ht = ops.chunk_gated_delta_rule(*leaf[:5], initial_state=leaf[5], output_final_state=True,
+                                           use_qk_l2norm_in_kernel=True, cu_seqlens=cu_t, skip_recompute=keep)
+        got.append((o, ht, *torch.autograd.grad([o, ht], leaf, [x["do"].cuda(), x["dht"].cuda()])))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
