@@ -119,6 +119,7 @@ struct KdaWorkspace {
                           //                        written when the recurrence forms the output itself or a backward pass follows
   int64_t VF;             // T [chunks,H,V/32,2]    v_new
   int64_t HF;             // T [chunks,H,V/32,K/32] state before each chunk
+  int64_t SEGH, SEGM;     // as in ChunkWorkspace; the reverse recurrence puts its own there
   int64_t fwd_bytes;
   // kept for a backward pass
   int64_t TMR;            // T [chunks,H,64,64]     Tm row-major, as rounded for the tiles
@@ -149,6 +150,9 @@ inline KdaWorkspace kda_workspace_layout(const ChunkDims& d, int elem_bytes) {
   w.QBT = take(nc * 64 * H * d.K * elem_bytes);
   w.VF = take(nc * 64 * H * d.V * elem_bytes);
   w.HF = take(nc * H * d.V * d.K * elem_bytes);
+  const int64_t P = state_segments(d, elem_bytes), seg = P > 1 ? (int64_t)d.N * H * d.K * 4 : 0;
+  w.SEGH = take(seg * P * d.V);
+  w.SEGM = take(seg * (P - 1) * (d.V + d.K));
   w.fwd_bytes = off;
   w.TMR = take(nc * H * 64 * 64 * elem_bytes);
   w.DVF = take(nc * 64 * H * d.V * elem_bytes);

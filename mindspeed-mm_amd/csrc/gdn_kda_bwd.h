@@ -873,12 +873,28 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
   T* DUMP = reinterpret_cast<T*>(ws + L.DUMP);
   float* DD = reinterpret_cast<float*>(ws + L.DD);
   float* PART = reinterpret_cast<float*>(ws + L.PART);
+  const int segs = state_segments(d, (int)sizeof(T));
+  if constexpr (sizeof(T) == 2 && DK == 128 && NWS == 1) {
+    if (segs > 1) {   // as in the forward pass, from the other end
+      float* maps = reinterpret_cast<float*>(ws + L.SEGM);
+      float* starts = reinterpret_cast<float*>(ws + L.SEGH);
+      auto kern = chunk_state_bwd_kernel<T, DK, 2, NLS, STAGES, true, true>;
+      constexpr int smem = StateBwdSmem<T, DK, 2, STAGES, true>::bytes;
+      if (int e = set_lds_b(kern, smem)) return e;
+      GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st, K2F, K1F,
+                 QBT, Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr,
+                 cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
+      GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
+                 (const float*)maps, dht, starts, segs, H, d.V);
+      dht = starts;
+    }
+  }
   {
     auto kern = chunk_state_bwd_kernel<T, DK, NWS, NLS, STAGES, true>;
     constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES, true>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
-    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, K2F, K1F, QBT,
-               Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, 1);
+    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, K2F, K1F, QBT,
+               Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
   }
   {
     auto kern = chunk_bwd_local_kernel<T, DK, true>;
@@ -938,7 +954,7 @@ extern "C" int gdn_kda_bwd(const void* q, const void* k, const void* v, const vo
 #define GDN_KDAB(T_, DK_, NWS_, NLS_, ST_)                                                                              \
   return kda_bwd_launch<T_, DK_, NWS_, NLS_, ST_>(d, L, q, k, v, g, A_log, dt_bias, cu_seqlens, d_o, d_final_state, dq, dk, dv, \
                                                   dg, dbeta, dA_log, ddt_bias, d_initial_state, ws, scale, fl, st)
-  const bool one_slab = one_slab_per_workgroup(d, device_compute_units());
+  const bool one_slab = one_slab_per_workgroup(d, device_compute_units(), state_segments(d, dtype == 0 ? 4 : 2));
   if (dtype == 1) {
     if (K == 128) {
       if (one_slab) GDN_KDAB(bf16_t, 128, 1, 4, 2);

@@ -484,15 +484,32 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
                dt_bias, cu, (const int*)chunk_offsets, bhat, dec, Ai, AQ, K1F, K2F, QB, QBT, TMR, keep ? rstd : nullptr,
                keep ? rstd + (int64_t)nc * 64 * H : nullptr, d.T, d.N, H, scale, fl);
   }
+  const int segs = state_segments(d, (int)sizeof(T));
+  if constexpr (FUSE && DK == 128) {
+    if (segs > 1) {   // sequences in segments: their maps, then the state each of them starts from (gdn_segments.h)
+      float* maps = reinterpret_cast<float*>(ws + L.SEGM);
+      float* starts = reinterpret_cast<float*>(ws + L.SEGH);
+      auto kern = chunk_state_kernel<T, DK, 2, NLS, STAGES, false, true, true, true>;
+      constexpr int smem = StateSmem<T, DK, 2, STAGES, false, true, true>::bytes;
+      if (int e = set_lds(kern, smem)) return e;
+      GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
+                 (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const void*)bhat, 0,
+                 (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H,
+                 d.V, scale, (int64_t)H * d.V, (const T*)nullptr, segs);
+      GDN_LAUNCH(kKernStateFwd, st, (segment_chain_kernel<DK, false>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
+                 (const float*)maps, h0, starts, segs, H, d.V);
+      h0 = starts;
+    }
+  }
   if constexpr (FUSE) {
     auto kern = chunk_state_kernel<T, DK, NWS, NLS, STAGES, true, true, true>;
     constexpr int smem = StateSmem<T, DK, NWS, STAGES, true, true, true>::bytes;
     if (int e = set_lds(kern, smem)) return e;
     // the per-chunk states and v_new leave the kernel only for a backward pass
-    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS * (1 + StateOutWaves<NWS>::value) + NLS)),
+    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * (NWS * (1 + StateOutWaves<NWS>::value) + NLS)),
                smem, st, (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec,
                (const void*)bhat, 0, h0, ht, with_backward ? VF : (T*)nullptr, with_backward ? HF : (T*)nullptr, (T*)o, cu,
-               (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)QBT, 1);
+               (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)QBT, segs);
     return (int)hipGetLastError();
   }
   {
@@ -608,7 +625,7 @@ extern "C" int gdn_kda_fwd(const void* q, const void* k, const void* v, const vo
   return kda_fwd_launch<T_, DK_, NWO_, NWS_, NLS_, ST_>(d, L, q, k, v, g, beta, A_log, dt_bias, initial_state, cu_seqlens, o, \
                                                         final_state, ws, scale, fl, with_bwd, st)
   // a CU per 32-column slab of the state while there are no more slabs than CUs (see one_slab_per_workgroup)
-  const bool one_slab = one_slab_per_workgroup(d, device_compute_units());
+  const bool one_slab = one_slab_per_workgroup(d, device_compute_units(), state_segments(d, dtype == 0 ? 4 : 2));
   if (dtype == 1) {
     if (K == 128) {
       if (one_slab) GDN_KDA(bf16_t, 128, 2, 1, 4, 2);

@@ -89,3 +89,8 @@ def test_recurrences_in_segments(ops, T, Hqk, Hv, V, cu):
         got.append((o, ht, *torch.autograd.grad([o, ht], leaf, [x["do"].cuda(), x["dht"].cuda()])))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,H,cu", [(4097, 2, None), (12400, 1, [0, 130, 130, 12400])])
+def test_kda_recurrences_in_segments(ops, T, H, cu):
+    P.check_kda(ops, "cuda", 1, T, H, 128, 128, BF, cu=cu, backward=True)
