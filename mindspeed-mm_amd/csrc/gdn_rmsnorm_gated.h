@@ -13,15 +13,17 @@
 
 namespace gdn {
 
-// 16-bit types: reciprocal instruction and one Newton step (within an ulp, a third of the instructions of the IEEE
-// division, which made these kernels bound by vector issue instead of memory); the exponent is capped where the
-// sigmoid leaves the normal range, so that the step never meets an infinity
+// 16-bit types: reciprocal instruction and one Newton step, which lands on the correctly rounded quotient but for ties (the
+// first estimate is off by an ulp, the step squares that), in two thirds of the instructions of the IEEE division, which
+// made these kernels bound by vector issue instead of memory.  The reciprocal is taken of a quarter of 1 + e^-p: the
+// instruction flushes subnormal results, which a quarter never has.  v_div_fixup sets 0 where e^-p overflowed (the step
+// gives 0 x inf there) and hands a NaN on.
 template <typename T> __device__ __forceinline__ float sigmoid_(float p) {
   if constexpr (sizeof(T) == 4) {
     return 1.f / (1.f + __expf(-p));
   } else {
-    const float d = 1.f + __expf(fminf(-p, 88.f)), r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.f), r, r);
+    const float d = fmaf(__expf(-p), 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(d), r4 = 0.25f * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, r, 1.f), r4, r4), d, 1.f);
   }
 }
 

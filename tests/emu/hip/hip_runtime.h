@@ -267,6 +267,10 @@ static emu::GdimProxy gridDim;
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_rcpf(x) (1.0f / (x))
 #define __builtin_amdgcn_rsqf(x) (1.0f / sqrtf(x))
+// v_div_fixup_f32: the quotient n/d as computed, or its exact special value
+inline float __builtin_amdgcn_div_fixupf(float quotient, float d, float n) {
+  return isfinite(d) && d != 0.f && isfinite(n) ? copysignf(fabsf(quotient), signbit(d) == signbit(n) ? 1.f : -1.f) : n / d;
+}
 #define __builtin_amdgcn_logf(x) log2f(x)
 #define GDN_WAVES_PER_SIMD(n)
 #define GDN_KEEP_HERE(x) ((void)0)

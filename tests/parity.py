@@ -522,3 +522,33 @@ def check_kda(ops, device, B, T, H, K, V, dtype, cu=None, seed=0, with_h0=True, 
             errs["d" + n] = _err("d" + n, leaves[n].grad, ref[n].grad, dtype,
                                  kda_param_tol(ref[n].grad, B * T) if param else BF16_ABS_GRAD)
     return errs
+
+
+def check_far_gates(ops, device, activation):
+    """Gates at and beyond the ends of the exponential, infinite and NaN: bf16 against the same call in float32 on the same
+    values.  NaN and infinities lie where float32 has them; y is off by three roundings to bf16 (2^-9 each, the first shared
+    with float32's xn taken unrounded) and half the smallest bf16; dgate, a product with 1 - s and 1 + gate (1 - s), besides
+    by 2 ulp of s times what multiplies it."""
+    low = torch.finfo(torch.bfloat16).min
+    gate = torch.tensor([float("nan"), float("inf"), -float("inf"), low, -low, -1e36, 1e36, -1e4, -200.0, -105.0, -89.0, -88.5,
+                         -88.0, -87.5, -87.0, -17.0, 0.0, 17.0, 88.0, 1e4], dtype=torch.bfloat16)
+    N = 128
+    gen = torch.Generator().manual_seed(5)
+    x = torch.randn(40, N, generator=gen).to(torch.bfloat16)
+    g = gate.repeat(40 * N // gate.numel()).view(N, 40).t().contiguous()      # every row meets every gate
+    d = torch.randn(40, N, generator=gen).to(torch.bfloat16)
+    res = []
+    for dt in (torch.bfloat16, torch.float32):
+        leaf = [t.to(device, dt).requires_grad_(True) for t in (x, g)]
+        y = ops.rms_norm_gated(*leaf, torch.ones(N, device=device, dtype=dt), 1e-6, activation)
+        res.append([t.detach().cpu().double() for t in (y, *torch.autograd.grad([y], leaf, [d.to(device, dt)]))])
+    (y, dx, dg), (ry, rdx, rdg) = res
+    gd, xn = g.double(), x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-6)
+    ulp_s = 2.0 ** -22 * (d.double() * xn).abs() * (1 + (gd.abs().clamp(max=200.0) if activation == "silu" else 0))
+    for name, got, ref, slack in (("y", y, ry, 0.0), ("dgate", dg, rdg, ulp_s)):
+        assert torch.equal(got.isnan(), ref.isnan()), (name, "NaN")
+        assert torch.equal(got.isinf(), ref.isinf()), (name, "inf")
+        ok = ref.isfinite()
+        off = (got - ref).abs() - 2.0 ** -7 * ref.abs() - slack - 2.0 ** -134
+        assert off[ok].max() <= 0, (name, gd[ok][off[ok].argmax()], got[ok][off[ok].argmax()], ref[ok][off[ok].argmax()])
+    assert torch.equal(dx.isnan(), rdx.isnan())      # a NaN of the gate reaches its whole row of dx
