@@ -68,6 +68,7 @@ int device_compute_units();   // defined with the forward launcher
 constexpr int kMinSegmentChunks = 16, kMinCutChunks = 64;
 inline int state_segments(const ChunkDims& d, int elem_bytes) {
   if (elem_bytes != 2 || d.K != 128 || d.V != 128) return 1;
+  if (d.N <= 0 || d.Hv <= 0) return 1;   // the size queries ask before any dimension has been checked
   const int64_t slabs = (int64_t)d.N * d.Hv * (d.V / 32), chunks = d.tokens() / 64 / d.N;
   const int64_t fit = device_compute_units() / slabs, p = fit < chunks / kMinSegmentChunks ? fit : chunks / kMinSegmentChunks;
   return p >= 3 && chunks >= kMinCutChunks ? (int)p : 1;

@@ -72,6 +72,19 @@ def test_chunk_packed_with_empty_sequences(ops, cu):
     P.check_chunk(ops, "cpu", 1, cu[-1], 1, 2, 64, 64, F32, cu=cu, backward=True, wrap=guarded, h0_std=0.1)
 
 
+@pytest.mark.parametrize("B,T,cu", [(0, 64, None), (1, 64, [0])])
+def test_no_sequence_is_refused(ops, B, T, cu):
+    """A batch without a sequence raises, in the sizes whose recurrences may be cut into segments too."""
+    x = P.kda_inputs(1, T, 2, 128, 128, BF, N=1)
+    r = {n: x[n][:B] for n in ("q", "k", "v", "g", "beta")}
+    cu_t = torch.tensor(cu, dtype=torch.int64) if cu else None
+    with pytest.raises(ValueError):
+        ops.chunk_gated_delta_rule(r["q"], r["k"], r["v"], r["g"][..., 0].float(), r["beta"], cu_seqlens=cu_t)
+    with pytest.raises(ValueError):
+        ops.chunk_kda(r["q"], r["k"], r["v"], r["g"].float(), r["beta"], cu_seqlens=cu_t, A_log=x["A_log"],
+                      dt_bias=x["dt_bias"], use_gate_in_kernel=True)
+
+
 @pytest.mark.parametrize("dtype,B,T,Hqk,Hv,K,V,cu", [
     (BF, 1, 200, 1, 2, 128, 128, None), (F32, 1, 140, 1, 2, 64, 64, [0, 5, 70, 140]),
 ])
