@@ -74,6 +74,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
   const SegmentRun run = segment_run(ns, MAP ? segs - 1 : segs, MAP ? 1 : 0, segs, cu, chunk_offsets, T_len);
   const int64_t bos = run.bos, chunk_base = run.chunk_base;
   const int len = run.len, nchunks = run.nchunks;
+  if (MAP && nchunks == 0) return;
   // MAP: the workgroup's columns belong to A, which starts from the identity and sees no dO
   const bool of_a = MAP && (int)blockIdx.y * (32 * NW) >= V;
   const int col0 = of_a ? 0 : (int)blockIdx.y * (32 * NW);   // of the rows of dO it reads
@@ -1014,7 +1015,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
                    (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, beta, beta_same,
                    (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, segs);
         GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
-                   (const float*)maps, dht, starts, segs, d.Hv, d.V);
+                   (const float*)maps, dht, starts, cu, d.T, segs, d.Hv, d.V);
         dht = starts;
       }
     }

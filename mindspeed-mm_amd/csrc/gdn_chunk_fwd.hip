@@ -386,8 +386,8 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
                          ? nullptr : ht + ((int64_t)(MAP ? ns : run.n) * Hv + h) * DK * ldt;
   // number of barriers every wave passes: one per chunk, plus one that hands the last V' to the output waves
   const int nsteps = nchunks + (OUT ? 1 : 0);
-  if (nchunks == 0) {   // an empty sequence: its final state is its initial state
-    if (wave < NW && hto != nullptr) {
+  if (nchunks == 0) {   // an empty sequence: its final state is its initial state; an empty segment has no map
+    if (!MAP && wave < NW && hto != nullptr) {
       const int col = 32 * (blockIdx.y * NW + wave) + acc_col();
       for (int kt = 0; kt < NKT; ++kt)
         for (int r = 0; r < 16; ++r) {
@@ -1023,7 +1023,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
                    (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T,
                    d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr, segs);
         GDN_LAUNCH(kKernStateFwd, st, (segment_chain_kernel<DK, false>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
-                   (const float*)maps, h0, starts, segs, d.Hv, d.V);
+                   (const float*)maps, h0, starts, cu, d.T, segs, d.Hv, d.V);
       }
       h0 = starts;
     }

@@ -885,7 +885,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
                  QBT, Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr,
                  cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
       GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
-                 (const float*)maps, dht, starts, segs, H, d.V);
+                 (const float*)maps, dht, starts, cu, d.T, segs, H, d.V);
       dht = starts;
     }
   }

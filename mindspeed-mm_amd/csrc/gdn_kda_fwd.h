@@ -497,7 +497,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
                  (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H,
                  d.V, scale, (int64_t)H * d.V, (const T*)nullptr, segs);
       GDN_LAUNCH(kKernStateFwd, st, (segment_chain_kernel<DK, false>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
-                 (const float*)maps, h0, starts, segs, H, d.V);
+                 (const float*)maps, h0, starts, cu, d.T, segs, H, d.V);
       h0 = starts;
     }
   }

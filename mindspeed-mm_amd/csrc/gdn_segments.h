@@ -17,6 +17,9 @@
 
 namespace gdn {
 
+// chunks to a segment of a sequence of `nchunks`
+__device__ __forceinline__ int segment_chunks(int nchunks, int segs) { return (nchunks + segs - 1) / segs; }
+
 // the run of chunks a workgroup of a recurrence kernel walks
 struct SegmentRun {
   int n, p;            // sequence, segment
@@ -35,7 +38,7 @@ __device__ __forceinline__ SegmentRun segment_run(int ns, int per_seq, int first
   s.nchunks = (s.len + kChunk - 1) / kChunk;
   s.chunk_base = cu ? chunk_offsets[s.n] : (int64_t)s.n * ((T_len + kChunk - 1) / kChunk);
   if (segs > 1) {   // equal runs, the last ones of a short sequence shorter or empty
-    const int per = (s.nchunks + segs - 1) / segs, c0 = imin(s.p * per, s.nchunks);
+    const int per = segment_chunks(s.nchunks, segs), c0 = imin(s.p * per, s.nchunks);
     s.nchunks = imin(per, s.nchunks - c0);
     s.len = s.nchunks > 0 ? imin(s.len - c0 * kChunk, s.nchunks * kChunk) : 0;
     s.bos += (int64_t)c0 * kChunk;
@@ -46,18 +49,23 @@ __device__ __forceinline__ SegmentRun segment_run(int ns, int per_seq, int first
 
 // start[p + 1] = A_p start[p] + B_p along the segments of a sequence (REVERSE: start[p - 1] = A_p start[p] + B_p), from
 // `first` (null: zero).  map: f32 [N, P-1, Hv, K, V + K], the segments 0 .. P-2 (REVERSE: 1 .. P-1); start: f32
-// [N, P, Hv, K, V].  A workgroup owns 16 columns of one head's states, wave w their rows 16 w .. 16 w + 15.  Bound by
-// latency: a step is 32 fp32 matrix instructions per wave behind one barrier, its map requested a step ahead (3.2 us a
-// step; requested two steps ahead it takes the same).
+// [N, P, Hv, K, V].  An empty segment has no map: the state passes it as it is, infinities included (0 x inf in a product
+// with the identity would be NaN).  A workgroup owns 16 columns of one head's states, wave w their rows
+// 16 w .. 16 w + 15.  Bound by latency: a step is 32 fp32 matrix instructions per wave behind one barrier, its map
+// requested a step ahead (3.2 us a step; requested two steps ahead it takes the same).
 template <int DK, bool REVERSE>
 __global__ __launch_bounds__(4 * DK) void segment_chain_kernel(const float* __restrict__ map, const float* __restrict__ first,
-                                                               float* __restrict__ start, int segs, int Hv, int V) {
+                                                               float* __restrict__ start, const int64_t* __restrict__ cu,
+                                                               int T_len, int segs, int Hv, int V) {
   constexpr int LD = DK + 4, NM = DK / 16;
   __shared__ __align__(16) float hs[2][16 * LD];   // the running state, column-major
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, j = lane >> 4;
   const int n = blockIdx.x / Hv, h = blockIdx.x % Hv, v0 = 16 * blockIdx.y, ld = V + DK;
   const int row0 = 16 * wave + 4 * j;              // the lane's rows row0 .. row0 + 3 of column c
   auto start_at = [&](int p) { return start + ((((int64_t)n * segs + p) * Hv + h) * DK + row0) * V + v0 + c; };
+  const int nchunks = ((cu ? (int)(cu[n + 1] - cu[n]) : T_len) + kChunk - 1) / kChunk;
+  const int live = nchunks > 0 ? (nchunks - 1) / segment_chunks(nchunks, segs) + 1 : 0;   // segments with chunks
+  auto applies = [&](int s) { return s < segs && (REVERSE ? segs - s : s - 1) < live; };
   f32x4 A[NM], B, S;
   auto request = [&](int s) {                      // the map applied in step s = 1 .. segs - 1
     const int i = n * (segs - 1) + (REVERSE ? segs - 1 - s : s - 1);
@@ -67,7 +75,7 @@ __global__ __launch_bounds__(4 * DK) void segment_chain_kernel(const float* __re
 #pragma unroll
     for (int r = 0; r < 4; ++r) B[r] = m[(int64_t)(row0 + r) * ld + v0 + c];
   };
-  request(1);
+  if (applies(1)) request(1);
 #pragma unroll
   for (int r = 0; r < 4; ++r) S[r] = first ? first[(((int64_t)n * Hv + h) * DK + row0 + r) * V + v0 + c] : 0.f;
   for (int s = 1;; ++s) {
@@ -75,6 +83,10 @@ __global__ __launch_bounds__(4 * DK) void segment_chain_kernel(const float* __re
 #pragma unroll
     for (int r = 0; r < 4; ++r) out[(int64_t)r * V] = S[r];
     if (s == segs) break;
+    if (!applies(s)) {
+      if (applies(s + 1)) request(s + 1);
+      continue;
+    }
     float* hb = hs[s & 1];
     *reinterpret_cast<f32x4*>(hb + c * LD + row0) = S;
     __syncthreads();
@@ -82,7 +94,7 @@ __global__ __launch_bounds__(4 * DK) void segment_chain_kernel(const float* __re
     f32x4 a0 = B, a1 = {0.f, 0.f, 0.f, 0.f}, now[NM];
 #pragma unroll
     for (int k = 0; k < NM; ++k) now[k] = A[k];
-    if (s + 1 < segs) request(s + 1);
+    if (applies(s + 1)) request(s + 1);
 #pragma unroll
     for (int k = 0; k < NM; ++k) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(hb + c * LD + 16 * k + 4 * j);

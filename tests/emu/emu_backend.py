@@ -5,6 +5,7 @@ guard pages instead of GPU faults.  The shipped package never imports this modul
 import contextlib
 import ctypes
 import os
+import shutil
 import sys
 
 import torch
@@ -15,21 +16,33 @@ for p in (ROOT, os.path.join(ROOT, "mindspeed-mm_amd")):
     if p not in sys.path:
         sys.path.insert(0, p)
 
-from mindspeed_mm_amd._lib import GdnLibrary  # noqa: E402
+from mindspeed_mm_amd._lib import DTYPE_CODE, GdnLibrary  # noqa: E402
 from mindspeed_mm_amd.ops import GdnOps  # noqa: E402
 
-_ops = None
+_ops = {}
 
 
-def emu_ops() -> GdnOps:
-    global _ops
-    if _ops is None:
+def emu_ops(compute_units=None) -> GdnOps:
+    """The operators on the CPU build.  compute_units: on a copy of the library whose device has that many (the launchers
+    ask once per library); results are the same, the choice of launches is that of a device of this size."""
+    if compute_units not in _ops:
         from . import build_emu
         path = build_emu.build()
-        _ops = GdnOps(GdnLibrary(path, "cpu"))
-        _ops.lib.cdll.emu_guard_alloc.restype = ctypes.c_void_p
-        _ops.lib.cdll.emu_guard_alloc.argtypes = [ctypes.c_size_t, ctypes.c_int]
-    return _ops
+        if compute_units is not None:
+            copy = f"{path[:-3]}_{compute_units}.so"
+            shutil.copyfile(path, copy)
+            path = copy
+        ops = GdnOps(GdnLibrary(path, "cpu"))
+        ops.lib.cdll.emu_guard_alloc.restype = ctypes.c_void_p
+        ops.lib.cdll.emu_guard_alloc.argtypes = [ctypes.c_size_t, ctypes.c_int]
+        if compute_units is not None:
+            os.environ["GDN_EMU_COMPUTE_UNITS"] = str(compute_units)
+            try:
+                ops.lib.gdn_chunk_workspace_bytes(1, 64, 1, 1, 1, 128, 128, DTYPE_CODE[torch.bfloat16], 0)
+            finally:
+                del os.environ["GDN_EMU_COMPUTE_UNITS"]
+        _ops[compute_units] = ops
+    return _ops[compute_units]
 
 
 _keep = []

@@ -50,8 +50,13 @@ static inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 #define HIP_SYMBOL(x) (&(x))
 static inline hipError_t hipGetSymbolAddress(void** p, const void* sym) { *p = const_cast<void*>(sym); return hipSuccess; }
 enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount = 63 };
-// a small "device" so that the test shapes exercise both the one-slab-per-workgroup and the shared-tile launches
-static inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 8; return hipSuccess; }
+// a small "device" so that the test shapes exercise both the one-slab-per-workgroup and the shared-tile launches;
+// GDN_EMU_COMPUTE_UNITS: another size (a library asks once)
+static inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
+  const char* n = getenv("GDN_EMU_COMPUTE_UNITS");
+  *v = n ? atoi(n) : 8;
+  return hipSuccess;
+}
 typedef void* hipEvent_t;
 static inline hipError_t hipEventCreate(hipEvent_t* e) { *e = nullptr; return hipSuccess; }
 static inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }

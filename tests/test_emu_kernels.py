@@ -339,3 +339,32 @@ def test_kda_intermediate_states(ops, dtype, B, T, H, K, V, cu, kw):
     """The states at chunk entries, written out from the workspace's tiles in both layouts."""
     errs = P.check_kda(ops, "cpu", B, T, H, K, V, dtype, cu=cu, wrap=guarded, h0_std=0.1, states=True, **kw)
     assert "h" in errs
+
+
+@pytest.fixture(scope="module")
+def ops256():
+    """A device of 256 compute units: few heads and 64 chunks a sequence make the recurrences run cut into segments."""
+    return emu_ops(256)
+
+
+@pytest.mark.parametrize("kda", [False, True])
+def test_cut_launch_hands_the_state_of_an_empty_sequence_through(ops256, kda):
+    """An empty sequence beside a long one: its final state is its initial state and its initial state's gradient the final
+    state's, bit for bit, infinities and NaN included."""
+    T = 8193
+    x = (P.kda_inputs(1, T, 1, 128, 128, BF, N=2) if kda else P.gdn_inputs(1, T, 1, 1, 128, 128, BF, N=2))
+    h0, dht = x["h0"].clone(), torch.randn(x["h0"].shape, generator=torch.Generator().manual_seed(1))
+    h0[0, 0, 3, 5], h0[0, 0, 7, 9], dht[0, 0, 2, 11] = float("inf"), float("nan"), -float("inf")
+    leaf = {n: guarded(x[n]).requires_grad_(True) for n in ("q", "k", "v", "g", "beta")}
+    h0 = guarded(h0).requires_grad_(True)
+    kw = dict(initial_state=h0, output_final_state=True, use_qk_l2norm_in_kernel=True,
+              cu_seqlens=torch.tensor([0, 0, T], dtype=torch.int64))
+    if kda:
+        o, ht = ops256.chunk_kda(*leaf.values(), use_gate_in_kernel=True, use_beta_sigmoid_in_kernel=True,
+                                 A_log=guarded(x["A_log"]), dt_bias=guarded(x["dt_bias"]), **kw)
+    else:
+        o, ht = ops256.chunk_gated_delta_rule(*leaf.values(), **kw)
+    dh0, = torch.autograd.grad([o, ht], [h0], [torch.ones_like(o), dht])
+    assert torch.equal(ht[0].view(torch.int32), h0[0].view(torch.int32))
+    assert torch.equal(dh0[0].view(torch.int32), dht[0].view(torch.int32))
+    assert ht[1].isfinite().all() and dh0[1].isfinite().all()
