@@ -146,7 +146,8 @@ int gdn_recurrent_fwd_qkv(const void* qkv, int64_t token_stride, const void* a, 
  * replaces causal_conv1d_fwd_impl / causal_conv1d_bwd_impl / causal_conv1d_update_states,
  * mindspeed_mm/fsdp/ops/gdn/triton/convolution.py:517-588, 591-714, 762-787.
  * x,y,residual,dy,dx [B,T,D]; weight [W,D]; bias [D]; states [N,D,W]; activation 0 = none, 1 = SiLU.
- * W in 1..8; D % 8 == 0 (D % 4 for fp32).  dw [W,D] and db [D] are fp32.
+ * W in 1..8; D % 8 == 0 (D % 4 for fp32).  dw [W,D] and db [D] are fp32.  final_state may be initial_state itself; no
+ * other output may overlap an input.
  */
 int gdn_conv1d_fwd(const void* x, const void* weight, const void* bias, const void* residual,
                    const void* initial_state, const int64_t* cu_seqlens, void* y, void* final_state, int B, int T,

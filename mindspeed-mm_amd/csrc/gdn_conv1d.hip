@@ -140,11 +140,12 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) vo
   }
 }
 
-// final_state[n,d,w] = x[T_n - W + w] (falls back to the initial state / zero for T_n < W).  Packed input only, where a
-// sequence may be empty; the forward kernel writes the state of a dense batch itself.
+// final_state[n,d,w] = x[T_n - W + w] (falls back to the initial state / zero for T_n < W).  For packed input, where a
+// sequence may be empty, and where the state is updated in place (a thread reads ahead of what it writes, and only its own
+// channel); otherwise the forward kernel writes the state itself.
 template <typename T>
-__global__ void conv1d_final_state_kernel(const T* __restrict__ x, const T* __restrict__ init,
-                                          const int64_t* __restrict__ cu, T* __restrict__ fs, int T_len, int N, int D,
+__global__ void conv1d_final_state_kernel(const T* __restrict__ x, const T* init,
+                                          const int64_t* __restrict__ cu, T* fs, int T_len, int N, int D,
                                           int W) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (int64_t)N * D) return;
@@ -501,7 +502,9 @@ template <typename T> struct ConvLaunch {
     const int64_t nblocks = (int64_t)((D / V + kConvThreads - 1) / kConvThreads) * ((total + TT - 1) / TT);
     if (nblocks > 0x7fffffffLL) return -3;
     dim3 grid((unsigned)nblocks);
-    const bool fs_inside = cu == nullptr && total > 0;   // every sequence has a last token
+    // every sequence of a dense batch has a last token, whose tile can write the final state -- but not over the initial
+    // state, which the sequence's first tile may still be reading
+    const bool fs_inside = cu == nullptr && total > 0 && fs != init;
     if (total > 0) {
       auto launch = [&](auto kern) {
         GDN_LAUNCH(kKernConvFwd, st, kern, grid, dim3(kConvThreads), 0, st, (const T*)x, (const T*)weight, (const T*)bias,

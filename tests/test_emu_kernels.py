@@ -6,6 +6,7 @@ GPU fault.  The shipped library is not involved: these tests prove indexing/sync
 import pytest
 import torch
 
+from mindspeed_mm_amd._lib import kernel_timings, ptr
 from tests import parity as P
 from tests.emu.emu_backend import emu_ops, guarded, guarded_outputs
 
@@ -103,6 +104,24 @@ def test_chunk_backward_without_initial_state(ops):
 def test_conv1d(ops, dtype, B, T, D, W, cu):
     P.check_conv(ops, "cpu", B, T, D, W, dtype, cu=cu, residual=True, wrap=guarded)
     P.check_conv(ops, "cpu", B, T, D, W, dtype, cu=cu, bias=False, state=False, activation=None, wrap=guarded)
+
+
+@pytest.mark.parametrize("T", [2, 100])
+def test_conv1d_state_updated_in_place(ops, T):
+    """The C entry with final_state = initial_state: the state is written by a launch of its own, behind the one whose
+    first tiles read it."""
+    B, D, W = 2, 16, 4
+    gen = torch.Generator().manual_seed(0)
+    x, w = torch.randn(B, T, D, generator=gen), torch.randn(W, D, generator=gen)
+    h0 = torch.randn(B, D, W, generator=gen)
+    want_y, want_fs = ops.causal_conv1d(x, w, initial_state=h0, output_final_state=True)
+    y, lib = torch.empty_like(x), ops.lib
+    lib.gdn_profile_enable(1)
+    lib.check(lib.gdn_conv1d_fwd(ptr(x), ptr(w), None, None, ptr(h0), None, ptr(y), ptr(h0), B, T, B, D, W, 0, 0, None), "conv")
+    launched = kernel_timings(lib)
+    lib.gdn_profile_enable(0)
+    assert torch.equal(y, want_y) and torch.equal(h0, want_fs)
+    assert launched["conv1d_final_state_kernel"][1] == 1
 
 
 @pytest.mark.parametrize("dtype,B,T,D,W", [(F32, 2, 1, 16, 4), (BF, 3, 5, 8, 4), (F32, 1, 3, 8, 2)])
