@@ -29,22 +29,13 @@ struct RecurrentGates {   // either g, beta (fp32 [tokens,Hv]) or the projection
   const void* dt_bias;
 };
 
-// n consecutive values, n * sizeof(T) <= 16 bytes, in one load
+// n consecutive values, n * sizeof(T) <= 16 bytes, in one load; aligned as their type is, not as the load is wide
 template <typename T, int n> __device__ __forceinline__ void load_run(float* dst, const T* p) {
   constexpr int bytes = n * (int)sizeof(T);
+  static_assert(bytes == 2 || bytes == 4 || bytes == 8 || bytes == 16, "2 to 16 bytes");
   float f[Elem<T>::kVec];
   Vec16<T> x = zero16<T>();
-  if constexpr (bytes == 16) {
-    x = ld16(p);
-  } else if constexpr (bytes == 8) {
-    const u32x2 w = *reinterpret_cast<const u32x2*>(p);
-    x.raw[0] = w[0]; x.raw[1] = w[1];
-  } else if constexpr (bytes == 4) {
-    x.raw[0] = *reinterpret_cast<const uint32_t*>(p);
-  } else {
-    static_assert(bytes == 2, "2 to 16 bytes");
-    x.raw[0] = *reinterpret_cast<const uint16_t*>(p);
-  }
+  __builtin_memcpy(&x.raw, p, bytes);
   unpack16<T>(x, f);
 #pragma unroll
   for (int e = 0; e < n; ++e) dst[e] = f[e];

@@ -34,6 +34,21 @@ def test_recurrent(ops, dtype, B, T, Hqk, Hv, K, V):
     P.check_recurrent(ops, "cpu", B, T, Hqk, Hv, K, V, dtype, l2=False, with_state=False, wrap=guarded)
 
 
+@pytest.mark.parametrize("dtype,K", [(BF, 64), (BF, 128), (BF, 256), (F32, 128)])
+def test_recurrent_rows_on_any_element(ops, dtype, K):
+    """q and k may start on any element: the kernel's loads are wider than one, but promise no more alignment than that."""
+    x = P.gdn_inputs(2, 2, 1, 2, K, 64, dtype, seed=2)
+    want = ops.fused_recurrent_gated_delta_rule(*(x[n] for n in ("q", "k", "v", "g", "beta")), initial_state=x["h0"],
+                                                output_final_state=True, use_qk_l2norm_in_kernel=True)
+    for n in ("q", "k"):
+        x[n] = torch.cat([x[n].flatten()[:1], x[n].flatten()])[1:].view(x[n].shape)
+        assert x[n].data_ptr() % 4 or dtype == F32 and x[n].data_ptr() % 8
+    got = ops.fused_recurrent_gated_delta_rule(*(x[n] for n in ("q", "k", "v", "g", "beta")), initial_state=x["h0"],
+                                               output_final_state=True, use_qk_l2norm_in_kernel=True)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,T,cu,Hqk,Hv,K,V", [
     (F32, 12, [0, 3, 3, 8, 12], 1, 2, 64, 64), (BF, 9, [0, 1, 6], 1, 2, 128, 64),
 ])
