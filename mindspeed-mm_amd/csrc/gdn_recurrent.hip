@@ -44,35 +44,47 @@ template <typename T, int n> __device__ __forceinline__ void load_run(float* dst
 // A workgroup's slab is BV columns of one state, 4 of them per thread in RPT rows.  Everything a token needs is requested
 // at once: the slab, k and q (each wave normalises them by itself and keeps them in a part of the LDS of its own), v and
 // the gates; the only barrier of a token lies between the waves' partial sums over the rows.
+// The sums over the rows run in one order whatever BV is, so that a sequence's bits do not depend on the size of its batch,
+// which decides BV: 32 chains of the rows r, r + 32, ..., r = g + 8 m; then over m = 0 .. 3 in pairs, over the two g of a
+// wave, over the waves.  A thread holds BV / 32 of the m; the others and the second g are lanes of its wave.
 // waves per SIMD the registers have to allow: left to itself the compiler takes 280 for some of the smaller slabs
-constexpr int recurrent_waves(int dk, int bv) { return dk * bv < 128 * 128 ? 4 : 1; }
+constexpr int kRecurrentWaves = 4;
 
 template <typename T, typename TP, int DK, int BV, bool STREAM>
-__global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel(
+__global__ __launch_bounds__(256, kRecurrentWaves) void recurrent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int64_t sq, int64_t sk, int64_t sv,
     RecurrentGates gates, const float* state_in, float* state_out, T* __restrict__ o, const int64_t* __restrict__ cu,
     int T_len, int Hqk, int Hv, int V, float scale, int use_l2norm) {
   constexpr int CG = BV / 4;            // column groups (4 fp32 = 16 bytes each)
-  constexpr int NRG = kThreads / CG;    // row groups
-  constexpr int RPT = DK / NRG;         // state rows held by a thread: rg, rg + NRG, ...
+  constexpr int MC = BV / 32;           // chains of rows held by a thread
+  constexpr int NJ = DK / 32;           // rows of a chain
   constexpr int EPL = DK / 64;          // elements of k and q per lane for the norms
-  static_assert(DK % NRG == 0 && RPT >= 1 && CG <= 64, "tile shape");
+  static_assert(MC == 1 || MC == 2 || MC == 4, "tile shape");
   __shared__ float red[2][4][CG][8], kq_rows[4][DK][2];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int cg = tid % CG, rg = tid / CG;
+  const int cg = tid % CG, lrow = lane / CG;
+  const int row0 = 2 * wave + lrow / (4 / MC) + 8 * MC * (lrow % (4 / MC));
+  // the thread's rows are row0 + 32 j + 8 m
   // the slabs of a state are neighbours in the launch order: what is in flight then stays close together in memory
   const int nslab = V / BV, bh = blockIdx.x / nslab, b = bh / Hv, h = bh % Hv, hq = h / (Hv / Hqk);
   const int v0 = (blockIdx.x % nslab) * BV + cg * 4;
-  const int64_t sbase = ((int64_t)bh * DK + rg) * V + v0;
+  const int64_t sbase = ((int64_t)bh * DK + row0) * V + v0;
 
-  f32x4 S[RPT];
+  f32x4 S[NJ][MC];
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(state_in + sbase + (int64_t)(NRG * i) * V);
-    if (state_in == nullptr) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    else if constexpr (STREAM) S[i] = __builtin_nontemporal_load(p);
-    else S[i] = *p;
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int m = 0; m < MC; ++m) S[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (state_in != nullptr) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int m = 0; m < MC; ++m) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(state_in + sbase + (int64_t)(32 * j + 8 * m) * V);
+        if constexpr (STREAM) S[j][m] = __builtin_nontemporal_load(p);
+        else S[j][m] = *p;
+      }
   }
 
   // packed input (cu given): "sequence" b owns the tokens cu[b] .. cu[b+1] of the one batch row
@@ -118,13 +130,23 @@ __global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel
     GDN_WAVE_LDS_SYNC();
 
     // ---- one pass over the slab: S_old^T k and S_old^T q ----
-    float pk[4] = {0.f, 0.f, 0.f, 0.f}, pq[4] = {0.f, 0.f, 0.f, 0.f};
+    f32x4 ck[MC], cq[MC];
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const float kk = kw[rg + NRG * i][0], qq = kw[rg + NRG * i][1];
+    for (int m = 0; m < MC; ++m) ck[m] = cq[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < 4; ++c) { pk[c] += S[i][c] * kk; pq[c] += S[i][c] * qq; }
-    }
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int m = 0; m < MC; ++m) {
+        const float kk = kw[row0 + 32 * j + 8 * m][0], qq = kw[row0 + 32 * j + 8 * m][1];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          ck[m][c] = fmaf(S[j][m][c], kk, ck[m][c]);
+          cq[m][c] = fmaf(S[j][m][c], qq, cq[m][c]);
+        }
+      }
+    f32x4 pk = ck[0], pq = cq[0];
+    if constexpr (MC == 2) { pk = ck[0] + ck[1]; pq = cq[0] + cq[1]; }
+    if constexpr (MC == 4) { pk = (ck[0] + ck[1]) + (ck[2] + ck[3]); pq = (cq[0] + cq[1]) + (cq[2] + cq[3]); }
 #pragma unroll
     for (int m = CG; m < 64; m <<= 1) {
 #pragma unroll
@@ -141,17 +163,19 @@ __global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel
     for (int c = 0; c < 4; ++c) {
       const float skv = rd[0][cg][c] + rd[1][cg][c] + rd[2][cg][c] + rd[3][cg][c];
       const float sqv = rd[0][cg][4 + c] + rd[1][cg][4 + c] + rd[2][cg][4 + c] + rd[3][cg][4 + c];
-      delta[c] = bt * (vv[c] - eg * skv);
-      ov[c] = eg * sqv + kq * delta[c];
+      delta[c] = bt * fmaf(-eg, skv, vv[c]);
+      ov[c] = fmaf(eg, sqv, kq * delta[c]);
     }
     // ---- rank-1 update in registers ----
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const float kk = kw[rg + NRG * i][0];
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) S[i][c] = eg * S[i][c] + kk * delta[c];
-    }
-    if (rg == 0) {
+      for (int m = 0; m < MC; ++m) {
+        const float kk = kw[row0 + 32 * j + 8 * m][0];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) S[j][m][c] = fmaf(kk, delta[c], eg * S[j][m][c]);
+      }
+    if (wave == 0 && lrow == 0) {
       T* op = o + (tok * Hv + h) * V + v0;
       if constexpr (sizeof(T) == 4) {
         *reinterpret_cast<f32x4*>(op) = f32x4{ov[0], ov[1], ov[2], ov[3]};
@@ -162,9 +186,12 @@ __global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel
   }
 
   if (state_out != nullptr) {
+    GDN_WAIT_VMEM();   // once, where the compiler waits before every store (195 -> 184 us at 256 sequences of 32 heads)
 #pragma unroll
-    for (int i = 0; i < RPT; ++i)   // streaming store: the slab is not read again by this kernel
-      __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(state_out + sbase + (int64_t)(NRG * i) * V));
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int m = 0; m < MC; ++m)   // streaming store: the slab is not read again by this kernel
+        __builtin_nontemporal_store(S[j][m], reinterpret_cast<f32x4*>(state_out + sbase + (int64_t)(32 * j + 8 * m) * V));
   }
 }
 

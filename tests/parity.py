@@ -552,3 +552,16 @@ def check_far_gates(ops, device, activation):
         off = (got - ref).abs() - 2.0 ** -7 * ref.abs() - slack - 2.0 ** -134
         assert off[ok].max() <= 0, (name, gd[ok][off[ok].argmax()], got[ok][off[ok].argmax()], ref[ok][off[ok].argmax()])
     assert torch.equal(dx.isnan(), rdx.isnan())      # a NaN of the gate reaches its whole row of dx
+
+
+def check_recurrent_batch_bits(ops, device, batches, Hqk, Hv, K, V, dtype):
+    """A sequence's decode outputs and state are the same bits whatever else is in its batch."""
+    x = {n: t.to(device) for n, t in gdn_inputs(max(batches), 2, Hqk, Hv, K, V, dtype, seed=4).items()}
+    first = None
+    for B in batches:
+        o, s = ops.fused_recurrent_gated_delta_rule(*(x[n][:B].contiguous() for n in ("q", "k", "v", "g", "beta")),
+                                                    initial_state=x["h0"][:B].contiguous(), output_final_state=True,
+                                                    use_qk_l2norm_in_kernel=True)
+        if first is None:
+            first = (o[0], s[0])
+        assert torch.equal(o[0], first[0]) and torch.equal(s[0], first[1]), B

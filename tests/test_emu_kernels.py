@@ -49,6 +49,11 @@ def test_recurrent_rows_on_any_element(ops, dtype, K):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype,K,V", [(BF, 128, 128), (BF, 128, 192), (F32, 64, 128), (BF, 256, 128)])
+def test_recurrent_bits_do_not_depend_on_the_batch(ops, dtype, K, V):
+    P.check_recurrent_batch_bits(ops, "cpu", (1, 9), 1, 1, K, V, dtype)   # fewer and more states than compute units
+
+
 @pytest.mark.parametrize("dtype,T,cu,Hqk,Hv,K,V", [
     (F32, 12, [0, 3, 3, 8, 12], 1, 2, 64, 64), (BF, 9, [0, 1, 6], 1, 2, 128, 64),
 ])

@@ -72,6 +72,14 @@ def test_recurrent_edges(ops, dtype, B, T, Hqk, Hv, K, V):
     P.check_recurrent(ops, "cuda", B, T, Hqk, Hv, K, V, dtype)
 
 
+@pytest.mark.parametrize("dtype,K,V,batches", [
+    (BF, 128, 128, (1, 9, 17, 129)), (F32, 128, 128, (1, 9)), (BF, 128, 64, (1, 9, 40, 260)), (BF, 64, 128, (1, 33, 258)),
+    (BF, 256, 128, (1, 9, 20, 66)),
+])
+def test_recurrent_bits_do_not_depend_on_the_batch(ops, dtype, K, V, batches):
+    P.check_recurrent_batch_bits(ops, "cuda", batches, 16, 32, K, V, dtype)
+
+
 @pytest.mark.parametrize("T,Hqk,Hv,V,cu", [
     (4095, 1, 2, 128, None), (4096, 1, 2, 128, None), (4097, 2, 2, 128, None),   # a token short of being cut; uneven segments
     (4159, 1, 3, 128, None),                                                     # a group of three heads, a short last chunk
