@@ -3,9 +3,10 @@
 // (reference math: mindspeed_mm/fsdp/models/qwen3_5/modeling_qwen3_5.py:478-517).
 //
 // The kernel is bound by streaming the fp32 state [K,V] (64 KB at K=V=128) through HBM once in, once
-// out (a batch of 256 with 32 heads: 1.08 GB in 190 us = 5.7 TB/s on states that no cache holds; 217 us with the loads and
-// the launch order left to themselves).  One workgroup of 256
-// threads owns a [K, BV] column slab of one state; the slab lives in registers for all T tokens of the call.  With S_old the state before the token,
+// out (a batch of 256 with 32 heads: 1.08 GB in 183 us = 5.9 TB/s on states that no cache holds, 162 us = 6.7 TB/s where the
+// memory-side cache holds a part of them; 217 and 163 us with the loads left to themselves).  One workgroup of 256 threads
+// owns a [K, BV] column slab of one state; the slab lives in registers for all T tokens of the call.  With S_old the state
+// before the token,
 //     S^T k = e^g (S_old^T k),   S^T q = e^g (S_old^T q) + (k.q) delta
 // so both contractions are taken in ONE pass over the registers, then the rank-1 update is applied.
 // No MFMA: 6 flop per 8 bytes of state traffic, far below the matrix-core ridge.
@@ -48,10 +49,18 @@ template <typename T, int n> __device__ __forceinline__ void load_run(float* dst
 // which decides BV: 32 chains of the rows r, r + 32, ..., r = g + 8 m; then over m = 0 .. 3 in pairs, over the two g of a
 // wave, over the waves.  A thread holds BV / 32 of the m; the others and the second g are lanes of its wave.
 // waves per SIMD the registers have to allow: left to itself the compiler takes 280 for some of the smaller slabs
-constexpr int kRecurrentWaves = 4;
+constexpr int recurrent_waves(int dk, int bv) { return dk * bv <= 128 * 128 ? 4 : 2; }
 
-template <typename T, typename TP, int DK, int BV, bool STREAM>
-__global__ __launch_bounds__(256, kRecurrentWaves) void recurrent_kernel(
+// How the states are loaded.  kStream passes by the caches, which hold states that fit them (kCached) from one step to the
+// next.  Larger ones pass through the 256 MB memory-side cache for nothing and cost bandwidth on their way; kMixed leaves it
+// a fixed part of them, of every kKeepPeriod workgroups (about what the device has in flight) the first kKept, so that hits
+// and memory work side by side: 256 sequences of 32 heads (512 MB), the same states every step 162 us (kCached 163, kStream
+// 184), two or three sets of states in turn 162 (217, 183), six sets 183 (217, 182).
+enum class StateLoads { kCached, kStream, kMixed };
+constexpr int kKeepPeriod = 512, kKept = 80;
+
+template <typename T, typename TP, int DK, int BV, StateLoads LOADS>
+__global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int64_t sq, int64_t sk, int64_t sv,
     RecurrentGates gates, const float* state_in, float* state_out, T* __restrict__ o, const int64_t* __restrict__ cu,
     int T_len, int Hqk, int Hv, int V, float scale, int use_l2norm) {
@@ -77,14 +86,25 @@ __global__ __launch_bounds__(256, kRecurrentWaves) void recurrent_kernel(
 #pragma unroll
     for (int m = 0; m < MC; ++m) S[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (state_in != nullptr) {
+    auto load = [&](auto stream) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int m = 0; m < MC; ++m) {
-        const f32x4* p = reinterpret_cast<const f32x4*>(state_in + sbase + (int64_t)(32 * j + 8 * m) * V);
-        if constexpr (STREAM) S[j][m] = __builtin_nontemporal_load(p);
-        else S[j][m] = *p;
-      }
+        for (int m = 0; m < MC; ++m) {
+          const f32x4* p = reinterpret_cast<const f32x4*>(state_in + sbase + (int64_t)(32 * j + 8 * m) * V);
+          if constexpr (decltype(stream)::value) S[j][m] = __builtin_nontemporal_load(p);
+          else S[j][m] = *p;
+        }
+    };
+    if constexpr (LOADS == StateLoads::kCached) {
+      load(std::false_type{});
+    } else if (LOADS == StateLoads::kStream || blockIdx.x % kKeepPeriod >= kKept) {
+      load(std::true_type{});
+    } else {
+      asm volatile("" ::: "memory");   // or the compiler makes one branch of the two, and its loads plain
+      load(std::false_type{});
+      asm volatile("" ::: "memory");
+    }
   }
 
   // packed input (cu given): "sequence" b owns the tokens cu[b] .. cu[b+1] of the one batch row
@@ -200,36 +220,47 @@ static int launch_recurrent(const void* q, const void* k, const void* v, int64_t
                             const RecurrentGates& gates, const float* state_in, float* state_out, void* o, int B,
                             int T_len, int Hqk, int Hv, int K, int V, float scale, int use_l2norm, hipStream_t stream,
                             const int64_t* cu = nullptr) {
-  // Whole states (64 KB at K = V = 128) per workgroup where they give every CU one, else 32 columns: 8.1 -> 7.1 us for one
-  // sequence of 32 heads, 11.4 -> 10.4 for 8; 32 columns at 16 / 32 sequences 18 / 30 us against 14 / 24.
-  // State loads that pass by the caches, except where the states exceed the L2s and still fit the 256 MB memory-side cache,
-  // which then serves a part of them (64 sequences 46 us against 49; 128 sequences 107 against 97).
-  // Past that size two or three workgroups per CU instead of four (by the LDS they ask for): less memory in flight at
-  // once, 198 -> 190 us at 256 sequences; below it 47 -> 57 us at 64.
-  const int64_t states = (int64_t)B * Hv * (V / 128), bytes = (int64_t)B * Hv * K * V * 4;
-  const bool narrow = V % 128 != 0 || states <= device_compute_units(), beyond = bytes >= (256LL << 20);
-  const bool cached = bytes > (32LL << 20) && !beyond;
-#define GDN_REC(DK_, BV_, ST_, LDS_)                                                                                   \
-  GDN_LAUNCH(kKernRecurrent, stream, (recurrent_kernel<T, TP, DK_, BV_, ST_>), dim3((unsigned)(B * Hv * (V / BV_))),   \
-             dim3(kThreads), LDS_, stream, (const T*)q, (const T*)k, (const T*)v, sq, sk, sv, gates, state_in,         \
-             state_out, (T*)o, cu, T_len, Hqk, Hv, V, scale, use_l2norm)
-  // (K = 256: half as wide, which makes the slab the registers hold the same)
-#define GDN_REC_K(DK_)                                                           \
-  constexpr int kWide##DK_ = DK_ == 256 ? 64 : 128;                              \
-  if (K == DK_) {                                                                \
-    if (narrow && cached) GDN_REC(DK_, 32, false, 0);                            \
-    else if (narrow) GDN_REC(DK_, 32, true, 0);                                  \
-    else if (beyond) GDN_REC(DK_, kWide##DK_, true, 45000);                             \
-    else if (cached) GDN_REC(DK_, kWide##DK_, false, 0);                  \
-    else GDN_REC(DK_, kWide##DK_, true, 0);                                             \
-    return (int)hipGetLastError();                                               \
+  // Times in us, the same states every step / three sets of states in turn.
+  // 32 columns per workgroup while wider slabs would leave CUs without one (32 heads: one sequence 8.1 -> 7.1, 16 sequences
+  // 18 against 14), else 128, or 64 where V asks for it (V = 64, 32 sequences: 15.3 / 15.2 with 32 columns, 11.9 / 14.6).
+  // K = 256: 64 (V = 128, 1 GB of states 326 / 382, 128 columns 340 / 390), but 128 for states in the memory-side cache
+  // (64 MB 26.2 -> 24.3) and for rows of several such slabs beyond it (V = 256, 1 GB 349 / 403 -> 330 / 381).
+  // Loads: kCached between the L2s' 32 MB and the memory-side cache's 256 MB (128 MB 45 / 47; kStream 49), kMixed beyond, save
+  // for K = 64 in 128 columns, where the kept part earns nothing (512 MB 179 against 175).
+  // Beyond: two workgroups per CU instead of four (by the LDS they ask for), less memory in flight at once: 512 MB 198 -> 184
+  // with kStream.  Three for slabs of 16 KB (K = V = 64, 512 MB 169 / 171 -> 161 / 164).
+  constexpr int64_t MB = 1 << 20;
+  const int64_t bytes = (int64_t)B * Hv * K * V * 4;
+  const bool beyond = bytes >= 256 * MB, cached = bytes > 32 * MB && !beyond;
+  const int full = V % 128 != 0 || (K == 256 && !cached && !(beyond && V % 256 == 0)) ? 64 : 128;
+  const int bv = (int64_t)B * Hv * (V / full) <= device_compute_units() ? 32 : full;
+  const int lds = !beyond ? 0 : K * full > 64 * 64 ? 45000 : 30000;
+  auto launch = [&](auto kern) {
+    GDN_LAUNCH(kKernRecurrent, stream, kern, dim3((unsigned)((int64_t)B * Hv * (V / bv))), dim3(kThreads), lds, stream,
+               (const T*)q, (const T*)k, (const T*)v, sq, sk, sv, gates, state_in, state_out, (T*)o, cu, T_len, Hqk, Hv, V,
+               scale, use_l2norm);
+    return (int)hipGetLastError();
+  };
+#define GDN_REC(DK_, BV_, LOADS_) return launch(recurrent_kernel<T, TP, DK_, BV_, StateLoads::LOADS_>)
+#define GDN_REC_WIDTH(DK_, BV_, BEYOND_)               \
+  if (K == DK_ && bv == BV_) {                         \
+    if (beyond) GDN_REC(DK_, BV_, BEYOND_);            \
+    if (cached) GDN_REC(DK_, BV_, kCached);            \
+    GDN_REC(DK_, BV_, kStream);                        \
   }
-  GDN_REC_K(64)
-  GDN_REC_K(128)
-  GDN_REC_K(256)
-  return -3;
-#undef GDN_REC_K
+  if (K == 64 && bv == 32) GDN_REC(64, 32, kStream);
+  if (K == 128 && bv == 32) GDN_REC(128, 32, kStream);
+  if (K == 256 && bv == 32) GDN_REC(256, 32, kStream);
+  GDN_REC_WIDTH(64, 64, kMixed)
+  GDN_REC_WIDTH(64, 128, kStream)
+  GDN_REC_WIDTH(128, 64, kMixed)
+  GDN_REC_WIDTH(128, 128, kMixed)
+  GDN_REC_WIDTH(256, 64, kMixed)
+  if (K == 256 && cached) GDN_REC(256, 128, kCached);
+  if (K == 256) GDN_REC(256, 128, kMixed);
+#undef GDN_REC_WIDTH
 #undef GDN_REC
+  return -3;
 }
 
 static int recurrent_check(int B, int T, int Hqk, int Hv, int V) {

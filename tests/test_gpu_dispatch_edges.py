@@ -74,7 +74,7 @@ def test_recurrent_edges(ops, dtype, B, T, Hqk, Hv, K, V):
 
 @pytest.mark.parametrize("dtype,K,V,batches", [
     (BF, 128, 128, (1, 9, 17, 129)), (F32, 128, 128, (1, 9)), (BF, 128, 64, (1, 9, 40, 260)), (BF, 64, 128, (1, 33, 258)),
-    (BF, 256, 128, (1, 9, 20, 66)),
+    (BF, 256, 128, (1, 9, 20, 66)), (BF, 256, 256, (1, 33)),
 ])
 def test_recurrent_bits_do_not_depend_on_the_batch(ops, dtype, K, V, batches):
     P.check_recurrent_batch_bits(ops, "cuda", batches, 16, 32, K, V, dtype)
