@@ -63,8 +63,10 @@ __device__ __forceinline__ void load_hist(float* dst, const T* x, const T* init,
 // v_rcp_f32 (1 ulp) instead of an IEEE division: ten instructions fewer per element
 __device__ __forceinline__ float sigmoidf_(float p) { return __builtin_amdgcn_rcpf(1.f + __expf(-p)); }
 
-// TT tokens per workgroup.  A tile that lies inside one sequence, history included, takes straight-line code: its rows
-// and the W-1 before them are requested at once.  Tiles at a sequence's ends go token by token.
+// TT tokens per workgroup, their rows and the W-1 before them requested at once.  A tile that lies inside one sequence,
+// history included, takes straight-line code; one in which a sequence begins or ends looks at every token (32768 tokens
+// below in sequences of 8: 184 us as well; reading the W rows of each token anew 290).  The first tile, and a last one that
+// is not full, go token by token.
 // Bound by memory.  32768 x 8192 bf16, W = 4: 64 tokens per workgroup 206 us (5.2 TB/s), 16: 244, 8: 181 (5.9), 4: 189;
 // 4096 x 8192: 46 -> 23 us (64 tokens: too few waves in flight).
 template <typename T, int W, int TT, bool SILU, bool RES>
@@ -104,6 +106,17 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) vo
     for (int e = 0; e < V; ++e) bs[e] = 0.f;
     if (bias != nullptr) load_chan(bs, bias + d0);
   };
+  auto final_state = [&](int64_t t, int u) {   // dense batches: the window is the final state [W] of each channel
+    if (fs == nullptr || t + 1 != cur.eos) return;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      float f[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) f[e] = win[(u + (i * V + e) % W) % W][(i * V + e) / W];
+      const Vec16<T> piece = pack16<T>(f);
+      __builtin_memcpy(fs + ((int64_t)cur.n * D + d0) * W + i * V, &piece.raw, 16);
+    }
+  };
   if (t0 >= H && t0 + TT <= total) {
     // the rows exist whatever sequence they belong to: they are on their way while the sequence is looked up
     Vec16<T> xr[TT + H];
@@ -122,21 +135,37 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) vo
       }
       return;
     }
-  } else {
-    weights();
-    cur.init(cu, N, T_len, t0);
+    // a sequence begins or ends in the tile: the same rows, the window replaced where a sequence begins
+#pragma unroll
+    for (int w = 0; w < H; ++w) {
+      if (t0 - H + w >= cur.bos) unpack_chan(win[w], xr[w]);
+      else load_hist(win[w], x, init, t0 - H + w, cur, D, W, d0);
+    }
+#pragma unroll
+    for (int u = 0; u < TT; ++u) {
+      if (cur.advance_to(t0 + u)) {   // its first token
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          T row[W];
+          if (init != nullptr) __builtin_memcpy(row, init + ((int64_t)cur.n * D + d0 + e) * W, sizeof(row));
+#pragma unroll
+          for (int w = 0; w < H; ++w) win[(u + w) % W][e] = init != nullptr ? Elem<T>::to_f(row[w + 1]) : 0.f;
+        }
+      }
+      unpack_chan(win[(u + H) % W], xr[u + H]);
+      finish(t0 + u, u);
+      final_state(t0 + u, u);
+    }
+    return;
   }
-  for (int64_t t = t0; t < t0 + TT && t < total; ++t) {
+  weights();
+  cur.init(cu, N, T_len, t0);
+  for (int64_t t = t0; t < t0 + TT && t < total; ++t) {   // the first tile, and a last one that is not full
     cur.advance_to(t);
 #pragma unroll
     for (int w = 0; w < W; ++w) load_hist(win[w], x, init, t - H + w, cur, D, W, d0);
     finish(t, 0);
-    if (fs != nullptr && t + 1 == cur.eos) {   // the window is the sequence's final state [W] of each channel
-#pragma unroll
-      for (int e = 0; e < V; ++e)
-#pragma unroll
-        for (int w = 0; w < W; ++w) fs[((int64_t)cur.n * D + d0 + e) * W + w] = Elem<T>::from_f(win[w][e]);
-    }
+    final_state(t, 0);
   }
 }
 

@@ -120,6 +120,7 @@ def test_chunk_backward_without_initial_state(ops):
 @pytest.mark.parametrize("dtype,B,T,D,W,cu", [
     (F32, 2, 37, 16, 4, None), (BF, 1, 300, 32, 4, [0, 1, 3, 130, 131, 300]), (F32, 1, 9, 8, 3, [0, 2, 9]),
     (torch.float16, 2, 5, 8, 2, None), (F32, 3, 2, 8, 4, None), (F32, 1, 600, 8, 4, [0, 255, 257, 600]),
+    (BF, 1, 41, 16, 4, list(range(42))), (F32, 9, 5, 8, 4, None),    # sequences shorter than a window or a tile
 ])
 def test_conv1d(ops, dtype, B, T, D, W, cu):
     P.check_conv(ops, "cpu", B, T, D, W, dtype, cu=cu, residual=True, wrap=guarded)

@@ -53,6 +53,7 @@ def test_rms_norm_gated_far_gates(ops, activation):
 @pytest.mark.parametrize("dtype,B,T,D,W,cu", [
     (BF, 1, 8, 64, 4, None), (BF, 2, 11, 64, 4, None), (BF, 1, 19, 1032, 4, None),   # one tile; its halo; a ragged channel block
     (BF, 1, 600, 64, 4, [0, 3, 16, 19, 24, 24, 300, 303, 600]),       # boundaries on, just past and inside tile edges
+    (BF, 1, 41, 64, 4, list(range(42))), (F32, 1, 75, 64, 3, list(range(0, 76, 3))), (BF, 9, 5, 64, 4, None),   # shorter than a window or a tile
     (BF, 3, 64, 72, 4, None), (F32, 1, 257, 64, 3, [0, 128, 257]), (torch.float16, 1, 100, 64, 2, None),
     (BF, 1, 300, 64, 5, [0, 64, 65, 300]), (BF, 1, 200, 64, 8, None),  # windows wider than the straight-line backward tile
     (BF, 1, 16 * 256 + 5, 1024, 4, None),                              # tiles past the first of every backward workgroup
