@@ -193,9 +193,10 @@ __global__ void conv1d_final_state_kernel(const T* __restrict__ x, const T* init
 // Backward.  With p the pre-activation and dyp = dy * act'(p):
 //   dx[s]   = sum_u dyp[s+u] * weight[W-1-u]   (s+u inside the sequence of s)  (+ dht at the last W tokens)
 //   dw[w]   = sum_t dyp[t] * xpad[t-(W-1)+w],   db = sum_t dyp[t]
-// A workgroup walks the tiles by, by + G, by + 2 G, ... of its channels (G = gridDim.x / channel blocks), so that the
-// workgroups move through memory together, and writes one partial dw/db to part[by][W+1][D]; conv1d_reduce_kernel sums
-// them in a fixed order.
+// A workgroup walks one tile of its channels in every G (G = gridDim.x / channel blocks), so that the workgroups move
+// through memory together, and writes one partial dw/db to part[by][W+1][D]; conv1d_reduce_kernel sums them in a fixed
+// order.  The tile is the (by + k)-th of the k-th G, not always the by-th: sequences of equal length put their ends, whose
+// tiles take longer, at the same few places of every G (32768 x 8192 in sequences of 128 tokens: 360 us with the by-th, 324 now).
 template <typename T, int W, int TT, bool SILU>
 __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 2 : 1) void conv1d_bwd_kernel(
     const T* __restrict__ x, const T* __restrict__ dy, const T* __restrict__ weight, const T* __restrict__ bias,
@@ -362,7 +363,11 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 2 : 1) vo
     }
   };
   Vec16<T> xa[W], ga[W], xb[W], gb[W];
-  for (t0 = by * TT; t0 < total; t0 += (int64_t)groups * TT) {
+  const int64_t ntiles = (total + TT - 1) / TT;
+  int turn = (int)by;
+  for (int64_t first = 0; first < ntiles; first += groups, turn = turn + 1 == groups ? 0 : turn + 1) {
+    t0 = (first + turn) * TT;
+    if (t0 >= total) continue;
     t1 = t0 + TT < total ? t0 + TT : total;
     tend = t1 + (W - 1) < total ? t1 + (W - 1) : total;   // halo: dyp of later tokens feeds dx
     cur.init(cu, N, T_len, t0);
@@ -510,12 +515,15 @@ __global__ __launch_bounds__(256) void conv1d_update_rows_kernel(const T* __rest
 constexpr int kConvFwdTile = 8;
 // Tokens per tile of the backward pass.  Bound by vector issue (about 40 instruction slots per element, halo tokens
 // included).  W = 4, D = 8192 bf16, 360 / 4096 / 32768 tokens: tiles of 256 on one workgroup each 200 / 208 / 362 us,
-// tiles of 32 29 / 54 / 337, tiles of 16 20 / 52 / 330.
+// tiles of 32 29 / 54 / 337, tiles of 16 20 / 52 / 330 (321 with the tiles dealt in turn).  Sequences of one to three tokens
+// pay for the halo (32768 of one token each: 419 -> 447 us with the reduction).
 constexpr int conv_bwd_tile(int W) { return W <= 4 ? 16 : 64; }   // wide windows: fewer halo tokens computed twice
-constexpr int kConvMaxGroups = 256;
+constexpr int kConvMaxGroups = 1024;
 // workgroups (and partial sums of dw, db) per channel block of the backward pass: as many as fit the device at once, no
-// more partial sums than it takes (512 workgroups in all instead of 1024: 427 us at 32768 x 8192, 2048: 328)
+// more partial sums than it takes (512 workgroups in all instead of 1024: 427 us at 32768 x 8192, 2048: 328; with at most 256
+// per channel block few channels leave the device idle: 262144 x 512 494 us, now 224)
 static int conv_bwd_groups(int64_t total, int nbd, int W) {
+  if (nbd < 1) nbd = 1;
   const int64_t ntiles = (total + conv_bwd_tile(W) - 1) / conv_bwd_tile(W);
   int most = 1024 / nbd;
   most = most < 64 ? 64 : most > kConvMaxGroups ? kConvMaxGroups : most;
@@ -625,9 +633,9 @@ static int conv_check(int B, int T_len, int N, int D, int W, int dtype) {
 }  // namespace gdn
 
 extern "C" int64_t gdn_conv1d_bwd_workspace_bytes(int B, int T, int D, int W) {
-  const int64_t total = (int64_t)B * T;
-  int64_t groups = (total + gdn::conv_bwd_tile(W) - 1) / gdn::conv_bwd_tile(W);
-  if (groups > gdn::kConvMaxGroups) groups = gdn::kConvMaxGroups;
+  if (D <= 0) return 256;   // refused by the call itself
+  // the 16-bit types have half as many channel blocks as fp32, and as many groups or more
+  const int groups = gdn::conv_bwd_groups((int64_t)B * T, (D / 8 + gdn::kConvThreads - 1) / gdn::kConvThreads, W);
   return (groups > 0 ? groups : 1) * (int64_t)(W + 1) * D * (int64_t)sizeof(float);
 }
 
