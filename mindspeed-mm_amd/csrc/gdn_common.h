@@ -77,6 +77,11 @@ template <typename T> __device__ __host__ constexpr int lds_ld(int cols) { retur
 // Instruction-scheduling fence: nothing is moved across it.  Used to pin hand-made software pipelines (issue the
 // LDS reads of the next group, then the matrix instructions of this group) that the scheduler would otherwise
 // serialise into read -> wait -> multiply.
+// work-items of one launch: the dispatch packet counts them in 32 bits (the CPU test build sets a small bound, so that its
+// tests meet launches in parts)
+#ifndef GDN_MAX_LAUNCH_THREADS
+#define GDN_MAX_LAUNCH_THREADS 0xffffffffLL
+#endif
 #define GDN_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 // Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by their linear index.  The recurrence kernels
 // number their workgroups so that the value heads of one q/k group, which read the same K / Q^T tiles, share an XCD:

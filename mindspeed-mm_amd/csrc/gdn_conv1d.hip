@@ -73,11 +73,11 @@ template <typename T, int W, int TT, bool SILU, bool RES>
 __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) void conv1d_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ weight, const T* __restrict__ bias, const T* __restrict__ residual,
     const T* __restrict__ init, const int64_t* __restrict__ cu, T* __restrict__ y, T* __restrict__ fs, int64_t total,
-    int T_len, int N, int D) {
+    int64_t first_tile, int T_len, int N, int D) {
   constexpr int V = Elem<T>::kVec, H = W - 1;
   // one linear grid, channel blocks fastest: the number of token tiles is not bounded by the y dimension's 65535
   const int nbd = (D / V + kConvThreads - 1) / kConvThreads, bx = blockIdx.x % nbd;
-  const int64_t t0 = (int64_t)(blockIdx.x / nbd) * TT;
+  const int64_t t0 = (first_tile + blockIdx.x / nbd) * TT;
   const int d0 = (bx * kConvThreads + threadIdx.x) * V;
   if (d0 >= D) return;
   float wgt[W][V], bs[V], win[W][V];
@@ -536,16 +536,19 @@ template <typename T> struct ConvLaunch {
                  hipStream_t st) {
     constexpr int V = Elem<T>::kVec, TT = kConvFwdTile;
     const int64_t total = (int64_t)B * T_len;
-    const int64_t nblocks = (int64_t)((D / V + kConvThreads - 1) / kConvThreads) * ((total + TT - 1) / TT);
-    if (nblocks > 0x7fffffffLL) return -3;
-    dim3 grid((unsigned)nblocks);
+    const int nbd = (D / V + kConvThreads - 1) / kConvThreads;
+    if ((int64_t)nbd * kConvThreads > GDN_MAX_LAUNCH_THREADS) return -3;
+    const int64_t ntiles = (total + TT - 1) / TT, most = GDN_MAX_LAUNCH_THREADS / ((int64_t)nbd * kConvThreads);
     // every sequence of a dense batch has a last token, whose tile can write the final state -- but not over the initial
     // state, which the sequence's first tile may still be reading
     const bool fs_inside = cu == nullptr && total > 0 && fs != init;
     if (total > 0) {
       auto launch = [&](auto kern) {
-        GDN_LAUNCH(kKernConvFwd, st, kern, grid, dim3(kConvThreads), 0, st, (const T*)x, (const T*)weight, (const T*)bias,
-                   (const T*)residual, (const T*)init, cu, (T*)y, fs_inside ? (T*)fs : (T*)nullptr, total, T_len, N, D);
+        for (int64_t t = 0; t < ntiles; t += most) {   // 8 channels: 4 GB of x to a launch
+          const dim3 grid((unsigned)(nbd * (ntiles - t < most ? ntiles - t : most)));
+          GDN_LAUNCH(kKernConvFwd, st, kern, grid, dim3(kConvThreads), 0, st, (const T*)x, (const T*)weight, (const T*)bias,
+                     (const T*)residual, (const T*)init, cu, (T*)y, fs_inside ? (T*)fs : (T*)nullptr, total, t, T_len, N, D);
+        }
       };
       switch (W) {
 #define GDN_CASE(W_)                                                                                \

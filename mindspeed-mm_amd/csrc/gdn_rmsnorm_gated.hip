@@ -156,15 +156,17 @@ static int rmsnorm_bwd_blocks(int64_t rows, int rpb) {
 template <typename T, typename TW, int LPR>
 static int rmsnorm_fwd_launch(const void* x, const void* gate, const void* weight, void* y, float* rstd, int64_t rows,
                               float eps, int act, hipStream_t st) {
-  const int64_t nb = (rows + kThreads / LPR - 1) / (kThreads / LPR);
-  if (nb > 0x7fffffffLL) return -3;
-  const dim3 grid((unsigned)nb);
-  if (act == 0)
-    GDN_LAUNCH(kKernRmsNormFwd, st, (rmsnorm_gated_fwd_kernel<T, TW, LPR, 0>), grid, dim3(kThreads), 0, st, (const T*)x,
-               (const T*)gate, (const TW*)weight, (T*)y, rstd, rows, eps);
-  else
-    GDN_LAUNCH(kKernRmsNormFwd, st, (rmsnorm_gated_fwd_kernel<T, TW, LPR, 1>), grid, dim3(kThreads), 0, st, (const T*)x,
-               (const T*)gate, (const TW*)weight, (T*)y, rstd, rows, eps);
+  constexpr int N = LPR * Elem<T>::kVec, RPB = kThreads / LPR;
+  constexpr int64_t most = GDN_MAX_LAUNCH_THREADS / kThreads * RPB;   // rows of one launch (4 KB of x to a workgroup: 68 GB)
+  for (int64_t r = 0; r < rows; r += most) {
+    const int64_t n = rows - r < most ? rows - r : most;
+    auto launch = [&](auto kern) {
+      GDN_LAUNCH(kKernRmsNormFwd, st, kern, dim3((unsigned)((n + RPB - 1) / RPB)), dim3(kThreads), 0, st, (const T*)x + r * N,
+                 (const T*)gate + r * N, (const TW*)weight, (T*)y + r * N, rstd + r, n, eps);
+    };
+    if (act == 0) launch(rmsnorm_gated_fwd_kernel<T, TW, LPR, 0>);
+    else launch(rmsnorm_gated_fwd_kernel<T, TW, LPR, 1>);
+  }
   return (int)hipGetLastError();
 }
 

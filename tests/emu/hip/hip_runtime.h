@@ -29,6 +29,7 @@
 #define __shared__ thread_local
 #define __align__(n) __attribute__((aligned(n)))
 #define HIP_KERNEL_NAME(...) __VA_ARGS__
+#define GDN_MAX_LAUNCH_THREADS 8192   // kernels that are launched in parts come in parts of this size
 
 struct dim3 {
   unsigned x, y, z;

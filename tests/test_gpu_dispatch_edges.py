@@ -63,6 +63,19 @@ def test_conv1d_edges(ops, dtype, B, T, D, W, cu):
     P.check_conv(ops, "cuda", B, T, D, W, dtype, cu=cu, bias=False, state=False, activation=None)
 
 
+def test_conv1d_more_work_items_than_a_launch(ops):
+    """8 channels: 2^25 workgroups of 128 take 2^28 tokens, and a launch counts fewer than 2^32 work-items."""
+    T, D, W, n = (1 << 28) + 1000, 8, 4, 4000
+    w = torch.randn(W, D, device="cuda", dtype=BF)
+    x = torch.empty(1, T, D, device="cuda", dtype=BF).uniform_(-1, 1)
+    with torch.no_grad():
+        y, _ = ops.causal_conv1d(x, w, activation="silu")
+        for at in (0, T // 2, T - n):
+            lo = max(0, at - 8)
+            part, _ = ops.causal_conv1d(x[:, lo:at + n].contiguous(), w, activation="silu")
+            assert torch.equal(y[:, at:at + n], part[:, at - lo:])
+
+
 @pytest.mark.parametrize("dtype,B,T,Hqk,Hv,K,V", [
     (BF, 8, 1, 16, 32, 128, 128), (BF, 9, 1, 16, 32, 128, 128),    # as many states as compute units; more: whole states
     (BF, 17, 1, 16, 32, 128, 128),                                 # states larger than the L2s
