@@ -565,3 +565,43 @@ def check_recurrent_batch_bits(ops, device, batches, Hqk, Hv, K, V, dtype):
         if first is None:
             first = (o[0], s[0])
         assert torch.equal(o[0], first[0]) and torch.equal(s[0], first[1]), B
+
+
+def run_cut_case(ops, x, kda, cu=None, tile=1):
+    """Outputs and every gradient of a call on x (gdn_inputs / kda_inputs on the device); tile: the heads repeated that
+    often, of which the first set's results are returned."""
+    names = ("q", "k", "v", "g", "beta", "h0") + (("A_log", "dt_bias") if kda else ())
+    head = {"q": 2, "k": 2, "v": 2, "g": 2, "beta": 2, "do": 2, "h0": 1, "dht": 1, "A_log": 0, "dt_bias": 0}
+    n = {k: t.shape[head[k]] for k, t in x.items()}
+    leaf = {k: torch.cat([t] * tile, head[k]).contiguous().requires_grad_(k in names) for k, t in x.items()}
+    cu_t = torch.tensor(cu, dtype=torch.int64, device=x["q"].device) if cu is not None else None
+    args, kw = [leaf[k] for k in ("q", "k", "v", "g", "beta")], dict(
+        initial_state=leaf["h0"], output_final_state=True, use_qk_l2norm_in_kernel=True, cu_seqlens=cu_t)
+    if kda:
+        o, ht = ops.chunk_kda(*args, use_gate_in_kernel=True, use_beta_sigmoid_in_kernel=True, A_log=leaf["A_log"],
+                              dt_bias=leaf["dt_bias"], **kw)
+    else:
+        o, ht = ops.chunk_gated_delta_rule(*args, **kw)
+    grads = torch.autograd.grad([o, ht], [leaf[k] for k in names], [leaf["do"], leaf["dht"]])
+    res = {"o": o.detach().narrow(2, 0, n["v"]), "ht": ht.detach().narrow(1, 0, n["h0"])}
+    res.update({"d" + k: t.narrow(head[k], 0, n[k]) for k, t in zip(names, grads)})
+    return res
+
+
+def check_cut_against_uncut(ops, device, T, Hqk, Hv, kda, cu=None, B=1, seed=0, uncut_ops=None, tile=1, wrap=lambda t: t):
+    """Slow decays (a state outlives several segments: exp of the summed decay over 1000 tokens is 0.5 to 0.9), where the
+    maps between segments matter: a call that is cut into segments against one that is not -- other operators (uncut_ops)
+    or the heads repeated until the device is full.  Each is within 6e-3 of float64 in the 2-norm (bf16 operands, 2^-9 a
+    rounding), 8e-3 for KDA, so they lie within twice that of each other."""
+    N = len(cu) - 1 if cu is not None else B
+    slow = dict(seed=seed, N=N, a_log=(0.5, 2.0), dt_bias=(-9.0, -8.0), h0_std=0.1)
+    x = kda_inputs(B, T, Hv, 128, 128, torch.bfloat16, **slow) if kda else \
+        gdn_inputs(B, T, Hqk, Hv, 128, 128, torch.bfloat16, **slow)
+    x = {k: wrap(t.to(device)) for k, t in x.items()}
+    cut = run_cut_case(ops, x, kda, cu)
+    uncut = run_cut_case(uncut_ops or ops, x, kda, cu, tile=tile)
+    off = {k: ((cut[k].double() - uncut[k].double()).norm() / uncut[k].double().norm()).item() for k in cut}
+    print(f"cut against uncut T{T} H{Hv} kda={kda}:", {k: f"{e:.1e}" for k, e in off.items()}, flush=True)
+    assert any(not torch.equal(cut[k], uncut[k]) for k in cut), "neither of the calls, or both, ran cut"
+    assert max(off.values()) <= (1.6e-2 if kda else 1.2e-2), off
+    return off

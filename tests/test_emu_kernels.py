@@ -408,3 +408,9 @@ def test_cut_launch_hands_the_state_of_an_empty_sequence_through(ops256, kda):
     assert torch.equal(ht[0].view(torch.int32), h0[0].view(torch.int32))
     assert torch.equal(dh0[0].view(torch.int32), dht[0].view(torch.int32))
     assert ht[1].isfinite().all() and dh0[1].isfinite().all()
+
+
+@pytest.mark.parametrize("kda", [False, True])
+def test_cut_launch_carries_a_slowly_decaying_state(ops, ops256, kda):
+    """The maps, the chain and the cut recurrences against guard pages, and against the uncut recurrences."""
+    P.check_cut_against_uncut(ops256, "cpu", 4097, 1, 1, kda, uncut_ops=ops, wrap=guarded)

@@ -118,3 +118,44 @@ def test_recurrences_in_segments(ops, T, Hqk, Hv, V, cu):
 @pytest.mark.parametrize("T,H,cu", [(4097, 2, None), (12400, 1, [0, 130, 130, 12400])])
 def test_kda_recurrences_in_segments(ops, T, H, cu):
     P.check_kda(ops, "cuda", 1, T, H, 128, 128, BF, cu=cu, backward=True)
+
+
+@pytest.mark.parametrize("T,Hqk,Hv,kda,B,cu", [
+    (4097, 1, 2, False, 1, None), (4159, 1, 1, True, 1, None),
+    (8192, 4, 8, False, 1, None), (8192, 8, 8, True, 1, None),      # as many slabs as compute units: refill with two to a workgroup
+    (4160, 2, 2, False, 2, None), (4160, 2, 2, True, 2, None),      # a dense batch
+    (12400, 1, 2, False, 1, [0, 130, 130, 12400]), (12400, 1, 1, True, 1, [0, 130, 130, 12400]),
+])
+def test_cut_sequences_carry_a_slowly_decaying_state(ops, T, Hqk, Hv, kda, B, cu):
+    N = B if cu is None else len(cu) - 1
+    P.check_cut_against_uncut(ops, "cuda", T, Hqk, Hv, kda, cu=cu, B=B, tile=-(-24 // (N * Hv)))
+
+
+def test_cut_sequences_through_the_strided_entry_and_the_norm(ops):
+    """The unsplit convolution output and the gated norm in one call, cut: the bits of the separate operators on copies."""
+    T, H, K = 4200, 2, 128
+    x = P.gdn_inputs(1, T, H, H, K, K, BF, seed=6, a_log=(0.5, 2.0), dt_bias=(-9.0, -8.0))
+    d = {n: t.cuda() for n, t in x.items()}
+    qkv = torch.cat([d[n].flatten(2) for n in ("q", "k", "v")], -1)
+    z, w = torch.randn(1, T, H, K, device="cuda", dtype=BF), torch.rand(K, device="cuda").to(BF)
+    with torch.no_grad():
+        y, ht = ops.chunk_gated_delta_rule_qkv(qkv, d["g"], d["beta"], H, H, K, K, initial_state=d["h0"],
+                                               output_final_state=True, use_qk_l2norm_in_kernel=True, gate=z, norm_weight=w)
+        o, ht2 = ops.chunk_gated_delta_rule(d["q"], d["k"], d["v"], d["g"], d["beta"], initial_state=d["h0"],
+                                            output_final_state=True, use_qk_l2norm_in_kernel=True)
+        assert torch.equal(y, ops.rms_norm_gated(o, z, w)) and torch.equal(ht, ht2)
+
+
+def test_sequence_bits_alone_and_in_a_batch(ops):
+    """Uncut, a sequence's bits do not depend on what is packed with it; a call that is cut has the bits of its own number of
+    segments."""
+    x = {n: t.cuda() for n, t in P.gdn_inputs(1, 8192, 8, 32, 128, 128, BF, seed=8, N=2).items()}
+
+    def first(T, N, cu):
+        with torch.no_grad():
+            o, ht = ops.chunk_gated_delta_rule(*(x[n][:, :T].contiguous() for n in ("q", "k", "v", "g", "beta")),
+                                               initial_state=x["h0"][:N].contiguous(), output_final_state=True,
+                                               use_qk_l2norm_in_kernel=True, cu_seqlens=cu)
+        return o[:, :4096], ht[:1]
+    alone, packed = first(4096, 1, [0, 4096]), first(8192, 2, [0, 4096, 8192])
+    assert torch.equal(alone[0], packed[0]) and torch.equal(alone[1], packed[1])
