@@ -44,6 +44,10 @@ extern "C" {
  * call in a 16-bit dtype that writes o (and no fused norm) needs the prep part only.  gdn_chunk_bwd_parts takes the
  * two parts as separate buffers, so that a caller can keep the prep part of its forward call (0.28 GB at B=2, T=8192,
  * Hqk=16, Hv=32, d=128 in bf16, against 1.2 GB for both) and have the backward pass rebuild the state part.
+ *
+ * Bits.  The decode entries give a sequence the same bits whatever else is in the call.  So do the chunk entries, except
+ * where they cut sequences into segments (16-bit types, K = V = 128, few sequences and heads, 64 chunks a sequence or
+ * more): the number of segments follows from the call's sequences, heads and tokens, and moves the rounding.
  */
 int64_t gdn_chunk_workspace_bytes(int B, int T, int N, int Hqk, int Hv, int K, int V, int dtype, int with_backward);
 

@@ -61,10 +61,11 @@ int device_compute_units();   // defined with the forward launcher
 // many dependent steps as one.  Sequences of kMinCutChunks on average pay for the two launches in front of each
 // recurrence.  Forward pass, 128-wide heads, not cut -> cut: 4 heads 114 -> 80 us at 64 chunks, 207 -> 89 at 128; 8
 // heads 407 -> 145 at 256; 16 heads (4 segments) 114 -> 83 at 64, 829 -> 459 at 512.  At 48 chunks it is still 91 -> 77,
-// but a training step of that length waits for the host, and two more launches a pass cost it 235 -> 250.  Wider value
-// heads stay uncut: cut, they are as far from float32 in the mean (dg of slowly decaying heads 4.3e-3 to 5.2e-3, uncut
-// 4.3e-3 to 5.0e-3), but where the largest differences fall changes, and those lie at the stated bound (0.046 to 0.086
-// uncut, 0.050 to 0.082 cut, of a dg of 15).
+// but a training step of that length waits for the host, and two more launches a pass cost it 235 -> 250.  The number
+// follows from the sequences, heads and tokens of the call: a sequence's bits, cut, are those of its call's number of
+// segments.  Heads of other sizes stay uncut: K = 64 has no such kernels, and with V = 256 single entries of dg of slowly
+// decaying heads moved past the bound this project states for them (0.050 to 0.082 cut, 0.046 to 0.086 uncut, of a dg of
+// 15), at the same mean error; whether cutting pays there is open.
 constexpr int kMinSegmentChunks = 16, kMinCutChunks = 64;
 inline int state_segments(const ChunkDims& d, int elem_bytes) {
   if (elem_bytes != 2 || d.K != 128 || d.V != 128) return 1;

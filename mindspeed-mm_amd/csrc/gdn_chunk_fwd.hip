@@ -1006,8 +1006,9 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
                (const int*)chunk_offsets, G, Ai, AQ, KAF, QTF, rstd, rstd + (int64_t)nc * 64 * d.Hqk, d.T, d.N, d.Hqk,
                d.Hv, scale, l2norm, ts);
   }
-  // decided for the two-slab variant, the largest one: results must not depend on how many slabs a launch happens
-  // to give a workgroup (a sequence computes the same bits alone and inside a packed batch)
+  // decided for the two-slab variant, the largest one: results must not depend on how many slabs a launch happens to give a
+  // workgroup.  (Uncut, a sequence computes the same bits alone and inside a packed batch; into how many segments it is cut
+  // follows from the whole call, see state_segments.)
   constexpr bool PRE = StatePre<T, DK, 2, STAGES, FUSE>::value && StatePre<T, DK, NWS, STAGES, FUSE>::value;
   const int segs = state_segments(d, (int)sizeof(T));
   if constexpr (FUSE && DK == 128 && NW == 4) {

@@ -6,8 +6,8 @@
 // Row-wise and bandwidth-bound: forward reads x, gate and writes y; backward reads x, gate, dy and writes dx, dgate.
 // The forward pass gives every workgroup 4 KB of each tensor and nothing more: handed out in order, such pieces keep what
 // is in flight close together, which the memory rewards (1M rows of 128 bf16: 164 us = 4.9 TB/s with 2048 workgroups
-// striding over the rows and element-wise conversions, 127 us = 6.3 TB/s now; the card's copy of 4 KB pieces reaches 6.2
-// to 6.5, of 32 KB pieces 5.4).  The backward pass needs few partial sums of dweight and strides (276 -> 234 us).
+// striding over the rows and element-wise conversions, 127 to 133 us = 6.1 to 6.3 TB/s now; the card's copy of 4 KB pieces reaches 6.2
+// to 6.5, of 32 KB pieces 5.4).  The backward pass needs few partial sums of dweight and strides (276 -> 234 to 243 us).
 // A row of N elements is held by N/VEC neighbouring lanes (16 bytes each); row sums use data-parallel-primitive moves.
 // With gate_activation = 1 the gate passes through a sigmoid instead (the KDA layer's norm, KimiK_3_MoeRMSNormGated,
 // mindspeed_mm/fsdp/models/kimi_k3/modeling_kimi_linear.py:75-96): s = cast(sigmoid(gate)).

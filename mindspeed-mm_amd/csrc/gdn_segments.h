@@ -10,8 +10,9 @@
 //   3. the recurrence kernel proper, every segment from its own start
 // The reverse recurrence does the same from the other end.  2 n / P dependent steps instead of n.  32768 tokens, 8 heads
 // of 128, 8 segments: maps 100 us, chain 23, recurrence 117 where the recurrence alone took 0.8 ms; forward and backward
-// 1820 -> 795 us.  The error against float64 is the uncut recurrence's, also with decays near 1 over a whole segment
-// (3200 to 4100 tokens: o 4.75e-3 against 4.76e-3, final state 3.82e-3 against 3.84e-3, dq 4.61e-3 against 4.62e-3).
+// 1820 -> 795 us.  The error against float64 is the uncut recurrence's (4160 to 16384 tokens, 2 to 8 heads, four seeds each:
+// o 4.745e-3 and 4.745e-3 with decays near 1 over a whole segment, final state 3.78e-3 and 3.78e-3, dg 5.58e-3 to 5.95e-3
+// uncut, 5.60e-3 to 5.90e-3 cut, smaller in five of eight cases).
 #pragma once
 #include "gdn_common.h"
 
