@@ -147,10 +147,12 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_gated_dw_reduce_kernel(const
 
 // Two workgroups per CU, each a trip ahead with its requests.  Five streams share the memory: what counts is that the
 // rows in flight stay close together (2048 workgroups: 5.3 TB/s, 1024: 5.2, 768: 5.5, 512: 5.75, 384: 5.25, 256: 5.0 at
-// 1M rows of 128 bf16).
-static int rmsnorm_bwd_blocks(int64_t rows, int rpb) {
-  const int64_t need = (rows + rpb - 1) / rpb;
-  return (int)(need < 512 ? (need > 0 ? need : 1) : 512);
+// 1M rows of 128 bf16).  Three per CU for 16-bit tensors of up to 100 MB, which the memory-side cache holds in part (262144
+// rows, with the reduction: 70 to 72 -> 69 us; 131072: 39 -> 37.5; 524288, 134 MB: 121 -> 126; fp32, 67 MB: 64 -> 66).
+template <typename T> static int rmsnorm_bwd_blocks(int64_t rows, int rpb) {
+  const int64_t need = (rows + rpb - 1) / rpb, tensor = need * (kThreads * 16);
+  const int most = sizeof(T) == 2 && tensor <= 100 * 1000 * 1000 ? 768 : 512;
+  return (int)(need < most ? (need > 0 ? need : 1) : most);
 }
 
 template <typename T, typename TW, int LPR>
@@ -174,7 +176,7 @@ template <typename T, typename TW, int LPR>
 static int rmsnorm_bwd_launch(const void* x, const void* gate, const void* weight, const float* rstd, const void* dy,
                               void* dx, void* dgate, float* dw, float* part, int64_t rows, int act, hipStream_t st) {
   constexpr int N = LPR * Elem<T>::kVec;
-  const int nb = rmsnorm_bwd_blocks(rows, kThreads / LPR);
+  const int nb = rmsnorm_bwd_blocks<T>(rows, kThreads / LPR);
   if (act == 0)
     GDN_LAUNCH(kKernRmsNormBwd, st, (rmsnorm_gated_bwd_kernel<T, TW, LPR, 0>), dim3(nb), dim3(kThreads), 0, st, (const T*)x,
                (const T*)gate, (const TW*)weight, rstd, (const T*)dy, (T*)dx, (T*)dgate, part, rows);

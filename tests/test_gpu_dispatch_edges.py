@@ -22,6 +22,7 @@ def ops():
 @pytest.mark.parametrize("dtype,rows,N", [
     (BF, 1, 128), (BF, 17, 128),                   # one row; one row past a workgroup of the forward kernel
     (BF, 16 * 512 + 1, 128), (BF, 3 * 16 * 512, 128),   # one row past the backward grid; whole trips of it
+    (BF, 16 * 768 + 1, 128),                       # one row past the larger backward grid of 16-bit tensors
     (BF, 4 * 512 + 3, 512), (F32, 64 * 512 + 5, 16),    # a row on a whole wave; a row on four lanes
 ])
 @pytest.mark.parametrize("activation", ["silu", "sigmoid"])
