@@ -146,6 +146,15 @@ int gdn_recurrent_fwd_qkv(const void* qkv, int64_t token_stride, const void* a, 
                           int Hqk, int Hv, int K, int V, float scale, int use_qk_l2norm, int dtype, int param_dtype,
                           void* stream);
 
+/* A decode step whole: gdn_conv1d_update on hidden [B,D] (D = 2 Hqk K + Hv V, one token per sequence, state_len = W), then
+ * gdn_recurrent_fwd_qkv with the l2 norm on its output, in one launch and with the bits of the two.  conv_state [B,D,W] and
+ * state [B,Hv,K,V] are updated in place; conv_weight [D,W], conv_bias [D] or null; o [B,Hv,V].  W = 4 and K = 128; -3 for
+ * what needs the two calls: other sizes, value heads of one q/k head whose slabs (of 64 columns while the states are 32 MB
+ * or less, else of 128) are not 1, 2 or 4 in number, rows of conv_state or conv_weight not aligned to their size. */
+int gdn_decode_step(const void* hidden, void* conv_state, const void* conv_weight, const void* conv_bias, const void* a,
+                    const void* b, const void* A_log, const void* dt_bias, float* state, void* o, int B, int Hqk, int Hv,
+                    int K, int V, int W, int activation, float scale, int dtype, int param_dtype, void* stream);
+
 /* -------- causal short depthwise conv1d --------------------------------------------------------
  * replaces causal_conv1d_fwd_impl / causal_conv1d_bwd_impl / causal_conv1d_update_states,
  * mindspeed_mm/fsdp/ops/gdn/triton/convolution.py:517-588, 591-714, 762-787.

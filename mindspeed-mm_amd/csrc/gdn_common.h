@@ -164,6 +164,7 @@ template <typename T> __device__ __forceinline__ void gate_st(void* p, int same,
   }
   reinterpret_cast<float*>(p)[i] = x;
 }
+__device__ __forceinline__ float sigmoidf_(float p) { return __builtin_amdgcn_rcpf(1.f + __expf(-p)); }   // of the convolution's SiLU
 __device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
 __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
 

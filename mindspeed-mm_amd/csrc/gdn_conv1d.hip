@@ -61,7 +61,6 @@ __device__ __forceinline__ void load_hist(float* dst, const T* x, const T* init,
 }
 
 // v_rcp_f32 (1 ulp) instead of an IEEE division: ten instructions fewer per element
-__device__ __forceinline__ float sigmoidf_(float p) { return __builtin_amdgcn_rcpf(1.f + __expf(-p)); }
 
 // TT tokens per workgroup, their rows and the W-1 before them requested at once.  A tile that lies inside one sequence,
 // history included, takes straight-line code; one in which a sequence begins or ends looks at every token (32768 tokens

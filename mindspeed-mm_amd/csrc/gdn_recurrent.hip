@@ -30,6 +30,16 @@ struct RecurrentGates {   // either g, beta (fp32 [tokens,Hv]) or the projection
   const void* dt_bias;
 };
 
+// A decode step's convolution update, where the kernel does it too: one token per sequence, S = W taps, the rows of
+// conv_state [B,D,W] and weight [D,W] one vector load each, D = 2 Hqk K + Hv V.
+struct RecurrentConv {
+  const void* hidden;   // [B,D]
+  void* state;
+  const void* weight;
+  const void* bias;     // [D] or null
+  int silu;
+};
+
 // n consecutive values, n * sizeof(T) <= 16 bytes, in one load; aligned as their type is, not as the load is wide
 template <typename T, int n> __device__ __forceinline__ void load_run(float* dst, const T* p) {
   constexpr int bytes = n * (int)sizeof(T);
@@ -59,26 +69,79 @@ constexpr int recurrent_waves(int dk, int bv) { return dk * bv <= 128 * 128 ? 4 
 enum class StateLoads { kCached, kStream, kMixed };
 constexpr int kKeepPeriod = 512, kKept = 80;
 
-template <typename T, typename TP, int DK, int BV, StateLoads LOADS>
-__global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel(
+// CONV = 0: q, k, v come from memory.  CONV = n: a decode step with its convolution update in one launch.  A workgroup is n
+// groups of 256 threads, a slab each, and covers all slabs of all value heads of one q/k head: it alone reads and rolls the
+// convolution states of its channels, so no other workgroup can meet them half done.  Its threads form the convolution's
+// outputs, a channel at a time, and leave them in LDS while the slabs are on their way.
+template <typename T, typename TP, int DK, int BV, StateLoads LOADS, int CONV = 0>
+__global__ __launch_bounds__(256 * (CONV ? CONV : 1), recurrent_waves(DK, BV)) void recurrent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int64_t sq, int64_t sk, int64_t sv,
     RecurrentGates gates, const float* state_in, float* state_out, T* __restrict__ o, const int64_t* __restrict__ cu,
-    int T_len, int Hqk, int Hv, int V, float scale, int use_l2norm) {
+    int T_len, int Hqk, int Hv, int V, float scale, int use_l2norm, RecurrentConv conv) {
+  constexpr int UN = CONV ? CONV : 1;   // slabs of the workgroup
   constexpr int CG = BV / 4;            // column groups (4 fp32 = 16 bytes each)
   constexpr int MC = BV / 32;           // chains of rows held by a thread
   constexpr int NJ = DK / 32;           // rows of a chain
   constexpr int EPL = DK / 64;          // elements of k and q per lane for the norms
   static_assert(MC == 1 || MC == 2 || MC == 4, "tile shape");
-  __shared__ float red[2][4][CG][8], kq_rows[4][DK][2];
+  __shared__ float red_[UN][2][4][CG][8], kq_rows_[UN][4][DK][2];
+  __shared__ float conv_out[CONV ? 2 * DK + UN * BV : 1];   // q, k, then v of the value heads in their order
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int unit = CONV ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  auto& red = red_[unit];
+  auto& kq_rows = kq_rows_[unit];
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int cg = tid % CG, lrow = lane / CG;
   const int row0 = 2 * wave + lrow / (4 / MC) + 8 * MC * (lrow % (4 / MC));
   // the thread's rows are row0 + 32 j + 8 m
   // the slabs of a state are neighbours in the launch order: what is in flight then stays close together in memory
-  const int nslab = V / BV, bh = blockIdx.x / nslab, b = bh / Hv, h = bh % Hv, hq = h / (Hv / Hqk);
-  const int v0 = (blockIdx.x % nslab) * BV + cg * 4;
+  const int nslab = V / BV, slab = blockIdx.x * UN + unit, bh = slab / nslab, b = bh / Hv, h = bh % Hv, hq = h / (Hv / Hqk);
+  const int v0 = (slab % nslab) * BV + cg * 4;
   const int64_t sbase = ((int64_t)bh * DK + row0) * V + v0;
+
+  // the convolution's operands are requested ahead of the slab and used behind its requests
+  constexpr int W = 4, NCH = 2 * DK + UN * BV, CPT = CONV ? (NCH + 256 * UN - 1) / (256 * UN) : 1;   // channels per thread
+  typedef uint32_t RowVec __attribute__((ext_vector_type(W * (int)sizeof(T) / 4)));
+  union Row { RowVec v; T e[W]; };
+  Row cs[CPT], cw[CPT];
+  T cx[CPT], cb[CPT];
+  auto channel = [&](int i) {   // (column of the convolution's output, place in conv_out) of the thread's i-th channel
+    const int c = imin((int)threadIdx.x + 256 * UN * i, NCH - 1);
+    return c < DK ? hq * DK + c : c < 2 * DK ? (Hqk + hq) * DK + c - DK : 2 * Hqk * DK + hq * (Hv / Hqk) * V + c - 2 * DK;
+  };
+  if constexpr (CONV != 0) {
+    const int D = 2 * Hqk * DK + Hv * V;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int d = channel(i);
+      cs[i].v = *reinterpret_cast<const RowVec*>(static_cast<const T*>(conv.state) + ((int64_t)b * D + d) * W);
+      cw[i].v = *reinterpret_cast<const RowVec*>(static_cast<const T*>(conv.weight) + (int64_t)d * W);
+      cx[i] = static_cast<const T*>(conv.hidden)[(int64_t)b * D + d];
+      if (conv.bias != nullptr) cb[i] = static_cast<const T*>(conv.bias)[d];
+    }
+    GDN_SCHED_FENCE();
+  }
+  // the arithmetic of the stand-alone update (conv1d_update_kernel): the same bits
+  auto convolve = [&]() {
+    const int D = 2 * Hqk * DK + Hv * V;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int c = (int)threadIdx.x + 256 * UN * i;
+      float st[W + 1], a = conv.bias != nullptr ? Elem<T>::to_f(cb[i]) : 0.f;
+#pragma unroll
+      for (int j = 0; j < W; ++j) st[j] = Elem<T>::to_f(cs[i].e[j]);
+      st[W] = Elem<T>::to_f(cx[i]);
+#pragma unroll
+      for (int w = 0; w < W; ++w) a += st[1 + w] * Elem<T>::to_f(cw[i].e[w]);
+      if (c < NCH) {
+        conv_out[c] = Elem<T>::to_f(Elem<T>::from_f(conv.silu ? a * sigmoidf_(a) : a));
+        Row r;
+#pragma unroll
+        for (int j = 0; j < W; ++j) r.e[j] = Elem<T>::from_f(st[1 + j]);
+        *reinterpret_cast<RowVec*>(static_cast<T*>(conv.state) + ((int64_t)b * D + channel(i)) * W) = r.v;
+      }
+    }
+  };
 
   f32x4 S[NJ][MC];
 #pragma unroll
@@ -95,29 +158,45 @@ __global__ __launch_bounds__(256, recurrent_waves(DK, BV)) void recurrent_kernel
           if constexpr (decltype(stream)::value) S[j][m] = __builtin_nontemporal_load(p);
           else S[j][m] = *p;
         }
+      if constexpr (CONV != 0) {
+        // here, inside the branch of the loads, at whose end the compiler waits for them; and nothing of it between the
+        // requests (47 registers spilled with slabs of 128 columns)
+        asm volatile("" ::: "memory");
+        GDN_SCHED_FENCE();
+        convolve();
+        asm volatile("" ::: "memory");
+      }
     };
     if constexpr (LOADS == StateLoads::kCached) {
       load(std::false_type{});
-    } else if (LOADS == StateLoads::kStream || blockIdx.x % kKeepPeriod >= kKept) {
+    } else if (LOADS == StateLoads::kStream || blockIdx.x % (kKeepPeriod / UN) >= kKept / UN) {
       load(std::true_type{});
     } else {
       asm volatile("" ::: "memory");   // or the compiler makes one branch of the two, and its loads plain
       load(std::false_type{});
       asm volatile("" ::: "memory");
     }
+  } else if constexpr (CONV != 0) {
+    convolve();
   }
+  if constexpr (CONV != 0) GDN_LDS_BARRIER();
 
   // packed input (cu given): "sequence" b owns the tokens cu[b] .. cu[b+1] of the one batch row
   const int64_t tok0 = cu != nullptr ? cu[b] : (int64_t)b * T_len;
   const int ntok = cu != nullptr ? (int)(cu[b + 1] - cu[b]) : T_len;
   for (int t = 0; t < ntok; ++t) {
     const int64_t tok = tok0 + t;
-    const T* kp = k + tok * sk + hq * DK;
-    const T* qp = q + tok * sq + hq * DK;
     float ke[EPL], qe[EPL], vv[4];
-    load_run<T, EPL>(ke, kp + lane * EPL);
-    load_run<T, EPL>(qe, qp + lane * EPL);
-    load_run<T, 4>(vv, v + tok * sv + h * V + v0);
+    if constexpr (CONV != 0) {
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) { qe[e] = conv_out[lane * EPL + e]; ke[e] = conv_out[DK + lane * EPL + e]; }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) vv[c] = conv_out[2 * DK + unit * BV + cg * 4 + c];
+    } else {
+      load_run<T, EPL>(ke, k + tok * sk + hq * DK + lane * EPL);
+      load_run<T, EPL>(qe, q + tok * sq + hq * DK + lane * EPL);
+      load_run<T, 4>(vv, v + tok * sv + h * V + v0);
+    }
     float eg, bt;
     if (gates.a == nullptr) {
       eg = __expf(gates.g[tok * Hv + h]);
@@ -238,7 +317,7 @@ static int launch_recurrent(const void* q, const void* k, const void* v, int64_t
   auto launch = [&](auto kern) {
     GDN_LAUNCH(kKernRecurrent, stream, kern, dim3((unsigned)((int64_t)B * Hv * (V / bv))), dim3(kThreads), lds, stream,
                (const T*)q, (const T*)k, (const T*)v, sq, sk, sv, gates, state_in, state_out, (T*)o, cu, T_len, Hqk, Hv, V,
-               scale, use_l2norm);
+               scale, use_l2norm, RecurrentConv{});
     return (int)hipGetLastError();
   };
 #define GDN_REC(DK_, BV_, LOADS_) return launch(recurrent_kernel<T, TP, DK_, BV_, StateLoads::LOADS_>)
@@ -260,6 +339,44 @@ static int launch_recurrent(const void* q, const void* k, const void* v, int64_t
   if (K == 256) GDN_REC(256, 128, kMixed);
 #undef GDN_REC_WIDTH
 #undef GDN_REC
+  return -3;
+}
+
+// A decode step with its convolution update in one launch; -3 for what needs the two launches: other key widths, and heads
+// whose slabs do not add up to 1, 2 or 4 groups of threads.
+// 16 q/k and 32 value heads of 128, us in the kernels / per step of a program, two launches -> one.  Small batches save the
+// host's share of a launch: 1 sequence 13.4 / 29.6 -> 9.7 / 16.5, 16 sequences 20.0 / 29.7 -> 15.2 / 16.5.  The same states
+// every step, 32 sequences 31 / 30 -> 23 / 22, 64: 54 / 49 -> 50 / 49, 128: 97 / 93 -> 90 / 89, 256: 180 / 177 -> 167 / 165;
+// states that no cache holds, 64 sequences 62 / 60 -> 53 / 53, 112: 107 / 103 -> 97 / 97, 256: 199 / 195 -> 195 / 194.
+// Slabs of 64 columns up to 32 MB of states, where few workgroups hold many waves each (1 sequence 9.7, with slabs of 128
+// columns 11.7); beyond, 128 columns and two workgroups a CU (17 sequences 21 -> 16, 256: 208 -> 167).  Loads: kStream to
+// 128 MB (64 sequences, five sets of states in turn, 53 against 56 with kCached; 32: 25 and 26), then kCached (112 sequences,
+// the same states every step, 81 against 86), kMixed from 256 MB on as in the rule alone.
+template <typename T, typename TP>
+static int launch_decode_step(const RecurrentConv& conv, const RecurrentGates& gates, float* state, void* o, int B, int Hqk,
+                              int Hv, int K, int V, float scale, hipStream_t stream) {
+  constexpr int64_t MB = 1 << 20;
+  const int64_t bytes = (int64_t)B * Hv * K * V * 4;
+  const int bv = bytes > 32 * MB ? 128 : 64;
+  if (K != 128 || V % bv != 0 || (int64_t)B * Hqk > 0x7fffffff) return -3;
+  const int64_t units = (int64_t)(Hv / Hqk) * (V / bv);
+  auto launch = [&](auto kern) {
+    GDN_LAUNCH(kKernRecurrent, stream, kern, dim3((unsigned)(B * Hqk)), dim3((unsigned)(kThreads * units)), 0, stream,
+               (const T*)nullptr, (const T*)nullptr, (const T*)nullptr, 0, 0, 0, gates, (const float*)state, state, (T*)o,
+               (const int64_t*)nullptr, 1, Hqk, Hv, V, scale, 1, conv);
+    return (int)hipGetLastError();
+  };
+#define GDN_STEP(UN_)                                                                                        \
+  if (units == UN_) {                                                                                        \
+    if (bytes <= 32 * MB) return launch(recurrent_kernel<T, TP, 128, 64, StateLoads::kStream, UN_>);         \
+    if (bytes <= 128 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kStream, UN_>);       \
+    if (bytes < 256 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kCached, UN_>);        \
+    return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kMixed, UN_>);                               \
+  }
+  GDN_STEP(1)
+  GDN_STEP(2)
+  GDN_STEP(4)
+#undef GDN_STEP
   return -3;
 }
 
@@ -333,4 +450,23 @@ extern "C" int gdn_recurrent_fwd_qkv(const void* qkv, int64_t token_stride, cons
                                             state_out, o, B, T, Hqk, Hv, K, V, scale, use_qk_l2norm, s);
   return launch_recurrent<bf16_t, float>(q, k, v, token_stride, token_stride, token_stride, gates, state_in, state_out,
                                          o, B, T, Hqk, Hv, K, V, scale, use_qk_l2norm, s);
+}
+
+extern "C" int gdn_decode_step(const void* hidden, void* conv_state, const void* conv_weight, const void* conv_bias,
+                               const void* a, const void* b, const void* A_log, const void* dt_bias, float* state, void* o,
+                               int B, int Hqk, int Hv, int K, int V, int W, int activation, float scale, int dtype,
+                               int param_dtype, void* stream) {
+  using namespace gdn;
+  if (!hidden || !conv_state || !conv_weight || !a || !b || !A_log || !dt_bias || !state || !o) return -1;
+  if (int e = recurrent_check(B, 1, Hqk, Hv, V)) return e;
+  if (dtype != 0 && dtype != 1) return -4;
+  if (param_dtype != 0 && param_dtype != dtype) return -4;
+  const int row = W * (dtype == 0 ? 4 : 2);
+  if (W != 4 || (((uintptr_t)conv_state | (uintptr_t)conv_weight) & (row - 1)) != 0 || ((uintptr_t)state & 15) != 0) return -3;
+  hipStream_t s = (hipStream_t)stream;
+  const RecurrentConv conv{hidden, conv_state, conv_weight, conv_bias, activation};
+  const RecurrentGates gates{nullptr, nullptr, a, b, A_log, dt_bias};
+  if (dtype == 0) return launch_decode_step<float, float>(conv, gates, state, o, B, Hqk, Hv, K, V, scale, s);
+  if (param_dtype == 1) return launch_decode_step<bf16_t, bf16_t>(conv, gates, state, o, B, Hqk, Hv, K, V, scale, s);
+  return launch_decode_step<bf16_t, float>(conv, gates, state, o, B, Hqk, Hv, K, V, scale, s);
 }

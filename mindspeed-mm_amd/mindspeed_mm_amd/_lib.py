@@ -24,6 +24,7 @@ SIGNATURES = {
     "gdn_recurrent_fwd": (I, [P] * 8 + [I] * 6 + [F, I, I, P]),
     "gdn_recurrent_fwd_packed": (I, [P] * 9 + [I] * 6 + [F, I, I, P]),
     "gdn_recurrent_fwd_qkv": (I, [P, L] + [P] * 7 + [I] * 6 + [F, I, I, I, P]),
+    "gdn_decode_step": (I, [P] * 10 + [I] * 7 + [F, I, I, P]),
     "gdn_conv1d_fwd": (I, [P] * 8 + [I] * 7 + [P]),
     "gdn_conv1d_bwd_workspace_bytes": (L, [I] * 4),
     "gdn_conv1d_bwd": (I, [P] * 12 + [L] + [I] * 7 + [P]),

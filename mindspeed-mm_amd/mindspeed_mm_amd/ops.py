@@ -80,6 +80,9 @@ def _check_packed_length(cu_seqlens, tokens):
                          f"({tokens}), got {cu[0]} ... {cu[-1]}")
 
 
+_ACTIVATIONS = (None, "silu", "swish")
+
+
 def _act_code(activation):
     if activation in ("silu", "swish"):
         return 1
@@ -440,13 +443,44 @@ class GdnOps:
     def decode_step(self, mixed_qkv, a, b, conv_state, recurrent_state, conv_weight, conv_bias, A_log, dt_bias,
                     num_k_heads, num_v_heads, head_k_dim, head_v_dim, activation="silu"):
         """The decode branch of Qwen3_5GatedDeltaNet.forward between the input projections and the gated norm
-        (modeling_qwen3_5.py:738-744, 808-848, 877-890) in two launches: convolution update (conv_state [B,D,S] rolled
-        in place), then the rule on its unsplit output with the gates formed in the kernel (recurrent_state
-        [B,Hv,K,V] fp32 updated in place).  mixed_qkv [B,T,D], a, b [B,T,Hv]; conv_weight [D,W].  Returns o [B,T,Hv,V]."""
+        (modeling_qwen3_5.py:738-744, 808-848, 877-890): convolution update (conv_state [B,D,S] rolled in place), then
+        the rule on its unsplit output with the gates formed in the kernel (recurrent_state [B,Hv,K,V] fp32 updated in
+        place).  mixed_qkv [B,T,D], a, b [B,T,Hv]; conv_weight [D,W].  Returns o [B,T,Hv,V].  One launch where the library
+        takes the step whole (gdn_decode_step), else the two operators in turn; the same bits."""
+        o = self._decode_step_whole(mixed_qkv, a, b, conv_state, recurrent_state, conv_weight, conv_bias, A_log, dt_bias,
+                                    int(num_k_heads), int(num_v_heads), int(head_k_dim), int(head_v_dim), activation)
+        if o is not None:
+            return o
         y = self.causal_conv1d_update(mixed_qkv, conv_state, conv_weight, conv_bias, activation)
         o, _ = self.fused_recurrent_gated_delta_rule_qkv(y, a, b, A_log, dt_bias, num_k_heads, num_v_heads, head_k_dim,
                                                          head_v_dim, initial_state=recurrent_state,
                                                          use_qk_l2norm_in_kernel=True, inplace_state=True)
+        return o
+
+    def _decode_step_whole(self, x, a, b, conv_state, state, weight, bias, A_log, dt_bias, Hqk, Hv, K, V, activation):
+        """The step in one launch, or None where it is not one token per sequence of plain dense operands (the two
+        operators then convert, copy or refuse)."""
+        if x.dim() != 3 or x.shape[1] != 1 or K != 128 or weight.dim() != 2 or weight.shape[1] != 4:
+            return None
+        B, dt, D, pdt = x.shape[0], x.dtype, x.shape[2], A_log.dtype
+        if dt not in (torch.float32, torch.bfloat16) or D != 2 * Hqk * K + Hv * V or activation not in _ACTIVATIONS or \
+                (pdt != dt and pdt != torch.float32) or dt_bias.dtype != pdt or \
+                not (a.dtype == b.dtype == conv_state.dtype == weight.dtype == dt) or \
+                (bias is not None and (bias.dtype != dt or bias.shape != (D,))) or state.dtype != torch.float32 or \
+                a.shape != (B, 1, Hv) or b.shape != (B, 1, Hv) or weight.shape != (D, 4) or \
+                conv_state.shape != (B, D, 4) or state.shape != (B, Hv, K, V) or A_log.shape != (Hv,) or \
+                dt_bias.shape != (Hv,):
+            return None
+        operands = (x, conv_state, weight, bias, a, b, A_log, dt_bias, state)
+        for t in operands:
+            if t is not None and not (t.is_contiguous() and t.device.type == self.lib.device_type):
+                return None
+        o = torch.empty(B, 1, Hv, V, dtype=dt, device=x.device)
+        code = self.lib.gdn_decode_step(*map(ptr, operands), o.data_ptr(), B, Hqk, Hv, K, V, 4, _act_code(activation),
+                                        K ** -0.5, DTYPE_CODE[dt], DTYPE_CODE[pdt], self.lib.stream())
+        if code == -3:   # a shape or an alignment it does not take
+            return None
+        self.lib.check(code, "gdn_decode_step")
         return o
 
     # ------------------------------------------------------------------ conv1d

@@ -211,6 +211,15 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt, wrap=guarded)
 
 
+@pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,K,V,W,pdt", [
+    (BF, 2, 2, 1, 1, 128, 64, 4, None), (F32, 1, 2, 1, 1, 128, 128, 4, None), (BF, 3, 1, 1, 4, 128, 64, 4, torch.float32),
+    (BF, 1, 1, 1, 8, 128, 64, 4, None),
+])
+def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
+    """1, 2 and 4 slabs to a workgroup, and 8, which take the two launches."""
+    P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt, wrap=guarded)
+
+
 @pytest.mark.parametrize("dtype,B,T,D,W,S", [(F32, 2, 3, 16, 4, 6), (BF, 2, 2, 8, 3, 3), (BF, 1, 1, 8, 4, 3)])
 def test_conv1d_update_general_state_length(ops, dtype, B, T, D, W, S):
     P.check_conv_update(ops, "cpu", B, T, D, W, dtype, S=S, wrap=guarded)

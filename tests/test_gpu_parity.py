@@ -529,6 +529,17 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt)
 
 
+@pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,K,V,W,pdt", [
+    (BF, 2, 2, 1, 1, 128, 64, 4, None), (F32, 1, 2, 1, 1, 128, 128, 4, None), (BF, 3, 1, 1, 4, 128, 64, 4, torch.float32),
+    (BF, 1, 1, 1, 8, 128, 64, 4, None), (BF, 16, 1, 16, 32, 128, 128, 4, None), (BF, 17, 1, 16, 32, 128, 128, 4, None),
+    (BF, 65, 1, 8, 32, 128, 128, 4, None), (F32, 127, 1, 32, 32, 128, 128, 4, None),
+    (BF, 128, 1, 16, 32, 128, 128, 4, torch.float32), (BF, 128, 1, 32, 32, 128, 128, 4, None),
+])
+def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
+    """1, 2 and 4 slabs to a workgroup, and 8, which take the two launches; states on either side of 32, 128 and 256 MB."""
+    P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt)
+
+
 def test_decode_cache_prefill_then_steps(ops):
     """Prefill with the chunked operators, hand both states to the cache, decode two more tokens, reorder the beams:
     equal to running the chunked operators over the longer sequences of the reordered batch."""
