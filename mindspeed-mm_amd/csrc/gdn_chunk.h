@@ -34,6 +34,8 @@ struct ChunkWorkspace {
   int64_t chunk_offsets;  // int32 [N+1]      chunks before each packed sequence
   int64_t rstd;           // f32 [2][chunks,Hqk,64] 1/|q|, 1/|k| of the in-kernel l2 norm, 64 contiguous values per chunk
   int64_t G;              // f32 [chunks,Hv,64]      chunk-local cumulative log decay
+  int64_t Bt;             // f32 [chunks,Hv,64]      beta of the chunk's tokens, 0 past its last: as [tokens,Hv] a wave's read of a
+                          //   column of it touches a cache line per token
   int64_t Ai;             // T [chunks,Hv,2,2]       Tm = (I + L)^-1 as A operand: tile = (32 rows) x (32 columns)
   int64_t AQ;             // T [chunks,Hv,2,2]       scale tril(Q K^T . Gam), accumulator tiles: lane <-> column, registers <-> row
   int64_t KAF;            // T [chunks,Hqk,K/32,2]   K as A operand: tile = (32 tokens) x (32 columns of K)
@@ -85,6 +87,7 @@ inline ChunkWorkspace chunk_workspace_layout(const ChunkDims& d, int elem_bytes)
   w.chunk_offsets = take((int64_t)(d.N + 1) * 4);
   w.rstd = take(2 * nc * 64 * d.Hqk * 4);
   w.G = take(nc * 64 * d.Hv * 4);
+  w.Bt = take(nc * 64 * d.Hv * 4);
   w.Ai = take(nc * 64 * d.Hv * 64 * elem_bytes);
   w.AQ = take(nc * 64 * d.Hv * 64 * elem_bytes);
   w.KAF = take(nc * 64 * d.Hqk * d.K * elem_bytes);
@@ -110,7 +113,7 @@ inline ChunkWorkspace chunk_workspace_layout(const ChunkDims& d, int elem_bytes)
 struct KdaWorkspace {
   int64_t chunk_offsets;  // int32 [N+1]
   int64_t rstd;           // f32 [2][chunks,H,64]   1/|q|, 1/|k| of the in-kernel l2 norm
-  int64_t bhat;           // f32 [tokens,H]         beta as the recurrence uses it (after the optional sigmoid)
+  int64_t bhat;           // f32 [chunks,H,64]      beta as the recurrence uses it (after the optional sigmoid), 0 past a chunk's end
   int64_t dec;            // f32 [chunks,H,K]       e^{G_last}: decay of each key channel over the whole chunk
   int64_t Ai;             // T [chunks,H,2,2]       Tm = (I + L)^-1 tiles
   int64_t AQ;             // T [chunks,H,2,2]       scale tril(sum_d q_i k_j e^{G_i-G_j}) tiles
@@ -142,7 +145,7 @@ inline KdaWorkspace kda_workspace_layout(const ChunkDims& d, int elem_bytes) {
   const int64_t nc = d.max_chunks(), H = d.Hv;
   w.chunk_offsets = take((int64_t)(d.N + 1) * 4);
   w.rstd = take(2 * nc * 64 * H * 4);
-  w.bhat = take(d.tokens() * H * 4);
+  w.bhat = take(nc * 64 * H * 4);
   w.dec = take(nc * H * d.K * 4);
   w.Ai = take(nc * 64 * H * 64 * elem_bytes);
   w.AQ = take(nc * 64 * H * 64 * elem_bytes);

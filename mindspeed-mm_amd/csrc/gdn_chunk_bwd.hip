@@ -57,7 +57,7 @@ template <int PIECES, int NT> struct DealB { static constexpr int kPer = (PIECES
 template <typename T, int DK, int NW, int NL, int STAGES, bool KDA = false, bool MAP = false>
 __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 && NL >= 4) ? 2 : 1) void chunk_state_bwd_kernel(
     const T* __restrict__ kaf, const T* __restrict__ kaf2, const T* __restrict__ qtf, const T* __restrict__ ai, const T* __restrict__ aqf,
-    const T* __restrict__ dO, const float* __restrict__ G, const void* __restrict__ beta, int beta_same,
+    const T* __restrict__ dO, const float* __restrict__ G, const float* __restrict__ bt,
     const float* __restrict__ dht,
     float* __restrict__ dh0, T* __restrict__ dvf, T* __restrict__ dhf, const int64_t* __restrict__ cu,
     const int* __restrict__ chunk_offsets, int T_len, int Hqk, int Hv, int V, float scale, int segs) {
@@ -85,8 +85,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
     const int lt = tid - 64 * NW;
     constexpr int DEPTH = (STAGES == 2) ? 2 : 1;
     Vec16<T> pk[DEPTH][CK], pk2[DEPTH][KDA ? CK : 1], pq[DEPTH][CK], ptm[DEPTH][CTM], pa[DEPTH][CTM], pd[DEPTH][CD];
-    float pgl[DEPTH], pgk[DEPTH][2], pgd[DEPTH][CD];
-    uint32_t pbk[DEPTH][2];   // beta as fetched
+    float pgl[DEPTH], pgk[DEPTH][2], pbk[DEPTH][2], pgd[DEPTH][CD];
     int pnv[DEPTH];
     static_assert(NT % (sizeof(T) == 2 ? 128 : 32) == 0, "a thread's pieces sit at one place of their tiles");
     const int krow = frag_piece_row<T>(lt & 127);
@@ -131,7 +130,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         pgk[set][j] = gc[32 * j + krow];
-        pbk[set][j] = gate_raw<T>(beta, beta_same, (tok0 + imin(32 * j + krow, nvalid - 1)) * Hv + h);
+        pbk[set][j] = bt[ch * 64 + 32 * j + krow];
       }
     };
     auto commit = [&](int set, int buf) {
@@ -141,7 +140,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           f1[j] = __expf(pgl[set] - pgk[set][j]);
-          f2[j] = (32 * j + krow < pnv[set]) ? -gate_val<T>(pbk[set][j], beta_same) * __expf(pgk[set][j]) : 0.f;
+          f2[j] = (32 * j + krow < pnv[set]) ? -pbk[set][j] * __expf(pgk[set][j]) : 0.f;
         }
       }
 #pragma unroll
@@ -403,10 +402,10 @@ template <typename T, int DK> struct BwdLocalSmem {
 //   [dQb = dO S^T | dK2 = V' dS'^T | P = dV' S^T : 64 x DK each][dAq = dO V'^T | a2 = dV' V^T : 64 x 64 each, lower tiles]
 // rounded to T like every other tensor that passes between two kernels (they are the largest of them: in fp32 they made
 // up half of what the backward pass moved), and dD = sum_v dS' . S [DK] in kda_dd, in fp32,
-// for kda_bwd_finish_kernel; G is not read and beta is the transformed beta in fp32.
+// for kda_bwd_finish_kernel; G is not read and bt is the transformed beta.  beta_same: the type dbeta leaves in.
 template <typename T, int DK, bool KDA = false>
 __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_local_kernel(
-    const T* __restrict__ qtf, const T* __restrict__ kaf, const T* __restrict__ v, const void* __restrict__ beta, int beta_same,
+    const T* __restrict__ qtf, const T* __restrict__ kaf, const T* __restrict__ v, const float* __restrict__ bt, int beta_same,
     const float* __restrict__ G, const T* __restrict__ Ai, const T* __restrict__ vf, const T* __restrict__ dvf,
     const T* __restrict__ dO, const T* __restrict__ hf, const T* dhf_in, const float* __restrict__ rstd_q,
     const float* __restrict__ rstd_k, T* dq, T* dk, T* __restrict__ dv_out, void* __restrict__ dbeta,
@@ -514,7 +513,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
   if (tid < 64) {   // the row vectors: all requests first, the same ones on every path
     const int tc = imin(tid, nvalid - 1);
     const float gv = KDA ? 0.f : G[ch * 64 + tc], gl = KDA ? 0.f : G[ch * 64 + nvalid - 1];
-    const uint32_t braw = gate_raw<T>(beta, beta_same, (tok0 + tc) * Hv + h);
+    const float bv = bt[ch * 64 + tid];   // 0 past the end
     float rq1 = 1.f, rk1v = 1.f;
     if (l2) {
       rq1 = rstd_q[((int64_t)blockIdx.x * Hqk + hq) * 64 + tc];
@@ -524,7 +523,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     egs[tid] = __expf(gv);
     sgs[tid] = scale * __expf(gv);
     egl[tid] = __expf(gl - gv);
-    bs[tid] = tid < nvalid ? gate_val<T>(braw, beta_same) : 0.f;
+    bs[tid] = bv;
     rsq[tid] = rq1;
     rsk[tid] = rk1v;
   }
@@ -983,7 +982,7 @@ template <typename K> static int set_lds_b(K kernel, int bytes) {
 
 template <typename T, int DK, int NW, int NWS, int NLS, int STAGES>
 static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const void* q, const void* k, const void* v,
-                            const void* beta, int beta_same, const int64_t* cu, const void* dO, const float* dht, void* dq,
+                            int beta_same, const int64_t* cu, const void* dO, const float* dht, void* dq,
                             void* dk, void* dv, float* dg, void* dbeta, float* dh0, unsigned char* ws, unsigned char* ws_state,
                             int phases, float scale, int l2norm, hipStream_t st) {
   // ws, ws_state: bases of the workspace's prep part and state part (see ChunkWorkspace); phases: 2 = the reverse
@@ -992,6 +991,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
   const int* chunk_offsets = reinterpret_cast<const int*>(ws + L.chunk_offsets);
   (void)q; (void)k;   // q and k reach the backward kernels as the forward pass's fragment tiles
   const float* G = reinterpret_cast<const float*>(ws + L.G);
+  const float* Bt = reinterpret_cast<const float*>(ws + L.Bt);
   const T* Ai = reinterpret_cast<const T*>(ws + L.Ai);
   const T* AQ = reinterpret_cast<const T*>(ws + L.AQ);
   const T* VF = reinterpret_cast<const T*>(ws_state + L.VF);
@@ -1012,7 +1012,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         constexpr int smem = StateBwdSmem<T, DK, 2, STAGES>::bytes;
         if (int e = set_lds_b(kern, smem)) return e;
         GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
-                   (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, beta, beta_same,
+                   (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, Bt,
                    (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, segs);
         GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
                    (const float*)maps, dht, starts, cu, d.T, segs, d.Hv, d.V);
@@ -1023,7 +1023,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
     constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
     GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)KAF,
-               (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, beta, beta_same, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V,
+               (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, Bt, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V,
                scale, segs);
   }
   if (phases & 4) {
@@ -1037,7 +1037,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
     if (int e = set_lds_b(kern, smem)) return e;
     for (int hh = 0; hh < d.Hv / d.Hqk; ++hh)
       GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, d.Hqk), dim3(kThreads), smem, st, QTF, (const T*)KAF, (const T*)v,
-                 beta, beta_same, G, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, rstd_q, rstd_k, (T*)dq, (T*)dk,
+                 Bt, beta_same, G, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, rstd_q, rstd_k, (T*)dq, (T*)dk,
                  (T*)dv, dbeta, dg, cu, chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, hh, d.strides(), (T*)nullptr, (float*)nullptr,
                  device_compute_units());
   }
@@ -1090,7 +1090,7 @@ static int chunk_bwd_entry(const void* q, const void* k, const void* v, int64_t 
     if (!(phases & 6)) return 0;
   }
 #define GDN_BWD(T_, DK_, NW_, NWS_, NLS_, ST_)                                                       \
-  return chunk_bwd_launch<T_, DK_, NW_, NWS_, NLS_, ST_>(d, L, q, k, v, beta, beta_same, cu_seqlens, d_o, d_final_state, dq, \
+  return chunk_bwd_launch<T_, DK_, NW_, NWS_, NLS_, ST_>(d, L, q, k, v, beta_same, cu_seqlens, d_o, d_final_state, dq, \
                                                           dk, dv, dg, dbeta, d_initial_state, ws, ws_state, phases, scale, \
                                                           use_qk_l2norm, st)
   const bool wide = (V % 128 == 0);

@@ -178,7 +178,7 @@ template <typename T, int DK>
 __global__ __launch_bounds__(kThreads) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 4 : 3) void chunk_prep_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const float* __restrict__ g, const void* __restrict__ beta,
     int beta_same, const int64_t* __restrict__ cu, const int* __restrict__ chunk_offsets, float* __restrict__ G_out,
-    T* __restrict__ Ai_out, T* __restrict__ Aq_out, T* __restrict__ KA_out, T* __restrict__ QT_out,
+    float* __restrict__ Bt_out, T* __restrict__ Ai_out, T* __restrict__ Aq_out, T* __restrict__ KA_out, T* __restrict__ QT_out,
     float* __restrict__ rstd_q_out, float* __restrict__ rstd_k_out, int T_len, int N, int Hqk, int Hv, float scale,
     int l2norm, TokenStrides ts) {
   using SM = PrepSmem<T, DK>;
@@ -220,6 +220,7 @@ __global__ __launch_bounds__(kThreads) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 4 : 3
     Gs[hh * 128 + lane] = x;
     Gs[hh * 128 + 64 + lane] = b;
     G_out[((int64_t)blockIdx.x * Hv + h) * 64 + lane] = x;   // 64 contiguous values per chunk and head
+    Bt_out[((int64_t)blockIdx.x * Hv + h) * 64 + lane] = b;
   };
   if (wave < grp) head_gates(wave, g_first, b_first);
   for (int hh = wave + 4; hh < grp; hh += 4) {
@@ -347,7 +348,7 @@ template <typename T, int DK, int NW, int STAGES, bool OUT, bool PRE_, bool KDA 
 template <int PIECES, int NT> struct Deal { static constexpr int kPer = (PIECES + NT - 1) / NT; };
 
 // KDA (one decay per key channel): kaf and qtf hold the two K images ready-made, rows scaled by -beta e^{G} and by
-// e^{G_last-G} channel by channel, G holds e^{G_last} [chunks,Hv,DK] and beta the transformed beta in fp32; the state's
+// e^{G_last-G} channel by channel, G holds e^{G_last} [chunks,Hv,DK] and bt the transformed beta; the state's
 // rows decay each by their own factor.  With OUT the output waves take (scale q . e^{G})^T from a third image, qim,
 // whose rows carry every factor of the output's first term (the other modes read their Q^T image through qtf).
 // segs: segments of a sequence, each with its own initial state (gdn_segments.h); MAP: their maps [B | A] into ht.
@@ -355,7 +356,7 @@ template <typename T, int DK, int NW, int NL, int STAGES, bool OUT, bool PRE_, b
 __global__ __launch_bounds__(64 * (NW + (OUT ? NW * StateOutWaves<NW>::value : 0) + NL)) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 2 : 1)
 void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, const T* __restrict__ ai,
                         const T* __restrict__ aqf, const T* __restrict__ v, const float* __restrict__ G,
-                        const void* __restrict__ beta, int beta_same, const float* __restrict__ h0, float* __restrict__ ht,
+                        const float* __restrict__ bt, const float* __restrict__ h0, float* __restrict__ ht,
                         T* __restrict__ vf, T* __restrict__ hf, T* __restrict__ o, const int64_t* __restrict__ cu,
                         const int* __restrict__ chunk_offsets, int T_len, int Hqk, int Hv, int V, float scale,
                         int64_t v_stride, const T* __restrict__ qim, int segs) {
@@ -407,7 +408,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     Vec16<T> pk[DEPTH][CK], ptm[DEPTH][CTM], pv[DEPTH][CV], pq[DEPTH][OUT || KDA ? CK : 1], pa[DEPTH][OUT ? CTM : 1];   // KDA: pq = second K image
     Vec16<T> pq2[DEPTH][OUT && KDA ? CK : 1];   // KDA with output waves: the Q^T image
     float pgl[DEPTH], pg[DEPTH], pgk[DEPTH][2];
-    uint32_t pb[DEPTH], pbk[DEPTH][2], pbv[DEPTH][CV];   // beta as fetched
+    float pb[DEPTH], pbk[DEPTH][2], pbv[DEPTH][CV];   // beta
     int pnv[DEPTH];
     constexpr bool PRE = SM::PRE;
     static_assert(NT % (sizeof(T) == 2 ? 128 : 32) == 0, "a thread's pieces sit at one place of their tiles");
@@ -437,7 +438,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       for (int i = 0; i < CV; ++i) {   // rows past the end of the sequence repeat the last one (their beta is 0)
         const int idc = imin(lt + i * NT, PV - 1), row = imin(idc / VPR, nvalid - 1), cc = idc % VPR;
         pv[set][i] = ld16(v + (tok0 + row) * v_stride + (int64_t)h * V + col0 + cc * VEC);
-        if constexpr (PRE) pbv[set][i] = gate_raw<T>(beta, beta_same, (tok0 + row) * Hv + h);
+        if constexpr (PRE) pbv[set][i] = bt[ch * 64 + row];
       }
       pnv[set] = nvalid;
       if constexpr (KDA) {
@@ -450,14 +451,14 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       // short chunk.
       pgl[set] = gc[63];
       pg[set] = gc[t];
-      pb[set] = gate_raw<T>(beta, beta_same, (tok0 + imin(t, nvalid - 1)) * Hv + h);
+      if constexpr (!PRE) pb[set] = bt[ch * 64 + t];
       if constexpr (PRE) {
         // In the K tiles every 16-byte piece belongs to one token, 32 (tile & 1) + the row of its place, and this
         // thread's pieces all sit at the same place of their tiles: the gates of two tokens cover them.
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           pgk[set][j] = gc[32 * j + krow];
-          pbk[set][j] = gate_raw<T>(beta, beta_same, (tok0 + imin(32 * j + krow, nvalid - 1)) * Hv + h);
+          pbk[set][j] = bt[ch * 64 + 32 * j + krow];
         }
       }
     };
@@ -467,7 +468,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       if constexpr (PRE && !KDA) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          f1[j] = (32 * j + krow < pnv[set]) ? -gate_val<T>(pbk[set][j], beta_same) * __expf(pgk[set][j]) : 0.f;
+          f1[j] = (32 * j + krow < pnv[set]) ? -pbk[set][j] * __expf(pgk[set][j]) : 0.f;
           f2[j] = __expf(pgl[set] - pgk[set][j]);
         }
       }
@@ -496,7 +497,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       for (int i = 0; i < CV; ++i) {
         const int idc = imin(lt + i * NT, PV - 1);
         if (of_a) st16(st + SM::off_v + idc * VEC, zero16<T>());   // not v x 0: v may hold infinities
-        else if constexpr (PRE) st16(st + SM::off_v + idc * VEC, scale16<T>(pv[set][i], idc / VPR < pnv[set] ? gate_val<T>(pbv[set][i], beta_same) : 0.f));
+        else if constexpr (PRE) st16(st + SM::off_v + idc * VEC, scale16<T>(pv[set][i], idc / VPR < pnv[set] ? pbv[set][i] : 0.f));
         else st16(st + SM::off_v + idc * VEC, pv[set][i]);
       }
       float* row = reinterpret_cast<float*>(gdn_smem + buf * SM::stage + SM::off_row);
@@ -505,9 +506,10 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
         return;
       }
       if (lt < 64) {
-        const float b = lt < pnv[set] ? gate_val<T>(pb[set], beta_same) : 0.f, eg = __expf(pg[set]);
+        const float eg = __expf(pg[set]);
         row[lt] = scale * eg;
         if constexpr (!PRE) {
+          const float b = pb[set];
           row[68 + lt] = __expf(pgl[set] - pg[set]);
           row[132 + lt] = b * eg;
           row[196 + lt] = b;
@@ -981,6 +983,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
   if (cu != nullptr && !skip_prep) GDN_LAUNCH(kKernChunkTable, st, chunk_table_kernel, dim3(1), dim3(kThreads), 0, st, cu, chunk_offsets, d.N);
   float* rstd = reinterpret_cast<float*>(ws + L.rstd);
   float* G = reinterpret_cast<float*>(ws + L.G);
+  float* Bt = reinterpret_cast<float*>(ws + L.Bt);
   T* Ai = reinterpret_cast<T*>(ws + L.Ai);
   T* AQ = reinterpret_cast<T*>(ws + L.AQ);
   T* KAF = reinterpret_cast<T*>(ws + L.KAF);
@@ -1003,7 +1006,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
     const int smem = PrepSmem<T, DK>::launch_bytes(d.Hv / d.Hqk);
     if (int e = set_lds(kern, smem)) return e;
     GDN_LAUNCH(kKernPrep, st, kern, dim3(nc, d.Hqk), dim3(kThreads), smem, st, qq, kk, g, beta, beta_same, cu,
-               (const int*)chunk_offsets, G, Ai, AQ, KAF, QTF, rstd, rstd + (int64_t)nc * 64 * d.Hqk, d.T, d.N, d.Hqk,
+               (const int*)chunk_offsets, G, Bt, Ai, AQ, KAF, QTF, rstd, rstd + (int64_t)nc * 64 * d.Hqk, d.T, d.N, d.Hqk,
                d.Hv, scale, l2norm, ts);
   }
   // decided for the two-slab variant, the largest one: results must not depend on how many slabs a launch happens to give a
@@ -1020,7 +1023,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         constexpr int smem = StateSmem<T, DK, 2, STAGES, false, PRE>::bytes;
         if (int e = set_lds(kern, smem)) return e;
         GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
-                   (const T*)KAF, (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, beta, beta_same,
+                   (const T*)KAF, (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, (const float*)Bt,
                    (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T,
                    d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr, segs);
         GDN_LAUNCH(kKernStateFwd, st, (segment_chain_kernel<DK, false>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
@@ -1032,7 +1035,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
   auto launch_state = [&](auto kern, int smem, int waves, T* op) -> int {
     if (int e = set_lds(kern, smem)) return e;
     GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * waves), smem, st, (const T*)KAF,
-               (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, beta, beta_same, h0, ht, VF, HF, op, cu,
+               (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, (const float*)Bt, h0, ht, VF, HF, op, cu,
                (const int*)chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr, segs);
     return 0;
   };

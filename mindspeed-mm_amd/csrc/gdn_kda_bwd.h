@@ -210,7 +210,7 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
   }
   // beta: requested by every wave alike and with the early group (loads arrive in the order of their requests: the
   // store of the row vectors below then waits for P and Tm, not for the requests made behind the gate)
-  const float bh = bhat[(tok0 + imin(lane, nvalid - 1)) * H + h];
+  const float bh = bhat[ch * 64 + lane];   // 0 past the end
   // G: the gate's log decay of every token and channel (0 on the rows past the end) into the place Kp will take,
   // summed down the tokens there, and back into this thread's registers until Kp is consumed
   {
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
     }
   }
   if (tid < 64) {
-    bs[tid] = tid < nvalid ? bh : 0.f;
+    bs[tid] = bh;
     rsq[tid] = 1.f;
     rsk[tid] = 1.f;
   }
@@ -882,7 +882,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
       constexpr int smem = StateBwdSmem<T, DK, 2, STAGES, true>::bytes;
       if (int e = set_lds_b(kern, smem)) return e;
       GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st, K2F, K1F,
-                 QBT, Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr,
+                 QBT, Ai, AQ, (const T*)dO, dec, bhat, (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr,
                  cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
       GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
                  (const float*)maps, dht, starts, cu, d.T, segs, H, d.V);
@@ -894,14 +894,14 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES, true>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
     GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, K2F, K1F, QBT,
-               Ai, AQ, (const T*)dO, dec, (const void*)bhat, 0, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
+               Ai, AQ, (const T*)dO, dec, bhat, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
   }
   {
     auto kern = chunk_bwd_local_kernel<T, DK, true>;
     constexpr int smem = BwdLocalSmem<T, DK>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
     TokenStrides ts = d.strides();
-    GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(kThreads), smem, st, QBT, K1F, (const T*)v, (const void*)bhat, 0,
+    GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(kThreads), smem, st, QBT, K1F, (const T*)v, bhat, 0,
                (const float*)nullptr, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, (const float*)nullptr,
                (const float*)nullptr, (T*)nullptr, (T*)nullptr, (T*)dv, (void*)nullptr, (float*)nullptr, cu, chunk_offsets, d.T,
                d.N, H, H, d.V, scale, 0, ts, DUMP, DD, device_compute_units());

@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kThreads) GDN_WAVES_PER_SIMD(2) void kda_prep_kerne
     }
     if (fl.beta_sigmoid) b = kda_sigmoid(b) * (fl.beta_x2 ? 2.f : 1.f);
     bs[lane] = lane < nvalid ? b : 0.f;
-    if (lane < nvalid) bhat_out[beta_at] = b;
+    bhat_out[ch * 64 + lane] = lane < nvalid ? b : 0.f;
   }
   {
     const int64_t roff = ch * 64;
@@ -493,7 +493,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
       constexpr int smem = StateSmem<T, DK, 2, STAGES, false, true, true>::bytes;
       if (int e = set_lds(kern, smem)) return e;
       GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
-                 (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const void*)bhat, 0,
+                 (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const float*)bhat,
                  (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H,
                  d.V, scale, (int64_t)H * d.V, (const T*)nullptr, segs);
       GDN_LAUNCH(kKernStateFwd, st, (segment_chain_kernel<DK, false>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
@@ -508,7 +508,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     // the per-chunk states and v_new leave the kernel only for a backward pass
     GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * (NWS * (1 + StateOutWaves<NWS>::value) + NLS)),
                smem, st, (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec,
-               (const void*)bhat, 0, h0, ht, with_backward ? VF : (T*)nullptr, with_backward ? HF : (T*)nullptr, (T*)o, cu,
+               (const float*)bhat, h0, ht, with_backward ? VF : (T*)nullptr, with_backward ? HF : (T*)nullptr, (T*)o, cu,
                (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)QBT, segs);
     return (int)hipGetLastError();
   }
@@ -517,7 +517,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     constexpr int smem = StateSmem<T, DK, NWS, STAGES, false, true, true>::bytes;
     if (int e = set_lds(kern, smem)) return e;
     GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)K1F,
-               (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const void*)bhat, 0, h0, ht, VF, HF,
+               (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const float*)bhat, h0, ht, VF, HF,
                (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)nullptr, 1);
   }
   {
