@@ -76,8 +76,10 @@ class GdnLibrary:
             setattr(self, name, fn)
 
     def stream(self):
+        """The current stream of the current device as the C ABI takes it; asked of torch's C layer, since building a
+        torch.cuda.Stream around it on every call costs 2.8 us."""
         if self.device_type == "cuda":
-            return torch.cuda.current_stream().cuda_stream
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
         return None
 
     def check(self, code: int, what: str):

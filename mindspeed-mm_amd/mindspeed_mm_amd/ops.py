@@ -19,6 +19,7 @@ C ABI per operator.  The kernels themselves are the HIP library; nothing in this
 """
 import functools
 import os
+import threading
 import warnings
 from typing import Optional
 
@@ -27,23 +28,44 @@ import torch
 from ._lib import DTYPE_CODE, GdnLibrary, default_library, ptr
 
 
-def _input_guard(fn):
-    """Runs an autograd function's forward / backward with the device of its first tensor argument current, as the
-    reference's input_guard does (mindspeed_mm/fsdp/ops/gdn/triton/utils.py:210-239): the backward pass is called
-    from the autograd engine's thread, where another device may be current."""
+def _on_device_of(args, fn, ctx):
+    """fn(ctx, *args) with the device of the first tensor among args current, as the reference's input_guard does
+    (mindspeed_mm/fsdp/ops/gdn/triton/utils.py:210-239): the backward pass is called by autograd on another thread."""
+    for a in args:
+        if isinstance(a, torch.Tensor):
+            if a.is_cuda and a.get_device() != torch._C._cuda_getDevice():
+                with torch.cuda.device(a.get_device()):
+                    return fn(ctx, *args)
+            break
+    return fn(ctx, *args)
+
+
+def _forward(fn):
+    """An autograd function's forward: on the device of its tensors; the autocast state is noted for the backward pass
+    (triton/utils.py:194-197)."""
     @functools.wraps(fn)
     def wrapper(ctx, *args):
-        dev = next((a.device for a in args if isinstance(a, torch.Tensor)), None)
-        if dev is not None and dev.type == "cuda":
-            with torch.cuda.device(dev):
-                return fn(ctx, *args)
-        return fn(ctx, *args)
+        ctx.autocast = (torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda"))
+        return _on_device_of(args, fn, ctx)
     return wrapper
 
 
-# forward and backward keep the autocast state of the forward call (triton/utils.py:194-197)
-_custom_fwd = functools.partial(torch.amp.custom_fwd, device_type="cuda")
-_custom_bwd = functools.partial(torch.amp.custom_bwd, device_type="cuda")
+def _backward(fn):
+    """Its backward: the same, under the autocast state of the forward call.  Entering an autocast region costs more host
+    time than the launches inside (15 us of a backward pass), so it is entered only where the state differs."""
+    @functools.wraps(fn)
+    def wrapper(ctx, *args):
+        enabled, dtype = ctx.autocast
+        if torch.is_autocast_enabled("cuda") == enabled and torch.get_autocast_dtype("cuda") == dtype:
+            return _on_device_of(args, fn, ctx)
+        with torch.autocast("cuda", dtype=dtype, enabled=enabled):
+            return _on_device_of(args, fn, ctx)
+    return wrapper
+
+
+def _as(t, dtype):
+    """t in `dtype`; None stays None."""
+    return t if t is None or t.dtype == dtype else t.to(dtype)
 
 
 def _out_grad(grad, like):
@@ -60,7 +82,7 @@ def _beta_arg(beta, act_dtype):
     is bf16, modeling_qwen3_5.py:833), else as float32.  Returns (tensor, dtype code)."""
     if beta.dtype == act_dtype and act_dtype == torch.bfloat16:
         return beta.detach().contiguous(), 1
-    return beta.detach().to(torch.float32).contiguous(), 0
+    return _as(beta.detach(), torch.float32).contiguous(), 0
 
 
 def _check_packed_length(cu_seqlens, tokens):
@@ -97,6 +119,7 @@ class GdnOps:
     def __init__(self, lib: GdnLibrary):
         self.lib = lib
         self._helpers = {}
+        self._events = threading.local()
         # False: the backward pass of the chunked rule runs its two recurrences one after the other on the caller's stream
         self.two_stream_backward = os.environ.get("GDN_TWO_STREAM_BACKWARD", "1") != "0"
 
@@ -112,19 +135,34 @@ class GdnOps:
             self._helpers[key] = torch.cuda.Stream(device=key)
         return self._helpers[key]
 
+    def order_after(self, later, earlier, slot):
+        """What `later` is given from here on runs behind what `earlier` holds.  The event between them is kept, one per
+        thread, device and slot (two threads must not record the same one); making and destroying one on every call costs
+        15 us.  While a graph is captured a new one is made: the capture keeps what it records."""
+        if torch.cuda.is_current_stream_capturing():
+            later.wait_stream(earlier)
+            return
+        kept = self._events.__dict__
+        key = (slot, earlier.device_index)
+        if key not in kept:
+            kept[key] = torch.cuda.Event()
+        kept[key].record(earlier)
+        kept[key].wait(later)
+
     # ------------------------------------------------------------------ helpers
     def _need(self, *tensors):
+        cuda = self.lib.device_type == "cuda"
         for t in tensors:
             if not isinstance(t, torch.Tensor):   # None, or cu_seqlens given as a list
                 continue
-            if t.device.type != self.lib.device_type:
+            if not (t.is_cuda if cuda else t.is_cpu):
                 raise RuntimeError(
                     f"tensor on {t.device}; these operators run only on {self.lib.device_type} tensors "
                     "(there is no host fallback)")
 
     @staticmethod
     def _f32(t):
-        return None if t is None else t.detach().to(torch.float32).contiguous()
+        return None if t is None else _as(t.detach(), torch.float32).contiguous()
 
     @staticmethod
     def _no_grad_views(*tensors):
@@ -418,7 +456,7 @@ class GdnOps:
         if D % vec != 0:
             raise ValueError(f"the width of mixed_qkv must be a multiple of {vec} elements")
         pdt = dt if (A_log.dtype == dt and dt_bias.dtype == dt) else torch.float32
-        Ac, dc = A_log.detach().to(pdt).contiguous(), dt_bias.detach().to(pdt).contiguous()
+        Ac, dc = _as(A_log.detach(), pdt).contiguous(), _as(dt_bias.detach(), pdt).contiguous()
         ac, bc = a.contiguous(), b.contiguous()
         o = torch.empty(B, T, Hv, V, dtype=dt, device=x.device)
         s_in = None
@@ -472,8 +510,9 @@ class GdnOps:
                 dt_bias.shape != (Hv,):
             return None
         operands = (x, conv_state, weight, bias, a, b, A_log, dt_bias, state)
+        cuda = self.lib.device_type == "cuda"
         for t in operands:
-            if t is not None and not (t.is_contiguous() and t.device.type == self.lib.device_type):
+            if t is not None and not (t.is_contiguous() and (t.is_cuda if cuda else t.is_cpu)):
                 return None
         o = torch.empty(B, 1, Hv, V, dtype=dt, device=x.device)
         code = self.lib.gdn_decode_step(*map(ptr, operands), o.data_ptr(), B, Hqk, Hv, K, V, 4, _act_code(activation),
@@ -506,8 +545,8 @@ class GdnOps:
         x = hidden_states.contiguous()
         state = conv_state if conv_state.dtype == dt else conv_state.to(dt)
         out = torch.empty_like(x)
-        wc = weight.to(dt).contiguous()
-        bc = None if bias is None else bias.to(dt).contiguous()
+        wc = _as(weight, dt).contiguous()
+        bc = None if bias is None else _as(bias, dt).contiguous()
         code = self.lib.gdn_conv1d_update(ptr(x), ptr(state), ptr(wc), ptr(bc), ptr(out), B, T, D,
                                           W, S, _act_code(activation), DTYPE_CODE[dt], self.lib.stream())
         self.lib.check(code, "gdn_conv1d_update")
@@ -547,9 +586,17 @@ def _chunk_workspace(lib, device, B, T, N, Hqk, Hv, K, V, code, need_grad):
     """A 256-byte aligned workspace; need_grad: False / True for a forward-only or a forward + backward workspace,
     2 / 3 for its prep part / state part alone (gdn_chunk_workspace_bytes)."""
     nbytes = lib.gdn_chunk_workspace_bytes(B, T, N, Hqk, Hv, K, V, code, int(need_grad))
+    return _aligned_bytes(nbytes, device), nbytes
+
+
+def _aligned_bytes(nbytes, device):
+    """nbytes bytes from a 256-byte boundary on, where torch's GPU allocator puts every tensor by itself."""
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if ws.data_ptr() % 256 == 0:
+        return ws
     ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=device)
     off = (-ws.data_ptr()) % 256
-    return ws[off:off + nbytes], nbytes
+    return ws[off:off + nbytes]
 
 
 def _chunk_forward_call(ops, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
@@ -599,24 +646,23 @@ def _chunk_backward_call(ops, saved, meta, do, dht):
         # the prep part was kept: the state part is rebuilt beside the reverse recurrence, then the chunk-local kernels
         ws_state, nstate = _chunk_workspace(lib, dev, B, T, N, Hqk, Hv, K, V, code, 3)
 
-        def phase(ph):
-            rc = lib.gdn_chunk_bwd_parts(ptr(qc), ptr(kc), ptr(vc), sq, sk, sv, ptr(g32), ptr(bc), ptr(h0), ptr(cu),
-                                         ptr(do), ptr(dht), ptr(dq), ptr(dk), ptr(dv), 0, 0, 0, ptr(dg), ptr(db),
-                                         ptr(dh0), ptr(ws), nbytes, ptr(ws_state), nstate, ph, 1, B, T, N, Hqk, Hv, K,
-                                         V, scale, l2, code, bcode, lib.stream())
-            lib.check(rc, "gdn_chunk_bwd_parts")
-        helper = ops.helper_stream(dev)
+        operands = (ptr(qc), ptr(kc), ptr(vc), sq, sk, sv, ptr(g32), ptr(bc), ptr(h0), ptr(cu), ptr(do), ptr(dht), ptr(dq),
+                    ptr(dk), ptr(dv), 0, 0, 0, ptr(dg), ptr(db), ptr(dh0), ptr(ws), nbytes, ptr(ws_state), nstate)
+        sizes = (1, B, T, N, Hqk, Hv, K, V, scale, l2, code, bcode)
+
+        def phase(ph, stream):
+            lib.check(lib.gdn_chunk_bwd_parts(*operands, ph, *sizes, stream), "gdn_chunk_bwd_parts")
+        helper, stream = ops.helper_stream(dev), lib.stream()
         if helper is None:
-            phase(7)
+            phase(7, stream)
         else:
             main = torch.cuda.current_stream(dev)
-            helper.wait_stream(main)
-            with torch.cuda.stream(helper):
-                phase(1)
-            phase(2)
-            main.wait_stream(helper)
-            phase(4)
-        return dq, dk, dv, dg.to(g_dt), db.to(b_dt), None if dh0 is None else dh0.to(h_dt)
+            ops.order_after(helper, main, "fork")
+            phase(1, helper.cuda_stream)
+            phase(2, stream)
+            ops.order_after(main, helper, "join")
+            phase(4, stream)
+        return dq, dk, dv, _as(dg, g_dt), _as(db, b_dt), None if dh0 is None else _as(dh0, h_dt)
     if ws is None:   # nothing was kept: refill a workspace (no output is written when o is null)
         ws, nbytes = _chunk_workspace(lib, dev, B, T, N, Hqk, Hv, K, V, code, True)
         rc = lib.gdn_chunk_fwd_strided(ptr(qc), ptr(kc), ptr(vc), sq, sk, sv, ptr(g32), ptr(bc), ptr(h0), ptr(cu),
@@ -628,7 +674,7 @@ def _chunk_backward_call(ops, saved, meta, do, dht):
                                    ptr(dh0), ptr(ws), nbytes, B, T, N, Hqk, Hv, K, V, scale, l2, code, bcode,
                                    lib.stream())
     lib.check(rc, "gdn_chunk_bwd_strided")
-    return dq, dk, dv, dg.to(g_dt), db.to(b_dt), None if dh0 is None else dh0.to(h_dt)
+    return dq, dk, dv, _as(dg, g_dt), _as(db, b_dt), None if dh0 is None else _as(dh0, h_dt)
 
 
 class _ChunkGatedDeltaRule(torch.autograd.Function):
@@ -644,8 +690,7 @@ class _ChunkGatedDeltaRule(torch.autograd.Function):
     gdn_chunk_workspace_bytes with with_backward=1) and skips that work.  All give the same gradients, bit for bit."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                 use_qk_l2norm_in_kernel, skip_recompute, ops):
         need_grad = any(ctx.needs_input_grad[:5]) or (initial_state is not None and ctx.needs_input_grad[6])
@@ -660,8 +705,7 @@ class _ChunkGatedDeltaRule(torch.autograd.Function):
         return o, ht
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, do, dht):
         do = _out_grad(do, ctx.o_like)
         dq, dk, dv, dg, db, dh0 = _chunk_backward_call(ctx.ops, ctx.saved_tensors, ctx.meta, do, dht)
@@ -673,8 +717,7 @@ class _ChunkGatedDeltaRuleNorm(torch.autograd.Function):
     (the forward then also writes `o` and 1/rms, which they need)."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, q, k, v, g, beta, gate, norm_weight, eps, scale, initial_state, output_final_state, cu_seqlens,
                 use_qk_l2norm_in_kernel, ops):
         lib = ops.lib
@@ -691,7 +734,7 @@ class _ChunkGatedDeltaRuleNorm(torch.autograd.Function):
         code = DTYPE_CODE[dt]
         w_dt = dt if norm_weight.dtype == dt else torch.float32
         gc = gate.detach().to(dt).contiguous().view(B, T, Hv, V)
-        wc = norm_weight.detach().to(w_dt).contiguous()
+        wc = _as(norm_weight.detach(), w_dt).contiguous()
         ws, nbytes = _chunk_workspace(lib, q.device, B, T, N, Hqk, Hv, K, V, code, rule_grad)
         y = torch.empty(B, T, Hv, V, dtype=dt, device=v.device)
         o = torch.empty(B, T, Hv, V, dtype=dt, device=v.device) if need_grad else None
@@ -713,8 +756,7 @@ class _ChunkGatedDeltaRuleNorm(torch.autograd.Function):
         return y, ht
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, dy, dht):
         qc, kc, vc, g32, b32, h0, cu, ws, o, gc, wc, rstd = ctx.saved_tensors
         (B, T, N, Hqk, Hv, K, V, scale, l2, code, nbytes, g_dt, b_dt, h_dt, sq, sk, sv, w_dt, weight_dt, gate_dt,
@@ -745,9 +787,9 @@ class _ChunkGatedDeltaRuleNorm(torch.autograd.Function):
                                            ptr(db), ptr(dh0), ptr(ws), nbytes, B, T, N, Hqk, Hv, K, V, scale, l2,
                                            code, bcode, lib.stream())
             lib.check(rc, "gdn_chunk_bwd_strided")
-            dg, db = dg.to(g_dt), db.to(b_dt)
-            dh0 = None if dh0 is None else dh0.to(h_dt)
-        return (dq, dk, dv, dg, db, dgate.view(gate_shape).to(gate_dt), dw.to(weight_dt), None, None, dh0, None,
+            dg, db = _as(dg, g_dt), _as(db, b_dt)
+            dh0 = None if dh0 is None else _as(dh0, h_dt)
+        return (dq, dk, dv, dg, db, dgate.view(gate_shape).to(gate_dt), _as(dw, weight_dt), None, None, dh0, None,
                 None, None, None)
 
 
@@ -757,8 +799,7 @@ class _ChunkGatedDeltaRuleQKV(torch.autograd.Function):
     backward pass writes dq, dk, dv into one [B,T,D] gradient, so neither the split nor its backward copies."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, qkv, g, beta, Hqk, Hv, K, V, scale, initial_state, output_final_state, cu_seqlens,
                 use_qk_l2norm_in_kernel, ops):
         lib = ops.lib
@@ -791,8 +832,7 @@ class _ChunkGatedDeltaRuleQKV(torch.autograd.Function):
         return o, ht
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, do, dht):
         x, g32, b32, h0, cu, ws = ctx.saved_tensors
         B, T, D, N, Hqk, Hv, K, V, scale, l2, code, nbytes, g_dt, b_dt, h_dt, bcode = ctx.meta
@@ -811,7 +851,7 @@ class _ChunkGatedDeltaRuleQKV(torch.autograd.Function):
                                        D, ptr(dg), ptr(db), ptr(dh0), ptr(ws), nbytes, B, T, N, Hqk, Hv, K, V, scale,
                                        l2, code, bcode, lib.stream())
         lib.check(rc, "gdn_chunk_bwd_strided")
-        return (dx, dg.to(g_dt), db.to(b_dt), None, None, None, None, None, None if dh0 is None else dh0.to(h_dt),
+        return (dx, _as(dg, g_dt), _as(db, b_dt), None, None, None, None, None, None if dh0 is None else _as(dh0, h_dt),
                 None, None, None, None)
 
 
@@ -820,8 +860,7 @@ class _ChunkKda(torch.autograd.Function):
     between the passes when a gradient is asked for)."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, q, k, v, g, beta, A_log, dt_bias, scale, initial_state, output_final_state, l2norm, use_gate,
                 beta_sigmoid, allow_neg, cu_seqlens, lower_bound, want_states, transposed_states, ops):
         lib = ops.lib
@@ -838,9 +877,7 @@ class _ChunkKda(torch.autograd.Function):
         cu = _i64(cu_seqlens, q)
         # the per-chunk states stay in the workspace only when it has the size that serves a backward pass
         nbytes = lib.gdn_kda_workspace_bytes(B, T, N, H, K, V, int(need_grad or want_states), code)
-        ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=q.device)
-        off = (-ws.data_ptr()) % 256
-        ws = ws[off:off + nbytes]
+        ws = _aligned_bytes(nbytes, q.device)
         o = torch.empty(B, T, H, V, dtype=v.dtype, device=v.device)
         ht = torch.empty(N, H, K, V, dtype=torch.float32, device=q.device) if output_final_state else None
         opts = (int(l2norm), int(use_gate), int(lower_bound is not None),
@@ -873,8 +910,7 @@ class _ChunkKda(torch.autograd.Function):
         return o, ht, hs
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, do, dht, _dhs=None):
         qc, kc, vc, gc, a32, d32, cu, ws = ctx.saved_tensors
         B, T, N, H, K, V, scale, opts, nbytes, g_dt, b_dt, bc_dt, a_dt, d_dt, h_dt = ctx.meta
@@ -892,8 +928,8 @@ class _ChunkKda(torch.autograd.Function):
                              ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dA), ptr(dD), ptr(dh0), ptr(ws), nbytes, B, T, N, H, K,
                              V, scale, *opts, lib.stream())
         lib.check(rc, "gdn_kda_bwd")
-        return (dq, dk, dv, dg.to(g_dt), db.to(b_dt), None if dA is None else dA.to(a_dt),
-                None if dD is None else dD.to(d_dt[0]).reshape(d_dt[1]), None, None if dh0 is None else dh0.to(h_dt),
+        return (dq, dk, dv, _as(dg, g_dt), _as(db, b_dt), None if dA is None else _as(dA, a_dt),
+                None if dD is None else dD.to(d_dt[0]).reshape(d_dt[1]), None, None if dh0 is None else _as(dh0, h_dt),
                 None, None, None, None, None, None, None, None, None, None)
 
 
@@ -901,14 +937,13 @@ class _GdnGates(torch.autograd.Function):
     """beta = sigmoid(b), g = -exp(A_log.float()) * softplus(a.float() + dt_bias), modeling_qwen3_5.py:833-841."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, a, b, A_log, dt_bias, ops):
         lib = ops.lib
         Hv = a.shape[-1]
         ac, bc = a.contiguous(), b.contiguous()
         pdt = a.dtype if (A_log.dtype == a.dtype and dt_bias.dtype == a.dtype) else torch.float32
-        Ac, dc = A_log.detach().to(pdt).contiguous(), dt_bias.detach().to(pdt).contiguous()
+        Ac, dc = _as(A_log.detach(), pdt).contiguous(), _as(dt_bias.detach(), pdt).contiguous()
         tokens = ac.numel() // Hv
         g = torch.empty(ac.shape, dtype=torch.float32, device=a.device)
         beta = torch.empty_like(bc)
@@ -921,8 +956,7 @@ class _GdnGates(torch.autograd.Function):
         return g, beta
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, dg, dbeta):
         ac, bc, Ac, dc = ctx.saved_tensors
         tokens, Hv, A_dt, d_dt = ctx.meta
@@ -938,15 +972,14 @@ class _GdnGates(torch.autograd.Function):
                               ptr(dd), ptr(ws), nbytes, tokens, Hv, DTYPE_CODE[ac.dtype], DTYPE_CODE[Ac.dtype],
                               lib.stream())
         lib.check(rc, "gdn_gate_bwd")
-        return da, db, dA.to(A_dt), dd.to(d_dt), None
+        return da, db, _as(dA, A_dt), _as(dd, d_dt), None
 
 
 class _CausalConv1d(torch.autograd.Function):
     """Argument order as CausalConv1dFunction.forward (models/qwen3_5/causal_conv1d.py:27-38)."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, x, weight, bias, residual, initial_state, activation, cu_seqlens, output_final_state, ops):
         lib = ops.lib
         B, T, D = x.shape
@@ -954,8 +987,8 @@ class _CausalConv1d(torch.autograd.Function):
         N = (len(cu_seqlens) - 1) if cu_seqlens is not None else B
         dt = x.dtype
         xc = x.contiguous()
-        wc = weight.to(dt).contiguous()
-        bc = None if bias is None else bias.to(dt).contiguous()
+        wc = _as(weight, dt).contiguous()
+        bc = None if bias is None else _as(bias, dt).contiguous()
         rc_ = None if residual is None else residual.to(dt).contiguous()
         h0 = None if initial_state is None else initial_state.to(dt).contiguous()
         cu = _i64(cu_seqlens, x)
@@ -972,13 +1005,12 @@ class _CausalConv1d(torch.autograd.Function):
         return y, fs
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, dy, dfs):
         xc, wc, bc, h0, cu = ctx.saved_tensors
         B, T, N, D, W, act, dt, w_dt, b_dt, has_res, r_dt, h_dt = ctx.meta
         lib = ctx.ops.lib
-        dy = dy.to(dt).contiguous()
+        dy = _as(dy, dt).contiguous()
         dfs = None if dfs is None else dfs.to(dt).contiguous()
         dx = torch.empty_like(xc)
         dw = torch.empty(W, D, dtype=torch.float32, device=xc.device)
@@ -989,8 +1021,8 @@ class _CausalConv1d(torch.autograd.Function):
         code = lib.gdn_conv1d_bwd(ptr(xc), ptr(dy), ptr(wc), ptr(bc), ptr(h0), ptr(dfs), ptr(cu), ptr(dx), ptr(dw),
                                   ptr(db), ptr(dh0), ptr(ws), nbytes, B, T, N, D, W, act, DTYPE_CODE[dt], lib.stream())
         lib.check(code, "gdn_conv1d_bwd")
-        return (dx, dw.to(w_dt), None if db is None else db.to(b_dt), dy.to(r_dt) if has_res else None,
-                None if dh0 is None else dh0.to(h_dt), None, None, None, None)
+        return (dx, _as(dw, w_dt), None if db is None else _as(db, b_dt), dy.to(r_dt) if has_res else None,
+                None if dh0 is None else _as(dh0, h_dt), None, None, None, None)
 
 
 _GATE_ACTIVATION = {"silu": 0, "swish": 0, "sigmoid": 1}
@@ -1000,8 +1032,7 @@ class _RMSNormGated(torch.autograd.Function):
     """y = (weight * rmsnorm(x)) * act(gate) over the last axis, act = silu (code 0) or sigmoid (code 1)."""
 
     @staticmethod
-    @_input_guard
-    @_custom_fwd
+    @_forward
     def forward(ctx, x, gate, weight, eps, ops, act=0):
         lib = ops.lib
         dt = x.dtype
@@ -1014,8 +1045,8 @@ class _RMSNormGated(torch.autograd.Function):
             raise ValueError(f"weight shape {tuple(weight.shape)}, expected ({N},)")
         w_dt = dt if weight.dtype == dt else torch.float32   # same dtype as the input, else fp32 as in the reference
         xc = x.contiguous().view(-1, N)
-        gc = gate.to(dt).contiguous().view(-1, N)
-        wc = weight.detach().to(w_dt).contiguous()
+        gc = _as(gate, dt).contiguous().view(-1, N)
+        wc = _as(weight.detach(), w_dt).contiguous()
         rows = xc.shape[0]
         y = torch.empty_like(xc)
         rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
@@ -1028,13 +1059,12 @@ class _RMSNormGated(torch.autograd.Function):
         return y.view(x.shape)
 
     @staticmethod
-    @_input_guard
-    @_custom_bwd
+    @_backward
     def backward(ctx, dy):
         xc, gc, wc, rstd = ctx.saved_tensors
         rows, N, dt, w_dt, weight_dt, gate_dt, shape, act = ctx.meta
         lib = ctx.ops.lib
-        dyc = dy.to(dt).contiguous().view(-1, N)
+        dyc = _as(dy, dt).contiguous().view(-1, N)
         dx = torch.empty_like(xc)
         dg = torch.empty_like(xc)
         dw = torch.empty(N, dtype=torch.float32, device=xc.device)
@@ -1043,7 +1073,7 @@ class _RMSNormGated(torch.autograd.Function):
         code = lib.gdn_rmsnorm_gated_bwd(ptr(xc), ptr(gc), ptr(wc), ptr(rstd), ptr(dyc), ptr(dx), ptr(dg), ptr(dw),
                                          ptr(ws), nbytes, rows, N, DTYPE_CODE[dt], DTYPE_CODE[w_dt], act, lib.stream())
         lib.check(code, "gdn_rmsnorm_gated_bwd")
-        return dx.view(shape), dg.view(shape).to(gate_dt), dw.to(weight_dt), None, None, None
+        return dx.view(shape), dg.view(shape).to(gate_dt), _as(dw, weight_dt), None, None, None
 
 
 # ---------------------------------------------------------------------- module-level entry points

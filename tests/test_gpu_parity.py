@@ -1,6 +1,8 @@
 """GPU parity tests proper: the shipped HIP library (through the package's C-ABI binding) against the CPU
 oracle on the same seeded inputs.  Run with `-m gpu` on an MI355X."""
 import pytest
+import threading
+
 import torch
 
 from oracle import gdn_oracle as O
@@ -803,3 +805,57 @@ def test_kda_random_shapes(ops, seed):
     errs = P.check_kda(ops, "cuda", B, T, H, K, V, dtype, cu=cu, backward=True, seed=seed, **kw)
     print("   ", {n: f"{e:.2e}" for n, e in errs.items()}, flush=True)
 
+
+
+def _training_call(ops, x):
+    leaf = {n: x[n].detach().requires_grad_(True) for n in ("q", "k", "v", "g", "beta")}
+    o, _ = ops.chunk_gated_delta_rule(*leaf.values(), use_qk_l2norm_in_kernel=True)
+    return [o.detach(), *torch.autograd.grad([o], list(leaf.values()), [x["do"]])]
+
+
+def test_backward_on_two_streams_from_two_threads(ops):
+    """The events that order the backward pass's two streams are kept from call to call: two threads, each on a stream of its
+    own, and calls of other sizes in between, get the gradients of calls that run alone."""
+    xs = [{n: t.cuda() for n, t in P.gdn_inputs(1, T, 2, 4, 128, 128, BF, seed=T).items()} for T in (700, 2000)]
+    want = [_training_call(ops, x) for x in xs]
+    torch.cuda.synchronize()
+    got, errors = {}, []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for n in range(8):
+                    got[i] = _training_call(ops, xs[(i + n + 1) % 2])
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:   # noqa: BLE001 -- shown by the assertion below
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for i in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(got[i], want[i]))
+
+
+def test_training_call_in_a_graph(ops):
+    """Forward and two-stream backward captured and replayed several times, with eager calls in between."""
+    x = {n: t.cuda() for n, t in P.gdn_inputs(1, 300, 2, 4, 128, 128, BF, seed=3).items()}
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = _training_call(ops, x)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = _training_call(ops, x)
+    for n in range(4):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, want)), n
+        assert all(torch.equal(a, b) for a, b in zip(_training_call(ops, x), want)), n
+        torch.cuda.synchronize()
