@@ -16,6 +16,7 @@
 // chunk_o.py:19-284, chunk_delta_h.py:307-513, wy_fast.py:17-141, chunk_gated_delta_rule.py:88-174), with
 // the dG row/column sums rewritten as row dot products with dQ/dK so that Q K^T need not be rebuilt.
 #include "gdn_chunk.h"
+#include "gdn_chunk_f32.h"
 #include "gdn_common.h"
 #include "gdn_profile.h"
 #include "gdn_segments.h"
@@ -1019,12 +1020,26 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         dht = starts;
       }
     }
-    auto kern = chunk_state_bwd_kernel<T, DK, NWS, NLS, STAGES>;
-    constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES>::bytes;
-    if (int e = set_lds_b(kern, smem)) return e;
-    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)KAF,
-               (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, Bt, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V,
-               scale, segs);
+    if constexpr (sizeof(T) == 4) {
+      auto launch_f32 = [&](auto kern, int smem, int cols) -> int {
+        if (int e = set_lds_b(kern, smem)) return e;
+        GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * d.Hv, d.V / cols), dim3(kF32Threads), smem, st, (const float*)KAF,
+                   (const float*)QTF, (const float*)Ai, (const float*)AQ, (const float*)dO, G, Bt, dht, dh0, (float*)DVF,
+                   (float*)DHF, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale);
+        return 0;
+      };
+      if (int e = f32_sixteen_columns(d.N, d.Hv, d.V, device_compute_units())
+                      ? launch_f32(chunk_state_bwd_f32_kernel<DK, 1>, StateBwdF32Smem<DK, 1>::bytes, 16)
+                      : launch_f32(chunk_state_bwd_f32_kernel<DK, 2>, StateBwdF32Smem<DK, 2>::bytes, 32))
+        return e;
+    } else {
+      auto kern = chunk_state_bwd_kernel<T, DK, NWS, NLS, STAGES>;
+      constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES>::bytes;
+      if (int e = set_lds_b(kern, smem)) return e;
+      GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st,
+                 (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, Bt, dht, dh0, DVF, DHF, cu,
+                 chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, segs);
+    }
   }
   if (phases & 4) {
     const TokenStrides gs = d.strides();

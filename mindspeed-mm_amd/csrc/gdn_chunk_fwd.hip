@@ -12,6 +12,7 @@
 //     chunk_out_kernel    per (chunk, head, 32-column block): O
 // A ragged last chunk is zero padded in LDS (k = v = beta = g = 0 is exact for this recurrence).
 #include "gdn_chunk.h"
+#include "gdn_chunk_f32.h"
 #include "gdn_common.h"
 #include "gdn_profile.h"
 #include "gdn_segments.h"
@@ -1047,9 +1048,22 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
       return (int)hipGetLastError();
     }
   }
-  if (int e = launch_state(chunk_state_kernel<T, DK, NWS, NLS, STAGES, false, PRE>,
-                           StateSmem<T, DK, NWS, STAGES, false, PRE>::bytes, NWS + NLS, (T*)nullptr))
+  if constexpr (sizeof(T) == 4) {
+    auto launch_f32 = [&](auto kern, int smem, int cols) -> int {
+      if (int e = set_lds(kern, smem)) return e;
+      GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * d.Hv, d.V / cols), dim3(kF32Threads), smem, st, (const float*)KAF,
+                 (const float*)Ai, (const float*)v, (const float*)G, (const float*)Bt, h0, ht, (float*)VF, (float*)HF, cu,
+                 (const int*)chunk_offsets, d.T, d.Hqk, d.Hv, d.V, ts.v);
+      return 0;
+    };
+    if (int e = f32_sixteen_columns(d.N, d.Hv, d.V, device_compute_units())
+                    ? launch_f32(chunk_state_f32_kernel<DK, 1>, StateF32Smem<DK, 1>::bytes, 16)
+                    : launch_f32(chunk_state_f32_kernel<DK, 2>, StateF32Smem<DK, 2>::bytes, 32))
+      return e;
+  } else if (int e = launch_state(chunk_state_kernel<T, DK, NWS, NLS, STAGES, false, PRE>,
+                                  StateSmem<T, DK, NWS, STAGES, false, PRE>::bytes, NWS + NLS, (T*)nullptr)) {
     return e;
+  }
   if (fill_only) return (int)hipGetLastError();
   auto launch_out = [&](auto kern, auto nm) -> int {
     constexpr int smem = OutSmem<T, DK, NW>::bytes;
