@@ -722,9 +722,20 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     // y = K S (PRE: z = beta v - beta e^G . (K S) at once), the two 32-token blocks are independent accumulation
     // chains.  The decay of S rides between the matrix instructions.
     f32x16 p0 = PRE ? Vb[0].unpack() : acc_zero(), p1 = PRE ? Vb[1].unpack() : acc_zero();
+    // What the chain needs next is read from LDS while the matrix pipe works on what it has: Tm ahead of the last pair of
+    // K tiles, the row factors between its products, K^T behind those with Tm.  The fences keep the compiler from moving
+    // the reads to their uses, where each would be waited for.  Forward only 2 x 8192, 32 heads 199 -> 193 us, four packed
+    // prompts 353 -> 344; K^T ahead of the last pair as well spills 33 registers and takes 393.
+    static_assert(NP <= 2, "two buffers of K tiles");
+    f32x16 b0, b1, e0, e1;                  // !PRE: beta and beta e^G of the rows
     GDN_SCHED_FENCE();
 #pragma unroll
     for (int kp = 0; kp < NP; ++kp) {
+      if (kp == NP - 1) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) Tf[t].load(Tm + t * 1024);
+        GDN_SCHED_FENCE();
+      }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         mma2(p0, Kf[kp & 1][0][j], Sb[2 * kp + j], p1, Kf[kp & 1][1][j], Sb[2 * kp + j]);
@@ -737,48 +748,59 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
           for (int r = 0; r < 16; ++r) S[2 * kp + j][r] *= eg;
         }
         GDN_INTERLEAVE_MFMA_VALU(2 * AccK<T>::kGroups, 16 / (2 * AccK<T>::kGroups));
+        if constexpr (!PRE) {
+          if (kp == NP - 1) {
+            GDN_SCHED_FENCE();
+            if (j == 0) { b0 = rows_ld(row + 196, 0); e0 = rows_ld(row + 132, 0); }
+            else { b1 = rows_ld(row + 196, 32); e1 = rows_ld(row + 132, 32); }
+            GDN_SCHED_FENCE();
+          }
+        }
       }
       GDN_SCHED_FENCE();
-      if (kp + 2 < NP) load_k(kp & 1, kp + 2);
-      GDN_SCHED_FENCE();
     }
+    if constexpr (!PRE) {   // z = beta (v - e^G . y), the B operand of Tm z
+      const f32x16 x0 = Vb[0].unpack();
 #pragma unroll
-    for (int t = 0; t < 3; ++t) Tf[t].load(Tm + t * 1024);
-    if constexpr (!PRE) {
-      // z = beta (v - e^G . y), the B operand of Tm z
-      const f32x16 b0 = rows_ld(row + 196, 0), b1 = rows_ld(row + 196, 32);
-      const f32x16 e0 = rows_ld(row + 132, 0), e1 = rows_ld(row + 132, 32);
-      const f32x16 x0 = Vb[0].unpack(), x1 = Vb[1].unpack();
-#pragma unroll
-      for (int r = 0; r < 16; ++r) { p0[r] = b0[r] * x0[r] - e0[r] * p0[r]; p1[r] = b1[r] * x1[r] - e1[r] * p1[r]; }
+      for (int r = 0; r < 16; ++r) p0[r] = b0[r] * x0[r] - e0[r] * p0[r];
     }
     Vb[0].pack(p0);
-    Vb[1].pack(p1);
+    // V' = Tm z (Tm lower triangular: tiles (0,0), (1,0), (1,1)); the second block's z is formed beside the first products
+    f32x16 w0 = acc_zero(), w1 = acc_zero();
+    mma2(w0, Tf[0], Vb[0], w1, Tf[1], Vb[0]);
+    GDN_SCHED_FENCE();
     load_kt(0, 0);
-    // V' = Tm z (Tm lower triangular: tiles (0,0), (1,0), (1,1))
-    p0 = acc_zero();
-    p1 = acc_zero();
-    mma2(p0, Tf[0], Vb[0], p1, Tf[1], Vb[0]);
-    mma32_ff<T>(p1, Tf[2], Vb[1]);
-    if (NP > 1) load_kt(1, 1);
-    Vb[0].pack(p0);
+    GDN_SCHED_FENCE();
+    if constexpr (!PRE) {
+      const f32x16 x1 = Vb[1].unpack();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p1[r] = b1[r] * x1[r] - e1[r] * p1[r];
+    }
     Vb[1].pack(p1);
-    if (!OUT && vf != nullptr) {
-      Vb[0].store_stream(vf + (tile0 * 2 + 0) * 1024);
-      Vb[1].store_stream(vf + (tile0 * 2 + 1) * 1024);
-    }
-    if constexpr (OUT) {
-      T* vx = xs + 2 * DK * 32 + (c & 1) * 2048;
-      Vb[0].store(vx);
-      Vb[1].store(vx + 1024);
-    }
+    f32x16 d0, d1;                          // !PRE: e^{G_last-G} of the rows
+    if constexpr (!PRE) { d0 = rows_ld(row + 68, 0); d1 = rows_ld(row + 68, 32); }
+    GDN_SCHED_FENCE();
+    mma32_ff<T>(w1, Tf[2], Vb[1]);
+    GDN_SCHED_FENCE();
+    if (NP > 1) load_kt(1, 1);
+    GDN_SCHED_FENCE();
+    Vb[0].pack(w0);
+    T* const vx = xs + 2 * DK * 32 + (c & 1) * 2048;   // OUT only
+    if constexpr (OUT) Vb[0].store(vx);
+    else if (vf != nullptr) Vb[0].store_stream(vf + (tile0 * 2 + 0) * 1024);
     if constexpr (!PRE) {
       // the decay of the state update rides on V': (e^{G_last - G} . K)^T V' = K^T (e^{G_last - G} . V')
-      const f32x16 d0 = rows_ld(row + 68, 0), d1 = rows_ld(row + 68, 32);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { p0[r] *= d0[r]; p1[r] *= d1[r]; }
-      Vb[0].pack(p0);
-      Vb[1].pack(p1);
+      for (int r = 0; r < 16; ++r) w0[r] *= d0[r];
+      Vb[0].pack(w0);
+    }
+    Vb[1].pack(w1);
+    if constexpr (OUT) Vb[1].store(vx + 1024);
+    else if (vf != nullptr) Vb[1].store_stream(vf + (tile0 * 2 + 1) * 1024);
+    if constexpr (!PRE) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) w1[r] *= d1[r];
+      Vb[1].pack(w1);
     }
     GDN_SCHED_FENCE();
     // S <- e^{G_last} S + K^T (e^{G_last - G} . V'); a finished tile of S is packed for the next chunk while the
