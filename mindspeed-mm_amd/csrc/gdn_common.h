@@ -894,7 +894,7 @@ __device__ __forceinline__ void tile_qk_finish(TileQK<T, DK, NT>& t, T* lds, int
 
 // ---------------------------------------------------------------------------------------------
 // Packed-sequence bookkeeping.  chunk_offsets[n] = number of 64-token chunks before sequence n
-// (chunk_offsets[N] = total); built on the device by gdn_chunk_table_kernel so that no host sync is
+// (chunk_offsets[N] = total); built on the device by chunk_table_kernel so that no host sync is
 // needed.  Without cu_seqlens every batch row is a sequence of T tokens.
 // ---------------------------------------------------------------------------------------------
 struct SeqInfo {
@@ -939,7 +939,7 @@ struct TailRows {
   int64_t row_stride[6];      // bytes between consecutive tokens
   int row_bytes[6];           // bytes to clear per token (a multiple of 2)
 };
-static __global__ void zero_tail_rows_kernel(const int64_t* __restrict__ cu, int N, int64_t tokens, TailRows t) {
+__device__ __forceinline__ void zero_tail_rows(const int64_t* cu, int N, int64_t tokens, const TailRows& t) {
   const int64_t covered = cu[N], lo = (int64_t)blockIdx.x * 64, hi = lo + 64 < tokens ? lo + 64 : tokens;
   if (hi <= covered) return;
   const int64_t first = lo > covered ? lo : covered;
@@ -956,6 +956,9 @@ static __global__ void zero_tail_rows_kernel(const int64_t* __restrict__ cu, int
         reinterpret_cast<uint16_t*>(b + (first + i / halves) * t.row_stride[a])[i % halves] = 0;
     }
   }
+}
+static __global__ void zero_tail_rows_kernel(const int64_t* __restrict__ cu, int N, int64_t tokens, TailRows t) {
+  zero_tail_rows(cu, N, tokens, t);
 }
 static inline void launch_zero_tail_rows(const int64_t* cu, int N, int64_t tokens, const TailRows& t, hipStream_t st) {
   if (cu == nullptr || tokens <= 0) return;

@@ -175,3 +175,36 @@ def test_sequence_bits_alone_and_in_a_batch(ops):
         return o[:, :4096], ht[:1]
     alone, packed = first(4096, 1, [0, 4096]), first(8192, 2, [0, 4096, 8192])
     assert torch.equal(alone[0], packed[0]) and torch.equal(alone[1], packed[1])
+
+
+@pytest.mark.parametrize("N", [1, 64, 65, 256, 257, 520])
+def test_chunk_table_of_many_sequences(ops, N):
+    """A wave and a workgroup of sequences, one more, several to a thread, empty ones among them: every sequence as in a
+    dense batch of its length, bit for bit, and zeros in the rows behind the last one."""
+    gen = torch.Generator().manual_seed(N)
+    kinds = [0, 1, 64, 65]
+    lengths = [kinds[i] for i in torch.randint(0, 4, (N,), generator=gen).tolist()]
+    lengths[-1] = 65
+    cu = [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    T, tail, K = cu[-1], 70, 64
+    x = P.gdn_inputs(1, T + tail, 1, 1, K, K, BF, seed=N)
+    x = {n: t.cuda() for n, t in x.items()}
+    print(f"chunk table: {N} sequences, {T} tokens", flush=True)
+
+    def rule(rows, h0, cu_t):
+        return ops.chunk_gated_delta_rule(*(rows(x[n]) for n in ("q", "k", "v", "g", "beta")), initial_state=h0,
+                                          output_final_state=True, use_qk_l2norm_in_kernel=True, cu_seqlens=cu_t)
+    h0 = torch.randn(N, 1, K, K, generator=gen).cuda()
+    with torch.no_grad():
+        o, ht = rule(lambda t: t, h0, torch.tensor(cu).cuda())
+        for L in kinds:
+            at = [n for n in range(N) if lengths[n] == L]
+            if L == 0 or not at:
+                assert all(torch.equal(ht[n], h0[n]) for n in at)
+                continue
+            idx = torch.tensor([[cu[n] + i for i in range(L)] for n in at]).cuda()
+            ob, hb = rule(lambda t: t[0][idx], h0[at], None)
+            assert torch.equal(o[0][idx], ob) and torch.equal(ht[at], hb)
+    assert not o[0, T:].any()
