@@ -60,6 +60,30 @@ __device__ __forceinline__ void load_hist(float* dst, const T* x, const T* init,
   }
 }
 
+// final_state[n, d, w] = x[T_n - W + w] (the initial state or zero ahead of the sequence) of V channels, bit for bit.  The
+// sequence may be empty, which is why no tile of tokens can be left to do it.  In workgroups of the forward launch: one of
+// its own behind it took 4.8 us (4 sequences of 8192 channels) and the host's share of a launch.
+template <typename T, int W>
+__device__ __forceinline__ void packed_final_state(const T* x, const T* init, const int64_t* cu, T* fs, int n, int D, int d0) {
+  constexpr int V = Elem<T>::kVec;
+  const int64_t bos = cu[n], len = cu[n + 1] - bos, at = ((int64_t)n * D + d0) * W;
+  T rows[W][V], out[W * V];
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    const int64_t src = len - W + w;
+    if (src >= 0) {
+      const Vec16<T> r = ld16(x + (bos + src) * D + d0);
+      __builtin_memcpy(rows[w], &r.raw, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e) rows[w][e] = init != nullptr ? init[at + e * W + src + W] : Elem<T>::from_f(0.f);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < W * V; ++i) out[i] = rows[i % W][i / W];
+  __builtin_memcpy(fs + at, out, sizeof(out));
+}
+
 // v_rcp_f32 (1 ulp) instead of an IEEE division: ten instructions fewer per element
 
 // TT tokens per workgroup, their rows and the W-1 before them requested at once.  A tile that lies inside one sequence,
@@ -80,6 +104,11 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) vo
   const int64_t t0 = (first_tile + blockIdx.x / nbd) * TT;
   const int d0 = (bx * kConvThreads + threadIdx.x) * V;
   if (d0 >= D) return;
+  if (t0 >= total) {   // behind the tiles of a packed batch: the final state of one sequence each
+    packed_final_state<T, W>(x, init, cu, fs, (int)(t0 / TT - (total + TT - 1) / TT), D, d0);
+    return;
+  }
+  if (cu != nullptr) fs = nullptr;   // the tiles write it for dense batches only
   float wgt[W][V], bs[V], win[W][V];
   SeqCursor cur;
   auto finish = [&](int64_t t, int u) {   // token t; the window's logical row j sits in slot (u + j) % W
@@ -162,9 +191,9 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) vo
   }
 }
 
-// final_state[n,d,w] = x[T_n - W + w] (falls back to the initial state / zero for T_n < W).  For packed input, where a
-// sequence may be empty, and where the state is updated in place (a thread reads ahead of what it writes, and only its own
-// channel); otherwise the forward kernel writes the state itself.
+// final_state[n,d,w] = x[T_n - W + w] (falls back to the initial state / zero for T_n < W).  Where the state is updated
+// in place (a thread reads ahead of what it writes, and only its own channel) or there is no token; otherwise the forward
+// kernel writes the state itself.
 template <typename T>
 __global__ void conv1d_final_state_kernel(const T* __restrict__ x, const T* init,
                                           const int64_t* __restrict__ cu, T* fs, int T_len, int N, int D,
@@ -531,10 +560,11 @@ template <typename T> struct ConvLaunch {
     const int64_t total = (int64_t)B * T_len;
     const int nbd = (D / V + kConvThreads - 1) / kConvThreads;
     if ((int64_t)nbd * kConvThreads > GDN_MAX_LAUNCH_THREADS) return -3;
-    const int64_t ntiles = (total + TT - 1) / TT, most = GDN_MAX_LAUNCH_THREADS / ((int64_t)nbd * kConvThreads);
-    // every sequence of a dense batch has a last token, whose tile can write the final state -- but not over the initial
-    // state, which the sequence's first tile may still be reading
-    const bool fs_inside = cu == nullptr && total > 0 && fs != init;
+    // every sequence of a dense batch has a last token, whose tile can write the final state, and workgroups behind the tiles
+    // write that of packed ones -- but not over the initial state, which the sequence's first tile may still be reading
+    const bool fs_inside = total > 0 && fs != init;
+    const int64_t ntiles = (total + TT - 1) / TT + (cu != nullptr && fs != nullptr && fs_inside ? N : 0);
+    const int64_t most = GDN_MAX_LAUNCH_THREADS / ((int64_t)nbd * kConvThreads);
     if (total > 0) {
       auto launch = [&](auto kern) {
         for (int64_t t = 0; t < ntiles; t += most) {   // 8 channels: 4 GB of x to a launch

@@ -78,6 +78,28 @@ def test_conv1d_more_work_items_than_a_launch(ops):
             assert torch.equal(y[:, at:at + n], part[:, at - lo:])
 
 
+@pytest.mark.parametrize("dtype,W,D", [(BF, 4, 1032), (BF, 1, 8), (BF, 8, 16), (F32, 3, 20)])
+@pytest.mark.parametrize("initial", ["none", "given", "in place"])
+@pytest.mark.parametrize("cu", [[0, 0, 1, 3, 3, 6, 10, 27, 32, 32], [0, 5], [0, 0, 0, 8]])
+def test_conv1d_final_states_of_packed_sequences(ops, dtype, W, D, initial, cu):
+    """Empty, shorter than the window, ending on a tile's edge and inside one: the states are copies, bit for bit."""
+    from mindspeed_mm_amd._lib import DTYPE_CODE, ptr
+    gen = torch.Generator().manual_seed(W)
+    T, N = cu[-1], len(cu) - 1
+    x, w = torch.randn(T, D, generator=gen).to(dtype), torch.randn(W, D, generator=gen).to(dtype)
+    init = None if initial == "none" else torch.randn(N, D, W, generator=gen).to(dtype)
+    want = torch.empty(N, D, W, dtype=dtype)
+    for n in range(N):
+        before = torch.zeros(D, W, dtype=dtype) if init is None else init[n]
+        want[n] = torch.cat([before, x[cu[n]:cu[n + 1]].t()], dim=1)[:, -W:]
+    xd, wd, cud, h0 = x.cuda(), w.cuda(), torch.tensor(cu).cuda(), None if init is None else init.cuda()
+    y, fs = torch.empty_like(xd), h0 if initial == "in place" else torch.empty(N, D, W, dtype=dtype, device="cuda")
+    print(f"conv1d packed final states {dtype} W{W} D{D} {initial} {cu}", flush=True)
+    ops.lib.check(ops.lib.gdn_conv1d_fwd(ptr(xd), ptr(wd), None, None, ptr(h0), ptr(cud), ptr(y), ptr(fs), 1, T, N, D, W, 0,
+                                         DTYPE_CODE[dtype], ops.lib.stream()), "gdn_conv1d_fwd")
+    assert torch.equal(fs.cpu(), want)
+
+
 @pytest.mark.parametrize("dtype,B,T,Hqk,Hv,K,V", [
     (BF, 8, 1, 16, 32, 128, 128), (BF, 9, 1, 16, 32, 128, 128),    # as many states as compute units; more: whole states
     (BF, 17, 1, 16, 32, 128, 128),                                 # states larger than the L2s
