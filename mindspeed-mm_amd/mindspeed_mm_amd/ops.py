@@ -498,8 +498,8 @@ class GdnOps:
     def _decode_step_whole(self, x, a, b, conv_state, state, weight, bias, A_log, dt_bias, Hqk, Hv, K, V, activation):
         """The step in one launch, or None where it is not one token per sequence of plain dense operands (the two
         operators then convert, copy or refuse)."""
-        if x.dim() != 3 or x.shape[1] != 1 or K != 128 or weight.dim() != 2 or weight.shape[1] != 4:
-            return None
+        if x.dim() != 3 or x.shape[1] != 1 or K != 128 or weight.dim() != 2 or weight.shape[1] != 4 or state is None:
+            return None   # (without a state the rule starts from zeros)
         B, dt, D, pdt = x.shape[0], x.dtype, x.shape[2], A_log.dtype
         if dt not in (torch.float32, torch.bfloat16) or D != 2 * Hqk * K + Hv * V or activation not in _ACTIVATIONS or \
                 (pdt != dt and pdt != torch.float32) or dt_bias.dtype != pdt or \

@@ -472,6 +472,18 @@ def check_decode_step(ops, device, B, steps, Hqk, Hv, K, V, W, dtype, param_dtyp
     return errs
 
 
+def check_decode_step_without_state(ops, device, B, Hqk, Hv, K, V, dtype, wrap=lambda t: t):
+    """recurrent_state=None: the outputs of a step from a state of zeros, bit for bit; the convolution's state is rolled."""
+    gen = torch.Generator().manual_seed(B)
+    D = 2 * Hqk * K + Hv * V
+    x, a, b, conv, cw, A, d = (wrap(torch.randn(*s, generator=gen).to(dtype).to(device)) for s in
+                               [(B, 1, D), (B, 1, Hv), (B, 1, Hv), (B, D, 4), (D, 4), (Hv,), (Hv,)])
+    convs = conv.clone(), conv.clone()
+    o = [ops.decode_step(x, a, b, c, S, cw, None, A, d, Hqk, Hv, K, V)
+         for c, S in zip(convs, (None, torch.zeros(B, Hv, K, V, device=device)))]
+    assert torch.equal(o[0], o[1]) and torch.equal(convs[0], convs[1]) and not torch.equal(convs[0], conv)
+
+
 def check_kda(ops, device, B, T, H, K, V, dtype, cu=None, seed=0, with_h0=True, gate_in_kernel=True, lower_bound=None,
               beta_sigmoid=True, allow_neg=False, l2=True, transpose_state=True, g_dtype=None, scale=None, backward=False,
               wrap=lambda t: t, states=False, **recipe):

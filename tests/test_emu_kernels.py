@@ -220,6 +220,11 @@ def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt, wrap=guarded)
 
 
+@pytest.mark.parametrize("dtype,V", [(BF, 64), (F32, 128)])
+def test_decode_step_without_a_state(ops, dtype, V):
+    P.check_decode_step_without_state(ops, "cpu", 2, 1, 1, 128, V, dtype, wrap=guarded)
+
+
 @pytest.mark.parametrize("dtype,B,T,D,W,S", [(F32, 2, 3, 16, 4, 6), (BF, 2, 2, 8, 3, 3), (BF, 1, 1, 8, 4, 3)])
 def test_conv1d_update_general_state_length(ops, dtype, B, T, D, W, S):
     P.check_conv_update(ops, "cpu", B, T, D, W, dtype, S=S, wrap=guarded)

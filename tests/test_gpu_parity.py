@@ -542,6 +542,11 @@ def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt)
 
 
+@pytest.mark.parametrize("dtype,V", [(BF, 64), (F32, 128)])
+def test_decode_step_without_a_state(ops, dtype, V):
+    P.check_decode_step_without_state(ops, "cuda", 2, 1, 1, 128, V, dtype)
+
+
 def test_decode_cache_prefill_then_steps(ops):
     """Prefill with the chunked operators, hand both states to the cache, decode two more tokens, reorder the beams:
     equal to running the chunked operators over the longer sequences of the reordered batch."""
