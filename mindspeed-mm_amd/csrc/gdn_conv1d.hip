@@ -309,8 +309,8 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 2 : 1) vo
           }
         }
         if (dht != nullptr) {
-          const int64_t wq = s_ - (lag.eos - W);   // final_state[n,d,wq] = x[s]
-          if (wq >= 0) {
+          const int64_t wq = s_ - (lag.eos - W);   // final_state[n,d,wq] = x[s]; W and more: rows of no sequence
+          if (wq >= 0 && wq < W) {
 #pragma unroll
             for (int e = 0; e < V; ++e) out[e] += Elem<T>::to_f(dht[((int64_t)lag.n * D + d0 + e) * W + wq]);
           }

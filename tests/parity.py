@@ -211,6 +211,23 @@ def check_conv(ops, device, B, T, D, W, dtype, activation="silu", cu=None, bias=
     return errs
 
 
+def check_conv_padded_rows(ops, device, T, W, dtype, cu, wrap=lambda t: t):
+    """Rows behind the last packed sequence: the gradient of the final states reaches the rows of its sequences alone, whose
+    gradients are those of a call on the covered rows, and nothing is read past its end (wrap: guarded copies)."""
+    D, N, covered = 8, len(cu) - 1, cu[-1]
+    gen = torch.Generator().manual_seed(T)
+    x, w, dy, dfs = (torch.randn(*s, generator=gen).to(dtype) for s in ((1, T, D), (W, D), (1, T, D), (N, D, W)))
+
+    def grad_x(rows, with_state):
+        xl = wrap(x[:, :rows].contiguous().to(device)).requires_grad_(True)
+        y, fs = ops.causal_conv1d(xl, wrap(w.to(device)), activation="silu", cu_seqlens=cu, output_final_state=True)
+        outs, grads = [y, fs][:1 + with_state], [wrap(t.contiguous().to(device)) for t in (dy[:, :rows], dfs)][:1 + with_state]
+        return torch.autograd.grad(outs, xl, grads)[0]
+    dx = grad_x(T, True)
+    assert torch.equal(dx[:, :covered], grad_x(covered, True))
+    assert torch.equal(dx[:, covered:], grad_x(T, False)[:, covered:])
+
+
 def check_conv_update(ops, device, B, T, D, W, dtype, seed=0, wrap=lambda t: t, S=None):
     """S: length of the state rows (default W, the layer's; a longer state takes the kernel's general path)."""
     gen = torch.Generator().manual_seed(seed)

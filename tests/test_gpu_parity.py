@@ -542,6 +542,11 @@ def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt)
 
 
+@pytest.mark.parametrize("dtype,T,W,cu", [(BF, 5, 4, [0, 3]), (F32, 64, 3, [0, 0, 2, 7]), (BF, 40, 8, [0, 17, 17]), (F32, 7, 1, [0, 5])])
+def test_conv1d_rows_behind_the_last_sequence(ops, dtype, T, W, cu):
+    P.check_conv_padded_rows(ops, "cuda", T, W, dtype, cu)
+
+
 @pytest.mark.parametrize("dtype,V", [(BF, 64), (F32, 128)])
 def test_decode_step_without_a_state(ops, dtype, V):
     P.check_decode_step_without_state(ops, "cuda", 2, 1, 1, 128, V, dtype)
