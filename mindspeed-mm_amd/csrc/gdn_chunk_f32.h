@@ -124,9 +124,8 @@ __device__ __forceinline__ f32x4 f32_cols(const float* lds, int t, int m, int co
   return a;
 }
 // the same as f32_rows from a tile in memory
-__device__ __forceinline__ f32x4 f32_rows_mem(const float* tile, int m, int row0) {
-  const int j = (threadIdx.x & 63) >> 4;
-  return reinterpret_cast<const f32x4*>(tile)[(4 * (m & 1) + j) * 32 + row0 + (threadIdx.x & 15)];
+__device__ __forceinline__ f32x4 f32_rows_mem(const float* tile, int m, int row0, int tid) {
+  return reinterpret_cast<const f32x4*>(tile)[(4 * (m & 1) + ((tid & 63) >> 4)) * 32 + row0 + (tid & 15)];
 }
 __device__ __forceinline__ f32x4 f32_ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
@@ -164,23 +163,24 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(2) void chunk_state
     f32x4 g, b;
     float gl;
   };
-  auto request = [&](int ch_, Set& p) {
+  auto request = [&](int ch_, Set& p, int on) {   // on: -1, or 0: every lane asks for what the first one does, and no one uses it
+    const int tid_ = tid & on, c_ = c & on, row_ = row & on;
     const int nvalid = imin(kChunk, run.len - ch_ * kChunk);
     const int64_t ch = (run.chunk_base + ch_) * Hv + h, tok0 = run.bos + (int64_t)ch_ * kChunk;
-    p.k.request(kaf + ((run.chunk_base + ch_) * Hqk + h / (Hv / Hqk)) * (64 * DK), tid);
+    p.k.request(kaf + ((run.chunk_base + ch_) * Hqk + h / (Hv / Hqk)) * (64 * DK), tid_);
 #pragma unroll
     for (int m = 0; m < 4; ++m)   // steps above the diagonal repeat the last one and are not used
-      p.t[m] = f32_rows_mem(ai + ch * 4096 + (2 * (wave >> 1) + (imin(m, wave) >> 1)) * 1024, m, 16 * (wave & 1));
+      p.t[m] = f32_rows_mem(ai + ch * 4096 + (2 * (wave >> 1) + (imin(m, wave) >> 1)) * 1024, m, 16 * (wave & 1), tid_);
 #pragma unroll
     for (int ct = 0; ct < CW; ++ct)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        p.v[ct][r] = v[(tok0 + imin(row + r, nvalid - 1)) * v_stride + (int64_t)h * V + v0 + 16 * ct + c];
-    p.g = f32_ld4(G + ch * 64 + row);
-    p.b = f32_ld4(bt + ch * 64 + row);
+        p.v[ct][r] = v[(tok0 + imin(row_ + r, nvalid - 1)) * v_stride + (int64_t)h * V + v0 + 16 * ct + c_];
+    p.g = f32_ld4(G + ch * 64 + row_);
+    p.b = f32_ld4(bt + ch * 64 + row_);
     p.gl = G[ch * 64 + 63];
   };
-  auto step = [&](int ci, Set& p) {
+  auto step = [&](int ci, Set& p, auto more) {   // more: a chunk follows (K = 64)
     const int64_t ch = (run.chunk_base + ci) * Hv + h;
     const int nvalid = imin(kChunk, run.len - ci * kChunk);
     p.k.place(Ks, tid);
@@ -208,7 +208,11 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(2) void chunk_state
 #pragma unroll
       for (int r = 0; r < 4; ++r) vv[ct][r] = p.v[ct][r];
     GDN_LDS_BARRIER();   // (not __syncthreads(), which would wait for the stores of S)
-    request(imin(ci + 1, run.nchunks - 1), p);   // past the end: the same requests, never used
+    // Behind the last chunk there is nothing to ask for, and asking for that chunk once more cost a sequence of one chunk up
+    // to a quarter of its time.  64 sequences of 64 tokens, 32 heads, us: K = V = 64 67 -> 60 with a last step of its own; K =
+    // V = 128, where that spills (4 x 1024 tokens 132 -> 182), 206 -> 167 with every lane asking for the same line (130).
+    if constexpr (DK == 128) request(imin(ci + 1, run.nchunks - 1), p, ci + 1 < run.nchunks ? -1 : 0);
+    else if constexpr (decltype(more)::value) request(ci + 1, p, -1);
     f32x4 acc[2][CW], kt[RT][4], xb[4][CW];
     // y = K S
     f32_zero<CW>(acc);
@@ -255,8 +259,10 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(2) void chunk_state
   };
   if (run.nchunks > 0) {
     Set set;
-    request(0, set);
-    for (int ci = 0; ci < run.nchunks; ++ci) step(ci, set);
+    request(0, set, -1);
+    const int steps = DK == 128 ? run.nchunks : run.nchunks - 1;
+    for (int ci = 0; ci < steps; ++ci) step(ci, set, std::true_type{});
+    if constexpr (DK != 128) step(steps, set, std::false_type{});
   }
   if (ht != nullptr) {
 #pragma unroll
@@ -311,7 +317,7 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(DK == 64 ? 2 : 1) v
     p.t.request(ai + ch * 4096, tid);
 #pragma unroll
     for (int m = 0; m < 4; ++m)   // the tiles of Aq are stored by columns: its transpose as it lies
-      p.a[m] = f32_rows_mem(aqf + ch * 4096 + (2 * (imax(m, wave) >> 1) + (wave >> 1)) * 1024, m, 16 * (wave & 1));
+      p.a[m] = f32_rows_mem(aqf + ch * 4096 + (2 * (imax(m, wave) >> 1) + (wave >> 1)) * 1024, m, 16 * (wave & 1), tid);
 #pragma unroll
     for (int ct = 0; ct < CW; ++ct)
 #pragma unroll
@@ -321,7 +327,7 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(DK == 64 ? 2 : 1) v
     p.b = f32_ld4(bt + ch * 64 + row);
     p.gl = G[ch * 64 + 63];
   };
-  auto step = [&](int ci, Set& p) {
+  auto step = [&](int ci, Set& p, auto more) {   // more: requests follow
     const int64_t ch = (run.chunk_base + ci) * Hv + h;
     const int nvalid = imin(kChunk, run.len - ci * kChunk);
     p.k.place(Ks, tid);
@@ -358,9 +364,9 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(DK == 64 ? 2 : 1) v
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) qt[rt][m] = f32_rows_mem(qc + ((2 * rt + (wave >> 1)) * 2 + (m >> 1)) * 1024, m, 16 * (wave & 1));
+        for (int m = 0; m < 4; ++m) qt[rt][m] = f32_rows_mem(qc + ((2 * rt + (wave >> 1)) * 2 + (m >> 1)) * 1024, m, 16 * (wave & 1), tid);
     }
-    request(imax(ci - 1, 0), p);
+    if constexpr (decltype(more)::value) request(imax(ci - 1, 0), p);
     f32x4 acc[2][CW], aq[2][CW], kt[RT][4], tt[4], db[4][CW], xb[4][CW];
     // dV'
     f32_zero<CW>(acc);
@@ -422,7 +428,11 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(DK == 64 ? 2 : 1) v
   if (run.nchunks > 0) {
     Set set;
     request(run.nchunks - 1, set);
-    for (int ci = run.nchunks - 1; ci >= 0; --ci) step(ci, set);
+    // K = 128: the last step without requests (64 sequences of 64 tokens, 32 heads of 128: 320 -> 278 us; 17 of 500: 556 -> 547).
+    // K = 64 repeats the requests of its last chunk: the step twice spills there (64 sequences of 64 tokens, 32 heads of 64: 86 -> 137 us).
+    constexpr int kLast = DK == 64 ? 0 : 1;
+    for (int ci = run.nchunks - 1; ci >= kLast; --ci) step(ci, set, std::true_type{});
+    if constexpr (kLast == 1) step(0, set, std::false_type{});
   }
   if (dh0 != nullptr) {
 #pragma unroll
