@@ -10,6 +10,8 @@ CPU oracle (oracle/gdn_oracle.py, oracle/kda_oracle.py).  Tolerances are the one
     bf16 vs the fp32 oracle on the same (bf16-valued) inputs: max abs error <= 2e-2 on o and on the final state,
           <= 5e-2 on dq/dk/dv/dg/dbeta (and on the gradient of the initial state).
 """
+import contextlib
+
 import torch
 
 from mindspeed_mm_amd.inputs import gdn_inputs, kda_inputs
@@ -444,10 +446,26 @@ def check_gdn_gates(ops, device, shape, Hv, dtype, param_dtype=None, seed=0, bac
     return errs
 
 
-def check_decode_step(ops, device, B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=None, seed=0, wrap=lambda t: t):
+@contextlib.contextmanager
+def _recorded(obj, name, results):
+    """While active, what obj.name(...) returns is also appended to `results`."""
+    def call(*args):
+        results.append(type(obj).__dict__[name](obj, *args))
+        return results[-1]
+    setattr(obj, name, call)
+    try:
+        yield
+    finally:
+        delattr(obj, name)
+
+
+def check_decode_step(ops, device, B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=None, seed=0, wrap=lambda t: t,
+                      one_launch=None):
     """`steps` consecutive decode tokens through decode_step (convolution update + rule on its unsplit output with the
     gates formed in the kernel, both states in place) against the oracle's chain conv update -> split -> gate recipe
-    -> recurrent rule, and bit for bit against this package's own unfused operators."""
+    -> recurrent rule, and bit for bit against this package's own unfused operators.  one_launch: whether every step has to
+    be taken whole (True) or by two operators (False), on dense inputs; None: a step's columns of all steps' tensor, either
+    way."""
     gen = torch.Generator().manual_seed(seed)
     r = lambda *s: torch.randn(*s, generator=gen)
     param_dtype = param_dtype or dtype
@@ -465,8 +483,11 @@ def check_decode_step(ops, device, B, steps, Hqk, Hv, K, V, W, dtype, param_dtyp
     errs = {}
     for t in range(steps):
         sl = slice(t, t + 1)
-        o = ops.decode_step(dev["mixed"][:, sl], dev["a"][:, sl], dev["b"][:, sl], conv1, S1, dev["cw"], dev["cb"],
-                            dev["A"], dev["d"], Hqk, Hv, K, V)
+        step = [dev[n][:, sl] if one_launch is None else wrap(dev[n][:, sl].contiguous()) for n in ("mixed", "a", "b")]
+        taken = []
+        with _recorded(ops, "_decode_step_whole", taken):
+            o = ops.decode_step(*step, conv1, S1, dev["cw"], dev["cb"], dev["A"], dev["d"], Hqk, Hv, K, V)
+        assert one_launch is None or [t is not None for t in taken] == [one_launch]
         # the same with this package's separate operators
         y2 = ops.causal_conv1d_update(dev["mixed"][:, sl], conv2, dev["cw"], dev["cb"], "silu")
         q2, k2, v2 = torch.split(y2, [nq, nq, nv], dim=-1)

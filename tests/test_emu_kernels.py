@@ -211,13 +211,14 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt, wrap=guarded)
 
 
-@pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,K,V,W,pdt", [
-    (BF, 2, 2, 1, 1, 128, 64, 4, None), (F32, 1, 2, 1, 1, 128, 128, 4, None), (BF, 3, 1, 1, 4, 128, 64, 4, torch.float32),
-    (BF, 1, 1, 1, 8, 128, 64, 4, None),
+@pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,V,pdt,whole", [
+    (BF, 2, 2, 1, 1, 64, None, True), (F32, 2, 2, 2, 2, 64, None, True), (F32, 1, 2, 1, 1, 128, None, True),
+    (BF, 3, 2, 2, 4, 64, None, True), (BF, 3, 2, 1, 4, 64, torch.float32, True), (BF, 2, 2, 1, 2, 128, None, True),
+    (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, False), (BF, 1, 1, 1, 3, 64, None, False),
 ])
-def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
-    """1, 2 and 4 slabs to a workgroup, and 8, which take the two launches."""
-    P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt, wrap=guarded)
+def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, V, pdt, whole):
+    """1, 2 and 4 slabs of 64 columns to a workgroup; 3 and 8 take the two launches."""
+    P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, 128, V, 4, dtype, param_dtype=pdt, wrap=guarded, one_launch=whole)
 
 
 @pytest.mark.parametrize("dtype,T,W,cu", [(BF, 5, 4, [0, 3]), (F32, 64, 3, [0, 0, 2, 7]), (BF, 40, 8, [0, 17, 17]), (F32, 7, 1, [0, 5])])

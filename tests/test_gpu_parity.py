@@ -531,15 +531,17 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt)
 
 
-@pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,K,V,W,pdt", [
-    (BF, 2, 2, 1, 1, 128, 64, 4, None), (F32, 1, 2, 1, 1, 128, 128, 4, None), (BF, 3, 1, 1, 4, 128, 64, 4, torch.float32),
-    (BF, 1, 1, 1, 8, 128, 64, 4, None), (BF, 16, 1, 16, 32, 128, 128, 4, None), (BF, 17, 1, 16, 32, 128, 128, 4, None),
-    (BF, 65, 1, 8, 32, 128, 128, 4, None), (F32, 127, 1, 32, 32, 128, 128, 4, None),
-    (BF, 128, 1, 16, 32, 128, 128, 4, torch.float32), (BF, 128, 1, 32, 32, 128, 128, 4, None),
+@pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,V,pdt,whole", [
+    (BF, 2, 2, 1, 1, 64, None, True), (F32, 1, 2, 1, 1, 128, None, True), (BF, 3, 2, 1, 4, 64, torch.float32, True),
+    (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, False), (BF, 16, 2, 16, 32, 128, None, True),
+    (BF, 17, 2, 16, 32, 128, None, True), (BF, 64, 1, 8, 32, 128, None, True), (BF, 65, 1, 8, 32, 128, None, True),
+    (F32, 127, 1, 32, 32, 128, None, True), (BF, 127, 1, 16, 32, 128, None, True), (BF, 128, 1, 16, 32, 128, torch.float32, True),
+    (BF, 128, 1, 32, 32, 128, None, True),
 ])
-def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
+def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, V, pdt, whole):
     """1, 2 and 4 slabs to a workgroup, and 8, which take the two launches; states on either side of 32, 128 and 256 MB."""
-    P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, K, V, W, dtype, param_dtype=pdt)
+    print(f"decode step in one launch {dtype} B{B} {Hqk}/{Hv} V{V}", flush=True)
+    P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, 128, V, 4, dtype, param_dtype=pdt, one_launch=whole)
 
 
 @pytest.mark.parametrize("dtype,T,W,cu", [(BF, 5, 4, [0, 3]), (F32, 64, 3, [0, 0, 2, 7]), (BF, 40, 8, [0, 17, 17]), (F32, 7, 1, [0, 5])])
