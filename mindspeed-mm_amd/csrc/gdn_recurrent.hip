@@ -352,6 +352,10 @@ static int launch_recurrent(const void* q, const void* k, const void* v, int64_t
 // columns 11.7); beyond, 128 columns and two workgroups a CU (17 sequences 21 -> 16, 256: 208 -> 167).  Loads: kStream to
 // 128 MB (64 sequences, five sets of states in turn, 53 against 56 with kCached; 32: 25 and 26), then kCached (112 sequences,
 // the same states every step, 81 against 86), kMixed from 256 MB on as in the rule alone.
+// Four slabs of 128 columns (four value heads to a q/k head) end at 128 MB: their 1024 threads have a CU to themselves, where
+// nothing loads while they compute, and past that size two launches are faster.  16 q/k and 64 value heads, us, one launch /
+// two: twelve sets of states in turn 64 MB 27 / 34, 128 MB 52 / 61, 160 MB 78 / 75, 256 MB 111 / 105, 512 MB 212 / 200; the same
+// states every step 96 MB 41 / 39, 160 MB 64 / 60, 256 MB 100 / 92, 512 MB 188 / 176.
 template <typename T, typename TP>
 static int launch_decode_step(const RecurrentConv& conv, const RecurrentGates& gates, float* state, void* o, int B, int Hqk,
                               int Hv, int K, int V, float scale, hipStream_t stream) {
@@ -360,6 +364,7 @@ static int launch_decode_step(const RecurrentConv& conv, const RecurrentGates& g
   const int bv = bytes > 32 * MB ? 128 : 64;
   if (K != 128 || V % bv != 0 || (int64_t)B * Hqk > 0x7fffffff) return -3;
   const int64_t units = (int64_t)(Hv / Hqk) * (V / bv);
+  if (units == 4 && bytes > 128 * MB) return -3;
   auto launch = [&](auto kern) {
     GDN_LAUNCH(kKernRecurrent, stream, kern, dim3((unsigned)(B * Hqk)), dim3((unsigned)(kThreads * units)), 0, stream,
                (const T*)nullptr, (const T*)nullptr, (const T*)nullptr, 0, 0, 0, gates, (const float*)state, state, (T*)o,
@@ -370,8 +375,10 @@ static int launch_decode_step(const RecurrentConv& conv, const RecurrentGates& g
   if (units == UN_) {                                                                                        \
     if (bytes <= 32 * MB) return launch(recurrent_kernel<T, TP, 128, 64, StateLoads::kStream, UN_>);         \
     if (bytes <= 128 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kStream, UN_>);       \
-    if (bytes < 256 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kCached, UN_>);        \
-    return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kMixed, UN_>);                               \
+    if constexpr (UN_ != 4) {                                                                                \
+      if (bytes < 256 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kCached, UN_>);      \
+      return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kMixed, UN_>);                             \
+    }                                                                                                        \
   }
   GDN_STEP(1)
   GDN_STEP(2)

@@ -534,12 +534,13 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
 @pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,V,pdt,whole", [
     (BF, 2, 2, 1, 1, 64, None, True), (F32, 1, 2, 1, 1, 128, None, True), (BF, 3, 2, 1, 4, 64, torch.float32, True),
     (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, False), (BF, 16, 2, 16, 32, 128, None, True),
-    (BF, 17, 2, 16, 32, 128, None, True), (BF, 64, 1, 8, 32, 128, None, True), (BF, 65, 1, 8, 32, 128, None, True),
+    (BF, 17, 2, 16, 32, 128, None, True), (BF, 64, 1, 8, 32, 128, None, True), (BF, 65, 1, 8, 32, 128, None, False),
     (F32, 127, 1, 32, 32, 128, None, True), (BF, 127, 1, 16, 32, 128, None, True), (BF, 128, 1, 16, 32, 128, torch.float32, True),
     (BF, 128, 1, 32, 32, 128, None, True),
 ])
 def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, V, pdt, whole):
-    """1, 2 and 4 slabs to a workgroup, and 8, which take the two launches; states on either side of 32, 128 and 256 MB."""
+    """1, 2 and 4 slabs to a workgroup; 8, and 4 beyond 128 MB, take the two launches; states on either side of 32, 128 and
+    256 MB."""
     print(f"decode step in one launch {dtype} B{B} {Hqk}/{Hv} V{V}", flush=True)
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, 128, V, 4, dtype, param_dtype=pdt, one_launch=whole)
 
