@@ -484,7 +484,7 @@ class GdnOps:
         (modeling_qwen3_5.py:738-744, 808-848, 877-890): convolution update (conv_state [B,D,S] rolled in place), then
         the rule on its unsplit output with the gates formed in the kernel (recurrent_state [B,Hv,K,V] fp32 updated in
         place).  mixed_qkv [B,T,D], a, b [B,T,Hv]; conv_weight [D,W].  Returns o [B,T,Hv,V].  One launch where the library
-        takes the step whole (gdn_decode_step), else the two operators in turn; the same bits."""
+        takes the step whole (gdn_decode_step) and that is the faster way, else the two operators in turn; the same bits."""
         o = self._decode_step_whole(mixed_qkv, a, b, conv_state, recurrent_state, conv_weight, conv_bias, A_log, dt_bias,
                                     int(num_k_heads), int(num_v_heads), int(head_k_dim), int(head_v_dim), activation)
         if o is not None:
@@ -514,6 +514,11 @@ class GdnOps:
         for t in operands:
             if t is not None and not (t.is_contiguous() and (t.is_cuda if cuda else t.is_cpu)):
                 return None
+        # Four slabs to a workgroup leave most CUs idle on few states, which only the host's share of a second launch makes up
+        # for.  A graph has no such share: 16 q/k and 32 value heads of 128, 24 layers, us a step there, whole / in two, 1
+        # sequence 8.1 / 6.3, 4 (8 MB) 8.9 / 8.2, 8 10.5 / 10.7; with two slabs (16 value heads) 1 sequence 5.8 / 6.1.
+        if Hv * V == 256 * Hqk and B * Hv * V <= 1 << 14 and cuda and torch._C._cuda_isCurrentStreamCapturing():
+            return None
         o = torch.empty(B, 1, Hv, V, dtype=dt, device=x.device)
         code = self.lib.gdn_decode_step(*map(ptr, operands), o.data_ptr(), B, Hqk, Hv, K, V, 4, _act_code(activation),
                                         K ** -0.5, DTYPE_CODE[dt], DTYPE_CODE[pdt], self.lib.stream())

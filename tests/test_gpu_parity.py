@@ -545,6 +545,39 @@ def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, V, pdt, whole)
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, 128, V, 4, dtype, param_dtype=pdt, one_launch=whole)
 
 
+@pytest.mark.parametrize("B,Hqk,Hv,whole", [(1, 16, 32, False), (4, 16, 32, False), (5, 16, 32, True), (1, 4, 4, True)])
+def test_decode_step_in_a_graph(ops, B, Hqk, Hv, whole):
+    """Captured and replayed on other inputs each time, with eager steps in between: the same bits as those.  Few states of two
+    value heads of 128 to a q/k head are captured as two launches, others as one."""
+    K = V = 128
+    D = 2 * Hqk * K + Hv * V
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    r = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(BF)
+    cw, cb, A, d = r(D, 4), r(D), r(Hv), r(Hv)
+    static = [r(B, 1, D), r(B, 1, Hv), r(B, 1, Hv)]
+    states = [r(B, D, 4), torch.randn(B, Hv, K, V, generator=gen, device="cuda")]
+    eager = [t.clone() for t in states]
+    step = lambda x, s: ops.decode_step(*x, *s, cw, cb, A, d, Hqk, Hv, K, V)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(static, [t.clone() for t in states])
+    torch.cuda.current_stream().wait_stream(side)
+    taken, graph = [], torch.cuda.CUDAGraph()
+    with P._recorded(ops, "_decode_step_whole", taken), torch.cuda.graph(graph):
+        out = step(static, states)
+    assert [t is not None for t in taken] == [whole]
+    for n in range(4):
+        x = [r(*t.shape) for t in static]
+        for t, new in zip(static, x):
+            t.copy_(new)
+        out.zero_()
+        graph.replay()
+        want = step(x, eager)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and all(torch.equal(a, b) for a, b in zip(states, eager)), n
+
+
 @pytest.mark.parametrize("dtype,T,W,cu", [(BF, 5, 4, [0, 3]), (F32, 64, 3, [0, 0, 2, 7]), (BF, 40, 8, [0, 17, 17]), (F32, 7, 1, [0, 5])])
 def test_conv1d_rows_behind_the_last_sequence(ops, dtype, T, W, cu):
     P.check_conv_padded_rows(ops, "cuda", T, W, dtype, cu)
