@@ -150,7 +150,8 @@ int gdn_recurrent_fwd_qkv(const void* qkv, int64_t token_stride, const void* a, 
  * gdn_recurrent_fwd_qkv with the l2 norm on its output, in one launch and with the bits of the two.  conv_state [B,D,W] and
  * state [B,Hv,K,V] are updated in place; conv_weight [D,W], conv_bias [D] or null; o [B,Hv,V].  W = 4 and K = 128; -3 for
  * what needs the two calls: other sizes, value heads of one q/k head whose slabs (of 64 columns while the states are 32 MB
- * or less, else of 128) are not 1, 2 or -- up to 128 MB of states -- 4 in number, rows of conv_state or conv_weight not aligned to their size. */
+ * or less and that makes no more than 4, else of 128) are not 1, 2 or, up to 128 MB of states, 4 in number, rows of
+ * conv_state or conv_weight not aligned to their size. */
 int gdn_decode_step(const void* hidden, void* conv_state, const void* conv_weight, const void* conv_bias, const void* a,
                     const void* b, const void* A_log, const void* dt_bias, float* state, void* o, int B, int Hqk, int Hv,
                     int K, int V, int W, int activation, float scale, int dtype, int param_dtype, void* stream);

@@ -361,7 +361,7 @@ static int launch_decode_step(const RecurrentConv& conv, const RecurrentGates& g
                               int Hv, int K, int V, float scale, hipStream_t stream) {
   constexpr int64_t MB = 1 << 20;
   const int64_t bytes = (int64_t)B * Hv * K * V * 4;
-  const int bv = bytes > 32 * MB ? 128 : 64;
+  const int bv = bytes > 32 * MB || (Hv / Hqk * (V / 64) > 4 && V % 128 == 0) ? 128 : 64;
   if (K != 128 || V % bv != 0 || (int64_t)B * Hqk > 0x7fffffff) return -3;
   const int64_t units = (int64_t)(Hv / Hqk) * (V / bv);
   if (units == 4 && bytes > 128 * MB) return -3;
@@ -373,7 +373,7 @@ static int launch_decode_step(const RecurrentConv& conv, const RecurrentGates& g
   };
 #define GDN_STEP(UN_)                                                                                        \
   if (units == UN_) {                                                                                        \
-    if (bytes <= 32 * MB) return launch(recurrent_kernel<T, TP, 128, 64, StateLoads::kStream, UN_>);         \
+    if (bv == 64) return launch(recurrent_kernel<T, TP, 128, 64, StateLoads::kStream, UN_>);                 \
     if (bytes <= 128 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kStream, UN_>);       \
     if constexpr (UN_ != 4) {                                                                                \
       if (bytes < 256 * MB) return launch(recurrent_kernel<T, TP, 128, 128, StateLoads::kCached, UN_>);      \

@@ -214,10 +214,11 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
 @pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,V,pdt,whole", [
     (BF, 2, 2, 1, 1, 64, None, True), (F32, 2, 2, 2, 2, 64, None, True), (F32, 1, 2, 1, 1, 128, None, True),
     (BF, 3, 2, 2, 4, 64, None, True), (BF, 3, 2, 1, 4, 64, torch.float32, True), (BF, 2, 2, 1, 2, 128, None, True),
-    (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, False), (BF, 1, 1, 1, 3, 64, None, False),
+    (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, True), (BF, 1, 1, 1, 3, 64, None, False),
+    (BF, 1, 1, 1, 3, 128, None, False), (F32, 1, 1, 1, 8, 128, None, False),
 ])
 def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, V, pdt, whole):
-    """1, 2 and 4 slabs of 64 columns to a workgroup; 3 and 8 take the two launches."""
+    """1, 2 and 4 slabs of 64 columns to a workgroup, 4 of 128 in place of 8; 3 of either and 8 of 128 take the two launches."""
     P.check_decode_step(ops, "cpu", B, steps, Hqk, Hv, 128, V, 4, dtype, param_dtype=pdt, wrap=guarded, one_launch=whole)
 
 

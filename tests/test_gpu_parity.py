@@ -533,22 +533,23 @@ def test_decode_step(ops, dtype, B, steps, Hqk, Hv, K, V, W, pdt):
 
 @pytest.mark.parametrize("dtype,B,steps,Hqk,Hv,V,pdt,whole", [
     (BF, 2, 2, 1, 1, 64, None, True), (F32, 1, 2, 1, 1, 128, None, True), (BF, 3, 2, 1, 4, 64, torch.float32, True),
-    (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, False), (BF, 16, 2, 16, 32, 128, None, True),
+    (BF, 1, 1, 1, 8, 64, None, False), (BF, 2, 2, 1, 4, 128, None, True), (BF, 8, 2, 16, 64, 128, None, True), (BF, 16, 2, 16, 32, 128, None, True),
     (BF, 17, 2, 16, 32, 128, None, True), (BF, 64, 1, 8, 32, 128, None, True), (BF, 65, 1, 8, 32, 128, None, False),
     (F32, 127, 1, 32, 32, 128, None, True), (BF, 127, 1, 16, 32, 128, None, True), (BF, 128, 1, 16, 32, 128, torch.float32, True),
     (BF, 128, 1, 32, 32, 128, None, True),
 ])
 def test_decode_step_in_one_launch(ops, dtype, B, steps, Hqk, Hv, V, pdt, whole):
-    """1, 2 and 4 slabs to a workgroup; 8, and 4 beyond 128 MB, take the two launches; states on either side of 32, 128 and
+    """1, 2 and 4 slabs to a workgroup, 4 of 128 columns in place of 8 of 64; 8 of 128, and 4 beyond 128 MB, take the two launches; states on either side of 32, 128 and
     256 MB."""
     print(f"decode step in one launch {dtype} B{B} {Hqk}/{Hv} V{V}", flush=True)
     P.check_decode_step(ops, "cuda", B, steps, Hqk, Hv, 128, V, 4, dtype, param_dtype=pdt, one_launch=whole)
 
 
-@pytest.mark.parametrize("B,Hqk,Hv,whole", [(1, 16, 32, False), (4, 16, 32, False), (5, 16, 32, True), (1, 4, 4, True)])
+@pytest.mark.parametrize("B,Hqk,Hv,whole", [(1, 16, 32, False), (4, 16, 32, False), (5, 16, 32, True), (1, 4, 4, True),
+                                             (1, 4, 16, False), (32, 4, 16, False), (33, 4, 16, True)])
 def test_decode_step_in_a_graph(ops, B, Hqk, Hv, whole):
     """Captured and replayed on other inputs each time, with eager steps in between: the same bits as those.  Few states of two
-    value heads of 128 to a q/k head are captured as two launches, others as one."""
+    or four value heads of 128 to a q/k head are captured as two launches, others as one."""
     K = V = 128
     D = 2 * Hqk * K + Hv * V
     gen = torch.Generator(device="cuda").manual_seed(B)
