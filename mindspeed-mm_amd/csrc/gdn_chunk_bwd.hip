@@ -1028,7 +1028,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
                    (float*)DHF, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale);
         return 0;
       };
-      if (int e = f32_sixteen_columns(d.N, d.Hv, d.V, device_compute_units())
+      if (int e = f32_sixteen_columns(d.N, d.Hv, d.V, device_compute_units(), DK == 64 ? 2 : 1)
                       ? launch_f32(chunk_state_bwd_f32_kernel<DK, 1>, StateBwdF32Smem<DK, 1>::bytes, 16)
                       : launch_f32(chunk_state_bwd_f32_kernel<DK, 2>, StateBwdF32Smem<DK, 2>::bytes, 32))
         return e;

@@ -8,8 +8,8 @@
 // an accumulator's four rows are the 16 bytes another wave reads as four steps of its contraction.  A chunk is then 48
 // (K = 64) to 80 instructions per wave and column tile instead of 176 to 304 that take twice as long.
 // Forward / backward recurrence, us, waves that own 32 columns -> this: 512 tokens, 4 heads, K = V = 64 54 / 90 -> 20 / 28,
-// K = V = 128 116 / 141 -> 27 / 40; 2 x 1024 tokens, 32 heads of 128 241 / 286 -> 94 / 133; 4 x 512, 32 heads, V = 256
-// 137 / 290 -> 136 / 249.  Of a chunk's 2.2 us (K = 64) the instructions are 0.65; the rest are the waits of the three
+// K = V = 128 116 / 141 -> 27 / 40; 2 x 1024 tokens, 32 heads of 128 241 / 286 -> 86 / 129; 4 x 512, 32 heads, V = 256
+// 137 / 290 -> 128 / 242.  Of a chunk's 2.2 us (K = 64) the instructions are 0.65; the rest are the waits of the three
 // exchanges and the address arithmetic and issue of the next chunk's requests.  Error against float64, 512 tokens, K = 64: o
 // 5.8e-7 -> 5.5e-7, final state 6.0e-7 -> 5.8e-7, dq 5.5e-7 -> 5.2e-7, dh0 2.8e-7 -> 2.1e-7.
 //
@@ -444,11 +444,13 @@ __global__ __launch_bounds__(kF32Threads) GDN_WAVES_PER_SIMD(DK == 64 ? 2 : 1) v
   }
 }
 
-// Columns to a workgroup: 16 while that leaves no more workgroups than compute units, else 32, which read the tiles half
-// as often; the same bits.  16 against 32 columns, forward / backward, us: 4 heads of 64 20 / 28 and 28 / 41; 32 heads, 4
-// sequences of 512 tokens, K = 128, V = 256 (2048 workgroups of 16 columns) 150 / 310 and 135 / 249.
-inline bool f32_sixteen_columns(int64_t sequences, int Hv, int V, int compute_units) {
-  return sequences * Hv * (V / 16) <= compute_units;
+// Columns to a workgroup: 16 while the compute units hold all of those workgroups at once (per_unit each: 2, but 1 for the
+// reverse recurrence with K = 128, whose registers fill a unit), else 32, which read the tiles half as often; the same bits.
+// 512 tokens, K = V, 16 / 32 columns, us, by the workgroups of 16 columns.  Forward, 64: 256 22 / 30, 512 31 / 33, 768 46 / 46,
+// 1024 62 / 49; 128: 256 31 / 44, 384 41 / 46, 512 44 / 47, 768 65 / 65, 1024 81 / 69.  Reverse, 64: 256 33 / 45, 512 46 / 48,
+// 768 69 / 68, 1024 93 / 72; 128: 256 44 / 63, 384 81 / 67, 512 84 / 68.
+inline bool f32_sixteen_columns(int64_t sequences, int Hv, int V, int compute_units, int per_unit) {
+  return sequences * Hv * (V / 16) <= (int64_t)per_unit * compute_units;
 }
 
 }  // namespace gdn

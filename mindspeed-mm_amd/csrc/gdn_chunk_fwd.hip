@@ -1098,7 +1098,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
                  (const int*)chunk_offsets, d.T, d.Hqk, d.Hv, d.V, ts.v);
       return 0;
     };
-    if (int e = f32_sixteen_columns(d.N, d.Hv, d.V, device_compute_units())
+    if (int e = f32_sixteen_columns(d.N, d.Hv, d.V, device_compute_units(), 2)
                     ? launch_f32(chunk_state_f32_kernel<DK, 1>, StateF32Smem<DK, 1>::bytes, 16)
                     : launch_f32(chunk_state_f32_kernel<DK, 2>, StateF32Smem<DK, 2>::bytes, 32))
       return e;

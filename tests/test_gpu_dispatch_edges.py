@@ -121,14 +121,14 @@ def test_recurrent_bits_do_not_depend_on_the_batch(ops, dtype, K, V, batches):
 @pytest.mark.parametrize("T,K,V", [(2, 64, 64), (130, 64, 64), (65, 128, 192), (64, 128, 128)])
 def test_chunk_fp32_bits_do_not_depend_on_the_batch(ops, T, K, V):
     """The fp32 recurrences give a workgroup 16 or 32 state columns by the size of the call: the same bits either way."""
-    x = {n: t.cuda() for n, t in P.gdn_inputs(24, T, 2, 4, K, V, F32, seed=T).items()}
+    x = {n: t.cuda() for n, t in P.gdn_inputs(40, T, 2, 4, K, V, F32, seed=T).items()}
 
     def call(n):
         leaf = {m: x[m][:n].clone().requires_grad_(True) for m in ("q", "k", "v", "g", "beta", "h0")}
         o, s = ops.chunk_gated_delta_rule(*list(leaf.values())[:5], initial_state=leaf["h0"], output_final_state=True,
                                           use_qk_l2norm_in_kernel=True)
         return [o, s, *torch.autograd.grad([o, s], list(leaf.values()), [x["do"][:n], x["dht"][:n]])]
-    for a, b in zip(call(1), call(24)):
+    for a, b in zip(call(1), call(40)):
         assert torch.equal(a[0], b[0])
 
 
