@@ -517,13 +517,15 @@ class GdnOps:
         # Four slabs to a workgroup leave most CUs idle on few states, which only the host's share of a second launch makes up
         # for.  A graph has no such share: 16 q/k heads, 24 layers, us a step there, whole / in two: 32 value heads of 128, 1
         # sequence 8.1 / 6.3, 4 (8 MB) 8.9 / 8.2, 8 10.5 / 10.7; 64 value heads, 1 sequence 12.4 / 6.8, 8 (32 MB) 16.7 / 15.9, 16
-        # 26.5 / 33.2.  With two slabs (16 value heads) the whole step is faster there too: 1 sequence 5.8 / 6.1.
-        if Hv * V >= 256 * Hqk and B * Hv * V <= (1 << 14 if Hv * V == 256 * Hqk else 1 << 16) and cuda and \
+        # 26.5 / 33.2.  With two slabs (16 value heads) the whole step is faster there too: 1 sequence 5.8 / 6.1.  (The default
+        # stream, 0, cannot be captured.)
+        stream = self.lib.stream()
+        if stream and Hv * V >= 256 * Hqk and B * Hv * V <= (1 << 14 if Hv * V == 256 * Hqk else 1 << 16) and \
                 torch._C._cuda_isCurrentStreamCapturing():
             return None
         o = torch.empty(B, 1, Hv, V, dtype=dt, device=x.device)
         code = self.lib.gdn_decode_step(*map(ptr, operands), o.data_ptr(), B, Hqk, Hv, K, V, 4, _act_code(activation),
-                                        K ** -0.5, DTYPE_CODE[dt], DTYPE_CODE[pdt], self.lib.stream())
+                                        K ** -0.5, DTYPE_CODE[dt], DTYPE_CODE[pdt], stream)
         if code == -3:   # a shape or an alignment it does not take
             return None
         self.lib.check(code, "gdn_decode_step")
