@@ -36,7 +36,7 @@ def test_rms_norm_gated_far_gates(ops, activation):
     what is not finite stays so."""
     gate = torch.tensor([-1e4, -200.0, -89.0, -88.0, -87.0, 0.0, 87.0, 89.0, 200.0, 1e4], device="cuda", dtype=BF)
     g = gate.repeat(13)[:128].repeat(40, 1)
-    x = torch.randn(40, 128, device="cuda", dtype=BF)
+    x = torch.randn(40, 128, generator=torch.Generator().manual_seed(40)).to("cuda", BF)
     w = torch.ones(128, device="cuda", dtype=BF)
     L = [t.clone().requires_grad_(True) for t in (x, g, w)]
     y = ops.rms_norm_gated(*L, 1e-6, activation)

@@ -861,19 +861,29 @@ def _training_call(ops, x):
 
 
 def test_backward_on_two_streams_from_two_threads(ops):
-    """The events that order the backward pass's two streams are kept from call to call: two threads, each on a stream of its
-    own, and calls of other sizes in between, get the gradients of calls that run alone."""
+    """The events that order the backward pass's two streams are kept from call to call, apart for each thread: two threads, each
+    on a stream of its own, with calls of two sizes in turn, get the gradients of calls that run alone.  The passes are called
+    directly: autograd would run the backward passes of both on its own single thread of the device."""
+    from mindspeed_mm_amd import ops as O_
+    names = ("q", "k", "v", "g", "beta")
     xs = [{n: t.cuda() for n, t in P.gdn_inputs(1, T, 2, 4, 128, 128, BF, seed=T).items()} for T in (700, 2000)]
     want = [_training_call(ops, x) for x in xs]
     torch.cuda.synchronize()
-    got, errors = {}, []
+    got, kept, errors = [], [], []
+    both = threading.Barrier(2, timeout=60)
 
     def work(i):
         try:
-            with torch.cuda.stream(torch.cuda.Stream()):
+            both.wait()
+            with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream()):
                 for n in range(8):
-                    got[i] = _training_call(ops, xs[(i + n + 1) % 2])
+                    x = xs[(i + n) % 2]
+                    o, _, saved, meta = O_._chunk_forward_call(ops, *(x[m] for m in names), 128 ** -0.5, None, False, None, True,
+                                                               True, False)
+                    got.append(((i + n) % 2, [o, *O_._chunk_backward_call(ops, saved, meta, x["do"], None)[:5]]))
                 torch.cuda.current_stream().synchronize()
+            kept.append(dict(ops._events.__dict__))
+            both.wait()   # neither thread's events are gone before the other's are looked at
         except Exception as e:   # noqa: BLE001 -- shown by the assertion below
             errors.append(e)
     threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
@@ -882,8 +892,11 @@ def test_backward_on_two_streams_from_two_threads(ops):
     for t in threads:
         t.join()
     assert not errors, errors
-    for i in range(2):
-        assert all(torch.equal(a, b) for a, b in zip(got[i], want[i]))
+    assert len(got) == 16
+    for i, tensors in got:
+        assert all(torch.equal(a, b) for a, b in zip(tensors, want[i]))
+    assert kept[0].keys() == kept[1].keys() and len(kept[0]) == 2
+    assert all(kept[0][k] is not kept[1][k] for k in kept[0])
 
 
 def test_training_call_in_a_graph(ops):
