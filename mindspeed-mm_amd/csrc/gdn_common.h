@@ -164,7 +164,8 @@ template <typename T> __device__ __forceinline__ void gate_st(void* p, int same,
   }
   reinterpret_cast<float*>(p)[i] = x;
 }
-__device__ __forceinline__ float sigmoidf_(float p) { return __builtin_amdgcn_rcpf(1.f + __expf(-p)); }   // of the convolution's SiLU
+// of the convolution's SiLU: v_rcp_f32 (1 ulp) instead of an IEEE division, ten instructions fewer per element
+__device__ __forceinline__ float sigmoidf_(float p) { return __builtin_amdgcn_rcpf(1.f + __expf(-p)); }
 __device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
 __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
 

@@ -84,8 +84,6 @@ __device__ __forceinline__ void packed_final_state(const T* x, const T* init, co
   __builtin_memcpy(fs + at, out, sizeof(out));
 }
 
-// v_rcp_f32 (1 ulp) instead of an IEEE division: ten instructions fewer per element
-
 // TT tokens per workgroup, their rows and the W-1 before them requested at once.  A tile that lies inside one sequence,
 // history included, takes straight-line code; one in which a sequence begins or ends looks at every token (32768 tokens
 // below in sequences of 8: 184 us as well; reading the W rows of each token anew 290).  The first tile too, and a last one
@@ -146,48 +144,46 @@ __global__ __launch_bounds__(kConvThreads) GDN_WAVES_PER_SIMD(W <= 4 ? 4 : 2) vo
       __builtin_memcpy(fs + ((int64_t)cur.n * D + d0) * W + i * V, &piece.raw, 16);
     }
   };
-  {
-    // the rows exist whatever sequence they belong to: they are on their way while the sequence is looked up.  Ahead of the
-    // first token and behind the last one a row that exists stands in and is not used.
-    Vec16<T> xr[TT + H];
-    const int lead = (int)(t0 < H ? H - t0 : 0), last = (int)(total - 1 - t0 < TT - 1 ? total - 1 - t0 : TT - 1) + H;
-    const T* xp = x + (t0 - H) * D;
+  // the rows exist whatever sequence they belong to: they are on their way while the sequence is looked up.  Ahead of the
+  // first token and behind the last one a row that exists stands in and is not used.
+  Vec16<T> xr[TT + H];
+  const int lead = (int)(t0 < H ? H - t0 : 0), last = (int)(total - 1 - t0 < TT - 1 ? total - 1 - t0 : TT - 1) + H;
+  const T* xp = x + (t0 - H) * D;
 #pragma unroll
-    for (int i = 0; i < TT + H; ++i) xr[i] = ld16(xp + (int64_t)imin(imax(i, lead), last) * D + d0);
-    weights();
-    cur.init(cu, N, T_len, t0);
-    if (t0 - H >= cur.bos && t0 + TT <= total && t0 + TT <= cur.eos - (fs != nullptr ? 1 : 0)) {
+  for (int i = 0; i < TT + H; ++i) xr[i] = ld16(xp + (int64_t)imin(imax(i, lead), last) * D + d0);
+  weights();
+  cur.init(cu, N, T_len, t0);
+  if (t0 - H >= cur.bos && t0 + TT <= total && t0 + TT <= cur.eos - (fs != nullptr ? 1 : 0)) {
 #pragma unroll
-      for (int w = 0; w < H; ++w) unpack_chan(win[w], xr[w]);
+    for (int w = 0; w < H; ++w) unpack_chan(win[w], xr[w]);
 #pragma unroll
-      for (int u = 0; u < TT; ++u) {   // sliding the window moves no register
-        unpack_chan(win[(u + H) % W], xr[u + H]);
-        finish(t0 + u, u);
-      }
-      return;
-    }
-    // a sequence begins or ends in the tile: the same rows, the window replaced where a sequence begins
-#pragma unroll
-    for (int w = 0; w < H; ++w) {
-      if (t0 - H + w >= cur.bos) unpack_chan(win[w], xr[w]);
-      else load_hist(win[w], x, init, t0 - H + w, cur, D, W, d0);
-    }
-#pragma unroll
-    for (int u = 0; u < TT; ++u) {
-      if (t0 + u >= total) break;
-      if (cur.advance_to(t0 + u)) {   // its first token
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-          T row[W];
-          if (init != nullptr) __builtin_memcpy(row, init + ((int64_t)cur.n * D + d0 + e) * W, sizeof(row));
-#pragma unroll
-          for (int w = 0; w < H; ++w) win[(u + w) % W][e] = init != nullptr ? Elem<T>::to_f(row[w + 1]) : 0.f;
-        }
-      }
+    for (int u = 0; u < TT; ++u) {   // sliding the window moves no register
       unpack_chan(win[(u + H) % W], xr[u + H]);
       finish(t0 + u, u);
-      final_state(t0 + u, u);
     }
+    return;
+  }
+  // a sequence begins or ends in the tile: the same rows, the window replaced where a sequence begins
+#pragma unroll
+  for (int w = 0; w < H; ++w) {
+    if (t0 - H + w >= cur.bos) unpack_chan(win[w], xr[w]);
+    else load_hist(win[w], x, init, t0 - H + w, cur, D, W, d0);
+  }
+#pragma unroll
+  for (int u = 0; u < TT; ++u) {
+    if (t0 + u >= total) break;
+    if (cur.advance_to(t0 + u)) {   // its first token
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        T row[W];
+        if (init != nullptr) __builtin_memcpy(row, init + ((int64_t)cur.n * D + d0 + e) * W, sizeof(row));
+#pragma unroll
+        for (int w = 0; w < H; ++w) win[(u + w) % W][e] = init != nullptr ? Elem<T>::to_f(row[w + 1]) : 0.f;
+      }
+    }
+    unpack_chan(win[(u + H) % W], xr[u + H]);
+    finish(t0 + u, u);
+    final_state(t0 + u, u);
   }
 }
 

@@ -4,9 +4,9 @@
 //
 // The kernel is bound by streaming the fp32 state [K,V] (64 KB at K=V=128) through HBM once in, once
 // out (a batch of 256 with 32 heads: 1.08 GB in 183 us = 5.9 TB/s on states that no cache holds, 162 us = 6.7 TB/s where the
-// memory-side cache holds a part of them; 217 and 163 us with the loads left to themselves).  One workgroup of 256 threads
-// owns a [K, BV] column slab of one state; the slab lives in registers for all T tokens of the call.  With S_old the state
-// before the token,
+// memory-side cache holds a part of them; 217 and 163 us with the loads left to themselves).  256 threads own a [K, BV] column
+// slab of one state, a workgroup one slab, or in a decode step with its convolution 1, 2 or 4; a slab lives in registers for
+// all T tokens of the call.  With S_old the state before the token,
 //     S^T k = e^g (S_old^T k),   S^T q = e^g (S_old^T q) + (k.q) delta
 // so both contractions are taken in ONE pass over the registers, then the rank-1 update is applied.
 // No MFMA: 6 flop per 8 bytes of state traffic, far below the matrix-core ridge.
@@ -14,7 +14,8 @@
 // q, k, v are read with a token stride, so they can be the column ranges of the convolution's [tokens, D] output, and
 // the gates can be formed here from the layer's projections (g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b)
 // rounded to b's dtype as the layer's `b.sigmoid()` is; modeling_qwen3_5.py:833-841) instead of being passed in: a
-// decode step of the layer is then the convolution update followed by this kernel, with no copies in between.
+// decode step of the layer is then the convolution update followed by this kernel, with no copies in between, or, where
+// launch_decode_step takes the sizes, this kernel alone (CONV).
 #include "gdn_chunk.h"
 #include "gdn_common.h"
 #include "gdn_profile.h"
@@ -344,12 +345,14 @@ static int launch_recurrent(const void* q, const void* k, const void* v, int64_t
 
 // A decode step with its convolution update in one launch; -3 for what needs the two launches: other key widths, and heads
 // whose slabs do not add up to 1, 2 or 4 groups of threads.
-// 16 q/k and 32 value heads of 128, us in the kernels / per step of a program, two launches -> one.  Small batches save the
-// host's share of a launch: 1 sequence 13.4 / 29.6 -> 9.7 / 16.5, 16 sequences 20.0 / 29.7 -> 15.2 / 16.5.  The same states
-// every step, 32 sequences 31 / 30 -> 23 / 22, 64: 54 / 49 -> 50 / 49, 128: 97 / 93 -> 90 / 89, 256: 180 / 177 -> 167 / 165;
-// states that no cache holds, 64 sequences 62 / 60 -> 53 / 53, 112: 107 / 103 -> 97 / 97, 256: 199 / 195 -> 195 / 194.
+// 16 q/k and 32 value heads of 128, 24 layers in turn, us a step in a graph / of an eager program, two launches -> one.  Small
+// batches save the host's share of a launch, not time on the device: 1 sequence 6.3 / 18.3 -> 8.1 / 10.2 (in the profiler 2.7 +
+// 5.1 -> 8.8), 4 sequences 8.2 / 17.9 -> 8.9 / 10.2, 16: 15.9 / 18.0 -> 15.1 / 15.3, 32: 33.5 -> 24.9, 64: 60.3 -> 52.8, 128: 105.0
+// -> 105.6.  The same states every step, 48 sequences 39.5 -> 36.6, 128: 93.5 -> 89.5, 256: 179.0 -> 167.6; three sets of states
+// in turn, 256: 198.4 -> 197.8.
 // Slabs of 64 columns up to 32 MB of states, where few workgroups hold many waves each (1 sequence 9.7, with slabs of 128
-// columns 11.7); beyond, 128 columns and two workgroups a CU (17 sequences 21 -> 16, 256: 208 -> 167).  Loads: kStream to
+// columns 11.7), but 128 where 64 would make eight slabs to a workgroup (64 value heads, 1 sequence eager 17.8 -> 12.7, 8
+// 18.3 -> 16.9); beyond, 128 columns and two workgroups a CU (17 sequences 21 -> 16, 256: 208 -> 167).  Loads: kStream to
 // 128 MB (64 sequences, five sets of states in turn, 53 against 56 with kCached; 32: 25 and 26), then kCached (112 sequences,
 // the same states every step, 81 against 86), kMixed from 256 MB on as in the rule alone.
 // Four slabs of 128 columns (four value heads to a q/k head) end at 128 MB: their 1024 threads have a CU to themselves, where
