@@ -20,6 +20,7 @@
 #include "gdn_common.h"
 #include "gdn_profile.h"
 #include "gdn_segments.h"
+#include "gdn_slab.h"
 
 namespace gdn {
 
@@ -31,33 +32,34 @@ namespace gdn {
 // (the last term is W^T dV' with W = Tm (beta e^G K) never materialised), dS, dV', R and the scaled dO used as B
 // operands straight from registers.  dS (gradient of the state AFTER the chunk) and dV' leave in fragment order.
 // Loader waves copy the A operands from contiguous fragment-order blocks: K and Q^T per q/k group, Tm and Aq per value
-// head; K^T and Tm^T are the same images read with the transposing LDS read, and so are the slab's raw dO rows on
-// their way into the B-operand layout.  The per-token factors never enter the compute wave's dependent chain: the
-// loaders write K twice, rows scaled by e^{G_last-G} (for K dS) and by -beta e^G (for the K^T product), and dO twice,
-// raw and with rows scaled by scale e^G.
+// head; K^T and Tm^T are read with the transposing LDS read, and so are the slab's raw dO rows on their way into the
+// B-operand layout.  The factors e^{G_last-G} and -beta e^G of the
+// tokens are applied to the accumulators of K dS and R in fp32; dO is staged twice, raw and with rows scaled by scale e^G.
 // ---------------------------------------------------------------------------------------------
 template <typename T, int DK, int NW, int STAGES, bool KDA = false> struct StateBwdSmem {
   // one stage, in elements of T
-  static constexpr int off_k = 0;                        // K images [2][K/32][2] tiles: rows x e^{G_last-G}, rows x -beta e^G
-  static constexpr int off_q = off_k + 2 * 64 * DK;      // Q^T image
+  static constexpr int off_k = 0;                        // K image as it lies [K/32][2] tiles
+  // that of the transposing reads: the same one, unless it arrives with factors of its own or lies otherwise
+  static constexpr int off_kt = KDA || SlabOf<T, NW>::type::kImageT ? off_k + 64 * DK : off_k;
+  static constexpr int off_q = off_kt + 64 * DK;         // Q^T image
   static constexpr int off_tm = off_q + 64 * DK;         // Tm tiles (0,0), (1,0), (1,1)
   static constexpr int off_aq = off_tm + 3 * 1024;       // Aq tiles (0,0), (1,0), (1,1)
   static constexpr int off_do = off_aq + 3 * 1024;       // dO rows of the slabs [2][64][32 NW]: raw, rows x scale e^G
-  static constexpr int off_row = (off_do + 2 * 64 * 32 * NW) * (int)sizeof(T);   // bytes: G_last; KDA: e^{G_last} per key channel [DK]
-  static constexpr int stage = off_row + (KDA ? DK * 4 : 16);
+  // bytes: e^{G_last-G} [64], -beta e^G [64], G_last; KDA: e^{G_last} per key channel [DK]
+  static constexpr int off_row = (off_do + 2 * 64 * 32 * NW) * (int)sizeof(T);
+  static constexpr int stage = off_row + (KDA ? DK * 4 : 132 * 4);
   static constexpr int bytes = STAGES * stage;
   static_assert(bytes <= 160 * 1024, "one CU's LDS");
 };
-
-template <int PIECES, int NT> struct DealB { static constexpr int kPer = (PIECES + NT - 1) / NT; };
 
 // KDA (one decay per key channel): kaf and kaf2 hold the two K images ready-made (rows x e^{G_last-G} and rows x
 // -beta e^{G}, channel by channel), qtf the transposed rows of q with scale and decay already applied (so dO is used
 // as it is), G holds e^{G_last} [chunks,Hv,DK]; the rows of dS decay each by their own factor.
 // segs, MAP: as in the forward recurrence; the map of a segment leaves in dh0.
+template <typename T> constexpr int state_bwd_waves(int nw, int nl) { return nw * slab_waves<T>(nw) + nl; }   // compute and loading
 template <typename T, int DK, int NW, int NL, int STAGES, bool KDA = false, bool MAP = false>
-__global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 && NL >= 4) ? 2 : 1) void chunk_state_bwd_kernel(
-    const T* __restrict__ kaf, const T* __restrict__ kaf2, const T* __restrict__ qtf, const T* __restrict__ ai, const T* __restrict__ aqf,
+__global__ __launch_bounds__(64 * state_bwd_waves<T>(NW, NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2) ? 2 : 1) void chunk_state_bwd_kernel(
+    const T* __restrict__ kaf, const T* __restrict__ kaf2, const T* __restrict__ qtf, const T* __restrict__ ai, const T* __restrict__ aqtf,
     const T* __restrict__ dO, const float* __restrict__ G, const float* __restrict__ bt,
     const float* __restrict__ dht,
     float* __restrict__ dh0, T* __restrict__ dvf, T* __restrict__ dhf, const int64_t* __restrict__ cu,
@@ -65,8 +67,10 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
   using SM = StateBwdSmem<T, DK, NW, STAGES, KDA>;
   static_assert(!KDA || 64 * NL >= DK, "a loader thread per key channel");
   constexpr int NT = 64 * NL, VEC = Elem<T>::kVec, NKT = DK / 32;   // NT loader threads
+  using SL = typename SlabOf<T, NW>::type;
+  constexpr int NWC = NW * SL::kWaves;   // compute waves
   constexpr int PK = 64 * DK / VEC, PTM = 3 * 1024 / VEC, PD = 64 * 32 * NW / VEC, DPR = 32 * NW / VEC;
-  constexpr int CK = DealB<PK, NT>::kPer, CTM = DealB<PTM, NT>::kPer, CD = DealB<PD, NT>::kPer;
+  constexpr int CK = Deal<PK, NT>::kPer, CTM = Deal<PTM, NT>::kPer, CD = Deal<PD, NT>::kPer;
   static_assert(STAGES == 1 || STAGES == 2, "one or two LDS stages");
 
   const int tid = threadIdx.x;
@@ -81,15 +85,13 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
   const int col0 = of_a ? 0 : (int)blockIdx.y * (32 * NW);   // of the rows of dO it reads
 
   // step s = 0 .. nchunks-1 handles chunk nchunks-1-s
-  if (wave >= NW) {
+  if (wave >= NWC) {
     // ================= loader waves =================
-    const int lt = tid - 64 * NW;
+    const int lt = tid - 64 * NWC;
     constexpr int DEPTH = (STAGES == 2) ? 2 : 1;
     Vec16<T> pk[DEPTH][CK], pk2[DEPTH][KDA ? CK : 1], pq[DEPTH][CK], ptm[DEPTH][CTM], pa[DEPTH][CTM], pd[DEPTH][CD];
-    float pgl[DEPTH], pgk[DEPTH][2], pbk[DEPTH][2], pgd[DEPTH][CD];
+    float pgl[DEPTH], pg[DEPTH], pb[DEPTH], pgd[DEPTH][CD];
     int pnv[DEPTH];
-    static_assert(NT % (sizeof(T) == 2 ? 128 : 32) == 0, "a thread's pieces sit at one place of their tiles");
-    const int krow = frag_piece_row<T>(lt & 127);
     auto tm_src = [&](int idc) {   // piece of the three kept tiles -> its place among the four stored ones
       const int t = idc / (1024 / VEC);
       return (t == 0 ? 0 : t + 1) * (1024 / VEC) + idc % (1024 / VEC);
@@ -101,20 +103,20 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
       const int64_t ch = (chunk_base + c) * Hv + h, chq = (chunk_base + c) * Hqk + h / (Hv / Hqk);
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = imin(lt + i * NT, PK - 1);
+        const int idc = dealt<PK, NT>(lt, i);
         pk[set][i] = ld16(kaf + chq * (64 * DK) + idc * VEC);
         if constexpr (KDA) pk2[set][i] = ld16(kaf2 + chq * (64 * DK) + idc * VEC);
         pq[set][i] = ld16(qtf + chq * (64 * DK) + idc * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int src = tm_src(imin(lt + i * NT, PTM - 1));
+        const int src = tm_src(dealt<PTM, NT>(lt, i));
         ptm[set][i] = ld16(ai + ch * 4096 + src * VEC);
-        pa[set][i] = ld16(aqf + ch * 4096 + src * VEC);
+        pa[set][i] = ld16(aqtf + ch * 4096 + src * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CD; ++i) {   // dO rows of the slabs; rows past the end repeat the last one and are cleared below
-        const int idc = imin(lt + i * NT, PD - 1), row = imin(idc / DPR, nvalid - 1), cc = idc % DPR;
+        const int idc = dealt<PD, NT>(lt, i), row = imin(idc / DPR, nvalid - 1), cc = idc % DPR;
         pd[set][i] = ld16(dO + ((tok0 + row) * Hv + h) * V + col0 + cc * VEC);
         if constexpr (!KDA) pgd[set][i] = G[ch * 64 + row];
       }
@@ -124,47 +126,30 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
         return;
       }
       const float* gc = G + ch * 64;
-      // raw values only: arithmetic here would wait for every load issued so far.  The array repeats G_last past the
-      // end of a short chunk.  In the K tiles every 16-byte piece belongs to one token, 32 (tile & 1) + the row of its
-      // place, and this thread's pieces all sit at the same place of their tiles: the gates of two tokens cover them.
+      // raw values only: arithmetic here would wait for every load issued so far.  The arrays repeat G_last past the
+      // end of a short chunk and hold a beta of 0 there.
       pgl[set] = gc[63];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        pgk[set][j] = gc[32 * j + krow];
-        pbk[set][j] = bt[ch * 64 + 32 * j + krow];
-      }
+      pg[set] = gc[lt & 63];
+      pb[set] = bt[ch * 64 + (lt & 63)];
     };
     auto commit = [&](int set, int buf) {
       T* st = reinterpret_cast<T*>(gdn_smem + buf * SM::stage);
-      float f1[2], f2[2];
-      if constexpr (!KDA) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          f1[j] = __expf(pgl[set] - pgk[set][j]);
-          f2[j] = (32 * j + krow < pnv[set]) ? -pbk[set][j] * __expf(pgk[set][j]) : 0.f;
-        }
-      }
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = imin(lt + i * NT, PK - 1), tj = (idc / (1024 / VEC)) & 1;
-        if constexpr (KDA) {
-          st16(st + SM::off_k + idc * VEC, pk[set][i]);
-          st16(st + SM::off_k + 64 * DK + idc * VEC, pk2[set][i]);
-        } else {
-          st16(st + SM::off_k + idc * VEC, scale16<T>(pk[set][i], f1[tj]));
-          st16(st + SM::off_k + 64 * DK + idc * VEC, scale16<T>(pk[set][i], f2[tj]));
-        }
+        const int idc = dealt<PK, NT>(lt, i);
+        st16(st + SM::off_k + idc * VEC, pk[set][i]);
+        if constexpr (SM::off_kt != SM::off_k) SL::st_t(st + SM::off_kt, idc, KDA ? pk2[set][i] : pk[set][i]);
         st16(st + SM::off_q + idc * VEC, pq[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int idc = imin(lt + i * NT, PTM - 1);
-        st16(st + SM::off_tm + idc * VEC, ptm[set][i]);
+        const int idc = dealt<PTM, NT>(lt, i);
+        SL::st_t(st + SM::off_tm, idc, ptm[set][i]);
         st16(st + SM::off_aq + idc * VEC, pa[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CD; ++i) {
-        const int idc = imin(lt + i * NT, PD - 1);
+        const int idc = dealt<PD, NT>(lt, i);
         const Vec16<T> x = idc / DPR < pnv[set] && !of_a ? pd[set][i] : zero16<T>();
         st16(st + SM::off_do + idc * VEC, x);
         if constexpr (KDA) st16(st + SM::off_do + 64 * 32 * NW + idc * VEC, x);
@@ -175,7 +160,11 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
         if (lt < DK) row[lt] = pgl[set];
         return;
       }
-      if (lt == 0) row[0] = pgl[set];
+      if (lt < 64) {
+        row[lt] = __expf(pgl[set] - pg[set]);
+        row[64 + lt] = -pb[set] * __expf(pg[set]);
+      }
+      if (lt == 0) row[128] = pgl[set];
     };
     if (nchunks == 0) return;
     if (STAGES == 2) {
@@ -218,71 +207,72 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
   }
 
   // ================= compute waves =================
-  const int vblk = blockIdx.y * NW + wave, v0 = 32 * vblk;
-  f32x16 dS[NKT];
+  const int slab = wave / SL::kWaves, strip = wave % SL::kWaves;   // of the workgroup's slabs; of the slab's strips of columns
+  const int vblk = blockIdx.y * NW + slab, v0 = 32 * vblk + SL::kCols * strip;
+  typename SL::Acc dS[NKT];
 #pragma unroll
   for (int kt = 0; kt < NKT; ++kt) {
-    dS[kt] = acc_zero();
+    dS[kt] = SL::zero();
     if constexpr (MAP) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) dS[kt][r] = v0 + acc_col() == V + 32 * kt + acc_row(r) ? 1.f : 0.f;
+      for (int r = 0; r < SL::kVals; ++r) dS[kt].set(r, v0 + SL::col() == V + 32 * kt + SL::row(r) ? 1.f : 0.f);
     } else if (dht != nullptr) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        dS[kt][r] = dht[(((int64_t)ns * Hv + h) * DK + 32 * kt + acc_row(r)) * V + v0 + acc_col()];
+      for (int r = 0; r < SL::kVals; ++r)
+        dS[kt].set(r, dht[(((int64_t)ns * Hv + h) * DK + 32 * kt + SL::row(r)) * V + v0 + SL::col()]);
     }
   }
   // As in the forward recurrence the vector work that does not depend on the running products (decay and packing of
   // dS) is written between the matrix instructions.
-  AccB<T> dSb[NKT];
+  typename SL::B dSb[NKT];
 #pragma unroll
   for (int kt = 0; kt < NKT; ++kt) dSb[kt].pack(dS[kt]);
-  // Two tile products into two accumulators, the matrix instructions of one alternating with those of the other: back
-  // to back on one accumulator a matrix instruction costs half as much again (49 cycles against 34, measured).
-  auto mma2 = [](f32x16& x0, const AccB<T>& a0, const AccB<T>& b0, f32x16& x1, const AccB<T>& a1, const AccB<T>& b1) {
-#pragma unroll
-    for (int kg = 0; kg < AccK<T>::kGroups; ++kg) {
-      mfma_kgroup<T>(x0, a0.f[kg], b0.f[kg]);
-      mfma_kgroup<T>(x1, a1.f[kg], b1.f[kg]);
-    }
-  };
   for (int st = 0; st < nchunks; ++st) {
     const int c = nchunks - 1 - st;
     const int buf = (STAGES == 2) ? (st & 1) : 0;
     GDN_LDS_BARRIER();                      // (A)
     const T* sm = reinterpret_cast<const T*>(gdn_smem + buf * SM::stage);
-    const T* Ka = sm + SM::off_k;              // rows x e^{G_last-G}
-    const T* Kn = Ka + 64 * DK;                // rows x -beta e^G
+    const T* Ka = sm + SM::off_k;              // KDA: rows x e^{G_last-G}
+    const T* Kn = sm + SM::off_kt;             // KDA: rows x -beta e^G
     const T* Qa = sm + SM::off_q;
     const T* Tm = sm + SM::off_tm;
     const T* Aq = sm + SM::off_aq;
-    const T* dOs = sm + SM::off_do;
+    const T* dOs = sm + SM::off_do + 32 * slab + SL::kCols * strip;
     const float* row = reinterpret_cast<const float*>(gdn_smem + buf * SM::stage + SM::off_row);
-    // dO of this wave's 32 columns as B operand (lane <-> V column, registers <-> token), raw and scaled by scale e^G
+    // dO of this wave's columns as B operand (lane <-> V column, registers <-> token), raw and scaled by scale e^G
     // of its token: the factor of the Q^T product rides on dO, so that the Q^T tiles are the same for every value head
     // of a q/k group
-    AccB<T> dob[2], dos[2], aq[3];
-    dob[0].load_cols(dOs + 32 * wave, 32 * NW);
-    dob[1].load_cols(dOs + 32 * (32 * NW) + 32 * wave, 32 * NW);
-    dos[0].load_cols(dOs + 64 * 32 * NW + 32 * wave, 32 * NW);
-    dos[1].load_cols(dOs + 64 * 32 * NW + 32 * (32 * NW) + 32 * wave, 32 * NW);
-    aq[0].load(Aq);                           // tiles (0,0), (1,0), (1,1)
+    typename SL::B dob[2], dos[2];
+    typename SL::A aq[3];
+    dob[0].load_cols(dOs, 32 * NW);
+    dob[1].load_cols(dOs + 32 * (32 * NW), 32 * NW);
+    dos[0].load_cols(dOs + 64 * 32 * NW, 32 * NW);
+    dos[1].load_cols(dOs + 64 * 32 * NW + 32 * (32 * NW), 32 * NW);
+    // tiles (0,0), (1,0), (1,1), whose rows (token j of Q K^T's columns) become accumulator rows
+    aq[0].load(Aq);
     aq[1].load(Aq + 1024);
     aq[2].load(Aq + 2048);
-    const float eg = KDA ? 1.f : __expf(row[0]);
+    const float eg = KDA ? 1.f : __expf(row[128]);
     const int64_t tile0 = ((chunk_base + c) * Hv + h) * (V / 32) + vblk;
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
-      if constexpr (!MAP) dSb[kt].store_stream(dhf + (tile0 * NKT + kt) * 1024);
-    // dV' = (scale tril(Q K^T . Gam))^T dO (from the forward pass's tiles) + (e^{G_last-G} . K) dS, one accumulation
+      if constexpr (!MAP) dSb[kt].store_stream(dhf + (tile0 * NKT + kt) * 1024, strip);
+    // dV' = (scale tril(Q K^T . Gam))^T dO (from the forward pass's tiles) + e^{G_last-G} . (K dS), one accumulation
     // chain per 32-token block.  The pair of A-operand tiles of K tile kt + 1 is requested from LDS before the matrix
     // instructions of K tile kt are issued (two register buffers); the decay of dS rides in between.
-    f32x16 a0 = acc_zero(), a1 = acc_zero();
-    AccB<T> af[2][2];                         // [buffer][tile of the pair]
+    typename SL::Acc a0 = SL::zero(), a1 = SL::zero();
+    typename SL::A af[2][2];                  // [buffer][tile of the pair]
+    typename SL::Rows fd, fn;                 // e^{G_last-G} and -beta e^G of the tokens; KDA: see below
+    if constexpr (!KDA) {
+      fd.load(row);
+      fn.load(row + 64);
+    }
+    typename SL::Acc u0 = SL::zero(), u1 = SL::zero();   // !KDA: the first sum, to which the scaled K dS is added
+    typename SL::Acc &c0 = KDA ? a0 : u0, &c1 = KDA ? a1 : u1;
     af[0][0].load(Ka);
     af[0][1].load(Ka + 1024);
-    mma2(a0, aq[0], dob[0], a1, aq[2], dob[1]);
-    mma32_ff<T>(a0, aq[1], dob[1]);
+    SL::mma2(c0, aq[0], dob[0], c1, aq[2], dob[1]);
+    SL::mma(c0, aq[1], dob[1]);
     GDN_SCHED_FENCE();
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt) {        // K tile kt, both 32-token blocks: one accumulator each
@@ -290,30 +280,44 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
         af[(kt + 1) & 1][0].load(Ka + (2 * kt + 2) * 1024);
         af[(kt + 1) & 1][1].load(Ka + (2 * kt + 3) * 1024);
       }
-      mma2(a0, af[kt & 1][0], dSb[kt], a1, af[kt & 1][1], dSb[kt]);
+      SL::mma2(a0, af[kt & 1][0], dSb[kt], a1, af[kt & 1][1], dSb[kt]);
       if constexpr (KDA) {
-        const f32x16 dk = rows_ld(row, 32 * kt);   // the decay of each of the tile's 32 key channels
+        if ((kt & 1) == 0) fd.load(row + 32 * kt);   // the decay of each of the two tiles' key channels
+        fd.fetch(kt & 1);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) dS[kt][r] *= dk[r];
+        for (int r = 0; r < SL::kVals; ++r) dS[kt].set(r, dS[kt].get(r) * fd.get(kt & 1, r));
       } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) dS[kt][r] *= eg;
+        for (int r = 0; r < SL::kVals; ++r) dS[kt].set(r, dS[kt].get(r) * eg);
+        if (kt >= NKT - 2) {
+          GDN_SCHED_FENCE();
+          fd.fetch(kt - (NKT - 2));
+        }
       }
       GDN_SCHED_FENCE();
     }
-    AccB<T> dvb[2], rb[2], tf[3];
+    typename SL::B dvb[2], rb[2];
+    typename SL::A tf[3];
 #pragma unroll
-    for (int t = 0; t < 3; ++t) tf[t].load_t(Tm + t * 1024);   // Tm^T tiles: (lane <-> column of Tm, registers <-> row)
+    for (int t = 0; t < 3; ++t) tf[t].load_t(Tm + t * 1024);   // Tm^T tiles: columns of Tm <-> accumulator rows
+    if constexpr (!KDA) {
+#pragma unroll
+      for (int r = 0; r < SL::kVals; ++r) {
+        a0.set(r, c0.get(r) + fd.get(0, r) * a0.get(r));
+        a1.set(r, c1.get(r) + fd.get(1, r) * a1.get(r));
+      }
+    }
     dvb[0].pack(a0);
     dvb[1].pack(a1);
     if constexpr (!MAP) {
-      dvb[0].store_stream(dvf + (tile0 * 2 + 0) * 1024);
-      dvb[1].store_stream(dvf + (tile0 * 2 + 1) * 1024);
+      dvb[0].store_stream(dvf + (tile0 * 2 + 0) * 1024, strip);
+      dvb[1].store_stream(dvf + (tile0 * 2 + 1) * 1024, strip);
     }
     // R = Tm^T dV' (upper triangular: R_0 = Tm00^T dV'_0 + Tm10^T dV'_1, R_1 = Tm11^T dV'_1)
-    f32x16 y0 = acc_zero(), y1 = acc_zero();
-    mma2(y0, tf[0], dvb[0], y1, tf[2], dvb[1]);
-    mma32_ff<T>(y0, tf[1], dvb[1]);
+    typename SL::Acc y0 = SL::zero(), y1 = SL::zero();
+    SL::mma2(y0, tf[0], dvb[0], y1, tf[2], dvb[1]);
+    SL::mma(y0, tf[1], dvb[1]);
+    if constexpr (!KDA) { fn.fetch(0); fn.fetch(1); }
     // A operands of the update of dS, for the pair of 32-row tiles (2 pr, 2 pr + 1) of dS and product p = 2 tj + w:
     // w = 0 the Q^T tile as it lies, w = 1 the K image read transposed
     auto load_qk = [&](int b, int pr, int p) {
@@ -324,10 +328,17 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
       }
     };
     load_qk(0, 0, 0);
+    if constexpr (!KDA) {
+#pragma unroll
+      for (int r = 0; r < SL::kVals; ++r) {
+        y0.set(r, fn.get(0, r) * y0.get(r));
+        y1.set(r, fn.get(1, r) * y1.get(r));
+      }
+    }
     rb[0].pack(y0);
     rb[1].pack(y1);
     GDN_SCHED_FENCE();
-    // dS <- e^{G_last} dS + Q^T (scale e^G . dO) + (-beta e^G . K)^T R, two tiles of dS at a time so that consecutive
+    // dS <- e^{G_last} dS + Q^T (scale e^G . dO) + K^T (-beta e^G . R), two tiles of dS at a time so that consecutive
     // matrix instructions never accumulate into the same one; a finished pair is packed for the next step while the
     // matrix pipe works on the following one
     static_assert(NKT % 2 == 0, "tiles of dS are updated in pairs");
@@ -335,8 +346,8 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
     for (int m = 0; m < 2 * NKT; ++m) {       // m = 4 pr + p
       const int pr = m >> 2, pp = m & 3;
       if (m + 1 < 2 * NKT) load_qk((m + 1) & 1, (m + 1) >> 2, (m + 1) & 3);
-      const AccB<T>& bop = (pp & 1) ? rb[pp >> 1] : dos[pp >> 1];
-      mma2(dS[2 * pr], af[m & 1][0], bop, dS[2 * pr + 1], af[m & 1][1], bop);
+      const typename SL::B& bop = (pp & 1) ? rb[pp >> 1] : dos[pp >> 1];
+      SL::mma2(dS[2 * pr], af[m & 1][0], bop, dS[2 * pr + 1], af[m & 1][1], bop);
       if (pp == 1 && pr >= 1) {
         dSb[2 * pr - 2].pack(dS[2 * pr - 2]);
         dSb[2 * pr - 1].pack(dS[2 * pr - 1]);
@@ -354,7 +365,7 @@ __global__ __launch_bounds__(64 * (NW + NL)) GDN_WAVES_PER_SIMD((sizeof(T) == 2 
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) to[(int64_t)(32 * kt + acc_row(r)) * ldt + v0 + acc_col()] = dS[kt][r];
+      for (int r = 0; r < SL::kVals; ++r) to[(int64_t)(32 * kt + SL::row(r)) * ldt + v0 + SL::col()] = dS[kt].get(r);
   }
 }
 
@@ -1012,7 +1023,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         auto kern = chunk_state_bwd_kernel<T, DK, 2, NLS, STAGES, false, true>;
         constexpr int smem = StateBwdSmem<T, DK, 2, STAGES>::bytes;
         if (int e = set_lds_b(kern, smem)) return e;
-        GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
+        GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * state_bwd_waves<T>(2, NLS)), smem, st,
                    (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, Bt,
                    (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, cu, chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, segs);
         GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * d.Hv, d.V / 16), dim3(4 * DK), 0, st,
@@ -1036,7 +1047,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
       auto kern = chunk_state_bwd_kernel<T, DK, NWS, NLS, STAGES>;
       constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES>::bytes;
       if (int e = set_lds_b(kern, smem)) return e;
-      GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st,
+      GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * d.Hv, d.V / (32 * NWS)), dim3(64 * state_bwd_waves<T>(NWS, NLS)), smem, st,
                  (const T*)KAF, (const T*)nullptr, (const T*)QTF, Ai, AQ, (const T*)dO, G, Bt, dht, dh0, DVF, DHF, cu,
                  chunk_offsets, d.T, d.Hqk, d.Hv, d.V, scale, segs);
     }
@@ -1115,9 +1126,9 @@ static int chunk_bwd_entry(const void* q, const void* k, const void* v, int64_t 
   if (dtype == 1) {
     if (K == 128 && wide && solo) GDN_BWD(bf16_t, 128, 4, 1, 4, 2);
     if (K == 128 && wide) GDN_BWD(bf16_t, 128, 4, 2, 4, 2);
-    if (K == 128) GDN_BWD(bf16_t, 128, 2, 2, 2, 2);
-    if (wide) GDN_BWD(bf16_t, 64, 4, 2, 2, 2);
-    GDN_BWD(bf16_t, 64, 2, 2, 2, 2);
+    if (K == 128) GDN_BWD(bf16_t, 128, 2, 2, 4, 2);
+    if (wide) GDN_BWD(bf16_t, 64, 4, 2, 4, 2);
+    GDN_BWD(bf16_t, 64, 2, 2, 4, 2);
   } else {
     if (K == 128) GDN_BWD(float, 128, 2, 2, 2, 1);
     GDN_BWD(float, 64, 2, 2, 2, 1);

@@ -16,6 +16,7 @@
 #include "gdn_common.h"
 #include "gdn_profile.h"
 #include "gdn_segments.h"
+#include "gdn_slab.h"
 #include "gdn_rmsnorm_gated.h"
 
 namespace gdn {
@@ -339,6 +340,10 @@ __global__ __launch_bounds__(kThreads) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 4 : 3
 // element type and key width follows, so that all of them round alike.
 // output waves per slab: a workgroup with a single slab has room for two, one per 32-token block of the chunk
 template <int NW> struct StateOutWaves { static constexpr int value = NW == 1 ? 2 : 1; };
+// waves of a workgroup: of compute, output and loading
+template <typename T> constexpr int state_waves(int nw, int nl, bool out) {
+  return nw * (slab_waves<T>(nw) + (out ? (nw == 1 ? 2 : 1) : 0)) + nl;
+}
 template <typename T, int DK, int NW, int STAGES, bool FUSE> struct StatePre {
   static constexpr int x_elems = 2 * DK * 32 + 2 * 2048 + StateOutWaves<NW>::value * Patch<T>::kElems;
   static constexpr bool value = STAGES * ((2 * 64 * DK + 3 * 1024 + 64 * 32 * NW + (FUSE ? 64 * DK + 3 * 1024 : 0)) * (int)sizeof(T) + 68 * 4) +
@@ -348,8 +353,10 @@ template <typename T, int DK, int NW, int STAGES, bool OUT, bool PRE_, bool KDA 
   static constexpr int x_elems = 2 * DK * 32 + 2 * 2048 + StateOutWaves<NW>::value * Patch<T>::kElems;
   static constexpr bool PRE = PRE_;
   // one stage, in elements of T
-  static constexpr int off_k = 0;                                   // K image(s) [K/32][2] tiles
-  static constexpr int off_tm = off_k + (PRE ? 2 : 1) * 64 * DK;    // Tm tiles (0,0), (1,0), (1,1)
+  static constexpr int off_k = 0;                                   // K image as it lies [K/32][2] tiles
+  // that of the transposing reads: the same one, unless it carries factors of its own or lies otherwise
+  static constexpr int off_kt = PRE || SlabOf<T, NW>::type::kImageT ? 64 * DK : 0;
+  static constexpr int off_tm = off_kt + 64 * DK;                   // Tm tiles (0,0), (1,0), (1,1)
   static constexpr int off_v = off_tm + 3 * 1024;                   // raw v rows of the slabs [64][32 NW]
   static constexpr int off_q = off_v + 64 * 32 * NW;                // OUT: Q^T image
   static constexpr int off_aq = off_q + (OUT ? 64 * DK : 0);        // OUT: Aq tiles (0,0), (1,0), (1,1)
@@ -364,17 +371,13 @@ template <typename T, int DK, int NW, int STAGES, bool OUT, bool PRE_, bool KDA 
   static_assert(bytes <= 160 * 1024, "one CU's LDS");
 };
 
-// pieces [0, PIECES) of 16 bytes dealt to NT threads, the same number to each: indices past the end repeat the last
-// piece (the same loads on every path; the duplicate lands on the same LDS address with the same data)
-template <int PIECES, int NT> struct Deal { static constexpr int kPer = (PIECES + NT - 1) / NT; };
-
 // KDA (one decay per key channel): kaf and qtf hold the two K images ready-made, rows scaled by -beta e^{G} and by
 // e^{G_last-G} channel by channel, G holds e^{G_last} [chunks,Hv,DK] and bt the transformed beta; the state's
 // rows decay each by their own factor.  With OUT the output waves take (scale q . e^{G})^T from a third image, qim,
 // whose rows carry every factor of the output's first term (the other modes read their Q^T image through qtf).
 // segs: segments of a sequence, each with its own initial state (gdn_segments.h); MAP: their maps [B | A] into ht.
 template <typename T, int DK, int NW, int NL, int STAGES, bool OUT, bool PRE_, bool KDA = false, bool MAP = false>
-__global__ __launch_bounds__(64 * (NW + (OUT ? NW * StateOutWaves<NW>::value : 0) + NL)) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 2 : 1)
+__global__ __launch_bounds__(64 * state_waves<T>(NW, NL, OUT)) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 2 : 1)
 void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, const T* __restrict__ ai,
                         const T* __restrict__ aqf, const T* __restrict__ v, const float* __restrict__ G,
                         const float* __restrict__ bt, const float* __restrict__ h0, float* __restrict__ ht,
@@ -384,6 +387,8 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
   using SM = StateSmem<T, DK, NW, STAGES, OUT, PRE_, KDA>;
   static_assert(!KDA || 64 * NL >= DK, "a loader thread per key channel");
   constexpr int NT = 64 * NL, VEC = Elem<T>::kVec, NKT = DK / 32, OS = StateOutWaves<NW>::value, NWO = OUT ? NW * OS : 0;
+  using SL = typename SlabOf<T, NW>::type;
+  constexpr int NWC = NW * SL::kWaves;   // compute waves
   constexpr int PK = 64 * DK / VEC, PTM = 3 * 1024 / VEC, PV = 64 * 32 * NW / VEC, VPR = 32 * NW / VEC;
   constexpr int CK = Deal<PK, NT>::kPer, CTM = Deal<PTM, NT>::kPer, CV = Deal<PV, NT>::kPer;
   static_assert(STAGES == 1 || STAGES == 2, "one or two LDS stages");
@@ -409,20 +414,20 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
   // number of barriers every wave passes: one per chunk, plus one that hands the last V' to the output waves
   const int nsteps = nchunks + (OUT ? 1 : 0);
   if (nchunks == 0) {   // an empty sequence: its final state is its initial state; an empty segment has no map
-    if (!MAP && wave < NW && hto != nullptr) {
-      const int col = 32 * (blockIdx.y * NW + wave) + acc_col();
+    if (!MAP && wave < NWC && hto != nullptr) {
+      const int col = 32 * blockIdx.y * NW + SL::kCols * wave + SL::col();
       for (int kt = 0; kt < NKT; ++kt)
-        for (int r = 0; r < 16; ++r) {
-          const int row = 32 * kt + acc_row(r);
+        for (int r = 0; r < SL::kVals; ++r) {
+          const int row = 32 * kt + SL::row(r);
           hto[(int64_t)row * ldt + col] = initial(row, col);
         }
     }
     return;
   }
 
-  if (wave >= NW + NWO) {
+  if (wave >= NWC + NWO) {
     // ================= loader waves: 16-byte copies =================
-    const int lt = tid - 64 * (NW + NWO);
+    const int lt = tid - 64 * (NWC + NWO);
     // DEPTH register sets: chunk j sits in set j % DEPTH from the iteration that requests it (j - DEPTH - 1) to the
     // one that copies it to LDS (j - 1), so global loads have DEPTH chunk periods to arrive
     constexpr int DEPTH = (STAGES == 2) ? 2 : 1;
@@ -444,20 +449,20 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       const int64_t tok0 = bos + (int64_t)c * kChunk;
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = imin(lt + i * NT, PK - 1);
+        const int idc = dealt<PK, NT>(lt, i);
         pk[set][i] = ld16(kaf + chq * (64 * DK) + idc * VEC);   // shared by the value heads of the group
         if constexpr (OUT || KDA) pq[set][i] = ld16(qtf + chq * (64 * DK) + idc * VEC);
         if constexpr (OUT && KDA) pq2[set][i] = ld16(qim + chq * (64 * DK) + idc * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int src = tm_src(imin(lt + i * NT, PTM - 1));
+        const int src = tm_src(dealt<PTM, NT>(lt, i));
         ptm[set][i] = ld16(ai + ch * 4096 + src * VEC);
         if constexpr (OUT) pa[set][i] = ld16(aqf + ch * 4096 + src * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CV; ++i) {   // rows past the end of the sequence repeat the last one (their beta is 0)
-        const int idc = imin(lt + i * NT, PV - 1), row = imin(idc / VPR, nvalid - 1), cc = idc % VPR;
+        const int idc = dealt<PV, NT>(lt, i), row = imin(idc / VPR, nvalid - 1), cc = idc % VPR;
         pv[set][i] = ld16(v + (tok0 + row) * v_stride + (int64_t)h * V + col0 + cc * VEC);
         if constexpr (PRE) pbv[set][i] = bt[ch * 64 + row];
       }
@@ -495,28 +500,29 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       }
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = imin(lt + i * NT, PK - 1);
+        const int idc = dealt<PK, NT>(lt, i);
         if constexpr (KDA) {
           st16(st + SM::off_k + idc * VEC, pk[set][i]);
-          st16(st + SM::off_k + 64 * DK + idc * VEC, pq[set][i]);
+          SL::st_t(st + SM::off_kt, idc, pq[set][i]);
         } else if constexpr (PRE) {
           const int tj = (idc / (1024 / VEC)) & 1;
           st16(st + SM::off_k + idc * VEC, scale16<T>(pk[set][i], f1[tj]));
-          st16(st + SM::off_k + 64 * DK + idc * VEC, scale16<T>(pk[set][i], f2[tj]));
+          SL::st_t(st + SM::off_kt, idc, scale16<T>(pk[set][i], f2[tj]));
         } else {
           st16(st + SM::off_k + idc * VEC, pk[set][i]);
+          if constexpr (SM::off_kt != SM::off_k) SL::st_t(st + SM::off_kt, idc, pk[set][i]);
         }
         if constexpr (OUT) st16(st + SM::off_q + idc * VEC, KDA ? pq2[set][i] : pq[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int idc = imin(lt + i * NT, PTM - 1);
+        const int idc = dealt<PTM, NT>(lt, i);
         st16(st + SM::off_tm + idc * VEC, ptm[set][i]);
         if constexpr (OUT) st16(st + SM::off_aq + idc * VEC, pa[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CV; ++i) {
-        const int idc = imin(lt + i * NT, PV - 1);
+        const int idc = dealt<PV, NT>(lt, i);
         if (of_a) st16(st + SM::off_v + idc * VEC, zero16<T>());   // not v x 0: v may hold infinities
         else if constexpr (PRE) st16(st + SM::off_v + idc * VEC, scale16<T>(pv[set][i], idc / VPR < pnv[set] ? pbv[set][i] : 0.f));
         else st16(st + SM::off_v + idc * VEC, pv[set][i]);
@@ -579,12 +585,12 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
   }
 
   if constexpr (OUT) {
-    if (wave >= NW) {
-      // ================= output waves: O of the slab's 32 columns, one step behind the compute wave =================
+    if (wave >= NWC) {
+      // ================= output waves: O of the slab's 32 columns, one step behind the compute waves =================
       // OS == 2: wave `hw` of the slab's two owns the chunk's 32-token block hw (and that share of the stores for the
       // backward pass); OS == 1: one wave does both blocks.  Either way every row is accumulated by the same
       // instructions in the same order.
-      const int w = (wave - NW) / OS, hw = (wave - NW) % OS;
+      const int w = (wave - NWC) / OS, hw = (wave - NWC) % OS;
       const int vblk = blockIdx.y * NW + w, v0 = 32 * vblk;
       T* xs = reinterpret_cast<T*>(gdn_smem + SM::off_x) + w * SM::x_elems;
       T* patch = xs + 2 * DK * 32 + 2 * 2048 + hw * Patch<T>::kElems;
@@ -673,35 +679,27 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
   }
 
   // ================= compute waves =================
-  const int vblk = blockIdx.y * NW + wave, v0 = 32 * vblk;
-  f32x16 S[NKT];
+  const int slab = wave / SL::kWaves, strip = wave % SL::kWaves;   // of the workgroup's slabs; of the slab's strips of columns
+  const int vblk = blockIdx.y * NW + slab, v0 = 32 * vblk + SL::kCols * strip;
+  typename SL::Acc S[NKT];
 #pragma unroll
   for (int kt = 0; kt < NKT; ++kt) {
-    S[kt] = acc_zero();
+    S[kt] = SL::zero();
     if (MAP || h0 != nullptr) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) S[kt][r] = initial(32 * kt + acc_row(r), v0 + acc_col());
+      for (int r = 0; r < SL::kVals; ++r) S[kt].set(r, initial(32 * kt + SL::row(r), v0 + SL::col()));
     }
   }
-  // The wave issues its instructions in order and a matrix instruction occupies the matrix pipe for 32 cycles, in
-  // which eight vector instructions can issue: the loop body is written so that the vector work which does not
+  // The wave issues its instructions in order and a matrix instruction occupies the matrix pipe for 16 cycles (float: 32),
+  // in which vector instructions can issue: the loop body is written so that the vector work which does not
   // depend on the running product (decay of S, packing S for the next chunk) sits between the matrix instructions
   // instead of before or after them.
-  AccB<T> Sb[NKT];
-  T* xs = reinterpret_cast<T*>(gdn_smem + SM::off_x) + wave * SM::x_elems;   // OUT only
-  // Two tile products into two accumulators, the matrix instructions of one alternating with those of the other: back
-  // to back on one accumulator a matrix instruction costs half as much again (49 cycles against 34, measured).
-  auto mma2 = [](f32x16& x0, const AccB<T>& a0, const AccB<T>& b0, f32x16& x1, const AccB<T>& a1, const AccB<T>& b1) {
-#pragma unroll
-    for (int kg = 0; kg < AccK<T>::kGroups; ++kg) {
-      mfma_kgroup<T>(x0, a0.f[kg], b0.f[kg]);
-      mfma_kgroup<T>(x1, a1.f[kg], b1.f[kg]);
-    }
-  };
+  typename SL::B Sb[NKT];
+  T* xs = reinterpret_cast<T*>(gdn_smem + SM::off_x) + slab * SM::x_elems;   // OUT only
 #pragma unroll
   for (int kt = 0; kt < NKT; ++kt) {
     Sb[kt].pack(S[kt]);
-    if constexpr (OUT) Sb[kt].store(xs + kt * 1024);
+    if constexpr (OUT) Sb[kt].store(xs + kt * 1024, strip);
   }
   for (int c = 0; c < nchunks; ++c) {
     const int buf = (STAGES == 2) ? (c & 1) : 0;
@@ -709,45 +707,51 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     const T* st = reinterpret_cast<const T*>(gdn_smem + buf * SM::stage);
     constexpr bool PRE = SM::PRE;
     const T* Ka = st + SM::off_k;                        // PRE: rows scaled by -beta e^G
-    const T* Kb = Ka + (PRE ? 64 * DK : 0);              // PRE: rows scaled by e^{G_last-G}
+    const T* Kb = st + SM::off_kt;                       // PRE: rows scaled by e^{G_last-G}
     const T* Tm = st + SM::off_tm;
-    const T* Vs = st + SM::off_v;
+    const T* Vs = st + SM::off_v + 32 * slab + SL::kCols * strip;
     const float* row = reinterpret_cast<const float*>(gdn_smem + buf * SM::stage + SM::off_row);
     const int64_t tile0 = ((chunk_base + c) * Hv + h) * (V / 32) + vblk;
 
     constexpr int NP = NKT / 2;             // K tiles are processed two at a time
-    AccB<T> Kf[2][2][2];                    // [buffer][32-token block][K tile of the pair]; later [buffer][K tile][token block]
-    auto load_k = [&](int b, int kp) {      // K as it lies: (lane <-> token, registers <-> K column)
+    typename SL::A Kf[2][2][2];             // [buffer][32-token block][K tile of the pair]; later [buffer][K tile][token block]
+    auto load_k = [&](int b, int kp) {      // K as it lies: tokens <-> accumulator rows, k along the K columns
 #pragma unroll
       for (int ri = 0; ri < 2; ++ri)
 #pragma unroll
         for (int j = 0; j < 2; ++j) Kf[b][ri][j].load(Ka + ((2 * kp + j) * 2 + ri) * 1024);
     };
-    auto load_kt = [&](int b, int kp) {     // K^T: (lane <-> K column, registers <-> token)
+    auto load_kt = [&](int b, int kp) {     // K^T: K columns <-> accumulator rows, k along the tokens
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int tj = 0; tj < 2; ++tj) Kf[b][j][tj].load_t(Kb + ((2 * kp + j) * 2 + tj) * 1024);
     };
-    AccB<T> Vb[2], Tf[3];
-    Vb[0].load_cols(Vs + 32 * wave, 32 * NW);                     // raw v, (lane <-> V column, registers <-> token)
-    Vb[1].load_cols(Vs + 32 * (32 * NW) + 32 * wave, 32 * NW);
+    typename SL::B Vb[2];
+    typename SL::A Tf[3];
+    Vb[0].load_cols(Vs, 32 * NW);                                 // raw v: this wave's columns, registers <-> token
+    Vb[1].load_cols(Vs + 32 * (32 * NW), 32 * NW);
     load_k(0, 0);
     if (NP > 1) load_k(1, 1);
     const float eg = KDA ? 1.f : __expf(row[64]);
     if (!OUT && hf != nullptr) {   // with output waves the stores are theirs: they hold S and V' too and have the time
 #pragma unroll
-      for (int kt = 0; kt < NKT; ++kt) Sb[kt].store_stream(hf + (tile0 * NKT + kt) * 1024);
+      for (int kt = 0; kt < NKT; ++kt) Sb[kt].store_stream(hf + (tile0 * NKT + kt) * 1024, strip);
     }
     // y = K S (PRE: z = beta v - beta e^G . (K S) at once), the two 32-token blocks are independent accumulation
     // chains.  The decay of S rides between the matrix instructions.
-    f32x16 p0 = PRE ? Vb[0].unpack() : acc_zero(), p1 = PRE ? Vb[1].unpack() : acc_zero();
+    typename SL::Acc p0 = PRE ? Vb[0].unpack() : SL::zero(), p1 = PRE ? Vb[1].unpack() : SL::zero();
     // What the chain needs next is read from LDS while the matrix pipe works on what it has: Tm ahead of the last pair of
     // K tiles, the row factors between its products, K^T behind those with Tm.  The fences keep the compiler from moving
     // the reads to their uses, where each would be waited for.  Forward only 2 x 8192, 32 heads 199 -> 193 us, four packed
     // prompts 353 -> 344; K^T ahead of the last pair as well spills 33 registers and takes 393.
     static_assert(NP <= 2, "two buffers of K tiles");
-    f32x16 b0, b1, e0, e1;                  // !PRE: beta and beta e^G of the rows
+    typename SL::Rows fb, fe, fd;           // !PRE: beta, beta e^G and e^{G_last-G} of the tokens; KDA: see below
+    if constexpr (!PRE) {
+      fb.load(row + 196);
+      fe.load(row + 132);
+      fd.load(row + 68);
+    }
     GDN_SCHED_FENCE();
 #pragma unroll
     for (int kp = 0; kp < NP; ++kp) {
@@ -758,21 +762,23 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        mma2(p0, Kf[kp & 1][0][j], Sb[2 * kp + j], p1, Kf[kp & 1][1][j], Sb[2 * kp + j]);
+        SL::mma2(p0, Kf[kp & 1][0][j], Sb[2 * kp + j], p1, Kf[kp & 1][1][j], Sb[2 * kp + j]);
+        typename SL::Acc& Sj = S[2 * kp + j];
         if constexpr (KDA) {
-          const f32x16 dk = rows_ld(row + 68, 32 * (2 * kp + j));   // the decay of each of the tile's 32 key channels
+          if (j == 0) fd.load(row + 68 + 64 * kp);   // the decay of each of the tiles' 64 key channels
+          fd.fetch(j);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) S[2 * kp + j][r] *= dk[r];
+          for (int r = 0; r < SL::kVals; ++r) Sj.set(r, Sj.get(r) * fd.get(j, r));
         } else {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) S[2 * kp + j][r] *= eg;
+          for (int r = 0; r < SL::kVals; ++r) Sj.set(r, Sj.get(r) * eg);
         }
-        GDN_INTERLEAVE_MFMA_VALU(2 * AccK<T>::kGroups, 16 / (2 * AccK<T>::kGroups));
+        GDN_INTERLEAVE_MFMA_VALU(SL::kMma2, SL::kVals / SL::kMma2);
         if constexpr (!PRE) {
           if (kp == NP - 1) {
             GDN_SCHED_FENCE();
-            if (j == 0) { b0 = rows_ld(row + 196, 0); e0 = rows_ld(row + 132, 0); }
-            else { b1 = rows_ld(row + 196, 32); e1 = rows_ld(row + 132, 32); }
+            fb.fetch(j);
+            fe.fetch(j);
             GDN_SCHED_FENCE();
           }
         }
@@ -780,46 +786,45 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       GDN_SCHED_FENCE();
     }
     if constexpr (!PRE) {   // z = beta (v - e^G . y), the B operand of Tm z
-      const f32x16 x0 = Vb[0].unpack();
+      const typename SL::Acc x0 = Vb[0].unpack();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p0[r] = b0[r] * x0[r] - e0[r] * p0[r];
+      for (int r = 0; r < SL::kVals; ++r) p0.set(r, fb.get(0, r) * x0.get(r) - fe.get(0, r) * p0.get(r));
     }
     Vb[0].pack(p0);
     // V' = Tm z (Tm lower triangular: tiles (0,0), (1,0), (1,1)); the second block's z is formed beside the first products
-    f32x16 w0 = acc_zero(), w1 = acc_zero();
-    mma2(w0, Tf[0], Vb[0], w1, Tf[1], Vb[0]);
+    typename SL::Acc w0 = SL::zero(), w1 = SL::zero();
+    SL::mma2(w0, Tf[0], Vb[0], w1, Tf[1], Vb[0]);
     GDN_SCHED_FENCE();
     load_kt(0, 0);
     GDN_SCHED_FENCE();
     if constexpr (!PRE) {
-      const f32x16 x1 = Vb[1].unpack();
+      const typename SL::Acc x1 = Vb[1].unpack();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p1[r] = b1[r] * x1[r] - e1[r] * p1[r];
+      for (int r = 0; r < SL::kVals; ++r) p1.set(r, fb.get(1, r) * x1.get(r) - fe.get(1, r) * p1.get(r));
     }
     Vb[1].pack(p1);
-    f32x16 d0, d1;                          // !PRE: e^{G_last-G} of the rows
-    if constexpr (!PRE) { d0 = rows_ld(row + 68, 0); d1 = rows_ld(row + 68, 32); }
+    if constexpr (!PRE) { fd.fetch(0); fd.fetch(1); }
     GDN_SCHED_FENCE();
-    mma32_ff<T>(w1, Tf[2], Vb[1]);
+    SL::mma(w1, Tf[2], Vb[1]);
     GDN_SCHED_FENCE();
     if (NP > 1) load_kt(1, 1);
     GDN_SCHED_FENCE();
     Vb[0].pack(w0);
     T* const vx = xs + 2 * DK * 32 + (c & 1) * 2048;   // OUT only
-    if constexpr (OUT) Vb[0].store(vx);
-    else if (vf != nullptr) Vb[0].store_stream(vf + (tile0 * 2 + 0) * 1024);
+    if constexpr (OUT) Vb[0].store(vx, strip);
+    else if (vf != nullptr) Vb[0].store_stream(vf + (tile0 * 2 + 0) * 1024, strip);
     if constexpr (!PRE) {
       // the decay of the state update rides on V': (e^{G_last - G} . K)^T V' = K^T (e^{G_last - G} . V')
 #pragma unroll
-      for (int r = 0; r < 16; ++r) w0[r] *= d0[r];
+      for (int r = 0; r < SL::kVals; ++r) w0.set(r, w0.get(r) * fd.get(0, r));
       Vb[0].pack(w0);
     }
     Vb[1].pack(w1);
-    if constexpr (OUT) Vb[1].store(vx + 1024);
-    else if (vf != nullptr) Vb[1].store_stream(vf + (tile0 * 2 + 1) * 1024);
+    if constexpr (OUT) Vb[1].store(vx + 1024, strip);
+    else if (vf != nullptr) Vb[1].store_stream(vf + (tile0 * 2 + 1) * 1024, strip);
     if constexpr (!PRE) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) w1[r] *= d1[r];
+      for (int r = 0; r < SL::kVals; ++r) w1.set(r, w1.get(r) * fd.get(1, r));
       Vb[1].pack(w1);
     }
     GDN_SCHED_FENCE();
@@ -829,7 +834,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     for (int kp = 0; kp < NP; ++kp) {
 #pragma unroll
       for (int tj = 0; tj < 2; ++tj) {   // the pair's two tiles of S take turns
-        mma2(S[2 * kp], Kf[kp & 1][0][tj], Vb[tj], S[2 * kp + 1], Kf[kp & 1][1][tj], Vb[tj]);
+        SL::mma2(S[2 * kp], Kf[kp & 1][0][tj], Vb[tj], S[2 * kp + 1], Kf[kp & 1][1][tj], Vb[tj]);
         if (kp >= 1) Sb[2 * kp - 2 + tj].pack(S[2 * kp - 2 + tj]);
       }
       GDN_SCHED_FENCE();
@@ -839,7 +844,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     for (int kt = (NKT >= 2 ? NKT - 2 : 0); kt < NKT; ++kt) Sb[kt].pack(S[kt]);
     if constexpr (OUT) {   // the state before chunk c+1, for the output wave's next step
 #pragma unroll
-      for (int kt = 0; kt < NKT; ++kt) Sb[kt].store(xs + ((c + 1) & 1) * (DK * 32) + kt * 1024);
+      for (int kt = 0; kt < NKT; ++kt) Sb[kt].store(xs + ((c + 1) & 1) * (DK * 32) + kt * 1024, strip);
     }
     if (STAGES == 1 && c + 1 < nsteps) GDN_LDS_BARRIER();      // (B) done with the single stage
   }
@@ -848,7 +853,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) hto[(int64_t)(32 * kt + acc_row(r)) * ldt + v0 + acc_col()] = S[kt][r];
+      for (int r = 0; r < SL::kVals; ++r) hto[(int64_t)(32 * kt + SL::row(r)) * ldt + v0 + SL::col()] = S[kt].get(r);
   }
 }
 
@@ -1065,7 +1070,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         auto kern = chunk_state_kernel<T, DK, 2, NLS, STAGES, false, PRE, false, true>;
         constexpr int smem = StateSmem<T, DK, 2, STAGES, false, PRE>::bytes;
         if (int e = set_lds(kern, smem)) return e;
-        GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
+        GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * d.Hv, (d.V + DK) / 64), dim3(64 * state_waves<T>(2, NLS, false)), smem, st,
                    (const T*)KAF, (const T*)QTF, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)G, (const float*)Bt,
                    (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T,
                    d.Hqk, d.Hv, d.V, scale, ts.v, (const T*)nullptr, segs);
@@ -1085,7 +1090,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
   if constexpr (FUSE) {
     if (fuse) {
       if (int e = launch_state(chunk_state_kernel<T, DK, NWS, NLS, STAGES, true, PRE>,
-                               StateSmem<T, DK, NWS, STAGES, true, PRE>::bytes, NWS * (1 + StateOutWaves<NWS>::value) + NLS, (T*)o))
+                               StateSmem<T, DK, NWS, STAGES, true, PRE>::bytes, state_waves<T>(NWS, NLS, true), (T*)o))
         return e;
       return (int)hipGetLastError();
     }
@@ -1103,7 +1108,7 @@ static int chunk_fwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
                     : launch_f32(chunk_state_f32_kernel<DK, 2>, StateF32Smem<DK, 2>::bytes, 32))
       return e;
   } else if (int e = launch_state(chunk_state_kernel<T, DK, NWS, NLS, STAGES, false, PRE>,
-                                  StateSmem<T, DK, NWS, STAGES, false, PRE>::bytes, NWS + NLS, (T*)nullptr)) {
+                                  StateSmem<T, DK, NWS, STAGES, false, PRE>::bytes, state_waves<T>(NWS, NLS, false), (T*)nullptr)) {
     return e;
   }
   if (fill_only) return (int)hipGetLastError();

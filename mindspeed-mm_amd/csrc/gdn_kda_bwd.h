@@ -881,7 +881,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
       auto kern = chunk_state_bwd_kernel<T, DK, 2, NLS, STAGES, true, true>;
       constexpr int smem = StateBwdSmem<T, DK, 2, STAGES, true>::bytes;
       if (int e = set_lds_b(kern, smem)) return e;
-      GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st, K2F, K1F,
+      GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * state_bwd_waves<T>(2, NLS)), smem, st, K2F, K1F,
                  QBT, Ai, AQ, (const T*)dO, dec, bhat, (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr,
                  cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
       GDN_LAUNCH(kKernStateBwd, st, (segment_chain_kernel<DK, true>), dim3(d.N * H, d.V / 16), dim3(4 * DK), 0, st,
@@ -893,7 +893,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     auto kern = chunk_state_bwd_kernel<T, DK, NWS, NLS, STAGES, true>;
     constexpr int smem = StateBwdSmem<T, DK, NWS, STAGES, true>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
-    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, K2F, K1F, QBT,
+    GDN_LAUNCH(kKernStateBwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * state_bwd_waves<T>(NWS, NLS)), smem, st, K2F, K1F, QBT,
                Ai, AQ, (const T*)dO, dec, bhat, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
   }
   {
@@ -960,7 +960,7 @@ extern "C" int gdn_kda_bwd(const void* q, const void* k, const void* v, const vo
       if (one_slab) GDN_KDAB(bf16_t, 128, 1, 4, 2);
       GDN_KDAB(bf16_t, 128, 2, 4, 2);
     }
-    GDN_KDAB(bf16_t, 64, 2, 2, 2);
+    GDN_KDAB(bf16_t, 64, 2, 4, 2);
   } else {
     if (K == 128) GDN_KDAB(float, 128, 2, 2, 1);
     GDN_KDAB(float, 64, 2, 2, 1);

@@ -491,7 +491,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
       auto kern = chunk_state_kernel<T, DK, 2, NLS, STAGES, false, true, true, true>;
       constexpr int smem = StateSmem<T, DK, 2, STAGES, false, true, true>::bytes;
       if (int e = set_lds(kern, smem)) return e;
-      GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * (2 + NLS)), smem, st,
+      GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * (segs - 1) * H, (d.V + DK) / 64), dim3(64 * state_waves<T>(2, NLS, false)), smem, st,
                  (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const float*)bhat,
                  (const float*)nullptr, maps, (T*)nullptr, (T*)nullptr, (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H,
                  d.V, scale, (int64_t)H * d.V, (const T*)nullptr, segs);
@@ -505,7 +505,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     constexpr int smem = StateSmem<T, DK, NWS, STAGES, true, true, true>::bytes;
     if (int e = set_lds(kern, smem)) return e;
     // the per-chunk states and v_new leave the kernel only for a backward pass
-    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * (NWS * (1 + StateOutWaves<NWS>::value) + NLS)),
+    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * segs * H, d.V / (32 * NWS)), dim3(64 * state_waves<T>(NWS, NLS, true)),
                smem, st, (const T*)K1F, (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec,
                (const float*)bhat, h0, ht, with_backward ? VF : (T*)nullptr, with_backward ? HF : (T*)nullptr, (T*)o, cu,
                (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)QBT, segs);
@@ -515,7 +515,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     auto kern = chunk_state_kernel<T, DK, NWS, NLS, STAGES, false, true, true>;
     constexpr int smem = StateSmem<T, DK, NWS, STAGES, false, true, true>::bytes;
     if (int e = set_lds(kern, smem)) return e;
-    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * (NWS + NLS)), smem, st, (const T*)K1F,
+    GDN_LAUNCH(kKernStateFwd, st, kern, dim3(d.N * H, d.V / (32 * NWS)), dim3(64 * state_waves<T>(NWS, NLS, false)), smem, st, (const T*)K1F,
                (const T*)K2F, (const T*)Ai, (const T*)AQ, (const T*)v, (const float*)dec, (const float*)bhat, h0, ht, VF, HF,
                (T*)nullptr, cu, (const int*)chunk_offsets, d.T, H, H, d.V, scale, (int64_t)H * d.V, (const T*)nullptr, 1);
   }
