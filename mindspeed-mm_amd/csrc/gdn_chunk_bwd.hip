@@ -15,6 +15,7 @@
 // The equations are those of the reference's backward kernels (mindspeed_mm/fsdp/ops/gdn/triton/
 // chunk_o.py:19-284, chunk_delta_h.py:307-513, wy_fast.py:17-141, chunk_gated_delta_rule.py:88-174), with
 // the dG row/column sums rewritten as row dot products with dQ/dK so that Q K^T need not be rebuilt.
+#include "gdn_bwd_local16.h"
 #include "gdn_chunk.h"
 #include "gdn_chunk_f32.h"
 #include "gdn_common.h"
@@ -1058,6 +1059,17 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
     TailRows tail{{dq, dk, dv, dg, dbeta}, {gs.dq * es, gs.dk * es, gs.dv * es, (int64_t)d.Hv * 4, (int64_t)d.Hv * bb},
                   {d.Hqk * DK * es, d.Hqk * DK * es, d.Hv * d.V * es, d.Hv * 4, d.Hv * bb}};
     launch_zero_tail_rows(cu, d.N, d.tokens(), tail, st);
+    if constexpr (std::is_same<T, bf16_t>::value) {
+      if (d.V >= 128 || d.Hv == d.Hqk) {   // the sums over a group's heads need the place of a head's state gradients
+        auto kern = chunk_bwd_local16_kernel<DK>;
+        constexpr int smem = BwdLocal16Smem<DK>::bytes;
+        if (int e = set_lds_b(kern, smem)) return e;
+        GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, d.Hqk), dim3(512), smem, st, (const T*)QTF, (const T*)KAF, (const T*)v, Bt,
+                   beta_same, G, Ai, VF, (const T*)DVF, (const T*)dO, HF, DHF, rstd_q, rstd_k, (T*)dq, (T*)dk, (T*)dv, dbeta, dg, cu,
+                   chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, d.strides());
+        return (int)hipGetLastError();
+      }
+    }
     auto kern = chunk_bwd_local_kernel<T, DK>;
     constexpr int smem = BwdLocalSmem<T, DK>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;

@@ -105,6 +105,7 @@ __device__ __forceinline__ int xcd_grouped_head(int b, int total, int grp) {
 // behind the load and make the wave wait for it there, before the loads that follow have been issued.
 #ifndef GDN_KEEP_HERE
 #define GDN_KEEP_HERE(x) asm volatile("" : "+v"(x))
+#define GDN_KEEP_HERE_UNIFORM(x) asm volatile("" : "+s"(x))   // a wave-uniform value, in a scalar register
 #endif
 // The workgroups of a launch start together and, doing equal work, stay in step: they all load at the same time and
 // all compute at the same time, and the two workgroups that share a CU do not fill each other's waits.  Holding back
@@ -145,6 +146,11 @@ template <int UNITS> __device__ __forceinline__ void stagger_second_resident(int
 template <typename T> __device__ __forceinline__ void load16_to_lds(const T* src, T* lds_wave_base) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                    (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
+}
+// the same for data that is read once: it passes through the L2 without displacing what will be read again
+template <typename T> __device__ __forceinline__ void load16_to_lds_stream(const T* src, T* lds_wave_base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 2);   // nt
 }
 // beta (and its gradient) as the caller holds it: fp32, or, with `same` set, the 16-bit type T of q, k, v.  The value
 // is fetched raw and converted later, so that a loader can issue the fetch without waiting for it.
@@ -291,6 +297,44 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const void* p) {
   const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
   return __builtin_bit_cast(u32x2, v);
 }
+
+// 2 N of them at once, N operands of two halves each, waited for.  For kernels with direct global -> LDS copies in flight: behind
+// such a copy the compiler puts a wait for all of them in front of the builtin (it does not know that they go elsewhere).
+#ifndef GDN_LDS_READ_TR16
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+template <int N, typename T> __device__ __forceinline__ void lds_read_tr16_pairs(const T* const* p, u32x4* out) {
+  static_assert(N == 1 || N == 2 || N == 4, "asm blocks of 2, 4 and 8 reads");
+  u32x2 r[2 * N];
+  uint32_t a[2 * N];
+#pragma unroll
+  for (int i = 0; i < 2 * N; ++i) a[i] = lds_address(p[i]);
+  if constexpr (N == 1) {
+    asm volatile("ds_read_b64_tr_b16 %0, %2\n ds_read_b64_tr_b16 %1, %3\n s_waitcnt lgkmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]) : "v"(a[0]), "v"(a[1]) : "memory");
+  } else if constexpr (N == 2) {
+    asm volatile("ds_read_b64_tr_b16 %0, %4\n ds_read_b64_tr_b16 %1, %5\n ds_read_b64_tr_b16 %2, %6\n"
+                 " ds_read_b64_tr_b16 %3, %7\n s_waitcnt lgkmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]) : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]) : "memory");
+  } else {
+    asm volatile("ds_read_b64_tr_b16 %0, %8\n ds_read_b64_tr_b16 %1, %9\n ds_read_b64_tr_b16 %2, %10\n"
+                 " ds_read_b64_tr_b16 %3, %11\n ds_read_b64_tr_b16 %4, %12\n ds_read_b64_tr_b16 %5, %13\n"
+                 " ds_read_b64_tr_b16 %6, %14\n ds_read_b64_tr_b16 %7, %15\n s_waitcnt lgkmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+                 : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]) : "memory");
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = u32x4{r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]};
+}
+#else
+template <int N, typename T> inline void lds_read_tr16_pairs(const T* const* p, u32x4* out) {
+  for (int i = 0; i < N; ++i) {
+    const u32x2 x = lds_read_tr16(p[2 * i]), y = lds_read_tr16(p[2 * i + 1]);
+    out[i] = u32x4{x[0], x[1], y[0], y[1]};
+  }
+}
+#endif
 
 // contiguous: p points at element [row][k0]; the lane reads kVec consecutive k
 template <typename T> __device__ __forceinline__ u32x4 frag_contig(const T* p) {

@@ -283,11 +283,13 @@ inline float __builtin_amdgcn_div_fixupf(float quotient, float d, float n) {
 #define __builtin_amdgcn_logf(x) log2f(x)
 #define GDN_WAVES_PER_SIMD(n)
 #define GDN_KEEP_HERE(x) ((void)0)
+#define GDN_KEEP_HERE_UNIFORM(x) ((void)(x))
 #define __builtin_amdgcn_sched_group_barrier(m, n, s) ((void)0)
 #define __builtin_amdgcn_wave_barrier() emu::wave_sync()
 #define __builtin_amdgcn_s_sleep(x) emu::yield()
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)
+#define GDN_LDS_READ_TR16   // one by one, by the stand-in for the builtin
 #define __builtin_amdgcn_ds_read_tr16_b64_v4i16(p) emu::ds_read_tr16((const void*)(uintptr_t)(p))
 // direct global -> LDS load: lane l's `size` bytes land at dst + l*size (done at once: the emulator has no asynchrony)
 #define __builtin_amdgcn_global_load_lds(src, dst, size, off, aux) \

@@ -113,6 +113,18 @@ def test_chunk_backward_recompute_mode_equals_stored_mode(ops, dtype, B, T, Hqk,
     P.check_chunk_recompute_equals_stored(ops, "cpu", B, T, Hqk, Hv, K, V, dtype, cu=cu, wrap=guarded, h0_std=0.1)
 
 
+@pytest.mark.parametrize("T,Hqk,Hv,K,V,l2", [
+    (70, 1, 3, 64, 128, True),     # three heads to a group, half of the waves without columns of K of their own
+    (65, 1, 2, 128, 192, True),    # R in two parts, the second of two V blocks; a last chunk of one token
+    (64, 1, 1, 128, 64, False),    # one pair of V blocks; no l2 norm
+    (33, 1, 2, 64, 64, True),      # several heads and V = 64: the four-wave kernel
+    (130, 2, 2, 64, 256, False),
+])
+def test_chunk_local_backward_of_head_groups(ops, T, Hqk, Hv, K, V, l2):
+    """The chunk-local kernel where its tiles, its V blocks and the sums over a group's heads end."""
+    P.check_chunk(ops, "cpu", 1, T, Hqk, Hv, K, V, BF, l2=l2, backward=True, wrap=guarded, h0_std=0.1, seed=5)
+
+
 def test_chunk_backward_without_initial_state(ops):
     P.check_chunk(ops, "cpu", 1, 70, 1, 1, 64, 64, F32, backward=True, with_h0=False, wrap=guarded)
 
