@@ -1,4 +1,4 @@
-// chunk_bwd_local16_kernel: what chunk_bwd_local_kernel does, for 16-bit types and scalar gates.
+// chunk_bwd_local16_kernel: what chunk_bwd_local_kernel does, for 16-bit types; with KDA its main loop alone.
 //
 // With z = beta (v - e^G . K S), V' = (I + L)^-1 z and R = Tm^T dV' = dz (Tm = (I + L)^-1), the gradient of L is
 // -strict_tril(R V'^T), that of a triangular solve's matrix; no product with Tm is needed beyond R:
@@ -133,14 +133,17 @@ template <int DK> struct BwdLocal16Smem {
   static_assert(bytes <= 80 * 1024, "two workgroups to a CU");
 };
 
-template <int DK>
+// KDA: the kernel ends after its main loop and leaves the sums over V for kda_bwd_finish_kernel (KdaDump); G is not read, bt is
+// the transformed beta and there is one value head to a group.  2 x 8192 tokens of 32 heads: 299 us, the four-wave kernel 368.
+template <int DK, bool KDA = false>
 __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_kernel(
     const bf16_t* __restrict__ qtf, const bf16_t* __restrict__ kaf, const bf16_t* __restrict__ v, const float* __restrict__ bt,
     int beta_same, const float* __restrict__ G, const bf16_t* __restrict__ Ai, const bf16_t* __restrict__ vf,
     const bf16_t* __restrict__ dvf, const bf16_t* __restrict__ dO, const bf16_t* __restrict__ hf, bf16_t* dhf,
     const float* __restrict__ rstd_q, const float* __restrict__ rstd_k, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk,
     bf16_t* __restrict__ dv_out, void* __restrict__ dbeta, float* __restrict__ dg, const int64_t* __restrict__ cu,
-    const int* __restrict__ chunk_offsets, int T_len, int N, int Hqk, int Hv, int V, float scale, TokenStrides ts) {
+    const int* __restrict__ chunk_offsets, int T_len, int N, int Hqk, int Hv, int V, float scale, TokenStrides ts,
+    bf16_t* __restrict__ kda_dump, float* __restrict__ kda_dd) {
   using namespace bl16;
   using T = bf16_t;
   using SM = BwdLocal16Smem<DK>;
@@ -235,11 +238,14 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
     L = Lane::here();
     if (L.w == 0) {
       const int tc = imin(L.id, nvalid - 1);
-      const float gv = G[ch * 64 + tc], gl = G[ch * 64 + nvalid - 1], bv = bt[ch * 64 + L.id];   // beta: 0 past the end
-      Gs[L.id] = gv;
-      egs[L.id] = __expf(gv);
-      sgs[L.id] = scale * __expf(gv);
-      egl[L.id] = __expf(gl - gv);
+      const float bv = bt[ch * 64 + L.id];   // beta: 0 past the end
+      if constexpr (!KDA) {
+        const float gv = G[ch * 64 + tc], gl = G[ch * 64 + nvalid - 1];
+        Gs[L.id] = gv;
+        egs[L.id] = __expf(gv);
+        sgs[L.id] = scale * __expf(gv);
+        egl[L.id] = __expf(gl - gv);
+      }
       bs[L.id] = bv;
     }
 
@@ -314,7 +320,7 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
         issue_priv(ch, vblk + 1);
         if ((vblk & 1) == 0 && vblk + 2 < nblk) issue_raw(h, (vblk >> 1) + 1);   // its buffer was last read in block vblk - 1
         if ((vblk & 3) == 3) issue_dv(ch, vblk + 1);                             // read at the head of these four blocks
-      } else {
+      } else if constexpr (!KDA) {
         issue_k();
         issue_q();
       }
@@ -353,6 +359,40 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
       if (L.tiles() == 2) own(1, L.ti(1), L.tj(1));
     }
     L = Lane::here();
+    if constexpr (KDA) {
+      using KD = KdaDump<DK>;
+      T* const dump = kda_dump + ch * KD::elems;
+      if (L.w < DK / 16) {
+        // two accumulator tiles of 16 tokens are the piece of a 32x32 tile in fragment order that the lane and the one 32
+        // lanes on hold half of each: they trade, and each lane writes 16 bytes
+        auto sums_out = [&](const f32x4* acc, T* out) {
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            const u32x2 lo = pack1(acc[2 * b]), hi = pack1(acc[2 * b + 1]);
+            const auto x = __builtin_amdgcn_permlane32_swap(lo[0], hi[0], false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(lo[1], hi[1], false, false);
+            __builtin_nontemporal_store(u32x4{x[0], y[0], x[1], y[1]},
+                                        reinterpret_cast<u32x4*>(out + (b * NKT + (L.w >> 1)) * 1024 +
+                                                                 frag_slot<T>(L.g >> 1, 16 * (L.w & 1) + L.n + 32 * (L.g & 1)) * 8));
+          }
+        };
+        sums_out(dQ, dump + KD::dq);
+        sums_out(dK, dump + KD::dk2);
+        sums_out(P, dump + KD::dk1);
+        sds += __shfl_xor(sds, 16);
+        sds += __shfl_xor(sds, 32);
+        if (L.g == 0) kda_dd[ch * DK + 16 * L.w + L.n] = sds;
+      }
+      auto tile_out = [&](int x, int ti, int tj) {   // a quarter of a 32x32 tile; nobody reads what lies above the diagonal
+        const int at = (2 * (ti >> 1) + (tj >> 1)) * 1024 + frag_slot<T>(ti & 1, 16 * (tj & 1) + L.n + 32 * (L.g & 1)) * 8 + 4 * (L.g >> 1);
+        *reinterpret_cast<u32x2*>(dump + KD::ds + at) = pack1(ds[x]);
+        *reinterpret_cast<u32x2*>(dump + KD::rv + at) = pack1(rvn[x]);
+      };
+      tile_out(0, L.ti(0), L.tj(0));
+      if (L.tiles() == 2) tile_out(1, L.ti(1), L.tj(1));
+      if (L.w == 0) reinterpret_cast<float*>(dump + KD::dots)[L.id] = rv[L.id] + rv[64 + L.id];
+      return;
+    }
     sds = wave_sum(sds);
     if (L.id == 0) wsum[L.w] = sds;
     const Mat64 MS{base + SM::raw}, MD{base + SM::raw + 4096}, MB{base + SM::vn};   // ds^T, dM^T, (beta dM)^T

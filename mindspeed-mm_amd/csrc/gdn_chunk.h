@@ -127,15 +127,24 @@ struct KdaWorkspace {
   int64_t SEGH, SEGM;     // as in ChunkWorkspace; the reverse recurrence puts its own there
   int64_t fwd_bytes;
   // kept for a backward pass
-  int64_t TMR;            // T [chunks,H,64,64]     Tm row-major, as rounded for the tiles
+  int64_t TMR;            // fp32 only: [chunks,H,64,64] Tm row-major
   int64_t DVF;            // T [chunks,H,V/32,2]    d(v_new)
   int64_t DHF;            // T [chunks,H,V/32,K/32] gradient of the state AFTER each chunk
-  int64_t DUMP;           // T [chunks,H][dQb | dK2 | P : 64,K each][dAq | a2 : 64,64 each]  sums over V of the chunk-local pass;
-                          //   P as rows, the others as 32x32 tiles in fragment order: (token block, channel block), (row block, column block)
+  int64_t DUMP;           // T [chunks,H][dump_elems] sums over V of the chunk-local pass (KdaDump)
   int64_t DD;             // f32 [chunks,H,K]       sum over V of dS' . S: the gradient of the chunk's decay per channel
   int64_t PART;           // f32 [chunks,H][1 + K]  partial sums of dA_log and d(dt_bias)
   int64_t total_bytes;
   static int64_t dump_elems(int K) { return 3 * 64 * (int64_t)K + 2 * 64 * 64; }
+};
+
+// What the chunk-local pass of KDA leaves per chunk and head, rounded to T like every other tensor that passes between two
+// kernels (they are the largest of them), as 32x32 tiles in fragment order, (token block, channel block) resp. (row block,
+// column block): dQb = dO S^T, dK2 = V' dS'^T [64,K] each, dAq = dO V'^T [64,64], and
+//   16-bit types: with R = Tm^T dV', dK1 = R S^T and R V'^T; in the place of the latter's tile above the diagonal, which
+//   nobody needs, <R_i, v_i> of the 64 tokens in fp32;
+//   fp32: P = dV' S^T, as rows, and a2 = dV' V^T.
+template <int DK> struct KdaDump {
+  static constexpr int dq = 0, dk2 = 64 * DK, dk1 = 2 * 64 * DK, ds = 3 * 64 * DK, rv = ds + 64 * 64, dots = rv + 1024, elems = rv + 64 * 64;
 };
 
 inline KdaWorkspace kda_workspace_layout(const ChunkDims& d, int elem_bytes) {
@@ -159,7 +168,7 @@ inline KdaWorkspace kda_workspace_layout(const ChunkDims& d, int elem_bytes) {
   w.SEGH = take(seg * P * d.V);
   w.SEGM = take(seg * (P - 1) * (d.V + d.K));
   w.fwd_bytes = off;
-  w.TMR = take(nc * H * 64 * 64 * elem_bytes);
+  w.TMR = take(elem_bytes == 4 ? nc * H * 64 * 64 * 4 : 0);
   w.DVF = take(nc * 64 * H * d.V * elem_bytes);
   w.DHF = take(nc * H * d.V * d.K * elem_bytes);
   w.DUMP = take(nc * H * KdaWorkspace::dump_elems(d.K) * elem_bytes);

@@ -410,11 +410,8 @@ template <typename T, int DK> struct BwdLocalSmem {
   static_assert(4 * Patch<T>::kElems <= raw_elems && 2 * (DK / 32) * 1024 <= raw_elems, "epilogue tenants fit");
 };
 
-// KDA (one decay per key channel): the sums over V are the same, what follows them is not.  The kernel then stops after
-// its main loop (dv is written there) and leaves the sums in kda_dump, per chunk and head
-//   [dQb = dO S^T | dK2 = V' dS'^T | P = dV' S^T : 64 x DK each][dAq = dO V'^T | a2 = dV' V^T : 64 x 64 each, lower tiles]
-// rounded to T like every other tensor that passes between two kernels (they are the largest of them: in fp32 they made
-// up half of what the backward pass moved), and dD = sum_v dS' . S [DK] in kda_dd, in fp32,
+// KDA (one decay per key channel, fp32): the sums over V are the same, what follows them is not.  The kernel then stops after
+// its main loop (dv is written there) and leaves the sums in kda_dump (KdaDump), and dD = sum_v dS' . S [DK] in kda_dd,
 // for kda_bwd_finish_kernel; G is not read and bt is the transformed beta.  beta_same: the type dbeta leaves in.
 template <typename T, int DK, bool KDA = false>
 __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_local_kernel(
@@ -425,6 +422,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     float* __restrict__ dg, const int64_t* __restrict__ cu, const int* __restrict__ chunk_offsets, int T_len, int N,
     int Hqk, int Hv, int V, float scale, int hh, TokenStrides ts, T* __restrict__ kda_dump, float* __restrict__ kda_dd,
     int cus) {
+  static_assert(!KDA || sizeof(T) == 4, "16-bit KDA: chunk_bwd_local16_kernel");
   using SM = BwdLocalSmem<T, DK>;
   constexpr int NKT = DK / 32, VEC = Elem<T>::kVec, KG = AccK<T>::kGroups;
   static_assert(NKT <= 4, "one 32-column block of K per wave");
@@ -651,8 +649,8 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     }
   }
   if constexpr (KDA) {
-    constexpr int64_t kDumpElems = 3 * 64 * DK + 2 * 64 * 64;
-    T* dump = kda_dump + ch * kDumpElems;
+    using KD = KdaDump<DK>;
+    T* dump = kda_dump + ch * KD::elems;
     GDN_WAIT_VMEM();
     GDN_LDS_BARRIER();   // the last block's stage is consumed: its place takes the store patches
     T* patch = stage0 + SM::sh + wave * Patch<T>::kElems;
@@ -664,10 +662,10 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
       for (int ri = 0; ri < 2; ++ri) {
         AccB<T> f;
         f.pack(dQi[ri]);
-        f.store_stream(dump + (ri * NKT + cj) * 1024);
+        f.store_stream(dump + KD::dq + (ri * NKT + cj) * 1024);
         f.pack(dKi[ri]);
-        f.store_stream(dump + 64 * DK + (ri * NKT + cj) * 1024);
-        acc_store_rows<T, false>(dWa[ri], id, patch, dump + 2 * 64 * DK + 32 * ri * DK + 32 * cj, DK, 32);
+        f.store_stream(dump + KD::dk2 + (ri * NKT + cj) * 1024);
+        acc_store_rows<T, false>(dWa[ri], id, patch, dump + KD::dk1 + 32 * ri * DK + 32 * cj, DK, 32);
       }
       sds += __shfl_xor(sds, 32);   // the other half of the V block's rows
       if (lane < 32) kda_dd[ch * DK + 32 * cj + lane] = sds;
@@ -675,9 +673,9 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     if (lower) {
       AccB<T> f;
       f.pack(ds);
-      f.store_stream(dump + 3 * 64 * DK + (2 * ti + tj) * 1024);
+      f.store_stream(dump + KD::ds + (2 * ti + tj) * 1024);
       f.pack(a2);
-      f.store_stream(dump + 3 * 64 * DK + 64 * 64 + (2 * ti + tj) * 1024);
+      f.store_stream(dump + KD::rv + (2 * ti + tj) * 1024);
     }
     return;
   }
@@ -1066,7 +1064,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         if (int e = set_lds_b(kern, smem)) return e;
         GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, d.Hqk), dim3(512), smem, st, (const T*)QTF, (const T*)KAF, (const T*)v, Bt,
                    beta_same, G, Ai, VF, (const T*)DVF, (const T*)dO, HF, DHF, rstd_q, rstd_k, (T*)dq, (T*)dk, (T*)dv, dbeta, dg, cu,
-                   chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, d.strides());
+                   chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, d.strides(), (T*)nullptr, (float*)nullptr);
         return (int)hipGetLastError();
       }
     }

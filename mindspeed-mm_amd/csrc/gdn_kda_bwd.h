@@ -1,6 +1,6 @@
 // KDA (Kimi delta attention) backward.  Included at the end of gdn_chunk_bwd.hip: the reverse recurrence and the sums
-// over V of the chunk-local pass are that file's kernels in their KDA modes (chunk_state_bwd_kernel,
-// chunk_bwd_local_kernel, which also writes dv); this file turns those sums into the gradients of q, k, the gate input
+// over V of the chunk-local pass are that file's kernels in their KDA modes (chunk_state_bwd_kernel; chunk_bwd_local16_kernel
+// or, for fp32, chunk_bwd_local_kernel, which also write dv); this file turns those sums into the gradients of q, k, the gate input
 // and beta, which is where the decay per key channel changes the algebra.  The reference differentiates its pure
 // PyTorch statement with autograd (mindspeed_mm/fsdp/ops/kda/chunk_kda_naive.py:106-221); the equations below are the
 // hand-derived backward of that statement.
@@ -9,9 +9,13 @@
 //   Kp = k . e^{G}   K1 = -b Kp   K2 = k . e^{G_last-G}   Qb = scale q . e^{G}
 //   L_ij = b_i sum_d k_id k_jd e^{G_id-G_jd} (i>j)   Tm = (I+L)^-1   Aq_ij = scale sum_d q_id k_jd e^{G_id-G_jd} (i>=j)
 //   z = b v + K1 S    V' = Tm z    O = Qb S + Aq V'    S' = e^{G_last} . S + K2^T V'
-// What arrives (sums over V, rounded to T; dD in fp32): dQb = dO S^T, dK2 = V' dS'^T, P = dV' S^T, dAq = tril(dO V'^T), a2 = dV' V^T,
-// dD = sum_v dS' . S.  Then
-//   dTm = stril(b_j (a2 - P Kp^T))    dL = -stril(Tm^T dTm Tm^T)    dK1 = Tm^T P    <R_t, v_t> = sum_i Tm_it a2_it
+// What arrives (sums over V, rounded to T; dD and <R_t,v_t> in fp32): dQb = dO S^T, dK2 = V' dS'^T, dAq = tril(dO V'^T),
+// dD = sum_v dS' . S, and with R = Tm^T dV' = dz
+//   16-bit types: dK1 = R S^T, R V'^T, <R_t, v_t>.  dL = -stril(R V'^T), the gradient of a triangular solve's matrix;
+//   fp32: P = dV' S^T, a2 = dV' V^T.  dTm = stril(b_j (a2 - P Kp^T))    dL = -stril(Tm^T dTm Tm^T)    dK1 = Tm^T P
+//         <R_t, v_t> = sum_i Tm_it a2_it, the reference's way (the other one rounds less in 16 bits and saves four phases, but
+//         in fp32, where every pair's decay weighs more than they do, it left dg 1 % less exact).
+// Then
 //   U_i  = sum_{j<i}  dL_ij        k_j . e^{G_i-G_j}          Uq_i = sum_{j<=i} scale dAq_ij k_j . e^{G_i-G_j}
 //   W_j  = sum_{i>=j} (dL_ij b_i k_i + scale dAq_ij q_i) . e^{G_i-G_j}
 //   dq^ = scale e^{G} . dQb + Uq
@@ -28,8 +32,6 @@
 // scaled by their own factor.  The levels of 2 and 4 tokens stay inside a lane: a lane has one key channel and, per
 // accumulator group, four consecutive tokens, which are one block of 4.  (For fp32 operands every pair is summed term
 // by term in fp32 instead.)
-// What the chunk-local kernel leaves (the workspace's DUMP): P as rows, dQb, dK2, dAq and a2 as 32x32 tiles in
-// fragment order, which is how both kernels hold them in registers.
 #pragma once
 #include "gdn_kda_common.h"
 
@@ -40,33 +42,30 @@ template <typename T, int DK> struct KdaBwdSmem {
   static constexpr bool FULL = sizeof(T) == 4;   // no rescaled images: every pair term by term
   static constexpr int tile = 64 * LDK * (int)sizeof(T), gmat = 64 * LDG * 4, mat = 64 * L64 * (int)sizeof(T);
   static constexpr int off_ks = 0;                   // k^ rows
-  static constexpr int off_qs = off_ks + tile;       // P as T; FULL: then q^ rows
-  static constexpr int off_gs = off_qs + tile;       // first Kp as T (64 rows), then G rows (fp32)
-  static constexpr int off_m1 = off_gs + gmat;       // dTm, then dL; later, with the next one, the store patches
-  static constexpr int off_m2 = off_m1 + mat;        // X = Tm^T dTm, then scale dAq
-  static constexpr int off_tm = off_m2 + mat;        // Tm row-major
-  static constexpr int off_m2t = off_tm + mat;       // scale dAq transposed (not FULL)
-  // not FULL: q^ rows and dL transposed get places of their own, so that P and Tm live until dK1 = Tm^T P is formed
-  // where it is used, after the decay-weighted sums, instead of occupying registers through them
-  static constexpr int off_q2 = off_m2t + (FULL ? 0 : mat);
-  static constexpr int off_m1t = off_q2 + (FULL ? 0 : tile);
-  // not FULL: which entries of a coefficient fragment belong to a level's pairs: [5 levels][2 halves of the 32 columns]
-  // [row = earlier | later token][64 lanes] masks of 16 bytes (only the levels of 8, 16 and 32 tokens are filled and
-  // used).  They depend on nothing but the lane.
-  static constexpr int off_keep = off_m1t + (FULL ? 0 : mat);
-  static constexpr int off_row = off_keep + (FULL ? 0 : 5 * 2 * 2 * 64 * 16);
+  static constexpr int off_qs = off_ks + tile;       // q^ rows; FULL: first P
+  static constexpr int off_gs = off_qs + tile;       // G rows (fp32); FULL: for a while Kp as T (64 rows)
+  static constexpr int off_m1 = off_gs + gmat;       // dL (FULL: first dTm); at the end, with the next ones, the store patches
+  static constexpr int off_m2 = off_m1 + mat;        // scale dAq (FULL: first X = Tm^T dTm)
+  static constexpr int off_m1t = off_m2 + mat;       // b dL transposed; FULL: Tm row-major
+  static constexpr int off_m2t = off_m1t + (FULL ? 0 : mat);   // scale dAq transposed (not FULL)
+  // not FULL: which entries of a coefficient fragment belong to a level's pairs: [levels of 8, 16, 32 tokens][2 halves of the
+  // 32 columns][row = earlier | later token][64 lanes] masks of 16 bytes.  They depend on nothing but the lane.
+  static constexpr int off_keep = off_m2t + mat;
+  static constexpr int off_row = off_keep + (FULL ? 0 : 3 * 2 * 2 * 64 * 16);
   // beta, 1/|q|, 1/|k| [64 each]; row sums <q^,dq^>, <k^,dk^>, db, <R,v> [256 each]; per-wave scalars [8]; what the
   // two waves of a channel block exchange: parts of dG_last and d(dt_bias) [8][32 each], sum of dG over tokens 32.. [4][32]
   // ... and the diagonal of scale dAq [64]
   static constexpr int bytes = off_row + (3 * 64 + 4 * 256 + 8 + 2 * 256 + 128 + 64) * 4;
-  static_assert(tile <= gmat, "Kp fits where G will be");
-  static_assert(8 * Patch<T>::kElems * (int)sizeof(T) <= 3 * mat, "store patches fit");
+  static_assert(tile <= gmat, "Kp fits where G is");
+  static_assert(8 * Patch<T>::kElems * (int)sizeof(T) <= off_keep - off_m1, "store patches fit");
   static_assert(bytes <= 160 * 1024, "one CU's LDS");
 };
 
 // Eight waves, two per SIMD: the kernel is a chain of short dependent steps (LDS reads, exponentials, small matrix
-// products), and a second wave on the SIMD fills the waits of the first.  Waves 0..3 each own a 32x32 tile of the 64x64
-// matrices of phases A1..A4; in phase B wave w owns key channels 32 (w >> 1).. and tokens 32 (w & 1).. of the chunk.
+// products), and a second wave on the SIMD fills the waits of the first.  Waves 0..3 each bring a 32x32 tile of the 64x64
+// matrices into place; in phase B wave w owns key channels 32 (w >> 1).. and tokens 32 (w & 1).. of the chunk.
+// With the 64x64 chain dTm -> Tm^T dTm Tm^T and the product Tm^T P in front of phase B (four more barriers, P and Tm through LDS)
+// 2 x 8192 tokens of 32 heads took 641 us, without them 573; still bound by the steps of phase B, one workgroup to a CU.
 constexpr int kFinThreads = 512;
 
 // rowacc[i0 + i] += sum_j x[i][j] for the 32 rows of an accumulator tile (see rows_add; the caller picks the slot)
@@ -88,11 +87,9 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
   constexpr int LDK = SM::LDK, LDG = SM::LDG, L64 = SM::L64, VEC = Elem<T>::kVec, CPR = DK / VEC, NKT = DK / 32;
   constexpr bool FULL = SM::FULL;
   T* Ks = reinterpret_cast<T*>(gdn_smem + SM::off_ks);
-  T* Pt = reinterpret_cast<T*>(gdn_smem + SM::off_qs);
-  T* Qs = FULL ? Pt : reinterpret_cast<T*>(gdn_smem + SM::off_q2);
+  T* Qs = reinterpret_cast<T*>(gdn_smem + SM::off_qs);
   float* Gs = reinterpret_cast<float*>(gdn_smem + SM::off_gs);
-  T* Kp = reinterpret_cast<T*>(gdn_smem + SM::off_gs);
-  T* TmT = reinterpret_cast<T*>(gdn_smem + SM::off_tm);
+  T* Pt = Qs, *Kp = reinterpret_cast<T*>(Gs), *TmT = reinterpret_cast<T*>(gdn_smem + SM::off_m1t);   // FULL
   T* M1 = reinterpret_cast<T*>(gdn_smem + SM::off_m1);
   T* M2 = reinterpret_cast<T*>(gdn_smem + SM::off_m2);
   T* M1t = reinterpret_cast<T*>(gdn_smem + SM::off_m1t);
@@ -103,7 +100,7 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
   float* rq = rsk + 64;     // row sums, a slot of 64 rows per block of 32 key channels (rows_add_at / rows_ld4)
   float* rk = rq + 256;
   float* rb = rk + 256;
-  float* rv = rb + 256;     // <R_t, v_t>, a slot per tile wave
+  float* rv = rb + 256;     // <R_t, v_t>; FULL: a slot per tile wave
   float* wsum = rv + 256;   // [8]   per wave: its part of dA_log
   float* xgl = wsum + 8;    // [8][32] per wave and channel: its part of dG_last
   float* xdt = xgl + 256;   // [8][32] per wave and channel: its part of d(dt_bias)
@@ -121,13 +118,13 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
   const bool tile_wave = wave < 4, lower = tile_wave && tj <= ti;
   const int cj = wave >> 1, ri = wave & 1;
   const bool has_k = cj < NKT;
-  const T* dump = dumps + ch * (3 * 64 * DK + 2 * 64 * 64);
-  const T* dQb = dump, *dK2 = dump + 64 * DK, *Pm = dump + 2 * 64 * DK;
-  const T* dAq = dump + 3 * 64 * DK, *a2m = dAq + 64 * 64;
+  using KD = KdaDump<DK>;
+  const T* dump = dumps + ch * KD::elems;
+  const T* dQb = dump + KD::dq, *dK2 = dump + KD::dk2, *dK1m = dump + KD::dk1;
+  const T* dAq = dump + KD::ds, *rvm = dump + KD::rv;
   const float* dD = dd + ch * DK;
 
-  // ---- phase A0: G from the gate input; k^ rows; P and Tm as operands; beta.  The tile waves request their tiles of
-  //      a2 and dAq now ----
+  // ---- phase A: G from the gate input; k^ and q^ rows; dL and scale dAq; beta ----
   // This thread's pieces of the 64 x DK operands: VEC consecutive channels of a row each.  The gate input goes first
   // (loads arrive in the order of their requests): the cumulative decay is rebuilt from it, with the forward pass's own
   // operations, while the other operands are on their way.  (As bits, one branch around the whole round of requests.)
@@ -170,7 +167,7 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
   TileQK<T, DK, kFinThreads> kt;   // moved by every thread
   TileQK<T, DK> qt;                // moved by kThreads threads, see below
   tile_qk_request<T, DK>(kt, k + tok0 * hk + h * DK, hk, nvalid, tid);
-  AccB<T> a2f, daf;
+  AccB<T> rvf, daf;
   u32x4* keepT = reinterpret_cast<u32x4*>(gdn_smem + SM::off_keep);
   if constexpr (!FULL) {
     // Which of 8 consecutive entries of a coefficient row belong to a level's pairs, as a mask over the fragment (two
@@ -180,8 +177,8 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
     // In terms of bits: i and j share the block and sit in different halves of it when (i ^ j) >> (lg - 1) == 1, and
     // the row's own half is bit lg - 1 of its index.  (Plain bit arithmetic: written with comparisons of the halves
     // the compiler turns every entry into a branch.)
-    for (int idx = 2 * 2 * 2 * 64 + tid; idx < 5 * 2 * 2 * 64; idx += kFinThreads) {   // levels of 8, 16, 32 tokens
-      const int ln = idx & 63, second = (idx >> 6) & 1, kg = (idx >> 7) & 1, sh = idx >> 8;   // sh = lg - 1
+    for (int idx = tid; idx < 3 * 2 * 2 * 64; idx += kFinThreads) {   // levels of 8, 16, 32 tokens
+      const int ln = idx & 63, second = (idx >> 6) & 1, kg = (idx >> 7) & 1, sh = 2 + (idx >> 8);   // sh = lg - 1
       const int a = ln & 31, b0 = 16 * kg + 8 * (ln >> 5);
       const uint32_t rok = ((a >> sh) & 1) == second ? 0xffffffffu : 0u;
       u32x4 w;
@@ -195,24 +192,23 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
       keepT[idx] = w;
     }
   }
-  // this thread's pieces of P and Tm, all requested before the first wait
-  f32x4 gk[NIT][VEC / 4];
-  Vec16<T> pf[NIT], tmv[NTM];
+  Vec16<T> pf[NIT], tmv[NTM];   // FULL: this thread's pieces of P and Tm
+  if constexpr (FULL) {
 #pragma unroll
-  for (int it = 0; it < NIT; ++it) {
-    const int c = tid + it * kFinThreads;
-    pf[it] = ld16(Pm + (c / CPR) * DK + (c % CPR) * VEC);
-  }
+    for (int it = 0; it < NIT; ++it) {
+      const int c = tid + it * kFinThreads;
+      pf[it] = ld16(dK1m + (c / CPR) * DK + (c % CPR) * VEC);
+    }
 #pragma unroll
-  for (int it = 0; it < NTM; ++it) {
-    const int c = tid + it * kFinThreads;
-    tmv[it] = ld16(TMR + ch * 4096 + (c / C64) * 64 + (c % C64) * VEC);
+    for (int it = 0; it < NTM; ++it) {
+      const int c = tid + it * kFinThreads;
+      tmv[it] = ld16(TMR + ch * 4096 + (c / C64) * 64 + (c % C64) * VEC);
+    }
   }
-  // beta: requested by every wave alike and with the early group (loads arrive in the order of their requests: the
-  // store of the row vectors below then waits for P and Tm, not for the requests made behind the gate)
+  // beta and <R, v>: requested by every wave alike and with the early group (loads arrive in the order of their requests)
   const float bh = bhat[ch * 64 + lane];   // 0 past the end
-  // G: the gate's log decay of every token and channel (0 on the rows past the end) into the place Kp will take,
-  // summed down the tokens there, and back into this thread's registers until Kp is consumed
+  const float rvl = FULL ? 0.f : reinterpret_cast<const float*>(dump + KD::dots)[lane];
+  // G: the gate's log decay of every token and channel (0 on the rows past the end), summed down the tokens
   {
     const float a = fl.use_gate ? __expf(A_log[h]) : 0.f;
     const float au = a * KdaDecay<T>::kUnit, lbu = fl.lower_bound * KdaDecay<T>::kUnit;
@@ -239,11 +235,9 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
     else gate_rows(IntConst<2>());
     GDN_LDS_BARRIER();
   }
-  // a2 and dAq arrive as tiles in fragment order: a tile wave takes its own.  These requests come behind the gate: none
-  // of them is needed before phase A1, and requested ahead of the gate their branches made every wave wait for all of
-  // its earlier requests first.
-  // q^ rows: in the 16-bit kernel they have a place of their own, and the waves that own no tile of the 64x64 phases
-  // normalise them during those phases.
+  // R V'^T and dAq arrive as tiles in fragment order: a tile wave takes its own.  These requests come behind the gate:
+  // requested ahead of it their branches made every wave wait for all of its earlier requests first.
+  // q^ rows: in the 16-bit kernel the waves that bring no tile of the 64x64 matrices normalise them meanwhile.
   // Every wave makes the same number of requests here (K = 128: four): the waits further down can then leave exactly
   // these in flight.  The wave of the tile above the diagonal, which nobody wrote, asks for tile (0,0) again (cached)
   // and drops it.
@@ -259,21 +253,21 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
     for (int i = 0; i < TileQK<T, DK>::PT; ++i) {
       const int c = t + i * kThreads, row = imin(c / CPR, nvalid - 1), cc = c % CPR;
       const T* qa = q + (tok0 + row) * hk + h * DK + cc * VEC;
-      const T* ta = (i < AccB<T>::kG ? a2m : dAq) + tile_at + frag_slot<T>(i % AccB<T>::kG, lane) * AccB<T>::kVecElems;
+      const T* ta = (i < AccB<T>::kG ? rvm : dAq) + tile_at + frag_slot<T>(i % AccB<T>::kG, lane) * AccB<T>::kVecElems;
       qt.x[i] = ld16(tile_wave ? ta : qa);
     }
 #pragma unroll
-    for (int g = 0; g < AccB<T>::kG; ++g) { a2f.f[g] = qt.x[g].raw; daf.f[g] = qt.x[AccB<T>::kG + g].raw; }
+    for (int g = 0; g < AccB<T>::kG; ++g) { rvf.f[g] = qt.x[g].raw; daf.f[g] = qt.x[AccB<T>::kG + g].raw; }
   } else if constexpr (Q_BY_OTHERS) {
     if (tile_wave) {
-      a2f.load(a2m + tile_at);
+      rvf.load(rvm + tile_at);
       daf.load(dAq + tile_at);
     } else {
       tile_qk_request<T, DK>(qt, q + tok0 * hk + h * DK, hk, nvalid, tid & (kThreads - 1));
     }
   } else {
     if (tile_wave) {
-      a2f.load(a2m + tile_at);
+      rvf.load(rvm + tile_at);
       daf.load(dAq + tile_at);
       tile_qk_request<T, DK>(qt, q + tok0 * hk + h * DK, hk, nvalid, tid & (kThreads - 1));
     }
@@ -289,9 +283,11 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
       const int c = tid + it * kFinThreads, row = c / CPR, cc = c % CPR, part = row / (64 / PARTS);
 #pragma unroll
       for (int e4 = 0; e4 < VEC / 4; ++e4) {
-        gk[it][e4] = *reinterpret_cast<const f32x4*>(Gs + row * LDG + cc * VEC + 4 * e4);
+        f32x4* at = reinterpret_cast<f32x4*>(Gs + row * LDG + cc * VEC + 4 * e4);
+        f32x4 x = *at;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) gk[it][e4][e] += kda_cumsum_before<DK, PARTS>(tot, part, cc * VEC + 4 * e4 + e);
+        for (int e = 0; e < 4; ++e) x[e] += kda_cumsum_before<DK, PARTS>(tot, part, cc * VEC + 4 * e4 + e);
+        *at = x;
       }
     }
   }
@@ -300,83 +296,89 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
     rsq[tid] = 1.f;
     rsk[tid] = 1.f;
   }
-  if (tid < 256) { rq[tid] = 0.f; rk[tid] = 0.f; rb[tid] = 0.f; rv[tid] = 0.f; }
-#pragma unroll
-  for (int it = 0; it < NIT; ++it) {
-    const int c = tid + it * kFinThreads;
-    st16(Pt + (c / CPR) * LDK + (c % CPR) * VEC, pf[it]);
-  }
-#pragma unroll
-  for (int it = 0; it < NTM; ++it) {
-    const int c = tid + it * kFinThreads;
-    st16(TmT + (c / C64) * L64 + (c % C64) * VEC, tmv[it]);
-  }
-  GDN_LDS_BARRIER();   // the row vectors are initialised before the norm below writes 1/|k| over its entries; G is in registers
+  if (tid < 256) { rq[tid] = 0.f; rk[tid] = 0.f; rb[tid] = 0.f; rv[tid] = tid < 64 ? rvl : 0.f; }
+  GDN_LDS_BARRIER();   // the row vectors are initialised before the norms below write 1/|q|, 1/|k| over their entries
   tile_qk_finish<T, DK>(kt, Ks, LDK, nvalid, tid, fl.l2norm != 0, nullptr, 0, rsk, 1);
-  GDN_LDS_BARRIER();
+  f32x16 dK1 = acc_zero(), rvt = acc_zero();   // rvt: -dL below the diagonal
+  if constexpr (FULL) {
+    f32x4 gk[NIT][VEC / 4];   // this thread's pieces of G, out of the way of Kp
 #pragma unroll
-  for (int it = 0; it < NIT; ++it) {   // Kp = k^ . e^{G}
-    const int c = tid + it * kFinThreads, row = c / CPR, cc = c % CPR;
-    float f[VEC];
-    unpack16<T>(ld16(Ks + row * LDK + cc * VEC), f);
+    for (int it = 0; it < NIT; ++it) {
+      const int c = tid + it * kFinThreads;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) f[e] *= KdaDecay<T>::exp(gk[it][e / 4][e % 4]);
-    st16(Kp + row * LDK + cc * VEC, pack16<T>(f));
-  }
-  GDN_LDS_BARRIER();
-
-  if (Q_BY_OTHERS && q_wave) tile_qk_finish<T, DK>(qt, Qs, LDK, nvalid, tid & (kThreads - 1), fl.l2norm != 0, nullptr, 0, rsq, 1);
-  // ---- phase A1: dTm = stril(b_j (a2 - P Kp^T)), one 32x32 tile per tile wave; <R_t, v_t> from Tm and a2 ----
-  f32x16 a2t = acc_zero(), dat = acc_zero();
-  if (lower) a2t = a2f.unpack();
-  if (tile_wave) {
-    f32x16 x = acc_zero();
-    if (lower) mma32<T, DK, true, true>(x, Pt + 32 * ti * LDK, LDK, Kp + 32 * tj * LDK, LDK);
-    const int j = 32 * tj + l32;
-    const float bj = bs[j];
-    float sv = 0.f;
-    f32x16 tmt;   // this wave's tile of Tm as the accumulator holds a tile
-    if constexpr (FULL) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) tmt[r] = TmT[(32 * ti + acc_row(r)) * L64 + j];
-    } else {
-      AccB<T> t;
-      t.load_cols(TmT + 32 * ti * L64 + 32 * tj, L64);
-      tmt = t.unpack();
+      for (int e = 0; e < VEC / 4; ++e)
+        gk[it][e] = *reinterpret_cast<const f32x4*>(Gs + (c / CPR) * LDG + (c % CPR) * VEC + 4 * e);
+      st16(Pt + (c / CPR) * LDK + (c % CPR) * VEC, pf[it]);
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int i = 32 * ti + acc_row(r);
-      const float a2v = a2t[r];
-      sv += a2v * tmt[r];
-      M1[i * L64 + j] = Elem<T>::from_f(i > j ? bj * (a2v - x[r]) : 0.f);
+    for (int it = 0; it < NTM; ++it) {
+      const int c = tid + it * kFinThreads;
+      st16(TmT + (c / C64) * L64 + (c % C64) * VEC, tmv[it]);
     }
-    sv += __shfl_xor(sv, 32);
-    if (lane < 32) rv[wave * 64 + 32 * tj + lane] = sv;
-  }
-  GDN_LDS_BARRIER();
-  // ---- phase A2: X = Tm^T dTm (the tiles dL needs: a >= the column block) ----
-  if (tile_wave) {
-    f32x16 x = acc_zero();
-    if (lower) mma32<T, 64, false, false>(x, TmT + 32 * ti, L64, M1 + 32 * tj, L64);
+    GDN_LDS_BARRIER();
 #pragma unroll
-    for (int r = 0; r < 16; ++r) M2[(32 * ti + acc_row(r)) * L64 + 32 * tj + l32] = Elem<T>::from_f(x[r]);
-  }
-  GDN_LDS_BARRIER();
-  // ---- phase A3: dL = -stril(X Tm^T); dK1 = Tm^T P for this wave's tokens and key channels; scale dAq ----
-  f32x16 dK1 = acc_zero(), dl = acc_zero(), sa;
-  if (lower) mma32<T, 64, true, true>(dl, M2 + 32 * ti * L64, L64, TmT + 32 * tj * L64, L64);
-  if (FULL && has_k) mma32<T, 64, false, false>(dK1, TmT + 32 * ri, L64, Pt + 32 * cj, LDK);
-  if (lower) dat = daf.unpack();
+    for (int it = 0; it < NIT; ++it) {   // Kp = k^ . e^{G}
+      const int c = tid + it * kFinThreads, row = c / CPR, cc = c % CPR;
+      float f[VEC];
+      unpack16<T>(ld16(Ks + row * LDK + cc * VEC), f);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = 32 * ti + acc_row(r), j = 32 * tj + l32;
-    dl[r] = i > j ? -dl[r] : 0.f;
-    sa[r] = i >= j ? scale * dat[r] : 0.f;
+      for (int e = 0; e < VEC; ++e) f[e] *= KdaDecay<T>::exp(gk[it][e / 4][e % 4]);
+      st16(Kp + row * LDK + cc * VEC, pack16<T>(f));
+    }
+    GDN_LDS_BARRIER();
+    // dTm = stril(b_j (a2 - P Kp^T)), one 32x32 tile per tile wave; <R_t, v_t> from Tm and a2
+    if (tile_wave) {
+      f32x16 x = acc_zero(), a2t = acc_zero();
+      if (lower) {
+        a2t = rvf.unpack();
+        mma32<T, DK, true, true>(x, Pt + 32 * ti * LDK, LDK, Kp + 32 * tj * LDK, LDK);
+      }
+      const int j = 32 * tj + l32;
+      const float bj = bs[j];
+      float sv = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * ti + acc_row(r);
+        sv += a2t[r] * TmT[i * L64 + j];
+        M1[i * L64 + j] = Elem<T>::from_f(i > j ? bj * (a2t[r] - x[r]) : 0.f);
+      }
+      sv += __shfl_xor(sv, 32);
+      if (lane < 32) rv[wave * 64 + 32 * tj + lane] = sv;
+    }
+    GDN_LDS_BARRIER();
+    // X = Tm^T dTm (the tiles dL needs: a >= the column block)
+    if (tile_wave) {
+      f32x16 x = acc_zero();
+      if (lower) mma32<T, 64, false, false>(x, TmT + 32 * ti, L64, M1 + 32 * tj, L64);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) M2[(32 * ti + acc_row(r)) * L64 + 32 * tj + l32] = Elem<T>::from_f(x[r]);
+    }
+    GDN_LDS_BARRIER();
+    // dL = -stril(X Tm^T); dK1 = Tm^T P for this wave's tokens and key channels
+    if (lower) mma32<T, 64, true, true>(rvt, M2 + 32 * ti * L64, L64, TmT + 32 * tj * L64, L64);
+    if (has_k) mma32<T, 64, false, false>(dK1, TmT + 32 * ri, L64, Pt + 32 * cj, LDK);
+    GDN_LDS_BARRIER();   // dTm, X, Kp and P are consumed
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      const int c = tid + it * kFinThreads;
+#pragma unroll
+      for (int e = 0; e < VEC / 4; ++e)
+        *reinterpret_cast<f32x4*>(Gs + (c / CPR) * LDG + (c % CPR) * VEC + 4 * e) = gk[it][e];
+    }
   }
-  GDN_LDS_BARRIER();   // dTm, X, Kp are consumed (FULL: P too)
-  // ---- phase A4: the coefficient matrices in place of dTm and X; G in place of Kp; q^ rows (FULL: in place of P) ----
+  if (q_wave) tile_qk_finish<T, DK>(qt, Qs, LDK, nvalid, tid & (kThreads - 1), fl.l2norm != 0, nullptr, 0, rsq, 1);
   if (tile_wave) {
+    f32x16 dl = acc_zero(), sa = acc_zero();
+    if (lower) {
+      if constexpr (!FULL) rvt = rvf.unpack();
+      const f32x16 dat = daf.unpack();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * ti + acc_row(r), j = 32 * tj + l32;
+        dl[r] = i > j ? -rvt[r] : 0.f;
+        sa[r] = i >= j ? scale * dat[r] : 0.f;
+      }
+    }
     // the transposed dL carries the beta of its later token (its row in dL): the sum over i of dL_ij b_i k_i f_i then
     // takes the same rescaled rows k_i f_i as the sum over j
     const f32x16 bi = rows_ld(bs, 32 * ti);
@@ -404,14 +406,6 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
         *reinterpret_cast<u32x2*>(M2t + att) = w2;
       }
     }
-    if constexpr (!Q_BY_OTHERS) tile_qk_finish<T, DK>(qt, Qs, LDK, nvalid, tid, fl.l2norm != 0, nullptr, 0, rsq, 1);
-  }
-#pragma unroll
-  for (int it = 0; it < NIT; ++it) {
-    const int c = tid + it * kFinThreads;
-#pragma unroll
-    for (int e = 0; e < VEC / 4; ++e)
-      *reinterpret_cast<f32x4*>(Gs + (c / CPR) * LDG + (c % CPR) * VEC + 4 * e) = gk[it][e];
   }
   GDN_LDS_BARRIER();
 
@@ -419,7 +413,7 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
   //      in the wave's 32-token block ----
   const int d = 32 * cj + l32;
   float Gi[16], U[16], Uq[16], W[16];
-  AccB<T> lqf, lkf;   // the sums over V of this lane's rows (dQb, dK2) for phase B3
+  AccB<T> lqf, lkf, l1f;   // the sums over V of this lane's rows (dQb, dK2, dK1) for phase B3
   if (has_k) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -509,7 +503,7 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
           // offset that is the same for every lane: one addition per address instead of a shift, a mask and a product.
           const float* Gpm = Gs + (32 * ri + (lg <= 3 ? 8 * half : 0)) * LDG + d;
           const float* Gom = Gs + (32 * ri + (lg <= 2 ? 4 * half : 0)) * LDG + d;
-          const u32x4* keepL = keepT + (lg - 1) * 4 * 64 + lane;
+          const u32x4* keepL = keepT + (lg - 3) * 4 * 64 + lane;
           f32x16 cu = acc_zero(), cq = acc_zero(), cw = acc_zero();
 #pragma unroll
           for (int kg = 0; kg < 2; ++kg) {
@@ -543,9 +537,10 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
             }
           }
         };
-        // (phase B3's tiles are requested here, four levels ahead of their use: 16 registers)
+        // (phase B3's tiles are requested here, four levels ahead of their use: 24 registers)
         lqf.load(dQb + (ri * NKT + cj) * 1024);
         lkf.load(dK2 + (ri * NKT + cj) * 1024);
+        l1f.load(dK1m + (ri * NKT + cj) * 1024);
 #pragma unroll 1
         for (int lg = 3; lg <= 5; ++lg) level(lg, IntConst<1>());
       }
@@ -642,9 +637,10 @@ __global__ __launch_bounds__(kFinThreads) void kda_bwd_finish_kernel(
     if constexpr (FULL) {   // (tiles in fragment order: token block ri, channel block cj)
       lqf.load(dQb + (ri * NKT + cj) * 1024);
       lkf.load(dK2 + (ri * NKT + cj) * 1024);
+    } else {
+      dK1 = l1f.unpack();
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (!FULL) mma32<T, 64, false, false>(dK1, TmT + 32 * ri, L64, Pt + 32 * cj, LDK);
     if constexpr (FULL) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -866,7 +862,6 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
   const T* K2F = reinterpret_cast<const T*>(ws + L.K2F);
   const T* VF = reinterpret_cast<const T*>(ws + L.VF);
   const T* HF = reinterpret_cast<const T*>(ws + L.HF);
-  const T* TMR = reinterpret_cast<const T*>(ws + L.TMR);
   const T* QBT = reinterpret_cast<const T*>(ws + L.QBT);
   T* DVF = reinterpret_cast<T*>(ws + L.DVF);
   T* DHF = reinterpret_cast<T*>(ws + L.DHF);
@@ -897,14 +892,24 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
                Ai, AQ, (const T*)dO, dec, bhat, dht, dh0, DVF, DHF, cu, chunk_offsets, d.T, H, H, d.V, scale, segs);
   }
   {
-    auto kern = chunk_bwd_local_kernel<T, DK, true>;
-    constexpr int smem = BwdLocalSmem<T, DK>::bytes;
-    if (int e = set_lds_b(kern, smem)) return e;
     TokenStrides ts = d.strides();
-    GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(kThreads), smem, st, QBT, K1F, (const T*)v, bhat, 0,
-               (const float*)nullptr, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, (const float*)nullptr,
-               (const float*)nullptr, (T*)nullptr, (T*)nullptr, (T*)dv, (void*)nullptr, (float*)nullptr, cu, chunk_offsets, d.T,
-               d.N, H, H, d.V, scale, 0, ts, DUMP, DD, device_compute_units());
+    if constexpr (sizeof(T) == 2) {
+      auto kern = chunk_bwd_local16_kernel<DK, true>;
+      constexpr int smem = BwdLocal16Smem<DK>::bytes;
+      if (int e = set_lds_b(kern, smem)) return e;
+      GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(512), smem, st, QBT, K1F, (const T*)v, bhat, 0,
+                 (const float*)nullptr, Ai, VF, (const T*)DVF, (const T*)dO, HF, DHF, (const float*)nullptr,
+                 (const float*)nullptr, (T*)nullptr, (T*)nullptr, (T*)dv, (void*)nullptr, (float*)nullptr, cu, chunk_offsets, d.T,
+                 d.N, H, H, d.V, scale, ts, DUMP, DD);
+    } else {
+      auto kern = chunk_bwd_local_kernel<T, DK, true>;
+      constexpr int smem = BwdLocalSmem<T, DK>::bytes;
+      if (int e = set_lds_b(kern, smem)) return e;
+      GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(kThreads), smem, st, QBT, K1F, (const T*)v, bhat, 0,
+                 (const float*)nullptr, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, (const float*)nullptr,
+                 (const float*)nullptr, (T*)nullptr, (T*)nullptr, (T*)dv, (void*)nullptr, (float*)nullptr, cu, chunk_offsets, d.T,
+                 d.N, H, H, d.V, scale, 0, ts, DUMP, DD, device_compute_units());
+    }
   }
   {
     const int es = (int)sizeof(T), ge = fl.g_f32 ? 4 : es, be = fl.beta_f32 ? 4 : es;
@@ -918,7 +923,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
     constexpr int smem = KdaBwdSmem<T, DK>::bytes;
     if (int e = set_lds_b(kern, smem)) return e;
     GDN_LAUNCH(kKernKdaBwdFinish, st, kern, dim3(nc, H), dim3(kFinThreads), smem, st, (const T*)q, (const T*)k, g, A_log, dt_bias,
-               bhat, TMR, (const T*)DUMP, (const float*)DD, cu, chunk_offsets, (T*)dq, (T*)dk, dg, dbeta, PART, d.T, d.N, H, scale, fl);
+               bhat, reinterpret_cast<const T*>(ws + L.TMR), (const T*)DUMP, (const float*)DD, cu, chunk_offsets, (T*)dq, (T*)dk, dg, dbeta, PART, d.T, d.N, H, scale, fl);
   }
   if (fl.use_gate && (dA_log != nullptr || ddt_bias != nullptr))
     GDN_LAUNCH(kKernKdaBwdReduce, st, kda_bwd_reduce_kernel, dim3(H, (d.K + 32) / 32), dim3(kThreads), 0, st, (const float*)PART, cu,

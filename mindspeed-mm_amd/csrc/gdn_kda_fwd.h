@@ -438,7 +438,7 @@ __global__ __launch_bounds__(kThreads) GDN_WAVES_PER_SIMD(2) void kda_prep_kerne
   }
   tril_inverse_64(As, Ti, wave, lane);
   store_tm_tiles<T>(Ti, Tms, Ai_out + ch * 4096, tid, wave, lane);
-  if (TMR_out != nullptr) {   // the staging tile holds Tm row-major in operand precision
+  if (sizeof(T) == 4 && TMR_out != nullptr) {   // the staging tile holds Tm row-major in operand precision
     constexpr int C64 = 64 / VEC;
     for (int c = tid; c < 64 * C64; c += kThreads)
       st16(TMR_out + ch * 4096 + (c / C64) * 64 + (c % C64) * VEC, ld16(Tms + (c / C64) * SM::L64 + (c % C64) * VEC));
@@ -468,7 +468,7 @@ static int kda_fwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
   T* VF = reinterpret_cast<T*>(ws + L.VF);
   T* HF = reinterpret_cast<T*>(ws + L.HF);
   T* QBT = (with_backward || FUSE) ? reinterpret_cast<T*>(ws + L.QBT) : nullptr;
-  T* TMR = with_backward ? reinterpret_cast<T*>(ws + L.TMR) : nullptr;
+  T* TMR = with_backward && sizeof(T) == 4 ? reinterpret_cast<T*>(ws + L.TMR) : nullptr;
   {
     const int64_t ob = (int64_t)H * d.V * (int)sizeof(T);
     TailRows tail{{o}, {ob}, {(int)ob}};

@@ -125,6 +125,12 @@ def test_chunk_local_backward_of_head_groups(ops, T, Hqk, Hv, K, V, l2):
     P.check_chunk(ops, "cpu", 1, T, Hqk, Hv, K, V, BF, l2=l2, backward=True, wrap=guarded, h0_std=0.1, seed=5)
 
 
+@pytest.mark.parametrize("T,K,V", [(33, 64, 64), (70, 64, 192), (65, 128, 192)])
+def test_kda_backward_where_the_sums_over_v_end(ops, T, K, V):
+    """One pair of V blocks, R in two parts with the second cut short, waves without columns of K, a last chunk of one token."""
+    P.check_kda(ops, "cpu", 1, T, 1, K, V, BF, backward=True, wrap=guarded, h0_std=0.1, seed=6)
+
+
 def test_chunk_backward_without_initial_state(ops):
     P.check_chunk(ops, "cpu", 1, 70, 1, 1, 64, 64, F32, backward=True, with_h0=False, wrap=guarded)
 
