@@ -542,13 +542,38 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
   GDN_WAIT_VMEM();
   GDN_LDS_BARRIER();
 
-  // Tm^T tile (a, b) as an A operand (lane <-> column of Tm, registers <-> row): the stored tile (b, a) turned round
-  auto tm_t = [&](int a, int b) {
-    AccB<T> f, o;
-    f.load(TmF + (2 * b + a) * 1024);
-    o.pack(mfma_transpose<T>(f, id));
+  // A stored tile turned round.  In fp32 a pass through the matrix core takes sixteen instructions of 64 cycles, and a wave that
+  // has a SIMD to itself waits for each; reading the tile along its columns, eight lanes to a bank, takes a quarter of that
+  // (the kernel: 8 chunks of 4 heads of 64 47 -> 38 us, 64 chunks of 16 heads of 128 303 -> 250).
+  auto turned = [&](const T* tile) {
+    AccB<T> o;
+    if constexpr (sizeof(T) == 4) {
+      o.load_t(tile);
+    } else {
+      AccB<T> f;
+      f.load(tile);
+      o.pack(mfma_transpose<T>(f, id));
+    }
     return o;
   };
+  // the same for a tile that passes from wave to wave: 16-bit types turn it before it is stored, fp32 turns it as it is read
+  auto store_turned = [&](const AccB<T>& x, T* tile) {
+    if constexpr (sizeof(T) == 4) {
+      x.store(tile);
+    } else {
+      AccB<T> o;
+      o.pack(mfma_transpose<T>(x, id));
+      o.store(tile);
+    }
+  };
+  auto load_turned = [&](const T* tile) {
+    AccB<T> o;
+    if constexpr (sizeof(T) == 4) o.load_t(tile);
+    else o.load(tile);
+    return o;
+  };
+  // Tm^T tile (a, b) as an A operand (lane <-> column of Tm, registers <-> row): the stored tile (b, a)
+  auto tm_t = [&](int a, int b) { return turned(TmF + (2 * b + a) * 1024); };
   f32x16 ds = acc_zero(), a2 = acc_zero(), dQi[2], dKi[2], dWa[2];
 #pragma unroll
   for (int ri = 0; ri < 2; ++ri) { dQi[ri] = acc_zero(); dKi[ri] = acc_zero(); dWa[ri] = acc_zero(); }
@@ -566,12 +591,9 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     // the wave are compared against loop constants (fragments indexed at run time would go to scratch).
     AccB<T> f, Sf, dSf, dOt[2];
     if (has_k) {                             // (lane <-> K column, registers <-> V)
-      f.load(stage0 + SM::priv + wave * 2048);
-      const f32x16 sv = mfma_transpose<T>(f, id);
-      Sf.pack(sv);
-      f.load(stage0 + SM::priv + wave * 2048 + 1024);
-      const f32x16 dsv = mfma_transpose<T>(f, id);
-      dSf.pack(dsv);
+      Sf = turned(stage0 + SM::priv + wave * 2048);
+      dSf = turned(stage0 + SM::priv + wave * 2048 + 1024);
+      const f32x16 sv = Sf.unpack(), dsv = dSf.unpack();
 #pragma unroll
       for (int r = 0; r < 16; ++r) sds += sv[r] * dsv[r];
     }
@@ -594,9 +616,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     }
 #pragma unroll
     for (int ri = 0; ri < 2; ++ri) {
-      AccB<T> Vt;
-      f.load(st + ri * 1024);
-      Vt.pack(mfma_transpose<T>(f, id));
+      const AccB<T> Vt = turned(st + ri * 1024);
       if (has_k) mma32_ff<T>(dKi[ri], Vt, dSf);
       if (lower && ri == tj) {
         // the dO fragments of this wave's token block, picked register by register (an indexed fragment would go to
@@ -611,9 +631,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     }
 #pragma unroll
     for (int ri = 0; ri < 2; ++ri) {
-      AccB<T> dVt;
-      f.load(st + (2 + ri) * 1024);
-      dVt.pack(mfma_transpose<T>(f, id));
+      const AccB<T> dVt = turned(st + (2 + ri) * 1024);
       if (has_k) mma32_ff<T>(dWa[ri], dVt, Sf);
       if (lower && ri == ti) {
         SwizzledTile<T, 64>::frags(f, rb + 64 * 64, 32 * tj + l32, rk0);
@@ -623,7 +641,8 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     // dv = beta (Tm^T dV') of this V block.  The dV' tiles serve as they lie in
     // the stage, as the A operand: the product is dv^T (lane <-> token, registers <-> V column), of which every lane
     // stores four adjacent columns at a time without a detour through LDS.
-    const int job = (wave - 2 * vblk) & 3;   // the two token halves of a block go to two waves, rotating with the block
+    // the two token halves of a block go to two waves, rotating with the block or, where there are any, without columns of K
+    const int job = (wave - (DK <= 64 ? 2 : 2 * vblk)) & 3;
     if (job < 2) {
       const int rj = job;
       f32x16 Rt = acc_zero();
@@ -696,18 +715,14 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
   if (has_k) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      AccB<T> f;
-      f.load(EA + (2 * cj + t) * 1024);
-      KTf[t].pack(mfma_transpose<T>(f, id));
+      KTf[t] = turned(EA + (2 * cj + t) * 1024);
       QTf[t].load(EQ + wave * 2048 + t * 1024);
     }
 #pragma unroll
     for (int ri = 0; ri < 2; ++ri) {         // dW = -(dV' S^T): B operand of P in registers, A operand of a1 to LDS
       dWb[ri].pack(dWa[ri]);
       dWb[ri].negate();      // the sign on the packed pairs: half as many instructions as on the sixteen values
-      AccB<T> a;
-      a.pack(mfma_transpose<T>(dWb[ri], id));
-      a.store(dWF + (ri * NKT + cj) * 1024);
+      store_turned(dWb[ri], dWF + (ri * NKT + cj) * 1024);
     }
   }
   {
@@ -724,11 +739,10 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) ds[r] = (32 * ti + acc_row(r) >= j) ? scale * ds[r] * eg[r] : 0.f;
-    AccB<T> d, t;
+    AccB<T> d;
     d.pack(ds);
     d.store(tileD + wave * 1024);
-    t.pack(mfma_transpose<T>(d, id));
-    t.store(tileT + wave * 1024);
+    store_turned(d, tileT + wave * 1024);
   }
   GDN_LDS_BARRIER();
   float ski = 0.f;
@@ -744,7 +758,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
         for (int r = 0; r < 16; ++r) dQi[ri][r] *= fq[r];
         AccB<T> a;
 #pragma unroll
-        for (int t = 0; t <= ri; ++t) { a.load(tileT + (2 * ri + t) * 1024); mma32_ff<T>(dQi[ri], a, KTf[t]); }
+        for (int t = 0; t <= ri; ++t) { a = load_turned(tileT + (2 * ri + t) * 1024); mma32_ff<T>(dQi[ri], a, KTf[t]); }
         const f32x16 qq = QTf[ri].unpack();
         f32x16 p;
 #pragma unroll
@@ -819,7 +833,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
 #pragma unroll
       for (int kt = 0; kt < NKT; ++kt) {
         AccB<T> a, b;
-        a.load(dWF + (ti * NKT + kt) * 1024);
+        a = load_turned(dWF + (ti * NKT + kt) * 1024);
         b.load(EA + (2 * kt + tj) * 1024);
         mma32_ff<T>(a1, a, b);
       }
@@ -828,10 +842,9 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     const float bj = bs[j], ej = egs[j];
 #pragma unroll
     for (int r = 0; r < 16; ++r) a1[r] = (32 * ti + acc_row(r) > j) ? bj * (ej * a1[r] + a2[r]) : 0.f;
-    AccB<T> d, t;
+    AccB<T> d;
     d.pack(a1);
-    t.pack(mfma_transpose<T>(d, id));
-    t.store(tileT + wave * 1024);
+    store_turned(d, tileT + wave * 1024);
   }
   // <q_i, dQ_i> once per row, for the l2-norm backward of dq behind the next barrier (instead of every lane adding
   // up the four slots for each of its sixteen rows)
@@ -871,7 +884,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     f32x16 x = acc_zero();
     AccB<T> a, b;
     for (int t = 0; t <= imin(ti, tj); ++t) {
-      a.load(tileT + (2 * ti + t) * 1024);
+      a = load_turned(tileT + (2 * ti + t) * 1024);
       b.load(TmF + (2 * tj + t) * 1024);
       mma32_ff<T>(x, a, b);
     }
@@ -897,10 +910,9 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
       y[r] = (32 * ti + acc_row(r) > j) ? -y[r] * __expf(gi[r] - gj) : 0.f;
       yb[r] = y[r] * br[r];
     }
-    AccB<T> d, t;
+    AccB<T> d;
     d.pack(y);
-    t.pack(mfma_transpose<T>(d, id));
-    t.store(tileT + wave * 1024);
+    store_turned(d, tileT + wave * 1024);
     d.pack(yb);
     d.store(dMD + wave * 1024);
   }
@@ -917,7 +929,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
       f32x16 E = acc_zero(), Fm = acc_zero(), p;
       AccB<T> a;
 #pragma unroll
-      for (int t = 0; t <= ri; ++t) { a.load(tileT + (2 * ri + t) * 1024); mma32_ff<T>(E, a, KTf[t]); }
+      for (int t = 0; t <= ri; ++t) { a = load_turned(tileT + (2 * ri + t) * 1024); mma32_ff<T>(E, a, KTf[t]); }
 #pragma unroll
       for (int t = ri; t < 2; ++t) { a.load(dMD + (2 * t + ri) * 1024); mma32_ff<T>(Fm, a, KTf[t]); }
       const f32x16 kk = KTf[ri].unpack(), br = rows_ld(bs, 32 * ri);
