@@ -20,9 +20,10 @@
 //   epilogue: contractions over tokens take them in the order 32 b + {4 g + e, 16 + 4 g + e}, which is that of two packed
 //     accumulator tiles; the 64x64 matrices pass between the waves as bf16 matrices in LDS (Mat64), written in 8-byte units
 //     straight from accumulators and read along their rows or, with the transposing read, along their columns.
-// Bound by memory: 2 x 8192 tokens, 16 q/k and 32 value heads of 128 move 2.0 GB in 424 us (4.7 TB/s), where one launch per
-// value head of the four-wave kernel, which waited (two waves to a SIMD), moved 2.04 GB in 466; 4 x 1024 tokens 139 -> 111,
-// 32768 tokens of 8 heads 234 -> 204.  What is read once passes the L2 by (424 -> 406 on a build without the fourth row sum).
+// Bound by memory: 2 x 8192 tokens, 16 q/k and 32 value heads of 128 move 2.0 GB in 411 us (4.9 TB/s), where one launch per
+// value head of the four-wave kernel, which waited (two waves to a SIMD), moved 2.04 GB in 466; 4 x 1024 tokens 139 -> 108,
+// 32768 tokens of 8 heads 234 -> 193.  (With four spilled values, each of which waits for all requests in flight when it is read
+// back: 422, 111, 203.)  What is read once passes the L2 by (424 -> 406 on a build without the fourth row sum).
 #pragma once
 #include "gdn_chunk.h"
 #include "gdn_common.h"
@@ -116,7 +117,8 @@ struct Mat64 {
 // t = n / 4, e = n % 4 and the others take it by a data-parallel-primitive move
 struct Tokens {
   Slab16::Rows v;
-  __device__ __forceinline__ void load(Lane l, const float* arr) { v.f = arr[16 * (l.n >> 2) + 4 * l.g + (l.n & 3)]; }
+  static __device__ __forceinline__ int own(Lane l) { return 16 * (l.n >> 2) + 4 * l.g + (l.n & 3); }
+  __device__ __forceinline__ void load(Lane l, const float* arr) { v.f = arr[own(l)]; }
   __device__ __forceinline__ float get(int t, int e) const { return v.get(t >> 1, 4 * (t & 1) + e); }
 };
 
@@ -161,6 +163,7 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
   float* const rsb = rsa + 512;                                // per wave: e^G <P_i,k_i> + <E_i,k_i>
   float* const rsc = rsb + 512;                                // per wave: <k_i, dK_i>
   float* const rsd = rsc + 512;                                // per wave: beta (e^G <P_i,k_i> + <E_i,k_i>) - <k_i, dK1_i> - <F_i,k_i>
+  float* const rsn = rsd + 512;                                // 1/|q|, 1/|k| of the l2 norm [64 each]
 
   const SeqInfo s = locate_chunk(blockIdx.x, cu, chunk_offsets, N, T_len);
   if (s.nvalid <= 0) return;
@@ -395,9 +398,13 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
     }
     sds = wave_sum(sds);
     if (L.id == 0) wsum[L.w] = sds;
+    float norm = 0.f;   // 1/|q|, 1/|k| of the chunk's tokens, two waves' share: they wait in LDS for the last step
+    const bool has_norm = l2 && (L.w == 2 || L.w == 3);
+    if (has_norm) norm = (L.w == 2 ? rstd_q : rstd_k)[chq * 64 + L.id];
     const Mat64 MS{base + SM::raw}, MD{base + SM::raw + 4096}, MB{base + SM::vn};   // ds^T, dM^T, (beta dM)^T
     GDN_WAIT_VMEM();
     GDN_LDS_BARRIER();   // K and Q have landed; the last block's operands are consumed
+    if (has_norm) rsn[64 * (L.w - 2) + L.id] = norm;
 
     auto tiles_out = [&](int x, int ti, int tj) {
       const float gj = Gs[16 * tj + L.n];
@@ -523,28 +530,18 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
     GDN_LDS_BARRIER();   // the row sums are complete; the matrices are consumed
     L = Lane::here();
     if (!last) issue_head(h + 1);
-    const int own_token = 16 * (L.n >> 2) + 4 * L.g + (L.n & 3);   // see Tokens
     auto slots = [&](const float* a, int i) {
       float x = a[i];
 #pragma unroll
       for (int k = 1; k < DK / 16; ++k) x += a[64 * k + i];
       return x;
     };
-    Tokens dot_q, dot_k, rs_q, rs_k;
     u32x4 before[4];
     {
-      if (l2) {
-        rs_q.v.f = rstd_q[chq * 64 + own_token];
-        rs_k.v.f = rstd_k[chq * 64 + own_token];
-      }
       const T* from = hh != 0 ? (const T*)sums() : reinterpret_cast<const T*>(kZero16);   // the choice on the address: no branch to join
 #pragma unroll
       for (int b = 0; b < 4; ++b) before[b] = *reinterpret_cast<const u32x4*>(from + (hh != 0 ? 8 * b : 0));
-      if (l2) {
-        load_kq();
-        dot_q.v.f = slots(rsa, own_token);
-        dot_k.v.f = slots(rsc, own_token);
-      }
+      if (l2) load_kq();
     }
     if (l2) {
       GDN_KEEP_HERE(QT[0]);
@@ -558,8 +555,14 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
     // l2 norm, the sum over the group's heads, and after its last head the rows by way of a [DK][64] matrix in LDS
     const Mat64 MQ{base + SM::raw}, MK{base + SM::dv};
     static_assert(SM::priv - SM::raw == 64 * 128 && SM::r - SM::dv == 64 * 128, "they fit");
-    auto finish = [&](f32x4* d, const u32x4* y, const Tokens& dot, const Tokens& r, const u32x4* so_far, T* sum, const Mat64& to) {
+    // (the row sums and norms are read where they are used: held over the requests above they are spilled, and the wait
+    // for a spilled value is a wait for every request)
+    auto finish = [&](f32x4* d, const u32x4* y, const float* row_sums, const float* norms, const u32x4* so_far, T* sum, const Mat64& to) {
       if (l2) {
+        const Lane H = Lane::here();
+        Tokens dot, r;
+        dot.v.f = slots(row_sums, Tokens::own(H));
+        r.load(H, norms);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -582,8 +585,8 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
       }
     };
     {
-      finish(dQ, QT, dot_q, rs_q, before, sums(), MQ);
-      finish(dK, KT, dot_k, rs_k, before + 2, sums() + 16, MK);
+      finish(dQ, QT, rsa, rsn, before, sums(), MQ);
+      finish(dK, KT, rsc, rsn + 64, before + 2, sums() + 16, MK);
     }
     if (L.w == 0) {   // d(cumulative G) -> d(g): suffix sum inside the chunk
       // dG_i = <q,dQ> + beta (e^G <P,k> + <E,k>) - <k,dK1> - <F,k>, E = dM K, F = dM^T (beta K)
