@@ -49,8 +49,8 @@ TRAFFIC_SOURCE = "profiles/chunk_fwd_bwd_B2_T8192_bf16_hbm_traffic.md"
 
 
 def measured_traffic_bytes_per_launch():
-    """{kernel: bytes per launch} from the first table of TRAFFIC_SOURCE (rows `| kernel<...> | ... | bytes |`, the last
-    column being bytes per launch); empty when the file is missing, and the traffic fields are then null."""
+    """{kernel: bytes} from the first table of TRAFFIC_SOURCE (rows `| kernel<...> | ... | bytes |`, the last column being
+    bytes per launch and, of the chunk-local kernel's one launch, per value head of a q/k group); empty when the file is missing, and the traffic fields are then null."""
     out, in_main = {}, False
     try:
         with open(os.path.join(ROOT, TRAFFIC_SOURCE)) as f:
@@ -95,9 +95,8 @@ def kernel_matmul_flops(K, V, C=64):
         "chunk_state_kernel": g(C, V, K) + g(C, V, C) + g(K, V, C) + g(C, V, K) + g(C, V, C),
         # Aq^T dO, K dS, Tm^T dV', Q^T dO, K^T R
         "chunk_state_bwd_kernel": g(C, V, C) + g(C, V, K) + g(C, V, C) + 2 * g(K, V, C),
-        # dO V'^T, dO S^T, V' dS^T, dV' S^T, ds K, ds^T Q | Tm^T dW, dW K^T, Tm^T dV', dV' V^T, dTm Tm^T, Tm^T X, dM K, dM^T K
-        "chunk_bwd_local_kernel": g(C, C, V) + 3 * g(C, K, V) + 2 * g(C, K, C)
-                                  + g(C, K, C) + g(C, C, K) + g(C, V, C) + g(C, C, V) + 2 * g(C, C, C) + 2 * g(C, K, C),
+        # dO V'^T, R V'^T, dO S^T, V' dS^T, R S^T with R = Tm^T dV', ds K, ds^T Q, dM K, dM^T K
+        "chunk_bwd_local_kernel": 2 * g(C, C, V) + 3 * g(C, K, V) + g(C, V, C) + 4 * g(C, K, C),
     }
 
 
@@ -114,9 +113,9 @@ def kernel_algorithmic_bytes(K, V, grp, e=2, C=64):
         "chunk_state_kernel": 2 * tk // grp + 2 * tri + tv + 2 * row + tv + tv + st,
         # K, Q^T (per group), Tm, Aq, dO, G, beta -> dv_new, dS
         "chunk_state_bwd_kernel": 2 * tk // grp + 2 * tri + tv + 2 * row + tv + st,
-        # v_new, dv_new, dO, S, dS, v, K, q, Tm, row vectors -> dv, dg, dbeta, dq/dk (written by the first head of a
-        # group, read and re-written by the others)
-        "chunk_bwd_local_kernel": 3 * tv + 2 * st + tv + 2 * tk + cc + 5 * row + tv + 2 * row
+        # v_new, dv_new, dO, S, dS, v, K and Q^T (per group), Tm, row vectors -> dv, dg, dbeta, dq/dk (the sums over a
+        # group's heads are written by each head and read by the next)
+        "chunk_bwd_local_kernel": 3 * tv + 2 * st + tv + 2 * tk // grp + tri + 5 * row + tv + 2 * row
                                   + 2 * tk * (2 * grp - 1) // grp,
     }
 
@@ -211,8 +210,8 @@ def main():
     total_kernel_ms = sum(ms for ms, _ in timings.values()) / args.steps
     flops = kernel_matmul_flops(c["K"], c["V"])
     for name, (ms, cnt) in timings.items():
-        # a kernel launched several times per step (one launch per value head of a q/k group) splits the step's work
-        # evenly over its launches: avg_ms is per launch, step_ms per step
+        # a kernel launched several times per step splits the step's work evenly over its launches: avg_ms is per launch,
+        # step_ms per step
         launches = cnt / args.steps
         avg, step_ms = ms / cnt, ms / args.steps
         per_kernel[name] = {"avg_ms": round(avg, 4), "launches_per_step": round(launches, 2),
@@ -233,10 +232,12 @@ def main():
     path_tflops = ref_formula_flops(tokens, c["Hv"], c["K"], c["V"]) / (ms_per_step * 1e-3) / 1e12
     min_bytes = minimal_bytes(c["B"], c["T"], c["B"], c["Hqk"], c["Hv"], c["K"], c["V"])
     interface_total = sum(abytes[n] * nchunk_heads for n in per_kernel if n in abytes)
-    traffic_table = measured_traffic_bytes_per_launch()
+    grp = c["Hv"] // c["Hqk"]
+    traffic_step = {n: b * (grp if n == "chunk_bwd_local_kernel" else per_kernel[n]["launches_per_step"])
+                    for n, b in measured_traffic_bytes_per_launch().items() if n in per_kernel}
     traffic_total = None
-    if all(n in traffic_table for n in per_kernel if n in abytes):
-        traffic_total = sum(traffic_table[n] * per_kernel[n]["launches_per_step"] for n in per_kernel if n in abytes)
+    if all(n in traffic_step for n in per_kernel if n in abytes):
+        traffic_total = sum(traffic_step[n] for n in per_kernel if n in abytes)
     # the whole step against both roofs: the operator's minimal bytes (inputs and outputs only) and the reference's
     # FLOP count say what an ideal implementation would need; the kernels' own interfaces move more (intermediates
     # between the launches), which is what the per-kernel figures above are measured against
@@ -260,7 +261,7 @@ def main():
                              "stored_mode_kept_bytes": int(lib.gdn_chunk_workspace_bytes(
                                  c["B"], c["T"], c["B"], c["Hqk"], c["Hv"], c["K"], c["V"], 1, 1))}}
     roofline = {"kernel": dom, "bound": "hbm", "achieved": round(dom_gbps, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                "frac": round(dom_gbps / PEAK_HBM_GBS, 4), "traffic": traffic_table.get(dom),
+                "frac": round(dom_gbps / PEAK_HBM_GBS, 4), "traffic": int(traffic_step[dom] / launches) if dom in traffic_step else None,
                 "traffic_source": TRAFFIC_SOURCE + " (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, collected offline)",
                 "algorithmic_bytes_per_launch": int(bytes_per_launch), "launches_per_step": launches,
                 "avg_launch_ms": per_kernel[dom]["avg_ms"],

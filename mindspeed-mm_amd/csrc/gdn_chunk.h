@@ -178,7 +178,7 @@ inline KdaWorkspace kda_workspace_layout(const ChunkDims& d, int elem_bytes) {
   return w;
 }
 
-// The two sequential kernels give one compute wave a 32-column slab of the state.  What limits them is the rate at
+// The two sequential kernels give one or two compute waves a 32-column slab of the state.  What limits them is the rate at
 // which one CU gets its requests served (about 35 GB/s measured, loads and stores together), whatever the number of
 // slabs the workgroup serves, so when the whole problem has no more slabs than the device has CUs every slab gets a
 // workgroup (and a CU) of its own; larger problems put two slabs in a workgroup, which share the tiles.

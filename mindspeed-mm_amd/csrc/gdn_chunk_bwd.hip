@@ -12,6 +12,7 @@
 //     dbeta = e^G<P,k> + <R,v> + <dM K, k>;  dG2 = beta e^G<P,k> + beta<dM K,k> - <dM^T(beta K),k>
 //   dg = reverse chunk-local cumsum(dG1 + dG2); group sum of dq/dk over grouped heads and the
 //   l2-norm backward dx = (dy - <dy,y> y) rstd                                  (same kernel)
+// (chunk_bwd_local16_kernel, 16-bit types: dM = -strict_tril(R V'^T) . Gam, P = -R S^T instead of the line of P, R, dTm, dM)
 // The equations are those of the reference's backward kernels (mindspeed_mm/fsdp/ops/gdn/triton/
 // chunk_o.py:19-284, chunk_delta_h.py:307-513, wy_fast.py:17-141, chunk_gated_delta_rule.py:88-174), with
 // the dG row/column sums rewritten as row dot products with dQ/dK so that Q K^T need not be rebuilt.
@@ -26,8 +27,8 @@
 namespace gdn {
 
 // ---------------------------------------------------------------------------------------------
-// chunk_state_bwd_kernel: the reverse recurrence, mirror of chunk_state_kernel.  One compute wave owns a 32-column
-// slab of dS[K, 32] in fp32 accumulators and per chunk (last to first) does
+// chunk_state_bwd_kernel: the reverse recurrence, mirror of chunk_state_kernel.  A 32-column
+// slab of dS[K, 32] is in the fp32 accumulators of one compute wave or of two (gdn_slab.h), which per chunk (last to first) do
 //     dV' = e^{G_last-G} . (K dS) + (scale Aq)^T dO
 //     R = Tm^T dV'        dS <- e^{G_last} dS + Q^T (scale e^G . dO) - K^T (beta e^G . R)
 // (the last term is W^T dV' with W = Tm (beta e^G K) never materialised), dS, dV', R and the scaled dO used as B

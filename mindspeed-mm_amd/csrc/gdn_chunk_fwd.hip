@@ -320,18 +320,18 @@ __global__ __launch_bounds__(kThreads) GDN_WAVES_PER_SIMD(sizeof(T) == 2 ? 4 : 3
 
 // ---------------------------------------------------------------------------------------------
 // chunk_state_kernel: the inter-chunk recurrence, the only part of the forward pass that is sequential in the
-// chunks.  One compute wave owns a 32-column slab of the state S[K, 32] in fp32 registers for the whole sequence
-// and per chunk does
+// chunks.  A slab of 32 columns of the state, S[K, 32], stays in the fp32 registers of one compute wave for the whole
+// sequence or, in 16 bits where a workgroup has one slab, of two waves with 16 columns each (gdn_slab.h); per chunk
 //     y = K S     z = beta (v - e^G . y)     V' = Tm z     S <- e^{G_last} S + K^T (e^{G_last-G} . V')
 // which is V' = U - W S with W = Tm (beta e^G K), U = Tm (beta V) never materialised.  Every B operand (S, z, V')
 // comes straight from accumulator registers (frag_b_from_acc), so the chain never touches LDS.  The A operands are
 // fragment-order tiles prepared by chunk_prep_kernel (K per q/k group, Tm per value head), one contiguous block per
 // chunk; K^T is the same K image read with the transposing LDS read, and the slab's raw v rows are read the same way
 // into the accumulator layout.  NL loader waves of the workgroup copy the next chunks' operands global -> registers ->
-// LDS two chunks ahead (two LDS stages); the roles meet at one barrier per chunk.  Where LDS allows (PRE) the loaders
-// write K twice, rows scaled by -beta e^G and by e^{G_last-G}, and v scaled by beta, so that the per-token factors
-// never enter the compute wave's dependent chain: z is the accumulator of (-beta e^G K) S started from beta v.
-// OUT: a second wave per slab forms the output O = scale e^G . (Q S) + Aq V' of the same 32 columns from the state and
+// LDS two chunks ahead (two LDS stages); the roles meet at one barrier per chunk.  With K = 64 (PRE) the loaders
+// write K twice, rows scaled by -beta e^G and by e^{G_last-G}, and v scaled by beta: z is the accumulator of (-beta e^G K) S
+// started from beta v.  Elsewhere the factors are applied to the accumulators in fp32.
+// OUT: further waves form the output O = scale e^G . (Q S) + Aq V' of the same 32 columns from the state and
 // V' the compute wave leaves in LDS (Q read transposed from the Q^T image, Aq likewise), one step behind it, so that
 // neither S nor V' has to be re-read from memory; both are still stored when a backward pass will need them.
 // ---------------------------------------------------------------------------------------------
@@ -743,8 +743,8 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
     typename SL::Acc p0 = PRE ? Vb[0].unpack() : SL::zero(), p1 = PRE ? Vb[1].unpack() : SL::zero();
     // What the chain needs next is read from LDS while the matrix pipe works on what it has: Tm ahead of the last pair of
     // K tiles, the row factors between its products, K^T behind those with Tm.  The fences keep the compiler from moving
-    // the reads to their uses, where each would be waited for.  Forward only 2 x 8192, 32 heads 199 -> 193 us, four packed
-    // prompts 353 -> 344; K^T ahead of the last pair as well spills 33 registers and takes 393.
+    // the reads to their uses, where each would be waited for.  With 32 columns to a wave: four packed prompts
+    // 353 -> 344 us; K^T ahead of the last pair as well spills 33 registers and takes 393.
     static_assert(NP <= 2, "two buffers of K tiles");
     typename SL::Rows fb, fe, fd;           // !PRE: beta, beta e^G and e^{G_last-G} of the tokens; KDA: see below
     if constexpr (!PRE) {
