@@ -273,7 +273,13 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
         const T* from = v + (tok0 + imin(row, nvalid - 1)) * ts.v + (int64_t)h * V + 32 * vblk + 8 * L.g;
         u32x4 vv[2];
 #pragma unroll
-        for (int x = 0; x < 2; ++x) vv[x] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from + 32 * imin((L.w >> 2) + 2 * x, nb - 1)));
+        for (int x = 0; x < 2; ++x) {
+          const u32x4* at_v = reinterpret_cast<const u32x4*>(from + 32 * imin((L.w >> 2) + 2 * x, nb - 1));
+          // two waves share a line of v.  Kept in the L2 for the second of them: V = 256 5145 -> 5043 us, V = 128 no change, but
+          // KDA, which has nothing else to read twice, 300 -> 313.
+          if constexpr (KDA) vv[x] = __builtin_nontemporal_load(at_v);
+          else vv[x] = *at_v;
+        }
         const float bj = bs[row];
         float sv = 0.f;
         u32x4 tm1 = L.turned(base + SM::tm + (1 + jb) * 1024, t & 1, kPiece), tm0 = u32x4{0u, 0u, 0u, 0u};
