@@ -391,6 +391,9 @@ __global__ __launch_bounds__(64 * state_bwd_waves<T>(NW, NL)) GDN_WAVES_PER_SIMD
 //     D ("direct"):      pack(X)                  lane <-> j, registers <-> i
 //     T ("transposed"):  pack(transpose(pack(X)))  lane <-> i, registers <-> j
 //   dQ, dK, dv leave as 16-byte row pieces.
+// (Holding the second workgroups of the CUs back by half of a workgroup's time, once a launch, costs that time where, as in fp32,
+// only one fits a CU, and gains nothing where two do: fp32, 128 chunks of 32 heads of 128, two launches 978 us with, 949 without;
+// 16 bits with V = 64, 256 chunks of 32 heads, K = 64 295 and 284, K = 128 347 and 345.)
 // ---------------------------------------------------------------------------------------------
 template <typename T, int DK> struct BwdLocalSmem {
   // main loop, in elements:
@@ -421,8 +424,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
     const T* __restrict__ dO, const T* __restrict__ hf, const T* dhf_in, const float* __restrict__ rstd_q,
     const float* __restrict__ rstd_k, T* dq, T* dk, T* __restrict__ dv_out, void* __restrict__ dbeta,
     float* __restrict__ dg, const int64_t* __restrict__ cu, const int* __restrict__ chunk_offsets, int T_len, int N,
-    int Hqk, int Hv, int V, float scale, int hh, TokenStrides ts, T* __restrict__ kda_dump, float* __restrict__ kda_dd,
-    int cus) {
+    int Hqk, int Hv, int V, float scale, int hh, TokenStrides ts, T* __restrict__ kda_dump, float* __restrict__ kda_dd) {
   static_assert(!KDA || sizeof(T) == 4, "16-bit KDA: chunk_bwd_local16_kernel");
   using SM = BwdLocalSmem<T, DK>;
   constexpr int NKT = DK / 32, VEC = Elem<T>::kVec, KG = AccK<T>::kGroups;
@@ -445,7 +447,6 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
   float* sgs = rqc + 64;   // scale e^{G_i}: the row factor of the inter-chunk part of dQ
   float* egl = sgs + 64;   // e^{G_last - G_i}: that of dK (one exponential per row here instead of one per element there)
 
-  stagger_second_resident<127>(KDA ? 3 : 4, 8 * cus, cus);   // about half of a workgroup's duration
   const SeqInfo s = locate_chunk(blockIdx.x, cu, chunk_offsets, N, T_len);
   if (s.nvalid <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31;
@@ -1087,8 +1088,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
     for (int hh = 0; hh < d.Hv / d.Hqk; ++hh)
       GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, d.Hqk), dim3(kThreads), smem, st, QTF, (const T*)KAF, (const T*)v,
                  Bt, beta_same, G, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, rstd_q, rstd_k, (T*)dq, (T*)dk,
-                 (T*)dv, dbeta, dg, cu, chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, hh, d.strides(), (T*)nullptr, (float*)nullptr,
-                 device_compute_units());
+                 (T*)dv, dbeta, dg, cu, chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, hh, d.strides(), (T*)nullptr, (float*)nullptr);
   }
   return (int)hipGetLastError();
 }

@@ -107,20 +107,6 @@ __device__ __forceinline__ int xcd_grouped_head(int b, int total, int grp) {
 #define GDN_KEEP_HERE(x) asm volatile("" : "+v"(x))
 #define GDN_KEEP_HERE_UNIFORM(x) asm volatile("" : "+s"(x))   // a wave-uniform value, in a scalar register
 #endif
-// The workgroups of a launch start together and, doing equal work, stay in step: they all load at the same time and
-// all compute at the same time, and the two workgroups that share a CU do not fill each other's waits.  Holding back
-// the second workgroup of each CU once (workgroup ids are handed out breadth first, so with `cus` compute units these
-// are ids cus .. 2 cus - 1) shifts it, and every workgroup that later takes over its place, for the rest of the launch.
-// Worth 2 % on the chunk-local backward kernel, measured in alternation with the same build without the wait; nothing
-// on kernels whose phases are shorter or that run one workgroup per CU.  The wait costs its own length once, at the
-// end of the launch, so launches of fewer than `min_groups` workgroups skip it.
-// UNITS: 64 clock cycles each (the argument of s_sleep is an immediate, at most 127).
-template <int UNITS> __device__ __forceinline__ void stagger_second_resident(int times, int min_groups, int cus) {
-  const int lin = blockIdx.x + gridDim.x * blockIdx.y;
-  if ((int)(gridDim.x * gridDim.y) >= min_groups && lin >= cus && lin < 2 * cus) {
-    for (int i = 0; i < times; ++i) __builtin_amdgcn_s_sleep(UNITS);
-  }
-}
 // Asks the scheduler for the pattern (1 matrix instruction, nvalu vector instructions) x nmfma in the current
 // scheduling region.
 #define GDN_INTERLEAVE_MFMA_VALU(nmfma, nvalu)                        \

@@ -908,7 +908,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
       GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(kThreads), smem, st, QBT, K1F, (const T*)v, bhat, 0,
                  (const float*)nullptr, Ai, VF, (const T*)DVF, (const T*)dO, HF, (const T*)DHF, (const float*)nullptr,
                  (const float*)nullptr, (T*)nullptr, (T*)nullptr, (T*)dv, (void*)nullptr, (float*)nullptr, cu, chunk_offsets, d.T,
-                 d.N, H, H, d.V, scale, 0, ts, DUMP, DD, device_compute_units());
+                 d.N, H, H, d.V, scale, 0, ts, DUMP, DD);
     }
   }
   {
