@@ -406,7 +406,7 @@ __global__ __launch_bounds__(512) GDN_WAVES_PER_SIMD(4) void chunk_bwd_local16_k
     if (L.id == 0) wsum[L.w] = sds;
     float norm = 0.f;   // 1/|q|, 1/|k| of the chunk's tokens, two waves' share: they wait in LDS for the last step
     const bool has_norm = l2 && (L.w == 2 || L.w == 3);
-    if (has_norm) norm = (L.w == 2 ? rstd_q : rstd_k)[chq * 64 + L.id];
+    if (has_norm) norm = (L.w == 2 ? rstd_q : rstd_k)[chq * 64 + imin(L.id, nvalid - 1)];   // (written for the tokens there are)
     const Mat64 MS{base + SM::raw}, MD{base + SM::raw + 4096}, MB{base + SM::vn};   // ds^T, dM^T, (beta dM)^T
     GDN_WAIT_VMEM();
     GDN_LDS_BARRIER();   // K and Q have landed; the last block's operands are consumed

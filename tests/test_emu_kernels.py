@@ -125,6 +125,25 @@ def test_chunk_local_backward_of_head_groups(ops, T, Hqk, Hv, K, V, l2):
     P.check_chunk(ops, "cpu", 1, T, Hqk, Hv, K, V, BF, l2=l2, backward=True, wrap=guarded, h0_std=0.1, seed=5)
 
 
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 256)])
+def test_group_sums_read_nothing_that_was_not_written(ops, monkeypatch, K, V):
+    """The dq, dk sums that pass from head to head of a group hold the rows past a short last chunk's end too: with a
+    workspace of NaN patterns these stay finite, as nothing they are formed of is left over from before."""
+    import mindspeed_mm_amd.ops as M
+    T, Hqk, Hv = 70, 1, 3
+    parts, real = [], M._chunk_workspace
+
+    def filled(*args):
+        ws, nbytes = real(*args)
+        parts.append(ws.fill_(0xff))
+        return ws, nbytes
+    monkeypatch.setattr(M, "_chunk_workspace", filled)
+    P.check_chunk(ops, "cpu", 1, T, Hqk, Hv, K, V, BF, backward=True, wrap=guarded, h0_std=0.1)
+    assert len(parts) == 2   # the prep part, the state part: the gradients of the states are the last in it
+    states = parts[1][-2 * Hv * K * V * 2:].view(BF).view(2, Hv, K * V)
+    assert torch.isfinite(states).all()
+
+
 @pytest.mark.parametrize("T,K,V", [(33, 64, 64), (70, 64, 192), (65, 128, 192)])
 def test_kda_backward_where_the_sums_over_v_end(ops, T, K, V):
     """One pair of V blocks, R in two parts with the second cut short, waves without columns of K, a last chunk of one token."""
