@@ -75,8 +75,8 @@ struct Lane {
     const int e = n >> 2, q = n & 3, b = 2 * t + (q & 1);
     return tile + ((half ? (q & 1) : b) * 32 + ((first(o, i) + e + 4 * b) & 31)) * 8 + 4 * (q >> 1);
   }
-  __device__ __forceinline__ u32x4 turned(const bf16_t* tile, int t, Order o, bool half = false) const {
-    const bf16_t* p[2] = {turned_at(tile, t, o, 0, half), turned_at(tile, t, o, 1, half)};
+  __device__ __forceinline__ u32x4 turned(const bf16_t* tile, int t, Order o) const {
+    const bf16_t* p[2] = {turned_at(tile, t, o, 0), turned_at(tile, t, o, 1)};
     u32x4 x;
     lds_read_tr16_pairs<1>(p, &x);
     return x;

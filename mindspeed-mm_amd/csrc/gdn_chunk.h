@@ -49,8 +49,8 @@ struct ChunkWorkspace {
   int64_t HF;             // T [chunks,Hv,V/32,K/32] state BEFORE each chunk, tile = (32 rows of K) x (32 columns of V)
   int64_t fwd_bytes;
   int64_t DVF;            // T [chunks,Hv,V/32,2]    d(v_new)
-  int64_t DHF;            // T [chunks,Hv,V/32,K/32] gradient of the state AFTER each chunk; once the chunk-local kernel of a
-                          //   head has read its part it may leave the group's dq, dk sums there for the next head's launch
+  int64_t DHF;            // T [chunks,Hv,V/32,K/32] gradient of the state AFTER each chunk; once the chunk-local kernel has read
+                          //   a head's part it may leave the group's dq, dk sums there for the next head
   int64_t SEGD, SEGDM;    // as SEGH, SEGM, for the state gradients; not shared with them: several backward passes may read
                           // one forward pass's prep part at a time
   int64_t total_bytes;

@@ -373,7 +373,8 @@ __global__ __launch_bounds__(64 * state_bwd_waves<T>(NW, NL)) GDN_WAVES_PER_SIMD
 
 // ---------------------------------------------------------------------------------------------
 // chunk_bwd_local_kernel, per (chunk, head), 4 waves: everything of the backward pass that is local to a chunk once
-// the reverse recurrence has left dS' and dV' behind.  Wave w owns the 32 K-columns [32w, 32w+32) of dQ, dK, dW and
+// the reverse recurrence has left dS' and dV' behind, for fp32 and, in 16 bits, for grouped heads with V = 64 (the others:
+// chunk_bwd_local16_kernel).  Wave w owns the 32 K-columns [32w, 32w+32) of dQ, dK, dW and
 // the 32x32 tile (w/2, w%2) of the 64x64 intra-chunk matrices.
 //   main loop over 32-column V blocks:
 //     v_new, dV', dO, S, dS' arrive in fragment order with (lane <-> V column); the contractions run over V, so each
@@ -809,8 +810,9 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void chunk_bwd_lo
   // Where the state gradient of a (chunk, head) has room for them (V >= 128: V K elements against 2 x 64 K), the sums
   // travel from one head's launch to the next as fragment-order tiles in that place, which this launch has finished
   // reading (the reverse recurrence rewrites it in every backward pass): no pass through rows, and only the group's
-  // last head writes dq and dk.  Tiles: dq (token block, channel block), then dk likewise.
-  const bool frag_sums = V >= 128 && grp > 1, last_head = hh == grp - 1;
+  // last head writes dq and dk.  Tiles: dq (token block, channel block), then dk likewise.  (fp32 alone: in 16 bits heads with
+  // that room are chunk_bwd_local16_kernel's, and what comes here adds rows.)
+  const bool frag_sums = sizeof(T) == 4 && V >= 128 && grp > 1, last_head = hh == grp - 1;
   T* sums_out = const_cast<T*>(dhf_in) + ch * (int64_t)(V / 32) * NKT * 1024;
   const T* sums_in = sums_out - (int64_t)(V / 32) * NKT * 1024;   // the head before this one
   RowPieces<T> held[2];   // rows, or a tile in fragment order: one set of requests either way (rows_or_tile_request)

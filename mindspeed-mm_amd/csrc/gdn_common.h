@@ -291,7 +291,7 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 template <int N, typename T> __device__ __forceinline__ void lds_read_tr16_pairs(const T* const* p, u32x4* out) {
-  static_assert(N == 1 || N == 2 || N == 4, "asm blocks of 2, 4 and 8 reads");
+  static_assert(N == 1 || N == 2, "asm blocks of 2 and 4 reads");
   u32x2 r[2 * N];
   uint32_t a[2 * N];
 #pragma unroll
@@ -299,16 +299,10 @@ template <int N, typename T> __device__ __forceinline__ void lds_read_tr16_pairs
   if constexpr (N == 1) {
     asm volatile("ds_read_b64_tr_b16 %0, %2\n ds_read_b64_tr_b16 %1, %3\n s_waitcnt lgkmcnt(0)"
                  : "=&v"(r[0]), "=&v"(r[1]) : "v"(a[0]), "v"(a[1]) : "memory");
-  } else if constexpr (N == 2) {
+  } else {
     asm volatile("ds_read_b64_tr_b16 %0, %4\n ds_read_b64_tr_b16 %1, %5\n ds_read_b64_tr_b16 %2, %6\n"
                  " ds_read_b64_tr_b16 %3, %7\n s_waitcnt lgkmcnt(0)"
                  : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]) : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]) : "memory");
-  } else {
-    asm volatile("ds_read_b64_tr_b16 %0, %8\n ds_read_b64_tr_b16 %1, %9\n ds_read_b64_tr_b16 %2, %10\n"
-                 " ds_read_b64_tr_b16 %3, %11\n ds_read_b64_tr_b16 %4, %12\n ds_read_b64_tr_b16 %5, %13\n"
-                 " ds_read_b64_tr_b16 %6, %14\n ds_read_b64_tr_b16 %7, %15\n s_waitcnt lgkmcnt(0)"
-                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
-                 : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]) : "memory");
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) out[i] = u32x4{r[2 * i][0], r[2 * i][1], r[2 * i + 1][0], r[2 * i + 1][1]};
