@@ -132,6 +132,39 @@ def test_chunk_fp32_bits_do_not_depend_on_the_batch(ops, T, K, V):
         assert torch.equal(a[0], b[0])
 
 
+@pytest.mark.parametrize("T,Hqk,Hv,K,V,l2,cu", [
+    (70, 1, 3, 64, 128, True, None),      # three heads to a group whose sums just fill their place, waves without columns of K
+    (65, 1, 2, 128, 192, True, None),     # R in two parts, the second of two V blocks; a last chunk of one token
+    (64, 1, 1, 128, 64, False, None),     # one pair of V blocks; no l2 norm
+    (33, 1, 2, 64, 64, True, None),       # several heads and V = 64: the four-wave kernel
+    (130, 2, 2, 64, 256, False, None),
+    (1000, 2, 8, 64, 192, True, [0, 1, 1, 300, 364, 427, 990]),   # chunks of 1, 43, 63 and 64 tokens, rows of no sequence
+    (2100, 16, 32, 128, 128, True, [0, 700, 2100]),               # 544 workgroups, where the chip holds 512 at once
+])
+def test_chunk_local_backward_of_head_groups(ops, T, Hqk, Hv, K, V, l2, cu):
+    """The chunk-local kernel where its tiles, its V blocks and the sums over a group's heads end."""
+    end = cu[-1] if cu else T
+    P.check_chunk(ops, "cuda", 1, end, Hqk, Hv, K, V, BF, l2=l2, cu=cu, backward=True, h0_std=0.1, seed=5)
+    if end == T:
+        return
+    # rows of no sequence: zero gradients, and the others those of the call without them
+    x = P.gdn_inputs(1, T, Hqk, Hv, K, V, BF, seed=5, N=len(cu) - 1, l2norm_in_kernel=l2, h0_std=0.1)
+    cu_t = torch.tensor(cu, dtype=torch.int64, device="cuda")
+
+    def grads(rows):
+        leaf = [x[n][:, :rows].cuda().requires_grad_(True) for n in ("q", "k", "v", "g", "beta")]
+        o, _ = ops.chunk_gated_delta_rule(*leaf, initial_state=x["h0"].cuda(), use_qk_l2norm_in_kernel=l2, cu_seqlens=cu_t)
+        return torch.autograd.grad([o], leaf, [x["do"][:, :rows].cuda()])
+    for a, b in zip(grads(T), grads(end)):
+        assert torch.equal(a[:, :end], b) and not a[:, end:].any()
+
+
+@pytest.mark.parametrize("T,K,V", [(33, 64, 64), (70, 64, 192), (65, 128, 192)])
+def test_kda_backward_where_the_sums_over_v_end(ops, T, K, V):
+    """One pair of V blocks, R in two parts with the second cut short, waves without columns of K, a last chunk of one token."""
+    P.check_kda(ops, "cuda", 1, T, 1, K, V, BF, backward=True, h0_std=0.1, seed=6)
+
+
 @pytest.mark.parametrize("T,Hqk,Hv,V,cu", [
     (4095, 1, 2, 128, None), (4096, 1, 2, 128, None), (4097, 2, 2, 128, None),   # a token short of being cut; uneven segments
     (4159, 1, 3, 128, None),                                                     # a group of three heads, a short last chunk
