@@ -50,7 +50,7 @@ TRAFFIC_SOURCE = "profiles/chunk_fwd_bwd_B2_T8192_bf16_hbm_traffic.md"
 
 def measured_traffic_bytes_per_launch():
     """{kernel: bytes} from the first table of TRAFFIC_SOURCE (rows `| kernel<...> | ... | bytes |`, the last column being
-    bytes per launch and, of the chunk-local kernel's one launch, per value head of a q/k group); empty when the file is missing, and the traffic fields are then null."""
+    bytes per launch); empty when the file is missing, and the traffic fields are then null."""
     out, in_main = {}, False
     try:
         with open(os.path.join(ROOT, TRAFFIC_SOURCE)) as f:
@@ -96,7 +96,7 @@ def kernel_matmul_flops(K, V, C=64):
         # Aq^T dO, K dS, Tm^T dV', Q^T dO, K^T R
         "chunk_state_bwd_kernel": g(C, V, C) + g(C, V, K) + g(C, V, C) + 2 * g(K, V, C),
         # dO V'^T, R V'^T, dO S^T, V' dS^T, R S^T with R = Tm^T dV', ds K, ds^T Q, dM K, dM^T K
-        "chunk_bwd_local_kernel": 2 * g(C, C, V) + 3 * g(C, K, V) + g(C, V, C) + 4 * g(C, K, C),
+        "chunk_bwd_local16_kernel": 2 * g(C, C, V) + 3 * g(C, K, V) + g(C, V, C) + 4 * g(C, K, C),
     }
 
 
@@ -115,8 +115,8 @@ def kernel_algorithmic_bytes(K, V, grp, e=2, C=64):
         "chunk_state_bwd_kernel": 2 * tk // grp + 2 * tri + tv + 2 * row + tv + st,
         # v_new, dv_new, dO, S, dS, v, K and Q^T (per group), Tm, row vectors -> dv, dg, dbeta, dq/dk (the sums over a
         # group's heads are written by each head and read by the next)
-        "chunk_bwd_local_kernel": 3 * tv + 2 * st + tv + 2 * tk // grp + tri + 5 * row + tv + 2 * row
-                                  + 2 * tk * (2 * grp - 1) // grp,
+        "chunk_bwd_local16_kernel": 3 * tv + 2 * st + tv + 2 * tk // grp + tri + 5 * row + tv + 2 * row
+                                    + 2 * tk * (2 * grp - 1) // grp,
     }
 
 
@@ -232,8 +232,7 @@ def main():
     path_tflops = ref_formula_flops(tokens, c["Hv"], c["K"], c["V"]) / (ms_per_step * 1e-3) / 1e12
     min_bytes = minimal_bytes(c["B"], c["T"], c["B"], c["Hqk"], c["Hv"], c["K"], c["V"])
     interface_total = sum(abytes[n] * nchunk_heads for n in per_kernel if n in abytes)
-    grp = c["Hv"] // c["Hqk"]
-    traffic_step = {n: b * (grp if n == "chunk_bwd_local_kernel" else per_kernel[n]["launches_per_step"])
+    traffic_step = {n: b * per_kernel[n]["launches_per_step"]
                     for n, b in measured_traffic_bytes_per_launch().items() if n in per_kernel}
     traffic_total = None
     if all(n in traffic_step for n in per_kernel if n in abytes):

@@ -1078,7 +1078,7 @@ static int chunk_bwd_launch(const ChunkDims& d, const ChunkWorkspace& L, const v
         auto kern = chunk_bwd_local16_kernel<DK>;
         constexpr int smem = BwdLocal16Smem<DK>::bytes;
         if (int e = set_lds_b(kern, smem)) return e;
-        GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, d.Hqk), dim3(512), smem, st, (const T*)QTF, (const T*)KAF, (const T*)v, Bt,
+        GDN_LAUNCH(kKernBwdLocal16, st, kern, dim3(nc, d.Hqk), dim3(512), smem, st, (const T*)QTF, (const T*)KAF, (const T*)v, Bt,
                    beta_same, G, Ai, VF, (const T*)DVF, (const T*)dO, HF, DHF, rstd_q, rstd_k, (T*)dq, (T*)dk, (T*)dv, dbeta, dg, cu,
                    chunk_offsets, d.T, d.N, d.Hqk, d.Hv, d.V, scale, d.strides(), (T*)nullptr, (float*)nullptr);
         return (int)hipGetLastError();

@@ -897,7 +897,7 @@ static int kda_bwd_launch(const ChunkDims& d, const KdaWorkspace& L, const void*
       auto kern = chunk_bwd_local16_kernel<DK, true>;
       constexpr int smem = BwdLocal16Smem<DK>::bytes;
       if (int e = set_lds_b(kern, smem)) return e;
-      GDN_LAUNCH(kKernBwdLocal, st, kern, dim3(nc, H), dim3(512), smem, st, QBT, K1F, (const T*)v, bhat, 0,
+      GDN_LAUNCH(kKernBwdLocal16, st, kern, dim3(nc, H), dim3(512), smem, st, QBT, K1F, (const T*)v, bhat, 0,
                  (const float*)nullptr, Ai, VF, (const T*)DVF, (const T*)dO, HF, DHF, (const float*)nullptr,
                  (const float*)nullptr, (T*)nullptr, (T*)nullptr, (T*)dv, (void*)nullptr, (float*)nullptr, cu, chunk_offsets, d.T,
                  d.N, H, H, d.V, scale, ts, DUMP, DD);

@@ -9,7 +9,8 @@ enum KernelId {
   kKernChunkTable = 0, kKernPrep, kKernStateFwd, kKernOut, kKernStateBwd, kKernBwdLocal,
   kKernRecurrent, kKernConvFwd, kKernConvState, kKernConvBwd, kKernConvReduce,
   kKernConvDh0, kKernConvUpdate, kKernRmsNormFwd, kKernRmsNormBwd, kKernRmsNormReduce,
-  kKernGateFwd, kKernGateBwd, kKernGateReduce, kKernKdaPrep, kKernKdaBwdFinish, kKernKdaBwdReduce, kKernCount
+  kKernGateFwd, kKernGateBwd, kKernGateReduce, kKernKdaPrep, kKernKdaBwdFinish, kKernKdaBwdReduce,
+  kKernBwdLocal16, kKernCount
 };
 
 bool profile_on();

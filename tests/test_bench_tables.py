@@ -10,13 +10,11 @@ import bench  # noqa: E402
 def test_traffic_table_is_read_from_the_tracked_summary():
     t = bench.measured_traffic_bytes_per_launch()
     c = bench.CFG
-    grp = c["Hv"] // c["Hqk"]
-    algo = bench.kernel_algorithmic_bytes(c["K"], c["V"], grp)
+    algo = bench.kernel_algorithmic_bytes(c["K"], c["V"], c["Hv"] // c["Hqk"])
     units = c["B"] * (c["T"] // c["C"]) * c["Hv"]
     assert set(t) == set(algo)
     for name, measured in t.items():
-        launches = grp if name == "chunk_bwd_local_kernel" else 1
-        modelled = algo[name] * units / launches
+        modelled = algo[name] * units   # each of them is launched once
         # the counters may read somewhat more than the interface bytes (partial lines, re-reads), never far less
         assert 0.9 * modelled < measured < 1.5 * modelled, (name, measured, modelled)
 

@@ -125,6 +125,19 @@ def test_chunk_local_backward_of_head_groups(ops, T, Hqk, Hv, K, V, l2):
     P.check_chunk(ops, "cpu", 1, T, Hqk, Hv, K, V, BF, l2=l2, backward=True, wrap=guarded, h0_std=0.1, seed=5)
 
 
+@pytest.mark.parametrize("dtype,V,launched", [
+    (BF, 128, {"chunk_bwd_local16_kernel": 1}), (BF, 64, {"chunk_bwd_local_kernel": 2}), (F32, 128, {"chunk_bwd_local_kernel": 2}),
+])
+def test_chunk_local_backward_is_timed_under_its_kernels_name(ops, dtype, V, launched):
+    """Two heads to a group: one launch of the eight-wave kernel, or one launch per head of the four-wave one."""
+    ops.lib.gdn_profile_enable(1)
+    try:
+        P.check_chunk(ops, "cpu", 1, 64, 1, 2, 64, V, dtype, backward=True)
+        assert {n: c for n, (_, c) in kernel_timings(ops.lib).items() if n.startswith("chunk_bwd_local")} == launched
+    finally:
+        ops.lib.gdn_profile_enable(0)
+
+
 @pytest.mark.parametrize("K,V", [(128, 128), (64, 256)])
 def test_group_sums_read_nothing_that_was_not_written(ops, monkeypatch, K, V):
     """The dq, dk sums that pass from head to head of a group hold the rows past a short last chunk's end too: with a
