@@ -1152,8 +1152,13 @@ static int chunk_bwd_entry(const void* q, const void* k, const void* v, int64_t 
     if (K == 128 && wide && solo) GDN_BWD(bf16_t, 128, 4, 1, 4, 2);
     if (K == 128 && wide) GDN_BWD(bf16_t, 128, 4, 2, 4, 2);
     if (K == 128) GDN_BWD(bf16_t, 128, 2, 2, 4, 2);
-    if (wide) GDN_BWD(bf16_t, 64, 4, 2, 4, 2);
-    GDN_BWD(bf16_t, 64, 2, 2, 4, 2);
+    // K = 64: four loading waves shorten the chain of a reverse recurrence that has the chip to itself (32 heads of 64, 1 x 4096
+    // tokens: 78 us, with two 81; 2 x 8192 162 and 163); from 129 slabs on, or beside the refill of the states, they cost more than
+    // they give (1 x 4096 tokens of 32 value heads, alone: V = 192 87 and 82, V = 256 95 and 85; beside it: V = 128 95 and 85, V = 256
+    // 122 and 108, the call 353 and 338; 2 x 8192 of 16 heads of 64 165 and 159).
+    const bool four_loaders = !share_device && (int64_t)d.N * Hv * (V / 32) <= 128;
+    if (four_loaders) GDN_BWD(bf16_t, 64, 2, 2, 4, 2);
+    GDN_BWD(bf16_t, 64, 2, 2, 2, 2);
   } else {
     if (K == 128) GDN_BWD(float, 128, 2, 2, 2, 1);
     GDN_BWD(float, 64, 2, 2, 2, 1);

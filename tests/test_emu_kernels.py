@@ -108,6 +108,7 @@ def test_no_sequence_is_refused(ops, B, T, cu):
 
 @pytest.mark.parametrize("dtype,B,T,Hqk,Hv,K,V,cu", [
     (BF, 1, 200, 1, 2, 128, 128, None), (F32, 1, 140, 1, 2, 64, 64, [0, 5, 70, 140]),
+    (BF, 1, 135, 1, 2, 64, 192, [0, 5, 70, 135]),   # reverse recurrence with two loading waves, and with four
 ])
 def test_chunk_backward_recompute_mode_equals_stored_mode(ops, dtype, B, T, Hqk, Hv, K, V, cu):
     P.check_chunk_recompute_equals_stored(ops, "cpu", B, T, Hqk, Hv, K, V, dtype, cu=cu, wrap=guarded, h0_std=0.1)

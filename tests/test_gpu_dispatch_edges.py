@@ -165,6 +165,13 @@ def test_kda_backward_where_the_sums_over_v_end(ops, T, K, V):
     P.check_kda(ops, "cuda", 1, T, 1, K, V, BF, backward=True, h0_std=0.1, seed=6)
 
 
+@pytest.mark.parametrize("B,Hv,V", [(2, 32, 64), (3, 22, 64), (1, 24, 192)])
+def test_reverse_recurrence_with_two_and_four_loading_waves(ops, B, Hv, V):
+    """K = 64: four up to 128 slabs of 32 columns where the recurrence runs alone, else two; the same bits."""
+    P.check_chunk(ops, "cuda", B, 300, Hv // 2, Hv, 64, V, BF, backward=True, skip_recompute=True, h0_std=0.1)
+    P.check_chunk_recompute_equals_stored(ops, "cuda", B, 300, Hv // 2, Hv, 64, V, BF)
+
+
 @pytest.mark.parametrize("T,Hqk,Hv,V,cu", [
     (4095, 1, 2, 128, None), (4096, 1, 2, 128, None), (4097, 2, 2, 128, None),   # a token short of being cut; uneven segments
     (4159, 1, 3, 128, None),                                                     # a group of three heads, a short last chunk
