@@ -105,20 +105,20 @@ __global__ __launch_bounds__(64 * state_bwd_waves<T>(NW, NL)) GDN_WAVES_PER_SIMD
       const int64_t ch = (chunk_base + c) * Hv + h, chq = (chunk_base + c) * Hqk + h / (Hv / Hqk);
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = dealt<PK, NT>(lt, i);
+        const int idc = dealt<T, PK, NT>(lt, i);
         pk[set][i] = ld16(kaf + chq * (64 * DK) + idc * VEC);
         if constexpr (KDA) pk2[set][i] = ld16(kaf2 + chq * (64 * DK) + idc * VEC);
         pq[set][i] = ld16(qtf + chq * (64 * DK) + idc * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int src = tm_src(dealt<PTM, NT>(lt, i));
+        const int src = tm_src(dealt<T, PTM, NT>(lt, i));
         ptm[set][i] = ld16(ai + ch * 4096 + src * VEC);
         pa[set][i] = ld16(aqtf + ch * 4096 + src * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CD; ++i) {   // dO rows of the slabs; rows past the end repeat the last one and are cleared below
-        const int idc = dealt<PD, NT>(lt, i), row = imin(idc / DPR, nvalid - 1), cc = idc % DPR;
+        const int idc = dealt<T, PD, NT>(lt, i), row = imin(idc / DPR, nvalid - 1), cc = idc % DPR;
         pd[set][i] = ld16(dO + ((tok0 + row) * Hv + h) * V + col0 + cc * VEC);
         if constexpr (!KDA) pgd[set][i] = G[ch * 64 + row];
       }
@@ -138,20 +138,20 @@ __global__ __launch_bounds__(64 * state_bwd_waves<T>(NW, NL)) GDN_WAVES_PER_SIMD
       T* st = reinterpret_cast<T*>(gdn_smem + buf * SM::stage);
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = dealt<PK, NT>(lt, i);
+        const int idc = dealt<T, PK, NT>(lt, i);
         st16(st + SM::off_k + idc * VEC, pk[set][i]);
         if constexpr (SM::off_kt != SM::off_k) SL::st_t(st + SM::off_kt, idc, KDA ? pk2[set][i] : pk[set][i]);
         st16(st + SM::off_q + idc * VEC, pq[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int idc = dealt<PTM, NT>(lt, i);
+        const int idc = dealt<T, PTM, NT>(lt, i);
         SL::st_t(st + SM::off_tm, idc, ptm[set][i]);
         st16(st + SM::off_aq + idc * VEC, pa[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CD; ++i) {
-        const int idc = dealt<PD, NT>(lt, i);
+        const int idc = dealt<T, PD, NT>(lt, i);
         const Vec16<T> x = idc / DPR < pnv[set] && !of_a ? pd[set][i] : zero16<T>();
         st16(st + SM::off_do + idc * VEC, x);
         if constexpr (KDA) st16(st + SM::off_do + 64 * 32 * NW + idc * VEC, x);

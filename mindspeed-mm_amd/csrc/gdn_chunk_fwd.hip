@@ -449,20 +449,20 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       const int64_t tok0 = bos + (int64_t)c * kChunk;
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = dealt<PK, NT>(lt, i);
+        const int idc = dealt<T, PK, NT>(lt, i);
         pk[set][i] = ld16(kaf + chq * (64 * DK) + idc * VEC);   // shared by the value heads of the group
         if constexpr (OUT || KDA) pq[set][i] = ld16(qtf + chq * (64 * DK) + idc * VEC);
         if constexpr (OUT && KDA) pq2[set][i] = ld16(qim + chq * (64 * DK) + idc * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int src = tm_src(dealt<PTM, NT>(lt, i));
+        const int src = tm_src(dealt<T, PTM, NT>(lt, i));
         ptm[set][i] = ld16(ai + ch * 4096 + src * VEC);
         if constexpr (OUT) pa[set][i] = ld16(aqf + ch * 4096 + src * VEC);
       }
 #pragma unroll
       for (int i = 0; i < CV; ++i) {   // rows past the end of the sequence repeat the last one (their beta is 0)
-        const int idc = dealt<PV, NT>(lt, i), row = imin(idc / VPR, nvalid - 1), cc = idc % VPR;
+        const int idc = dealt<T, PV, NT>(lt, i), row = imin(idc / VPR, nvalid - 1), cc = idc % VPR;
         pv[set][i] = ld16(v + (tok0 + row) * v_stride + (int64_t)h * V + col0 + cc * VEC);
         if constexpr (PRE) pbv[set][i] = bt[ch * 64 + row];
       }
@@ -500,7 +500,7 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       }
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        const int idc = dealt<PK, NT>(lt, i);
+        const int idc = dealt<T, PK, NT>(lt, i);
         if constexpr (KDA) {
           st16(st + SM::off_k + idc * VEC, pk[set][i]);
           SL::st_t(st + SM::off_kt, idc, pq[set][i]);
@@ -516,13 +516,13 @@ void chunk_state_kernel(const T* __restrict__ kaf, const T* __restrict__ qtf, co
       }
 #pragma unroll
       for (int i = 0; i < CTM; ++i) {
-        const int idc = dealt<PTM, NT>(lt, i);
+        const int idc = dealt<T, PTM, NT>(lt, i);
         st16(st + SM::off_tm + idc * VEC, ptm[set][i]);
         if constexpr (OUT) st16(st + SM::off_aq + idc * VEC, pa[set][i]);
       }
 #pragma unroll
       for (int i = 0; i < CV; ++i) {
-        const int idc = dealt<PV, NT>(lt, i);
+        const int idc = dealt<T, PV, NT>(lt, i);
         if (of_a) st16(st + SM::off_v + idc * VEC, zero16<T>());   // not v x 0: v may hold infinities
         else if constexpr (PRE) st16(st + SM::off_v + idc * VEC, scale16<T>(pv[set][i], idc / VPR < pnv[set] ? pbv[set][i] : 0.f));
         else st16(st + SM::off_v + idc * VEC, pv[set][i]);
