@@ -20,10 +20,13 @@
 //   epilogue: contractions over tokens take them in the order 32 b + {4 g + e, 16 + 4 g + e}, which is that of two packed
 //     accumulator tiles; the 64x64 matrices pass between the waves as bf16 matrices in LDS (Mat64), written in 8-byte units
 //     straight from accumulators and read along their rows or, with the transposing read, along their columns.
-// Bound by memory: 2 x 8192 tokens, 16 q/k and 32 value heads of 128 move 2.0 GB in 411 us (4.9 TB/s), where one launch per
-// value head of the four-wave kernel, which waited (two waves to a SIMD), moved 2.04 GB in 466; 4 x 1024 tokens 139 -> 108,
-// 32768 tokens of 8 heads 234 -> 193.  (With four spilled values, each of which waits for all requests in flight when it is read
-// back: 422, 111, 203.)  What is read once passes the L2 by (424 -> 406 on a build without the fourth row sum).
+// Bound by bytes and vector instructions together: 2 x 8192 tokens, 16 q/k and 32 value heads of 128 move 1.96 GB in 390 to
+// 411 us (4.8 to 5.0 TB/s; the main loop alone, which is all that KDA runs, 6.2), where one launch per
+// value head of the four-wave kernel, which waited (two waves to a SIMD), moved 2.04 GB in 466; 4 x 1024 tokens 139 -> 106,
+// 32768 tokens of 8 heads 234 -> 193; K = 64, 2 x 8192 tokens, 16 heads of 64 142 -> 133, 32 value heads of 256 616 -> 555 (half
+// of the waves have no K columns there and repeat the others' main loop).  (With four spilled values, each of which waits for all
+// requests in flight when it is read back: 422, 111, 203.)  What is read once passes the L2 by: kept in it, 422, 111, 204, KDA
+// 302 -> 352, 65536 tokens of 64 heads of 256 4990 -> 5200.
 #pragma once
 #include "gdn_chunk.h"
 #include "gdn_common.h"

@@ -61,9 +61,11 @@ int device_compute_units();   // defined with the forward launcher
 // Segments a sequence is cut into for the two recurrences (gdn_segments.h); 1 = not cut.  As many as give every slab of
 // 32 state columns a compute unit of its own, none shorter than kMinSegmentChunks on average; two segments would take as
 // many dependent steps as one.  Sequences of kMinCutChunks on average pay for the two launches in front of each
-// recurrence.  Forward pass, 128-wide heads, not cut -> cut: 4 heads 114 -> 80 us at 64 chunks, 207 -> 89 at 128; 8
-// heads 407 -> 145 at 256; 16 heads (4 segments) 114 -> 83 at 64, 829 -> 459 at 512.  At 48 chunks it is still 91 -> 77,
-// but a training step of that length waits for the host, and two more launches a pass cost it 235 -> 250.  The number
+// recurrence.  Forward pass, 128-wide heads, not cut -> cut: 4 heads 90 -> 74 us at 64 chunks, 159 -> 86 at 128; 8
+// heads 307 -> 137 at 256; 16 heads (4 segments) 94 -> 81 at 64, 648 -> 431 at 512; 20 heads (3 segments), where it pays least,
+// 97 -> 96 at 64, 179 -> 160 at 128.  A training step at 64 chunks, what the forward pass left kept: 4 heads 203 -> 190, 20 heads
+// 277 -> 276; not kept, it waits for the host, and two more launches a pass cost it 245 -> 262 (at 96 chunks 283 -> 252 to 268),
+// 20 heads 278 -> 284 (at 96 379 -> 370).  The number
 // follows from the sequences, heads and tokens of the call: a sequence's bits, cut, are those of its call's number of
 // segments.  Heads of other sizes stay uncut: K = 64 has no such kernels, and with V = 256 single entries of dg of slowly
 // decaying heads moved past the bound this project states for them (0.050 to 0.082 cut, 0.046 to 0.086 uncut, of a dg of
