@@ -10,9 +10,10 @@
 //   3. the recurrence kernel proper, every segment from its own start
 // The reverse recurrence does the same from the other end.  2 n / P dependent steps instead of n.  32768 tokens, 8 heads
 // of 128, 8 segments: maps 98 us, chain 21, recurrence 92 (205 together) where the uncut recurrence takes 561; reverse maps 120,
-// chain 21, recurrence 164 beside the refill; forward and backward 1430 -> 728 us.  The error against float64 is the uncut recurrence's (4160
-// to 16384 tokens, 2 to 8 heads, four seeds each: o 4.745e-3 and 4.745e-3 with decays near 1 over a whole segment, final state
-// 3.79e-3 and 3.78e-3, dk 5.63e-3 and 5.63e-3, dg 5.19e-3 to 5.68e-3 uncut, 5.14e-3 to 5.65e-3 cut, smaller in two of four cases).
+// chain 21, recurrence 164 beside the refill; forward and backward 1430 -> 728 us.  The error against float64 is the uncut
+// recurrence's (4160 to 16384 tokens, 2 to 8 heads, four seeds each: o 4.745e-3 and 4.745e-3 with decays near 1 over a whole
+// segment, final state 3.79e-3 and 3.78e-3, dk 5.63e-3 and 5.63e-3, dg 5.19e-3 to 5.68e-3 uncut, 5.14e-3 to 5.65e-3 cut, smaller in
+// two of four cases).
 #pragma once
 #include "gdn_common.h"
 
